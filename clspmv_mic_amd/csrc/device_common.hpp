@@ -34,8 +34,10 @@ __device__ __forceinline__ int4 ld_stream(const int4* p) {
 // Stored matrix values: FP32, or BF16 / FP16 bits widened to FP32 when
 // loaded (products and sums stay FP32).  ld: one value; ld2 / ld4: two /
 // four consecutive values (8 / 16-byte aligned for FP32, 4 / 8 for 16-bit).
+// cvt: a stored value as a float.
 struct ValF32 {
     typedef float T;
+    static __device__ __forceinline__ float cvt(float v) { return v; }
     static __device__ __forceinline__ float ld(const float* p) { return ld_stream(p); }
     static __device__ __forceinline__ float2 ld2(const float* p) {
         return *reinterpret_cast<const float2*>(p);
@@ -51,6 +53,7 @@ struct ValF32 {
 template <class Cvt>
 struct Val16 {
     typedef unsigned short T;
+    static __device__ __forceinline__ float cvt(T v) { return Cvt::f(v); }
     typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
     static __device__ __forceinline__ float ld(const T* p) { return Cvt::f(ld_stream(p)); }
     static __device__ __forceinline__ float2 ld2(const T* p) {
@@ -88,6 +91,33 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
     const int x = b % kXcds, i = b / kXcds;
     return x * q + (x < r ? x : r) + i;
 }
+
+// Orders the LDS accesses of one wave's lanes before and after this point (a
+// wave's LDS operations execute in order: only the compiler has to be held).
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Vectors of N values (N = 1: the value itself); UVec: aligned to its
+// element only, for loads at any element.
+template <class T, int N>
+struct VecOf {
+    typedef T type __attribute__((ext_vector_type(N)));
+    static __device__ __forceinline__ T get(const type& v, int i) { return v[i]; }
+    static __device__ __forceinline__ void set(type& v, int i, T x) { v[i] = x; }
+};
+template <class T>
+struct VecOf<T, 1> {
+    typedef T type;
+    static __device__ __forceinline__ T get(const type& v, int) { return v; }
+    static __device__ __forceinline__ void set(type& v, int, T x) { v = x; }
+};
+template <class T, int N>
+struct UVec {
+    typedef typename VecOf<T, N>::type type __attribute__((aligned(sizeof(T))));
+};
 
 // The lane's value from another lane of its 16-lane row, by DPP (no LDS
 // crossbar round trip): CTRL 0xB1 = quad_perm(1,0,3,2) (lane ^ 1), 0x4E =

@@ -11,6 +11,8 @@
 // FP32 in a fixed order, FP64 for CSR rows longer than kLongRowF64; no
 // atomics.
 
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -18,6 +20,7 @@ namespace clspmv {
 namespace {
 
 using namespace dev;
+using launch::kDiaRun;
 
 // Loads right-hand sides qb .. qb+Q-1 of row c of X (zero where q >= k).
 template <int Q>
@@ -46,47 +49,192 @@ __device__ __forceinline__ void load_xq(const float* __restrict__ X, int c, int 
     for (int q = 0; q < Q; ++q) xv[q] = qb + q < k ? p[q] : 0.0f;
 }
 
-// DIA: L = KB / Q neighbouring lanes share a row, each with Q = min(KB, 4)
-// right-hand sides, so a wave's X load for one diagonal is one contiguous
-// run of 64 / L rows of X (16-byte pieces).
-template <int KB, class V>
+// DIA.  The diagonals come as segments {first diagonal, its offset, how many
+// (at most W) consecutive offsets, 0} in diagonal order.  A wave owns NR
+// consecutive rows; lane t takes rows R * (t / L) .. + R - 1 and right-hand
+// sides Q * (t % L) .. + Q - 1 (the last lane of a group ends at k, so every
+// X access is a whole Q-float piece).
+//
+// What bounds it: the texture addresser.  A lane reading its own X pieces for
+// every diagonal sends each X row through L1 once per diagonal, 27 times on
+// the 27-point stencil, 64 bytes a cycle per CU (TA busy 73 % of the time,
+// 99 us on 96^3 rows at k = 16 even with that loop tuned).  So per segment the
+// wave loads the X rows of its window (NR + W - 1 consecutive rows of X) and
+// the segment's values once, coalesced, into its own part of LDS, and reads
+// them there: R + W - 1 pieces for R * W products per lane.  The next
+// segment's loads are in flight in registers meanwhile; no work-group barrier.
+// LDS rows are padded by KB floats every R rows, which keeps the 16-byte reads
+// of lanes R rows apart on different banks.  96^3 27-point stencil, FP32,
+// k = 2 / 4 / 7 / 8 / 16: 26 / 31 / 38 / 41 / 73 us against 41 / 49 / 135 /
+// 94 / 183 us for lanes loading every diagonal's X row themselves (1.7 to 3.8
+// TB/s of the bytes that cannot be avoided); 5-point Laplacian on 900^2, k = 8 /
+// 16: 19 / 42 against 30 / 59 us.
+//
+// Each column is summed alone in diagonal order, one product at a time,
+// skipping columns outside x, whatever the tile: its result does not depend
+// on k.
+template <int Q, int L, int R, int W, class V>
 __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
-    int rows, int cols, int len, int ndiag, const int* __restrict__ off,
-    const typename V::T* __restrict__ data, int k, const float* __restrict__ X, bool vec,
-    float* __restrict__ Y, int ldy) {
-    constexpr int Q = KB < 4 ? KB : 4;
-    constexpr int L = KB / Q;
-    const int t = threadIdx.x;
-    const int qb = (t % L) * Q;
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * (kBlock / L) + t / L;
-    if (r >= rows) return;
-    float acc[Q];
+    int rows, int cols, int len, int nseg, const int4* __restrict__ seg,
+    const typename V::T* __restrict__ data, int k, const float* __restrict__ X, float* __restrict__ Y,
+    int ldy) {
+    typedef typename V::T T;
+    constexpr int NR = kWave / L * R;                    // rows per wave
+    constexpr int RW = kWave / L;                        // X rows per load instruction
+    constexpr int QP = Q == 3 ? 4 : Q;                   // LDS floats per piece
+    constexpr int KB = QP * L;                           // LDS floats per X row
+    constexpr int CS = (R + 1) * KB;                     // LDS floats per R rows
+    constexpr int NX = NR + W - 1;                       // X rows per window
+    constexpr int NLD = (NX + RW - 1) / RW;              // X pieces per lane
+    constexpr int ND = NR >= kWave ? NR / kWave : 1;     // values per lane and diagonal
+    constexpr int DL = NR / ND;                          // lanes that load values
+    typedef VecOf<float, Q> XV;
+    typedef VecOf<T, ND> DV;
+    typedef VecOf<float, ND> FV;
+    typedef VecOf<float, R> RV;
+    constexpr int kWaves = kBlock / kWave;
+    __shared__ __attribute__((aligned(16))) float sx[kWaves][(NX + R - 1) / R * CS];
+    __shared__ __attribute__((aligned(16))) float sd[kWaves][W * NR];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int w0 = __builtin_amdgcn_readfirstlane((xcd_tile(blockIdx.x, gridDim.x) * kWaves + wave) * NR);
+    if (w0 >= rows) return;  // the whole wave
+    float* xl = sx[wave];
+    float* dl = sd[wave];
+    const int g = lane / L, p = lane % L;
+    const int q0 = p * Q, qs = min(q0, k - Q);
+    float acc[R][Q];
 #pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q] = 0.0f;
-    // C diagonals per step, every load of the step issued before its first
-    // product (C * (1 + Q) values in flight per lane); each column is still
-    // summed in diagonal order, one product at a time, skipping columns
-    // outside x.
-    constexpr int C = Q == 4 ? 8 : 16;
-    for (int j0 = 0; j0 < ndiag; j0 += C) {  // wave-uniform
-        float d[C], xv[C][Q];
-        bool in[C];
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-        for (int u = 0; u < C; ++u) {
-            const int j = min(j0 + u, ndiag - 1);
-            d[u] = V::ld(data + (size_t)j * len + r);
-            const int c = r + off[j];
-            in[u] = j0 + u < ndiag && (unsigned)c < (unsigned)cols;
-            load_xq<Q>(X, in[u] ? c : 0, k, qb, vec, xv[u]);
+        for (int q = 0; q < Q; ++q) acc[r][q] = 0.0f;
+    const bool tail = w0 + NR > len;  // rows past the stored length
+    typename XV::type xr[NLD];
+    typename DV::type dr[W];
+    const unsigned xo = (unsigned)(g * k + qs), xlast = (unsigned)((NX - 1) * k + qs);
+    // Whether every X row of a segment's window exists.
+    auto inside = [&](int off) { return (long long)w0 + off >= 0 && (long long)w0 + off + NX <= cols; };
+    auto load = [&](const int4 sg) {
+        if (inside(sg.y)) {
+            const float* xw = X + (ptrdiff_t)(w0 + sg.y) * k;
+#pragma unroll
+            for (int u = 0; u < NLD; ++u) {
+                const unsigned o = xo + (unsigned)(u * RW) * k;
+                xr[u] = *reinterpret_cast<const typename UVec<float, Q>::type*>(
+                    xw + ((u + 1) * RW <= NX ? o : min(o, xlast)));
+            }
+        } else {  // rows outside X re-read the first or last one and are not added
+#pragma unroll
+            for (int u = 0; u < NLD; ++u) {
+                const int c = min(max(w0 + sg.y + g + u * RW, 0), cols - 1);
+                xr[u] = *reinterpret_cast<const typename UVec<float, Q>::type*>(X + (size_t)c * k + qs);
+            }
         }
+        // Diagonals past the segment's re-read its last one and are not added.
+        const T* dp = data + (size_t)sg.x * len + w0;
+        if (!tail) {
+            const int at = min(lane, DL - 1) * ND;
 #pragma unroll
-        for (int u = 0; u < C; ++u)
+            for (int n = 0; n < W; ++n)
+                dr[n] = __builtin_nontemporal_load(reinterpret_cast<const typename UVec<T, ND>::type*>(
+                    dp + (size_t)min(n, sg.z - 1) * len + at));
+        } else {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) acc[q] = in[u] ? fmaf(d[u], xv[u][q], acc[q]) : acc[q];
+            for (int n = 0; n < W; ++n)
+#pragma unroll
+                for (int h = 0; h < ND; ++h)
+                    DV::set(dr[n], h, dp[(size_t)min(n, sg.z - 1) * len + min(lane * ND + h, len - 1 - w0)]);
+        }
+    };
+    int4 sg = seg[0];
+    load(sg);
+    for (int s = 0; s < nseg; ++s) {
+        const int z = sg.z, off = sg.y;
+#pragma unroll
+        for (int u = 0; u < NLD; ++u) {
+            const int r = g + u * RW;
+            float* at = xl + r / R * CS + r % R * KB + p * QP;
+            if ((u + 1) * RW <= NX || r < NX) {
+                if constexpr (Q == 3) {
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) at[q] = xr[u][q];
+                } else {
+                    *reinterpret_cast<typename XV::type*>(at) = xr[u];
+                }
+            }
+        }
+        if (lane < DL) {
+#pragma unroll
+            for (int n = 0; n < W; ++n) {
+                typename FV::type f;
+#pragma unroll
+                for (int h = 0; h < ND; ++h) FV::set(f, h, V::cvt(DV::get(dr[n], h)));
+                *reinterpret_cast<typename FV::type*>(dl + n * NR + lane * ND) = f;
+            }
+        }
+        wave_lds_order();
+        sg = seg[min(s + 1, nseg - 1)];
+        load(sg);
+        // N diagonals from the segment's n0-th on; `all`: no column to skip.
+        auto add = [&](auto count, auto all, int n0) {
+            constexpr int N = decltype(count)::value;
+            typename XV::type xv[R + N - 1];
+            typename RV::type d[N];
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                d[n] = *reinterpret_cast<const typename RV::type*>(dl + (n0 + n) * NR + g * R);
+#pragma unroll
+            for (int i = 0; i < R + N - 1; ++i) {
+                const int r = N == W ? i : n0 + i;  // N == W: n0 is 0, the offsets are constants
+                const float* at = xl + (g + r / R) * CS + r % R * KB + p * QP;
+                if constexpr (Q == 3) {
+                    const f32x4 t = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) xv[i][q] = t[q];
+                } else {
+                    xv[i] = *reinterpret_cast<const typename XV::type*>(at);
+                }
+            }
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const bool in =
+                        decltype(all)::value || (unsigned)(w0 + off + n0 + n + g * R + r) < (unsigned)cols;
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) {
+                        const float a = fmaf(RV::get(d[n], r), XV::get(xv[n + r], q), acc[r][q]);
+                        acc[r][q] = in ? a : acc[r][q];
+                    }
+                }
+        };
+        using One = std::integral_constant<int, 1>;
+        if (!inside(off)) {
+            for (int n = 0; n < z; ++n) add(One{}, std::false_type{}, n);
+        } else if (z == W) {
+            add(std::integral_constant<int, W>{}, std::true_type{}, 0);
+        } else {
+            for (int n = 0; n < z; ++n) add(One{}, std::true_type{}, n);
+        }
+        wave_lds_order();
     }
+    const int r0 = w0 + g * R;
+    if (q0 >= k) return;
 #pragma unroll
-    for (int q = 0; q < Q; ++q)
-        if (qb + q < k) Y[(size_t)(qb + q) * ldy + r] += acc[q];
+    for (int q = 0; q < Q; ++q) {
+        if (qs + q < q0) continue;  // the lane before has this column
+        float* yp = Y + (size_t)(qs + q) * ldy + r0;
+        if (r0 + R <= rows) {
+            typedef typename UVec<float, R>::type YU;
+            typename RV::type v = *reinterpret_cast<const YU*>(yp);
+#pragma unroll
+            for (int r = 0; r < R; ++r) RV::set(v, r, RV::get(v, r) + acc[r][q]);
+            *reinterpret_cast<YU*>(yp) = v;
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r0 + r < rows) yp[r] += acc[r][q];
+        }
+    }
 }
 
 // Accumulates a[q] += val[j] * X[col[j]][qb + q] over j = j0, j0 + step, ...
@@ -295,25 +443,44 @@ __global__ __launch_bounds__(kBlock) void csr_multi_kernel(
 
 int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
-template <int KB, class V>
-hipError_t dia_multi_kb(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off,
-                        const void* data, int k, const float* X, float* Y, int ldy) {
-    constexpr int Q = KB < 4 ? KB : 4;
-    const bool vec = Q > 1 && k % Q == 0 && ((uintptr_t)X % (Q * sizeof(float))) == 0;
-    hipLaunchKernelGGL((dia_multi_kernel<KB, V>), dim3(ceil_div(rows, kBlock / (KB / Q))), dim3(kBlock), 0,
-                       s, rows, cols, len, ndiag, off, static_cast<const typename V::T*>(data), k, X, vec, Y,
-                       ldy);
+template <int Q, int L, int R, class V>
+hipError_t dia_multi_tile(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
+                          const void* data, int k, const float* X, float* Y, int ldy) {
+    const dim3 grid(ceil_div(rows, kBlock / L * R)), block(kBlock);
+    const typename V::T* d = static_cast<const typename V::T*>(data);
+    if (w == 1)
+        hipLaunchKernelGGL((dia_multi_kernel<Q, L, R, 1, V>), grid, block, 0, s, rows, cols, len, nseg, seg, d, k, X,
+                           Y, ldy);
+    else
+        hipLaunchKernelGGL((dia_multi_kernel<Q, L, R, kDiaRun, V>), grid, block, 0, s, rows, cols, len, nseg, seg, d,
+                           k, X, Y, ldy);
     return hipGetLastError();
 }
 
+// Rows per lane: more of them reuse each staged X row more often but leave
+// fewer waves, each with a longer chain of segments.  On the 27-point stencil
+// the wider tile wins from 80^3 to 96^3 rows on (96^3, k = 4 / 8: 31 / 41 us
+// against 36 / 48 us for the narrower one) and loses below (64^3: 11.2 / 13.3
+// against 10.2 / 12.6 us); with few segments it never pays at k >= 2 (5-point
+// Laplacian on 900^2, k = 4 / 8: 15.5 / 22.5 against 13.4 / 19.7 us).  At k > 8
+// a wave has 64 / 4 lane groups, and four rows each win from 32^3 rows on
+// (32^3: 9.8 us, 22^3: 10.3 against 7.9 us).
 template <class V>
-hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off,
+hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
                        const void* data, int k, const float* X, float* Y, int ldy) {
-    if (k <= 1) return dia_multi_kb<1, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy);
-    if (k <= 2) return dia_multi_kb<2, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy);
-    if (k <= 4) return dia_multi_kb<4, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy);
-    if (k <= 8) return dia_multi_kb<8, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy);
-    return dia_multi_kb<16, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy);
+    const bool large = rows >= (1 << 19);
+    const bool deep = large && nseg >= 6;
+#define CLSPMV_DIA_MULTI(Q, L, R) dia_multi_tile<Q, L, R, V>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy)
+    switch (k) {
+        case 1: return large ? CLSPMV_DIA_MULTI(1, 1, 4) : CLSPMV_DIA_MULTI(1, 1, 1);
+        case 2: return deep ? CLSPMV_DIA_MULTI(2, 1, 2) : CLSPMV_DIA_MULTI(2, 1, 1);
+        case 3: return deep ? CLSPMV_DIA_MULTI(3, 1, 2) : CLSPMV_DIA_MULTI(3, 1, 1);
+        case 4: return deep ? CLSPMV_DIA_MULTI(4, 1, 2) : CLSPMV_DIA_MULTI(4, 1, 1);
+        default: break;
+    }
+    if (k <= 8) return deep && w > 1 ? CLSPMV_DIA_MULTI(4, 2, 4) : CLSPMV_DIA_MULTI(4, 2, 2);
+    return rows >= (1 << 15) ? CLSPMV_DIA_MULTI(4, 4, 4) : CLSPMV_DIA_MULTI(4, 4, 2);
+#undef CLSPMV_DIA_MULTI
 }
 
 template <int KB, class V>
@@ -350,14 +517,14 @@ hipError_t csr_multi_v(hipStream_t s, int nblocks, const int* blocks, const int*
 
 namespace launch {
 
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int ndiag, const int* offsets,
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy) {
-    if (rows <= 0 || ndiag <= 0 || k <= 0) return hipSuccess;
+    if (rows <= 0 || cols <= 0 || nseg <= 0 || k <= 0) return hipSuccess;
     if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, ndiag, offsets, data, k, X, Y, ldy);
-        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, ndiag, offsets, data, k, X, Y, ldy);
-        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, ndiag, offsets, data, k, X, Y, ldy);
+        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
+        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
+        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
         default: return hipErrorInvalidValue;
     }
 }

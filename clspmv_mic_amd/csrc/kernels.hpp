@@ -134,7 +134,11 @@ hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
 // ---- multi-right-hand-side SpMV (k <= kMultiMax) --------------------------------
 // Y[:, q] += A X[:, q]; X row-major (X[c*k + q]), Y column-major (ldy).
 constexpr int kMultiMax = 16;
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int ndiag, const int* offsets,
+// DIA: the diagonals as nseg segments {first diagonal, its offset, how many
+// consecutive offsets follow each other (at most w), 0} in diagonal order;
+// w is 1 or kDiaRun.
+constexpr int kDiaRun = 3;
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy);
 // CSR over the adaptive row blocks (csr_adaptive's `blocks`).  kb > 0 runs
 // the kernel built for kb right-hand sides (k <= kb; 1, 2, 4, 8 or 16)

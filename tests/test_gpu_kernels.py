@@ -382,6 +382,47 @@ def test_spmv_multi(ctx, oracle, name, fmt, dtype, k):
             np.testing.assert_array_equal(Y[q, :A.height], y64.astype(np.float32))
         np.testing.assert_array_equal(Y[q, A.height:], Y0[q, A.height:])
 
+DIA_TILE_OFFSETS = {
+    "runs_and_lone": [-7, -1, 0, 1, 9],
+    "lone": [-30, -9, 0, 4, 11, 25],
+    "many_runs": [-29, -28, -27, -20, -19, -18, -17, -16, -15, -14, -9, -8, -3, -2, -1, 0, 1, 5, 7, 8, 9, 15],
+}
+
+
+@pytest.mark.parametrize("offsets", sorted(DIA_TILE_OFFSETS))
+@pytest.mark.parametrize("n,ks", [(33, range(1, 17)), (64, range(1, 17)), (257, range(1, 17)), (1030, (2, 5, 8, 11, 16)),
+                                  ((1 << 15) + 5, (9, 12, 15, 16)), ((1 << 19) + 37, (1, 2, 3, 4, 7, 8, 13))])
+def test_dia_multi_tiles(ctx, offsets, n, ks):
+    """The multi-vector DIA kernel at the edges of its row tiles, over runs of
+    consecutive offsets and lone ones, on operands aligned to one float only:
+    dyadic inputs, so every sum is exact and equals the FP64 product."""
+    off = DIA_TILE_OFFSETS[offsets]
+    A = matrices.banded(n, off, seed=n, dyadic=True)
+    dtypes = [cs.DT_F32, cs.DT_BF16] if n < 2000 else [cs.DT_F32]
+    # The DIA struct by hand: coo2dia refuses short diagonals of a small matrix.
+    length = cs.lib.clspmv_aligned_length(n, cs.GPU_ALIGNMENT)
+    data, o32 = np.zeros((len(off), length), np.float32), np.array(off, np.int32)
+    for j, o in enumerate(off):
+        at = A.col.astype(np.int64) - A.row == o
+        data[j, A.row[at]] = A.val[at]
+    m = cs.DiaMatrix(cs.MatInfo(n, n, A.nnz), len(off), n, length, cs._ip(o32), cs._fp(data))
+    dAs = [cs.DeviceMatrix(ctx, m, dtype=dt) for dt in dtypes]
+    rng = np.random.default_rng(n)
+    for k in ks:
+        X = (rng.integers(-64, 65, size=(n, k)) / 64.0).astype(np.float32)
+        Y0 = (rng.integers(-64, 65, size=(k, n + 1)) / 64.0).astype(np.float32)
+        ref = Y0.astype(np.float64)
+        for o in off:
+            r0, r1 = max(0, -o), min(n, n - o)
+            v = A.val[A.col.astype(np.int64) - A.row == o].astype(np.float64)
+            ref[:, r0:r1] += v * X[r0 + o:r1 + o].T
+        dX = cs.DeviceVector(ctx, X.size + 1, np.concatenate([[0.0], X.reshape(-1)]).astype(np.float32)).view(1)
+        for dA in dAs:
+            dY = cs.DeviceVector(ctx, Y0.size + 1, np.concatenate([[0.0], Y0.reshape(-1)]).astype(np.float32))
+            dA.spmv_multi(k, dX, dY.view(1), n + 1)
+            ctx.sync()
+            np.testing.assert_array_equal(dY.download()[1:].reshape(k, n + 1), ref.astype(np.float32))
+
 
 @pytest.mark.parametrize("name", ["rand_small", "rand_dyadic", "rand_long_rows"])
 @pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
