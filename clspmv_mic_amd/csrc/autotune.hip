@@ -194,11 +194,15 @@ int make_flat(hipStream_t s, int format, int dim, int width, int slice_h, clspmv
             m->max_row = width;
             st = b.alloc(dim + 1LL, &m->rp);
             if (!st) st = fillr(s, m->rp, dim + 1LL, width);
-            if (!st) st = b.alloc(nnz, &m->col);
-            if (!st) st = b.alloc(nnz, &m->val);
-            if (!st) st = fillc(s, m->col, nnz, width, dim, 3);
-            if (!st) st = fillf(s, m->val, nnz, 1.0f);
-            // Adaptive row blocks for constant row length.
+            // Padded as the upload pads them; the padding's columns are valid.
+            if (!st) st = b.alloc(nnz + launch::kWaveNnz, &m->col);
+            if (!st) st = b.alloc(nnz + launch::kWaveNnz, &m->val);
+            if (!st) st = fillc(s, m->col, nnz + launch::kWaveNnz, width, dim, 3);
+            if (!st) st = fillf(s, m->val, nnz + launch::kWaveNnz, 1.0f);
+            std::vector<int> rp(dim + 1);
+            for (int r = 0; r <= dim; ++r) rp[r] = r * width;
+            if (!st) st = build_csr_wave(m, rp.data(), dim, nullptr);
+            // Row blocks for constant row length.
             std::vector<int> blocks{0};
             if (width > launch::kAdaptiveNnz) {
                 for (int r = 1; r <= dim; ++r) blocks.push_back(r);

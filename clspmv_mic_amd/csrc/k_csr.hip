@@ -5,12 +5,10 @@
 //   kernel).  Lanes stride over the row, then a lane-group xor-shuffle sum
 //   replaces the reference's barrier-free "volatile" LDS tree
 //   (kernels/spmv_csr_vector.cl:32-38).
-// csr_adaptive: one work-group per host-built row block.  Short rows: the
-//   block's products val*x[col] are staged in LDS with coalesced loads, then
-//   each row is summed by a lane group sized to the block's row count.  A row
-//   longer than the LDS budget gets the whole work-group.  Every row belongs
-//   to exactly one block, so y is written without atomics and results do not
-//   depend on what else runs on the GPU.
+// csr_wave: one wave per host-built block of rows whose entries fit
+//   kWaveNnz, a work-group per longer row.  Every row belongs to exactly one
+//   of them, so y is written without atomics and results do not depend on
+//   what else runs on the GPU.
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -44,88 +42,163 @@ __global__ __launch_bounds__(kBlock) void csr_vector_kernel(
     if (lane == 0) y[row] += sum;
 }
 
-__global__ __launch_bounds__(kBlock) void csr_adaptive_kernel(
-    const int* __restrict__ blocks, const int* __restrict__ rp,
-    const int* __restrict__ col, const float* __restrict__ val,
-    const float* __restrict__ x, float* __restrict__ y) {
-    __shared__ float prod[launch::kAdaptiveNnz];
-    __shared__ float wave_part[kBlock / kWave];
-    const int b = blockIdx.x;
-    const int r0 = blocks[b], r1 = blocks[b + 1];
-    const int s = rp[r0], e = rp[r1];
-    const int nrows = r1 - r0;
+// One row longer than kWaveNnz by the whole work-group: it strides over the
+// row, U entries' loads in flight per thread (each thread's sum in index
+// order), the waves' sums are added in order.  Acc is double for rows longer
+// than kLongRowF64 of 16-bit values: their products are exact and the row is
+// rounded once, into y.
+template <class V, class Acc>
+__device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict__ col,
+                                             const typename V::T* __restrict__ val,
+                                             const float* __restrict__ x, float* __restrict__ y,
+                                             Acc* part) {
+    constexpr int U = 4, kThreads = kWave * launch::kCsrWaves;
     const int t = threadIdx.x;
-
-    constexpr int U = launch::kAdaptiveNnz / kBlock;  // nonzeros in flight per thread
-    if (nrows == 1 && e - s > launch::kAdaptiveNnz) {
-        // Long row: the whole work-group strides over it, U nonzeros' loads
-        // in flight per thread (each thread's sum still in index order).
-        float acc = 0.0f;
-        int k = s + t;
-        for (; k + (U - 1) * kBlock < e; k += U * kBlock) {
-            int c[U];
-            float v[U], xv[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                c[u] = ld_stream(col + k + u * kBlock);
-                v[u] = ld_stream(val + k + u * kBlock);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
-#pragma unroll
-            for (int u = 0; u < U; ++u) acc = fmaf(v[u], xv[u], acc);
-        }
-        for (; k < e; k += kBlock) acc = fmaf(ld_stream(val + k), x[ld_stream(col + k)], acc);
-        acc = group_sum<kWave>(acc);
-        if ((t & (kWave - 1)) == 0) wave_part[t / kWave] = acc;
-        __syncthreads();
-        if (t == 0) {
-            float tot = 0.0f;
-#pragma unroll
-            for (int w = 0; w < kBlock / kWave; ++w) tot += wave_part[w];
-            y[r0] += tot;
-        }
-        return;
-    }
-
-    // Stage products with coalesced loads, every load of the block in
-    // flight at once (e - s <= kAdaptiveNnz = U * kBlock).  A block of empty
-    // rows loads nothing (its s may be the matrix's last index + 1).
-    if (e > s) {
+    Acc acc = 0;
+    int k = s + t;
+    for (; k + (U - 1) * kThreads < e; k += U * kThreads) {
         int c[U];
         float v[U], xv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = t + u * kBlock;
-            const int kk = k < e - s ? s + k : s;  // past the block: a valid index, not stored
-            c[u] = ld_stream(col + kk);
-            v[u] = ld_stream(val + kk);
+            c[u] = ld_stream(col + k + u * kThreads);
+            v[u] = V::ld(val + k + u * kThreads);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (t + u * kBlock < e - s) prod[t + u * kBlock] = v[u] * xv[u];
+        for (int u = 0; u < U; ++u) acc = fma((Acc)v[u], (Acc)xv[u], acc);
     }
+    for (; k < e; k += kThreads) acc = fma((Acc)V::ld(val + k), (Acc)x[ld_stream(col + k)], acc);
+    for (int m = kWave >> 1; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, kWave);
+    if (t % kWave == 0) part[t / kWave] = acc;
     __syncthreads();
+    if (t == 0) {
+        Acc tot = 0;
+#pragma unroll
+        for (int w = 0; w < launch::kCsrWaves; ++w) tot += part[w];
+        *y = sizeof(Acc) == sizeof(double) ? (float)((double)*y + (double)tot) : *y + (float)tot;
+    }
+}
 
-    // Lane-group size: the largest power of two with nrows groups fitting
-    // in the work-group, at most one wave.  A block holds at most
-    // kAdaptiveRows (= kBlock) rows, so kBlock / g >= nrows and one pass
-    // covers every row; all lanes run the shuffles.
-    int g = kBlock / (nrows > 0 ? nrows : 1);
-    g = g >= 64 ? 64 : g >= 32 ? 32 : g >= 16 ? 16 : g >= 8 ? 8 : g >= 4 ? 4
-      : g >= 2 ? 2 : 1;
-    const int lane = t & (g - 1);
-    const int r = t / g;
-    const bool live = r < nrows;
+// What bounds it: the gathers of x, and before that the waves' chain of
+// dependent loads (block, columns, x).  A wave loads the up to kWaveNnz entries
+// of its block at once as 16-byte pieces (the arrays carry kWaveNnz entries
+// of padding, so no load is guarded), the x values of its 8 entries per lane
+// at once, and leaves the products in its own part of LDS, where lane groups
+// sized to the row count sum the rows: no barrier, 32 waves per CU.  Against
+// lanes striding over rows (csr_vector) and a work-group per 1024 entries
+// with a barrier: 27-point stencil 77^3 52 / 31 -> 24 us, 5-point Laplacian
+// 701^2 15 / 10.5 -> 8 us.
+//
+// WIN: the columns of neighbouring rows are near each other but scattered
+// within the lines (meshes): a gather instruction then touches up to 64
+// lines and L1's tag rate bounds the kernel.  The work-group stages the
+// x window of its waves' columns ({first column, count} in `win`) in LDS
+// while the waves' entries are in flight and gathers there: mesh of 500,009
+// rows, 12.5 M entries, windows of 4.5 K floats: 32 -> 22 us (75 us with
+// csr_vector).  A work-group whose window is too wide (count 0) gathers from
+// memory.
+template <class V, bool WIN>
+__global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
+    int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
+    const int2* __restrict__ win, int wmax, const int* __restrict__ rp, const int* __restrict__ col,
+    const typename V::T* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
+    constexpr int U = launch::kWaveNnz / kWave, P4 = kWave * 4;
+    typedef typename V::T T;
+    typedef typename UVec<T, 4>::type T4U;
+    extern __shared__ __attribute__((aligned(16))) float sm[];  // x window, then the products of each wave
+    if ((int)blockIdx.x < nlong) {  // the longest work first
+        const int r = longs[blockIdx.x], s = rp[r], e = rp[r + 1];
+        double* part = reinterpret_cast<double*>(sm);
+        if (sizeof(T) == 2 && e - s > launch::kLongRowF64)
+            csr_long_row<V, double>(s, e, col, val, x, y + r, part);
+        else
+            csr_long_row<V, float>(s, e, col, val, x, y + r, reinterpret_cast<float*>(part));
+        return;
+    }
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int wg = xcd_tile(blockIdx.x - nlong, gridDim.x - nlong);
+    const int b = __builtin_amdgcn_readfirstlane(wg * launch::kCsrWaves + wave);
+    if (!WIN && b >= nblk) return;
+    int4 B = blk[min(b, nblk - 1)];  // {first row, rows, first entry, entries}
+    if (WIN && b >= nblk) B.y = B.w = 0;
+    const int nrows = B.y, s = B.z, n = B.w;
+    i32x4 c[U / 4];
+    typename VecOf<T, 4>::type v[U / 4];
+#pragma unroll
+    for (int u = 0; u < U / 4; ++u) {
+        c[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<int, 4>::type*>(col + s + u * P4 + lane * 4));
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const T4U*>(val + s + u * P4 + lane * 4));
+    }
+    // Lane groups for the sums: the largest power of two with nrows groups in
+    // the wave (a block holds at most kWave rows).
+    const int sh = nrows > 32 ? 0 : nrows > 16 ? 1 : nrows > 8 ? 2 : nrows > 4 ? 3 : nrows > 2 ? 4 : nrows > 1 ? 5 : 6;
+    const int g = 1 << sh, gl = lane & (g - 1);
+    const bool live = (lane >> sh) < nrows;
+    const int r = B.x + (live ? lane >> sh : 0);
+    const int k0 = rp[r] - s, k1 = rp[r + 1] - s;
+    const float yv = y[r];
+    float* prod = sm + (WIN ? wmax : 0) + wave * launch::kWaveNnz;
+    int2 w = make_int2(0, 0);
+    if constexpr (WIN) {
+        w = win[wg];
+        for (int i = threadIdx.x * 4; i < w.y; i += kWave * launch::kCsrWaves * 4) {
+            if (i + 4 <= w.y)
+                *reinterpret_cast<f32x4*>(sm + i) = *reinterpret_cast<const UVec<float, 4>::type*>(x + w.x + i);
+            else
+                for (int h = i; h < w.y; ++h) sm[h] = x[w.x + h];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < U / 4; ++u) {
+        if (u * P4 + lane * 4 >= n) continue;
+        f32x4 p;
+        if (WIN && w.y > 0) {  // uniform; entries past the block clamp into the window
+#pragma unroll
+            for (int h = 0; h < 4; ++h)
+                p[h] = V::cvt(v[u][h]) * sm[min((unsigned)(c[u][h] - w.x), (unsigned)w.y - 1u)];
+        } else {
+            float xv[4];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) xv[h] = x[c[u][h]];
+#pragma unroll
+            for (int h = 0; h < 4; ++h) p[h] = V::cvt(v[u][h]) * xv[h];
+        }
+        *reinterpret_cast<f32x4*>(prod + u * P4 + lane * 4) = p;
+    }
+    wave_lds_order();
     float acc = 0.0f;
     if (live) {
-        const int a = rp[r0 + r] - s, z = rp[r0 + r + 1] - s;
-        for (int k = a + lane; k < z; k += g) acc += prod[k];
+        float a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
+        int k = k0 + gl;
+        for (; k + 3 * g < k1; k += 4 * g) {
+            acc += prod[k];
+            a1 += prod[k + g];
+            a2 += prod[k + 2 * g];
+            a3 += prod[k + 3 * g];
+        }
+        for (; k < k1; k += g) acc += prod[k];
+        acc = (acc + a1) + (a2 + a3);
     }
     acc = group_sum_rt(acc, g);
-    if (live && lane == 0) y[r0 + r] += acc;
+    if (live && gl == 0) y[r] = yv + acc;
+}
+
+template <class V>
+hipError_t csr_wave_v(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
+                      const float* x, float* y) {
+    const dim3 grid(W.nlong + (W.nblk + launch::kCsrWaves - 1) / launch::kCsrWaves), block(kWave * launch::kCsrWaves);
+    const size_t lds = sizeof(float) * launch::kWaveNnz * launch::kCsrWaves;
+    const typename V::T* v = static_cast<const typename V::T*>(val);
+    if (W.win)
+        hipLaunchKernelGGL((csr_wave_kernel<V, true>), grid, block, lds + sizeof(float) * W.wmax, s, W.nlong, W.longs,
+                           W.nblk, W.blk, W.win, W.wmax, rp, col, v, x, y);
+    else
+        hipLaunchKernelGGL((csr_wave_kernel<V, false>), grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, W.win,
+                           0, rp, col, v, x, y);
+    return hipGetLastError();
 }
 
 }  // namespace
@@ -150,13 +223,15 @@ hipError_t csr_vector(hipStream_t s, int rows, int lanes, const int* rp,
     return hipGetLastError();
 }
 
-hipError_t csr_adaptive(hipStream_t s, int nblocks, const int* blocks,
-                        const int* rp, const int* col, const float* val,
-                        const float* x, float* y) {
-    if (nblocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(csr_adaptive_kernel, dim3(nblocks), dim3(kBlock), 0, s,
-                       blocks, rp, col, val, x, y);
-    return hipGetLastError();
+hipError_t csr_wave(hipStream_t s, const CsrWave& W, const int* rp, const int* col, int dtype, const void* val,
+                    const float* x, float* y) {
+    if (W.nblk + W.nlong <= 0) return hipSuccess;
+    switch (dtype) {
+        case 0: return csr_wave_v<ValF32>(s, W, rp, col, val, x, y);
+        case 1: return csr_wave_v<ValBF16>(s, W, rp, col, val, x, y);
+        case 2: return csr_wave_v<ValF16>(s, W, rp, col, val, x, y);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 }  // namespace launch

@@ -4,7 +4,7 @@
 // X is row-major (the k values of column c are X[c*k .. c*k+k)), so the
 // gather of one column brings every right-hand side's value in one or a few
 // 16-byte loads: a random column costs one cache line for all k products
-// instead of one line per product.  CSR runs over the adaptive row blocks
+// instead of one line per product.  CSR runs over row blocks
 // (a work-group per block of short rows or per long row).  Y is
 // column-major (ldy), so each right-hand side's y stays a contiguous
 // vector.  Matrix values may be FP32 or 16-bit (widened on load); sums are
@@ -311,7 +311,7 @@ __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__
     }
 }
 
-// CSR over the adaptive row blocks (runs of at most kAdaptiveRows rows whose
+// CSR over row blocks (runs of at most kAdaptiveRows rows whose
 // nonzeros fit kAdaptiveNnz, or one longer row).  Each lane carries
 // Q = min(KB, 4) right-hand sides (one 16-byte gather of X per nonzero), and
 // L = KB / Q neighbouring lanes cover the k values of one nonzero.

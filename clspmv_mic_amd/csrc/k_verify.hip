@@ -68,7 +68,7 @@ __device__ inline double wave_sum(double v, int g) {
     return v;
 }
 
-// One work-group per adaptive row block (csr_adaptive's blocks): a run of
+// One work-group per row block: a run of
 // rows whose nonzeros fit kAdaptiveNnz, or one longer row.
 __global__ __launch_bounds__(kBlock) void verify_csr_kernel(
     const int* __restrict__ blocks, const int* __restrict__ rp, const int* __restrict__ col,

@@ -12,17 +12,34 @@ namespace launch {
 // Vector kernel: `lanes` (power of two, 1..64) lanes cooperate on one row.
 hipError_t csr_vector(hipStream_t s, int rows, int lanes, const int* rp,
                       const int* col, const float* val, const float* x, float* y);
-// Adaptive kernel over host-built row blocks (`blocks`, nblocks+1 row starts).
-// A block is either a run of rows whose entries fit kAdaptiveNnz, or one
+// Row blocks of the multi-vector and verification kernels: a block is a run
+// of at most kAdaptiveRows rows whose entries fit kAdaptiveNnz, or one
 // longer row.
 constexpr int kAdaptiveNnz = 1024;
 constexpr int kAdaptiveRows = 256;
 // Rows longer than this are accumulated in FP64 by the 16-bit-value and
 // multi-vector CSR paths, the panel row sums and the block SpMM.
 constexpr int kLongRowF64 = 4096;
-hipError_t csr_adaptive(hipStream_t s, int nblocks, const int* blocks,
-                        const int* rp, const int* col, const float* val,
-                        const float* x, float* y);
+// Wave kernel: blk holds {first row, rows (at most 64), first entry, entries
+// (at most kWaveNnz)} per wave, longs the rows with more entries; col and val
+// carry kWaveNnz entries of padding (column 0) after the last one.  win
+// (or null): {first column, columns} of x staged for each run of kCsrWaves
+// blocks, columns 0 where it gathers from memory; wmax the most columns of
+// one, at most kCsrWinMax, rounded up to a multiple of 4.
+constexpr int kWaveNnz = 512;
+constexpr int kCsrWaves = 8;
+constexpr int kCsrWinMax = 8192;
+static_assert(4 * (kWaveNnz * kCsrWaves + kCsrWinMax) <= 64 * 1024, "within the default LDS limit");
+struct CsrWave {
+    const int4* blk = nullptr;
+    int nblk = 0;
+    const int* longs = nullptr;
+    int nlong = 0;
+    const int2* win = nullptr;
+    int wmax = 0;
+};
+hipError_t csr_wave(hipStream_t s, const CsrWave& W, const int* rp, const int* col, int dtype, const void* val,
+                    const float* x, float* y);
 
 // ---- COO ------------------------------------------------------------------
 // Row-sorted COO in chunks of kCooChunk entries; 2 carry slots per chunk.
@@ -140,7 +157,7 @@ constexpr int kMultiMax = 16;
 constexpr int kDiaRun = 3;
 hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy);
-// CSR over the adaptive row blocks (csr_adaptive's `blocks`).  kb > 0 runs
+// CSR over the row blocks above.  kb > 0 runs
 // the kernel built for kb right-hand sides (k <= kb; 1, 2, 4, 8 or 16)
 // whatever k is, so that each right-hand side's summation order stays that
 // of kb; kb = 0 picks the smallest width that holds k.

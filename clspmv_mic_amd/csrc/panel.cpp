@@ -366,6 +366,9 @@ void drop_encoding(clspmv_dmat* d, bool panel) {
     release_array(d, &d->carry_row);
     release_array(d, &d->carry_val);
     release_array(d, &d->blocks);
+    release_array(d, &d->wblk);
+    release_array(d, &d->wlong);
+    release_array(d, &d->wwin);
     d->plain = false;
     d->use_panel = true;
 }

@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <cstring>
 #include <chrono>
+#include <climits>
 #include <cmath>
 #include <cstdint>
 #include <numeric>
@@ -59,9 +60,9 @@ clspmv_dmat* new_dmat(int format, const clspmv_matinfo& mi) {
     return m;
 }
 
-// Row blocks of the adaptive CSR kernel: a block is a maximal run of at most
+// Row blocks of the multi-vector and verification CSR kernels: a block is a maximal run of at most
 // kAdaptiveRows rows whose entries fit kAdaptiveNnz, or a single longer row.
-std::vector<int> adaptive_blocks(const int* rp, int rows) {
+std::vector<int> csr_row_blocks(const int* rp, int rows) {
     std::vector<int> b{0};
     int r = 0;
     while (r < rows) {
@@ -99,12 +100,68 @@ bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 }  // namespace
 
+int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
+    std::vector<int4> blk;
+    std::vector<int> longs;
+    for (int r = 0; r < rows;) {
+        if (rp[r + 1] - rp[r] > launch::kWaveNnz) {
+            longs.push_back(r++);
+            continue;
+        }
+        int e = r;
+        while (e < rows && e - r < 64 && rp[e + 1] - rp[r] <= launch::kWaveNnz) ++e;
+        blk.push_back(make_int4(r, e - r, rp[r], rp[e] - rp[r]));
+        r = e;
+    }
+    d->nwblk = (int)blk.size();
+    d->nwlong = (int)longs.size();
+    int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
+    if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
+    if (st || !col || blk.empty()) return st;
+    // x windows: the column range of each work-group's blocks.  They pay where
+    // a gather instruction (64 entries, 4 apart) touches many 128-byte lines
+    // of x and the range is narrow: mesh of 500,009 rows, 52 lines, 4.5 K
+    // columns: 22 us against 32; 27-point stencil 47^3, 16 lines, 4.6 K
+    // columns: 10.2 against 8.0 us.  The lines are sampled on up to 256 blocks,
+    // and a matrix has windows when nine in ten of its work-groups fit.
+    long long lines = 0, samples = 0;
+    for (size_t b = 0, step = std::max<size_t>(1, blk.size() / 256); b < blk.size(); b += step) {
+        if (blk[b].w < 256) continue;
+        int line[64];
+        for (int i = 0; i < 64; ++i) line[i] = col[blk[b].z + 4 * i] / 32;
+        std::sort(line, line + 64);
+        lines += std::unique(line, line + 64) - line;
+        ++samples;
+    }
+    if (samples == 0 || lines < 32 * samples) return CLSPMV_OK;
+    constexpr int W = launch::kCsrWaves;
+    const size_t ng = (blk.size() + W - 1) / W;
+    std::vector<int2> win(ng);
+    size_t wide = 0;
+    int wmax = 0;
+    for (size_t g = 0; g < ng && wide * 10 <= ng; ++g) {
+        int lo = INT_MAX, hi = -1;
+        for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
+            for (int k = blk[b].z; k < blk[b].z + blk[b].w; ++k) {
+                lo = std::min(lo, col[k]);
+                hi = std::max(hi, col[k]);
+            }
+        const int n = hi < 0 ? 0 : hi - lo + 1;
+        win[g] = n > 0 && n <= launch::kCsrWinMax ? make_int2(lo, n) : make_int2(0, 0);
+        wide += n > launch::kCsrWinMax;
+        wmax = std::max(wmax, win[g].y);
+    }
+    if (wide * 10 > ng) return CLSPMV_OK;
+    d->wwin_max = round_up(wmax, 4);
+    return upload_array(d, win.data(), win.size(), &d->wwin);
+}
+
 int auto_method(const clspmv_dmat* A) {
     switch (A->info.format) {
-        case CLSPMV_FMT_CSR: {
-            double avg = A->info.rows ? (double)A->info.nnz / A->info.rows : 0.0;
-            return A->max_row > 8.0 * std::max(avg, 4.0) ? 1 : 0;
-        }
+        // The wave kernel: lanes striding over rows are no faster at any row
+        // length (27-point stencil 77^3 24 against 52 us, 5-point Laplacian
+        // 256^2 4.7 against 4.6 us, power-law rows 1 M 108 against 225 us).
+        case CLSPMV_FMT_CSR: return 1;
         case CLSPMV_FMT_ELL: return A->hal % 4 == 0 ? 1 : 0;
         case CLSPMV_FMT_DIA: return 0;
         case CLSPMV_FMT_BDIA: return 0;
@@ -178,13 +235,13 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
     const bool xa = aligned16(x);
     switch (I.format) {
         case CLSPMV_FMT_CSR:
-            if (A->dtype) {  // 16-bit values: the multi-vector kernel with k = 1
-                e = launch::csr_multi(s, A->nblocks, A->blocks, A->rp, A->col, A->dtype, A->lpval, 1, x, y,
-                                      I.rows);
-                break;
-            }
-            e = method == 0 ? launch::csr_vector(s, I.rows, A->lanes, A->rp, A->col, A->val, x, y)
-                            : launch::csr_adaptive(s, A->nblocks, A->blocks, A->rp, A->col, A->val, x, y);
+            // 16-bit values have one kernel, whatever the method.
+            if (method == 0 && !A->dtype)
+                e = launch::csr_vector(s, I.rows, A->lanes, A->rp, A->col, A->val, x, y);
+            else
+                e = launch::csr_wave(
+                    s, launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->wwin, A->wwin_max}, A->rp, A->col,
+                    A->dtype, A->dtype ? (const void*)A->lpval : (const void*)A->val, x, y);
             break;
         case CLSPMV_FMT_COO:
             e = launch::coo_segreduce(s, I.nnz, A->row, A->col, A->val, x, y,
@@ -484,17 +541,18 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     double avg = rows ? (double)nnz / rows : 0.0;
     d->lanes = pow2_at_least((int)std::ceil(avg), 64);
     UPLOAD_CHECK(upload_array(d, m->csr_row_ptr, (size_t)rows + 1, &d->rp));
-    UPLOAD_CHECK(upload_array(d, m->csr_col_id, nnz, &d->col));
+    UPLOAD_CHECK(upload_padded(d, m->csr_col_id, nnz, launch::kWaveNnz, &d->col));
     if (o.dtype != CLSPMV_DT_F32) {
-        // Own arrays with 16-bit values (run by the multi-vector kernel).
+        // Own arrays with 16-bit values (every method runs the wave kernel).
         std::vector<unsigned short> lp(nnz);
         UPLOAD_CHECK(clspmv_convert_from_f32(m->csr_data, lp.data(), (size_t)nnz, o.dtype));
-        UPLOAD_CHECK(upload_array(d, lp.data(), lp.size(), &d->lpval));
+        UPLOAD_CHECK(upload_padded(d, lp.data(), lp.size(), launch::kWaveNnz, &d->lpval));
         d->dtype = o.dtype;
     } else {
-        UPLOAD_CHECK(upload_array(d, m->csr_data, nnz, &d->val));
+        UPLOAD_CHECK(upload_padded(d, m->csr_data, nnz, launch::kWaveNnz, &d->val));
     }
-    std::vector<int> blocks = adaptive_blocks(m->csr_row_ptr, rows);
+    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, m->csr_col_id));
+    std::vector<int> blocks = csr_row_blocks(m->csr_row_ptr, rows);
     d->nblocks = (int)blocks.size() - 1;
     UPLOAD_CHECK(upload_array(d, blocks.data(), blocks.size(), &d->blocks));
 

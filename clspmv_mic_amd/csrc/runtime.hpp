@@ -20,7 +20,10 @@ struct clspmv_dmat {
     int device = 0;
     std::vector<std::pair<void*, size_t>> bufs;  // device allocations owned by the matrix
 
-    // CSR: rp/col/val; adaptive row blocks; vector lanes per row.
+    // CSR: rp/col/val (col and val padded by launch::kWaveNnz entries);
+    // row blocks of the multi-vector and verification kernels; blocks, long
+    // rows and x windows of the wave kernel (launch::CsrWave); lanes per row
+    // of the vector kernel.
     int* rp = nullptr;
     int* col = nullptr;
     float* val = nullptr;
@@ -28,6 +31,10 @@ struct clspmv_dmat {
     int nblocks = 0;
     int lanes = 1;
     int max_row = 0;
+    int4* wblk = nullptr;
+    int* wlong = nullptr;
+    int2* wwin = nullptr;
+    int nwblk = 0, nwlong = 0, wwin_max = 0;
     // COO: row/col/val, carry slots (2 per chunk).
     int* row = nullptr;
     int* carry_row = nullptr;
@@ -122,6 +129,18 @@ int upload_array(clspmv_dmat* m, const T* host, size_t n, T** out) {
     return CLSPMV_OK;
 }
 
+// The same with `pad` zeros after the last element.
+template <class T>
+int upload_padded(clspmv_dmat* m, const T* host, size_t n, size_t pad, T** out) {
+    const int st = upload_array<T>(m, nullptr, n + pad, out);
+    if (st) return st;
+    const std::vector<T> zero(pad, T(0));
+    hipError_t e = n ? hipMemcpy(*out, host, sizeof(T) * n, hipMemcpyHostToDevice) : hipSuccess;
+    if (e == hipSuccess) e = hipMemcpy(*out + n, zero.data(), sizeof(T) * pad, hipMemcpyHostToDevice);
+    if (e != hipSuccess) return fail(CLSPMV_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
+    return CLSPMV_OK;
+}
+
 // Frees one allocation of `m` (no-op for null); the pointer is cleared.
 template <class T>
 void release_array(clspmv_dmat* m, T** p) {
@@ -135,6 +154,10 @@ void release_array(clspmv_dmat* m, T** p) {
         }
     *p = nullptr;
 }
+
+// Builds and uploads the wave kernel's tables of a CSR matrix from its host
+// row pointers; col (or null: no x windows) its host columns.
+int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col);
 
 // x-panel encoding (k_panel.hip) of row-sorted entries, built on the host
 // and uploaded into `d`.  pw: panel width (multiple of 8, at most

@@ -57,8 +57,8 @@ enum clspmv_format {
  * per-format GFLOP/s columns of the .ben tables read by the Cocktail
  * partitioner, so the counts equal the reference's *_IMP_NUM.
  *   CSR  0: vector kernel, lanes per row = power of two near nnz/row
- *        1: adaptive row blocks (short rows share an LDS-staged block,
- *           long rows take a whole work-group)
+ *        1: row blocks (a wave per block of short rows, whose products it
+ *           sums from LDS; long rows take a whole work-group)
  *   COO  0: one-pass segmented reduction + carry fix-up
  *   ELL  0: one row per lane          1: four rows per lane (128-bit loads)
  *   SELL 0/1: one row per lane (slice height is a property of the data)

@@ -423,6 +423,41 @@ def test_dia_multi_tiles(ctx, offsets, n, ks):
             ctx.sync()
             np.testing.assert_array_equal(dY.download()[1:].reshape(k, n + 1), ref.astype(np.float32))
 
+def _csr_wave_case(name):
+    """Dyadic matrices at the edges of the CSR wave kernel: rows at its 512
+    entries, runs of empty rows, blocks of 64 rows, and scattered columns in
+    narrow windows (staged in LDS), some of them too wide."""
+    rng = np.random.default_rng(11)
+    if name == "row_lengths":
+        width = 6000
+        lens = np.concatenate([[0, 1, 512, 513, 0, 0, 3, 511, 1, 600, 5000], np.zeros(130, int), np.ones(200, int),
+                               [2, 510, 256, 256, 1, 511, 4096, 4097], rng.integers(0, 20, 300), [0]])
+        rows = np.repeat(np.arange(lens.size), lens)
+        cols = np.concatenate([np.sort(rng.choice(width, n, replace=False)) for n in lens])
+        height = lens.size
+    else:
+        height = width = 20_001
+        lens = rng.integers(8, 41, height)
+        rows = np.repeat(np.arange(height), lens)
+        cols = np.clip(rows + rng.integers(-900, 901, rows.size), 0, width - 1)
+        if name == "windows_some_wide":
+            cols[(rows // 50) % 200 == 7] = rng.integers(0, width, int(((rows // 50) % 200 == 7).sum()))
+        key = np.unique(rows.astype(np.int64) * width + cols)
+        rows, cols = key // width, key % width
+    vals = (rng.integers(-64, 65, rows.size) / 64.0).astype(np.float32)
+    return cs.Coo(rows.astype(np.int32), cols.astype(np.int32), vals, height, width)
+
+
+@pytest.mark.parametrize("name", ["row_lengths", "windows", "windows_some_wide"])
+@pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16, cs.DT_F16])
+@pytest.mark.parametrize("x_offset", [0, 1])
+def test_csr_wave(ctx, oracle, name, dtype, x_offset):
+    """Method 1 (and the automatic method) on dyadic inputs: every partial sum
+    is exact, so y equals the FP64 product bit for bit."""
+    A = _csr_wave_case(name)
+    for method in (1, cs.METHOD_AUTO):
+        _run(ctx, oracle, A, cs.coo2csr(A.copy()), method, panel=0, x_offset=x_offset, dtype=dtype)
+
 
 @pytest.mark.parametrize("name", ["rand_small", "rand_dyadic", "rand_long_rows"])
 @pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
