@@ -14,25 +14,110 @@ namespace {
 
 using namespace dev;
 
-__global__ __launch_bounds__(kBlock) void ell_kernel(
-    int rows, int hal, int ellnum, const int* __restrict__ col,
-    const float* __restrict__ val, const float* __restrict__ x,
+// One row per lane, for ELL (ptr null: every row has `w0` slots `stride` apart)
+// and SELL (slices of h rows; a slot's entries are h apart).
+//
+// What bounds it: on large matrices HBM (padding slots are read too), on
+// small ones the chain of slots: column, then x.  kSlots slots' columns and
+// values load at once, and the next kSlots' are in flight while the present
+// ones' x values are gathered (two register sets taking turns, nothing
+// copied; the last, shorter group loads no more than its slots).  Two slots
+// at a time took 9.8 / 10.4 us (ELL / SELL) on the 27-point stencil 30^3 and
+// 14.4 / 15.2 us on a mesh of 40,000 rows; this takes 6.5 / 7.1 and 10.2 /
+// 11.1 us.
+//
+// WIN: where neighbouring rows' columns are near each other but scattered
+// over lines (meshes) the work-group stages the x window of its rows
+// ({first column, count} in `win`; 0: gather from memory) in LDS and gathers
+// there, past L1's tag rate: mesh of 500,009 rows 60 / 63 -> 29 / 29 us, of
+// which reading the padded slots takes 23 us.
+template <bool SELL, bool WIN, int kSlots>
+__global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
+    int rows, int h, int w0, const int* __restrict__ ptr, const int2* __restrict__ win,
+    const int* __restrict__ col, const float* __restrict__ val, const float* __restrict__ x,
     float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= rows) return;
-    float a0 = 0.0f, a1 = 0.0f;
+    extern __shared__ __attribute__((aligned(16))) float xs[];
+    const int wg = xcd_tile(blockIdx.x, gridDim.x);
+    const int row = wg * launch::kEllRows + (int)threadIdx.x;
+    const int r = min(row, rows - 1);  // lanes past the end shadow the last row
+    int w = w0;
+    const int* cp = col + r;
+    const float* vp = val + r;
+    if constexpr (SELL) {
+        const int sl = r / h, p0 = ptr[sl];
+        w = (ptr[sl + 1] - p0) / h;
+        // A lane whose slice is empty reads entry 0 beside its neighbours (the
+        // matrix has entries when they have any): at p0 there may be none.
+        cp = w > 0 ? col + p0 + (r - sl * h) : col;
+        vp = w > 0 ? val + p0 + (r - sl * h) : val;
+    }
+    // The widest row of the wave: its slots are walked, and slots past the
+    // lane's own last one re-read that one and are not added.
+    int wm = w;
+    if constexpr (SELL)
+        for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    wm = __builtin_amdgcn_readfirstlane(wm);
+    int c[2][kSlots];
+    float v[2][kSlots];
+    auto load = [&](int s, int* cc, float* vv) {
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) {
+            const size_t at = (size_t)(SELL ? max(min(s + u, w - 1), 0) : s + u) * h;
+            cc[u] = ld_stream(cp + at);
+            vv[u] = ld_stream(vp + at);
+        }
+    };
+    auto load_part = [&](int s, int* cc, float* vv) {  // slots below wm
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u) {
+            if (s + u >= wm) break;
+            const size_t at = (size_t)(SELL ? max(min(s + u, w - 1), 0) : s + u) * h;
+            cc[u] = ld_stream(cp + at);
+            vv[u] = ld_stream(vp + at);
+        }
+    };
+    if (kSlots <= wm) load(0, c[0], v[0]);
+    else load_part(0, c[0], v[0]);
+    int2 wn = make_int2(0, 0);
+    if constexpr (WIN) {
+        wn = win[wg];
+        for (int i = threadIdx.x * 4; i < wn.y; i += launch::kEllRows * 4) {
+            if (i + 4 <= wn.y)
+                *reinterpret_cast<f32x4*>(xs + i) = *reinterpret_cast<const UVec<float, 4>::type*>(x + wn.x + i);
+            else
+                for (int e = i; e < wn.y; ++e) xs[e] = x[wn.x + e];
+        }
+        __syncthreads();
+    }
+    float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](int s, const int* cc, const float* vv) {
+        float xv[kSlots];
+        if (WIN && wn.y > 0) {
+#pragma unroll
+            for (int u = 0; u < kSlots; ++u)
+                if (s + u < wm) xv[u] = xs[min((unsigned)(cc[u] - wn.x), (unsigned)wn.y - 1u)];
+        } else {
+#pragma unroll
+            for (int u = 0; u < kSlots; ++u)
+                if (s + u < wm) xv[u] = x[cc[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u)
+            if (s + u < wm) a[u % 4] = s + u < w ? fmaf(vv[u], xv[u], a[u % 4]) : a[u % 4];
+    };
     int s = 0;
-    for (; s + 1 < ellnum; s += 2) {
-        const size_t i0 = (size_t)s * hal + r, i1 = i0 + hal;
-        const int c0 = ld_stream(col + i0), c1 = ld_stream(col + i1);
-        a0 = fmaf(ld_stream(val + i0), x[c0], a0);
-        a1 = fmaf(ld_stream(val + i1), x[c1], a1);
+    for (; s + 3 * kSlots <= wm; s += 2 * kSlots) {
+        load(s + kSlots, c[1], v[1]);
+        add(s, c[0], v[0]);
+        load(s + 2 * kSlots, c[0], v[0]);
+        add(s + kSlots, c[1], v[1]);
     }
-    if (s < ellnum) {
-        const size_t i0 = (size_t)s * hal + r;
-        a0 = fmaf(ld_stream(val + i0), x[ld_stream(col + i0)], a0);
-    }
-    y[r] += a0 + a1;
+    if (s + kSlots < wm) load_part(s + kSlots, c[1], v[1]);
+    add(s, c[0], v[0]);
+    if (s + 2 * kSlots < wm) load_part(s + 2 * kSlots, c[0], v[0]);
+    if (s + kSlots < wm) add(s + kSlots, c[1], v[1]);
+    if (s + 2 * kSlots < wm) add(s + 2 * kSlots, c[0], v[0]);
+    if (row < rows) y[r] += (a[0] + a[1]) + (a[2] + a[3]);
 }
 
 // Four consecutive rows per lane; requires hal % 4 == 0.
@@ -58,54 +143,51 @@ __global__ __launch_bounds__(kBlock) void ell4_kernel(
     if (r + 3 < rows) y[r + 3] += a.w;
 }
 
-__global__ __launch_bounds__(kBlock) void sell_kernel(
-    int rows, int h, const int* __restrict__ ptr, const int* __restrict__ col,
-    const float* __restrict__ val, const float* __restrict__ x,
-    float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= rows) return;
-    const int sl = r / h, i = r - sl * h;
-    const int p0 = ptr[sl];
-    const int w = (ptr[sl + 1] - p0) / h;
-    const int* c = col + p0 + i;
-    const float* v = val + p0 + i;
-    float a0 = 0.0f, a1 = 0.0f;
-    int k = 0;
-    for (; k + 1 < w; k += 2) {
-        const int c0 = ld_stream(c + (size_t)k * h), c1 = ld_stream(c + (size_t)(k + 1) * h);
-        a0 = fmaf(ld_stream(v + (size_t)k * h), x[c0], a0);
-        a1 = fmaf(ld_stream(v + (size_t)(k + 1) * h), x[c1], a1);
-    }
-    if (k < w) a0 = fmaf(ld_stream(v + (size_t)k * h), x[ld_stream(c + (size_t)k * h)], a0);
-    y[r] += a0 + a1;
+// Slots in flight: eight while there are fewer than two waves per SIMD (131,072
+// rows), where the chain of slots sets the time (stencil 30^3 6.5 against 8.2
+// us), four above, where more waves cover it and the shorter last group
+// matters (stencil 77^3 19 against 22 us, 5-point Laplacian 701^2 5.9 against
+// 6.6 us).
+template <bool SELL, int kSlots>
+hipError_t ell_rows_k(hipStream_t s, int rows, int h, int w, const int* ptr, launch::EllWindows W, const int* col,
+                      const float* val, const float* x, float* y) {
+    const dim3 grid((rows + launch::kEllRows - 1) / launch::kEllRows), block(launch::kEllRows);
+    if (W.win)
+        hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots>), grid, block, sizeof(float) * W.max, s, rows, h, w, ptr,
+                           W.win, col, val, x, y);
+    else
+        hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots>), grid, block, 0, s, rows, h, w, ptr, W.win, col, val,
+                           x, y);
+    return hipGetLastError();
+}
+
+template <bool SELL>
+hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, launch::EllWindows W, const int* col,
+                    const float* val, const float* x, float* y) {
+    return rows < (1 << 17) ? ell_rows_k<SELL, 8>(s, rows, h, w, ptr, W, col, val, x, y)
+                            : ell_rows_k<SELL, 4>(s, rows, h, w, ptr, W, col, val, x, y);
 }
 
 }  // namespace
 
 namespace launch {
 
-hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane,
+hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, EllWindows W,
                const int* col, const float* val, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
-    if (rows_per_lane == 4) {
-        if (hal % 4 != 0) return hipErrorInvalidValue;
-        const int lanes = (rows + 3) / 4;
-        hipLaunchKernelGGL(ell4_kernel, dim3((lanes + kBlock - 1) / kBlock),
-                           dim3(kBlock), 0, s, rows, hal, ellnum, col, val, x, y);
-    } else {
-        hipLaunchKernelGGL(ell_kernel, dim3((rows + kBlock - 1) / kBlock),
-                           dim3(kBlock), 0, s, rows, hal, ellnum, col, val, x, y);
-    }
+    if (rows_per_lane != 4) return ell_rows<false>(s, rows, hal, ellnum, nullptr, W, col, val, x, y);
+    if (hal % 4 != 0) return hipErrorInvalidValue;
+    const int lanes = (rows + 3) / 4;
+    hipLaunchKernelGGL(ell4_kernel, dim3((lanes + kBlock - 1) / kBlock),
+                       dim3(kBlock), 0, s, rows, hal, ellnum, col, val, x, y);
     return hipGetLastError();
 }
 
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr,
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, EllWindows W,
                 const int* col, const float* val, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
     if (slice_height <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(sell_kernel, dim3((rows + kBlock - 1) / kBlock),
-                       dim3(kBlock), 0, s, rows, slice_height, ptr, col, val, x, y);
-    return hipGetLastError();
+    return ell_rows<true>(s, rows, slice_height, 0, ptr, W, col, val, x, y);
 }
 
 }  // namespace launch

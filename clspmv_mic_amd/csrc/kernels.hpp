@@ -110,9 +110,18 @@ hipError_t panel_pass2(hipStream_t s, const float* seg_val, int nblocks, const i
                        const int* longs, float* y);
 
 // ---- ELL / SELL --------------------------------------------------------------
-hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane,
+// win (or null): {first column, columns} of x for each kEllRows rows, staged
+// in LDS by their work-group; columns 0 where it gathers from memory; max the
+// most columns of one, at most kEllWinMax.
+constexpr int kEllRows = 512;
+constexpr int kEllWinMax = 8192;
+struct EllWindows {
+    const int2* win = nullptr;
+    int max = 0;
+};
+hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, EllWindows W,
                const int* col, const float* val, const float* x, float* y);
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr,
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, EllWindows W,
                 const int* col, const float* val, const float* x, float* y);
 
 // ---- DIA / BDIA -------------------------------------------------------------

@@ -98,6 +98,43 @@ std::vector<int4> dia_segments(const int* off, int ndiag, int rows, int cols, in
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
+// x windows (launch::CsrWave, launch::EllWindows) for `groups` work-groups,
+// where neighbouring rows' columns are near each other but scattered over the
+// 128-byte lines of x: a gather instruction then touches many lines and L1's
+// tag rate bounds the kernel, while the window costs one coalesced pass.
+// sample(g, cols) gives the 64 columns of one gather instruction of group g
+// (false: none); they are looked at on up to 256 groups and must touch 24
+// lines on average.  range(g, lo, hi) widens [*lo, *hi] by the group's columns; a
+// group wider than `limit` gathers from memory, and with more than one in
+// ten of those the matrix gets no windows.
+template <class Sample, class Range>
+int add_windows(clspmv_dmat* d, size_t groups, int limit, Sample&& sample, Range&& range) {
+    long long lines = 0, samples = 0;
+    for (size_t g = 0, step = std::max<size_t>(1, groups / 256); g < groups; g += step) {
+        int line[64];
+        if (!sample(g, line)) continue;
+        for (int& l : line) l /= 32;
+        std::sort(line, line + 64);
+        lines += std::unique(line, line + 64) - line;
+        ++samples;
+    }
+    if (samples == 0 || lines < 24 * samples) return CLSPMV_OK;
+    std::vector<int2> win(groups);
+    size_t wide = 0;
+    int wmax = 0;
+    for (size_t g = 0; g < groups; ++g) {
+        int lo = INT_MAX, hi = -1;
+        range(g, &lo, &hi);
+        const int n = hi < 0 ? 0 : hi - lo + 1;
+        win[g] = n > 0 && n <= limit ? make_int2(lo, n) : make_int2(0, 0);
+        wide += n > limit;
+        wmax = std::max(wmax, win[g].y);
+        if (wide * 10 > groups) return CLSPMV_OK;
+    }
+    d->wwin_max = round_up(wmax, 4);
+    return upload_array(d, win.data(), win.size(), &d->wwin);
+}
+
 }  // namespace
 
 int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
@@ -118,42 +155,24 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
     int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
     if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
     if (st || !col || blk.empty()) return st;
-    // x windows: the column range of each work-group's blocks.  They pay where
-    // a gather instruction (64 entries, 4 apart) touches many 128-byte lines
-    // of x and the range is narrow: mesh of 500,009 rows, 52 lines, 4.5 K
-    // columns: 22 us against 32; 27-point stencil 47^3, 16 lines, 4.6 K
-    // columns: 10.2 against 8.0 us.  The lines are sampled on up to 256 blocks,
-    // and a matrix has windows when nine in ten of its work-groups fit.
-    long long lines = 0, samples = 0;
-    for (size_t b = 0, step = std::max<size_t>(1, blk.size() / 256); b < blk.size(); b += step) {
-        if (blk[b].w < 256) continue;
-        int line[64];
-        for (int i = 0; i < 64; ++i) line[i] = col[blk[b].z + 4 * i] / 32;
-        std::sort(line, line + 64);
-        lines += std::unique(line, line + 64) - line;
-        ++samples;
-    }
-    if (samples == 0 || lines < 32 * samples) return CLSPMV_OK;
+    // x windows where they pay: mesh of 500,009 rows (a gather instruction
+    // touches 52 lines, windows of 4.5 K columns) 22 us against 32; 27-point
+    // stencil 47^3 (16 lines, 4.6 K columns) 10.2 against 8.0 us.
     constexpr int W = launch::kCsrWaves;
-    const size_t ng = (blk.size() + W - 1) / W;
-    std::vector<int2> win(ng);
-    size_t wide = 0;
-    int wmax = 0;
-    for (size_t g = 0; g < ng && wide * 10 <= ng; ++g) {
-        int lo = INT_MAX, hi = -1;
-        for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
-            for (int k = blk[b].z; k < blk[b].z + blk[b].w; ++k) {
-                lo = std::min(lo, col[k]);
-                hi = std::max(hi, col[k]);
-            }
-        const int n = hi < 0 ? 0 : hi - lo + 1;
-        win[g] = n > 0 && n <= launch::kCsrWinMax ? make_int2(lo, n) : make_int2(0, 0);
-        wide += n > launch::kCsrWinMax;
-        wmax = std::max(wmax, win[g].y);
-    }
-    if (wide * 10 > ng) return CLSPMV_OK;
-    d->wwin_max = round_up(wmax, 4);
-    return upload_array(d, win.data(), win.size(), &d->wwin);
+    return add_windows(
+        d, (blk.size() + W - 1) / W, launch::kCsrWinMax,
+        [&](size_t g, int* line) {
+            const int4 b = blk[g * W];
+            for (int i = 0; i < 64 && b.w >= 256; ++i) line[i] = col[b.z + 4 * i];
+            return b.w >= 256;
+        },
+        [&](size_t g, int* lo, int* hi) {
+            for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
+                for (int k = blk[b].z; k < blk[b].z + blk[b].w; ++k) {
+                    *lo = std::min(*lo, col[k]);
+                    *hi = std::max(*hi, col[k]);
+                }
+        });
 }
 
 int auto_method(const clspmv_dmat* A) {
@@ -162,7 +181,10 @@ int auto_method(const clspmv_dmat* A) {
         // length (27-point stencil 77^3 24 against 52 us, 5-point Laplacian
         // 256^2 4.7 against 4.6 us, power-law rows 1 M 108 against 225 us).
         case CLSPMV_FMT_CSR: return 1;
-        case CLSPMV_FMT_ELL: return A->hal % 4 == 0 ? 1 : 0;
+        // A row per lane: four rows per lane leave a quarter of the waves and
+        // gather x four rows apart (27-point stencil 77^3 30 against 19 us,
+        // 30^3 21 against 6.5 us; 5-point Laplacian 701^2 7.9 against 5.9 us).
+        case CLSPMV_FMT_ELL: return 0;
         case CLSPMV_FMT_DIA: return 0;
         case CLSPMV_FMT_BDIA: return 0;
         default: return 0;
@@ -250,10 +272,12 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
         case CLSPMV_FMT_ELL:
             if (method == 1 && A->hal % 4 != 0)
                 return fail(CLSPMV_ERR_UNSUPPORTED, "ELL method 1 needs height_aligned %% 4 == 0");
-            e = launch::ell(s, I.rows, A->hal, A->ellnum, method == 1 ? 4 : 1, A->col, A->val, x, y);
+            e = launch::ell(s, I.rows, A->hal, A->ellnum, method == 1 ? 4 : 1, launch::EllWindows{A->wwin, A->wwin_max},
+                            A->col, A->val, x, y);
             break;
         case CLSPMV_FMT_SELL:
-            e = launch::sell(s, I.rows, I.slice_height, A->sptr, A->col, A->val, x, y);
+            e = launch::sell(s, I.rows, I.slice_height, A->sptr, launch::EllWindows{A->wwin, A->wwin_max}, A->col,
+                             A->val, x, y);
             break;
         case CLSPMV_FMT_DIA: {
             const int span = A->max_off - A->min_off;
@@ -613,6 +637,24 @@ int clspmv_upload_ell(clspmv_ctx* ctx, const clspmv_ell_matrix* m, clspmv_dmat**
     d->info.stored = (long long)total;
     UPLOAD_CHECK(upload_array(d, m->ell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->ell_data, total, &d->val));
+    if (m->ell_num > 0) {
+        const int rows = m->matinfo.height, hal = m->ell_height_aligned;
+        constexpr int R = launch::kEllRows;
+        UPLOAD_CHECK(add_windows(
+            d, (rows + R - 1) / R, launch::kEllWinMax,
+            [&](size_t g, int* line) {
+                if ((int)g * R + 64 > rows) return false;
+                std::copy_n(m->ell_col_id + (size_t)(m->ell_num / 2) * hal + g * R, 64, line);
+                return true;
+            },
+            [&](size_t g, int* lo, int* hi) {
+                for (int s = 0; s < m->ell_num; ++s)
+                    for (int r = (int)g * R; r < std::min(rows, ((int)g + 1) * R); ++r) {
+                        *lo = std::min(*lo, m->ell_col_id[(size_t)s * hal + r]);
+                        *hi = std::max(*hi, m->ell_col_id[(size_t)s * hal + r]);
+                    }
+            }));
+    }
     *out = d;
     return CLSPMV_OK;
 }
@@ -633,6 +675,34 @@ int clspmv_upload_sell(clspmv_ctx* ctx, const clspmv_sell_matrix* m, clspmv_dmat
     UPLOAD_CHECK(upload_array(d, m->sell_slice_ptr, (size_t)ns + 1, &d->sptr));
     UPLOAD_CHECK(upload_array(d, m->sell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->sell_data, total, &d->val));
+    {
+        const int rows = m->matinfo.height;
+        const int* sp = m->sell_slice_ptr;
+        constexpr int R = launch::kEllRows;
+        UPLOAD_CHECK(add_windows(
+            d, (rows + R - 1) / R, launch::kEllWinMax,
+            [&](size_t g, int* line) {
+                // The middle slot of each of 64 rows.
+                for (int i = 0; i < 64; ++i) {
+                    const int r = (int)g * R + i, s = r / h;
+                    if (r >= rows || sp[s + 1] == sp[s]) return false;
+                    line[i] = m->sell_col_id[sp[s] + (sp[s + 1] - sp[s]) / h / 2 * h + r % h];
+                }
+                return true;
+            },
+            [&](size_t g, int* lo, int* hi) {
+                const int r1 = std::min(rows, ((int)g + 1) * R);
+                for (int r = (int)g * R; r < r1;) {  // the group's rows of each slice
+                    const int s = r / h, i0 = r % h, i1 = std::min(h, i0 + r1 - r);
+                    for (int k = sp[s]; k < sp[s + 1]; k += h)
+                        for (int i = i0; i < i1; ++i) {
+                            *lo = std::min(*lo, m->sell_col_id[k + i]);
+                            *hi = std::max(*hi, m->sell_col_id[k + i]);
+                        }
+                    r += i1 - i0;
+                }
+            }));
+    }
     *out = d;
     return CLSPMV_OK;
 }

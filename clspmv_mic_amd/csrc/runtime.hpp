@@ -33,8 +33,11 @@ struct clspmv_dmat {
     int max_row = 0;
     int4* wblk = nullptr;
     int* wlong = nullptr;
+    int nwblk = 0, nwlong = 0;
+    // x windows of CSR's wave kernel, ELL and SELL (null: absent), the
+    // columns of the widest one.
     int2* wwin = nullptr;
-    int nwblk = 0, nwlong = 0, wwin_max = 0;
+    int wwin_max = 0;
     // COO: row/col/val, carry slots (2 per chunk).
     int* row = nullptr;
     int* carry_row = nullptr;

@@ -458,6 +458,38 @@ def test_csr_wave(ctx, oracle, name, dtype, x_offset):
     for method in (1, cs.METHOD_AUTO):
         _run(ctx, oracle, A, cs.coo2csr(A.copy()), method, panel=0, x_offset=x_offset, dtype=dtype)
 
+@pytest.mark.parametrize("name", ["windows", "windows_some_wide"])
+@pytest.mark.parametrize("fmt", ["ell", "sell"])
+@pytest.mark.parametrize("x_offset", [0, 1])
+@pytest.mark.parametrize("repeat", [1, 7])
+def test_ell_windows(ctx, oracle, name, fmt, x_offset, repeat):
+    """ELL and SELL with x windows in LDS, some work-groups without one, below
+    and above the row count where the slots in flight change (`repeat` copies
+    of the matrix along the diagonal); dyadic inputs, exact sums."""
+    A = _csr_wave_case(name)
+    if repeat > 1:
+        i = np.arange(repeat, dtype=np.int32)[:, None]
+        A = cs.Coo((A.row[None] + i * A.height).ravel(), (A.col[None] + i * A.width).ravel(),
+                   np.tile(A.val, repeat), A.height * repeat, A.width * repeat)
+    for owned in ([cs.coo2ell(A)] if fmt == "ell" else [cs.coo2sell(A, 32), cs.coo2sell(A, 700)]):
+        _run(ctx, oracle, A, owned, 0, x_offset=x_offset)
+
+
+@pytest.mark.parametrize("width", [1, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 24, 27])
+@pytest.mark.parametrize("rows", [100, (1 << 17) + 3])
+def test_ell_slot_groups(ctx, oracle, width, rows):
+    """Row widths around the groups of slots in flight, both group sizes, SELL
+    slices of different widths in one wave; dyadic inputs, exact sums."""
+    rng = np.random.default_rng(width)
+    lens = np.where(np.arange(rows) % 64 < 32, width, width // 2)
+    r = np.repeat(np.arange(rows), lens)
+    first = np.cumsum(lens) - lens
+    c = np.minimum(r, rows - 40) + (np.arange(r.size) - first[r])  # consecutive columns, distinct per row
+    A = cs.Coo(r.astype(np.int32), c.astype(np.int32), (rng.integers(-64, 65, r.size) / 64.0).astype(np.float32),
+               rows, rows)
+    _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
+    _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
+
 
 @pytest.mark.parametrize("name", ["rand_small", "rand_dyadic", "rand_long_rows"])
 @pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
