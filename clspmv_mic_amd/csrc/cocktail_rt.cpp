@@ -143,6 +143,21 @@ int launch_all(hipStream_t s, const clspmv_cocktail_kernels* k) {
 
 constexpr int kGraphPasses = 16;
 
+// Kernel launches of one pass.
+int launches(const clspmv_cocktail_kernels* k) {
+    int n = 0;
+    for (const clspmv_dmat* A : k->gpu->parts)
+        n += A->info.format == CLSPMV_FMT_COO || dmat_has_prepass(A) ? 2 : 1;
+    return n;
+}
+
+// Passes that fill no graph of kGraphPasses go out as plain launches while
+// they are at most this many: a graph launch of one pass costs the host
+// about 14 us, a kernel launch about 3.5 us (2D Laplacian 256^2, one
+// kernel: do_spmv(1) 30 us as a graph, 13.6 us plain; one DIA and one x-panel
+// part, three kernels: 64.6 against 58.6 us).
+constexpr int kPlainLaunches = 4;
+
 // Captures `passes` consecutive passes into *graph / *exec.
 int capture_passes(clspmv_cocktail_kernels* k, int passes, hipGraph_t* graph, hipGraphExec_t* exec) {
     hipStream_t s = k->ctx->stream;
@@ -321,7 +336,11 @@ int clspmv_do_spmv_async(clspmv_cocktail_kernels* k, int ntimes) {
     }
     int i = 0;
     for (; i + kGraphPasses <= ntimes; i += kGraphPasses) CLSPMV_HIP(hipGraphLaunch(k->exec_many, k->ctx->stream));
-    for (; i < ntimes; ++i) CLSPMV_HIP(hipGraphLaunch(k->exec, k->ctx->stream));
+    const bool plain = !overlaps(k) && launches(k) <= kPlainLaunches;
+    for (; i < ntimes; ++i) {
+        if (!plain) CLSPMV_HIP(hipGraphLaunch(k->exec, k->ctx->stream));
+        else if ((st = launch_all(k->ctx->stream, k))) return st;
+    }
     return CLSPMV_OK;
 }
 
