@@ -4,8 +4,7 @@
 // X is row-major (the k values of column c are X[c*k .. c*k+k)), so the
 // gather of one column brings every right-hand side's value in one or a few
 // 16-byte loads: a random column costs one cache line for all k products
-// instead of one line per product.  CSR runs over row blocks
-// (a work-group per block of short rows or per long row).  Y is
+// instead of one line per product.  Y is
 // column-major (ldy), so each right-hand side's y stays a contiguous
 // vector.  Matrix values may be FP32 or 16-bit (widened on load); sums are
 // FP32 in a fixed order, FP64 for CSR rows longer than kLongRowF64; no
@@ -273,24 +272,28 @@ __device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
     }
 }
 
-// One row longer than kAdaptiveNnz by the whole work-group: each lane
-// strides the row with 4 * L nonzeros in flight (a whole work-group round
-// covers kAdaptiveNnz of them), the four waves' sums are combined in a
-// fixed order through LDS, and Y[:, r] is updated once per right-hand side.
-template <int KB, class V, class Acc>
+// Work-group of the CSR kernel: with 512 threads a row over kWaveNnz entries has
+// 1,024 of them in flight (a 5,000-entry row sets the time of a small
+// power-law matrix: 60,000 rows, k = 4: 19.7 us against 27.3 with 256 threads).
+constexpr int kMultiThreads = 512;
+
+// One row longer than kWaveNnz by the whole work-group, always with four
+// lanes per entry, so that a column's sum does not depend on k: each lane
+// group strides the row with 8 entries in flight, the eight waves' sums are
+// combined in a fixed order through LDS, and Y[:, r] is updated once per
+// right-hand side.
+template <class V, class Acc>
 __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__ val,
                                                const int* __restrict__ col, int r, int j0, int j1,
                                                const float* __restrict__ X, int k, bool vec,
-                                               float* __restrict__ Y, int ldy, Acc (*part)[KB]) {
-    constexpr int Q = KB < 4 ? KB : 4;
-    constexpr int L = KB / Q;
+                                               float* __restrict__ Y, int ldy, Acc (*part)[launch::kMultiMax]) {
+    constexpr int Q = 4, L = launch::kMultiMax / Q;
     const int t = threadIdx.x;
     const int qb = (t % L) * Q;
     Acc a[Q];
 #pragma unroll
     for (int q = 0; q < Q; ++q) a[q] = 0;
-    csr_multi_run<Q, V, Acc, launch::kAdaptiveNnz * L / kBlock>(col, val, j0 + t / L, j1, kBlock / L, X, k, qb,
-                                                                vec, a);
+    csr_multi_run<Q, V, Acc, 8>(col, val, j0 + t / L, j1, kMultiThreads / L, X, k, qb, vec, a);
 #pragma unroll
     for (int q = 0; q < Q; ++q)
         for (int m = kWave >> 1; m >= L; m >>= 1) a[q] += __shfl_xor(a[q], m, kWave);
@@ -299,10 +302,10 @@ __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__
         for (int q = 0; q < Q; ++q) part[t / kWave][qb + q] = a[q];
     }
     __syncthreads();
-    if (t < KB && t < k) {
+    if (t < k) {
         Acc tot = 0;
 #pragma unroll
-        for (int w = 0; w < kBlock / kWave; ++w) tot += part[w][t];
+        for (int w = 0; w < kMultiThreads / kWave; ++w) tot += part[w][t];
         float* yp = Y + (size_t)t * ldy + r;
         if constexpr (sizeof(Acc) == sizeof(double))
             *yp = (float)((double)*yp + tot);  // one rounding of the whole row
@@ -311,133 +314,191 @@ __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__
     }
 }
 
-// CSR over row blocks (runs of at most kAdaptiveRows rows whose
-// nonzeros fit kAdaptiveNnz, or one longer row).  Each lane carries
-// Q = min(KB, 4) right-hand sides (one 16-byte gather of X per nonzero), and
-// L = KB / Q neighbouring lanes cover the k values of one nonzero.
+// The value of lane P of each aligned group of L lanes (L at most 4), by a
+// DPP quad permute.
+template <int L, int P, class T>
+__device__ __forceinline__ T group_lane(T v) {
+    if constexpr (L == 1) return v;
+    constexpr int ctrl = L == 4 ? P * 0x55 : P | P << 2 | (P + 2) << 4 | (P + 2) << 6;
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false));
+}
+
+// CSR: a wave per block of short rows (the wave kernel's blocks), L lanes per
+// entry with Q right-hand sides each; a work-group per longer row.
 //
-// A block of short rows is streamed: its nonzeros are cut into G = kBlock / L
-// equal consecutive chunks, one per lane group, whatever the rows' lengths
-// (a row-per-group split left short rows' groups idle beside one long row's
-// and put the gathers of a group's rows one after another).  A group loads
-// every column, value and X row of its chunk at once, then walks the chunk
-// in order: a row that starts and ends inside it is summed there and added
-// to Y; the part of a row that began in an earlier chunk goes to LDS (head),
-// and a row that continues past the chunk is finished, after a barrier, by
-// the group where it starts (its tail, then the later chunks' heads in
-// order).  Each row is thus summed in nonzero order with one break per chunk
-// boundary, in FP32, the same way every time.
+// A block is cut into units of 8 consecutive entries, whatever the rows'
+// lengths (a lane group per row would leave groups idle beside one long row
+// and put a row's gathers one after another).  A lane group loads its unit's
+// columns and values (each lane a part, handed round by DPP) and its 8 rows
+// of X at once, then walks the unit: a row that starts in it goes to the row's
+// place in LDS, the part of a row that began in an earlier unit to the unit's
+// `head`.  Then each row adds the heads of the later units it runs through, in
+// order, and Y is updated a column at a time, a lane per row.  A row's sum is
+// thus one FP32 chain per unit and the units in order: it depends on the
+// block cut alone, not on k.
 //
-// A long row: the whole work-group, the four waves' partial sums combined in
-// a fixed order through LDS, in FP64 for rows longer than kLongRowF64
-// (products exact, one rounding into y).
-template <int KB, class V>
-__global__ __launch_bounds__(kBlock) void csr_multi_kernel(
-    const int* __restrict__ blocks, const int* __restrict__ rp, const int* __restrict__ col,
-    const typename V::T* __restrict__ val, int k, const float* __restrict__ X, bool vec,
-    float* __restrict__ Y, int ldy) {
-    constexpr int Q = KB < 4 ? KB : 4;
-    constexpr int L = KB / Q;
-    constexpr int G = kBlock / L;                   // lane groups
-    constexpr int CM = launch::kAdaptiveNnz / G;    // nonzeros per group at most
-    static_assert(CM * G == launch::kAdaptiveNnz, "a block's nonzeros must split evenly over the groups");
-    __shared__ float part[kBlock / kWave][KB];
-    __shared__ double part64[kBlock / kWave][KB];
-    __shared__ int srp[launch::kAdaptiveRows + 1];  // the block's row starts, from its first nonzero
-    __shared__ float head[G][KB];                   // each chunk's part of a row begun earlier
-    const int b = blockIdx.x;
-    const int r0 = blocks[b], r1 = blocks[b + 1];
-    const int nrows = r1 - r0;
-    const int t = threadIdx.x;
-    const int qb = (t % L) * Q;
-    if (nrows == 1 && rp[r1] - rp[r0] > launch::kAdaptiveNnz) {
-        if (rp[r1] - rp[r0] > launch::kLongRowF64)
-            csr_multi_long<KB, V, double>(val, col, r0, rp[r0], rp[r1], X, k, vec, Y, ldy, part64);
+// What bounds it: random rows of X.  A 32- or 64-byte row costs a whole
+// 128-byte line once X outgrows the L2s: 72 / 62 G rows/s at 19 / 32 MB of X
+// (k = 8), 58 / 54 G at 38 / 64 MB (k = 16) when nothing else runs.  Before,
+// a work-group of 1024 entries waited at two barriers, each finished row was
+// added to Y where it ended (a load and a store of one float per right-hand
+// side, waited for) and k not a multiple of 4 gathered single floats.
+// Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 156 / 184 us; 1 M
+// rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 284 / 273 / 311 us (50 G rows/s);
+// 27-point stencil 64^3, k = 8: 74 -> 31 us.
+constexpr int kUnit = 8;
+
+template <int Q, int L, class V>
+__global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
+    int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
+    const int* __restrict__ rp, const int* __restrict__ col, const typename V::T* __restrict__ val, int k,
+    const float* __restrict__ X, bool vec, float* __restrict__ Y, int ldy) {
+    typedef typename V::T T;
+    constexpr int QP = Q == 3 ? 4 : Q;              // LDS floats per piece
+    constexpr int KB = QP * L;                      // and per row or unit
+    constexpr int AS = KB == 1 ? 1 : KB + QP;       // LDS stride of the rows
+    constexpr int G = kWave / L;                    // lane groups of a wave
+    constexpr int NU = launch::kWaveNnz / kUnit;    // units of a block at most
+    constexpr int NE = kUnit / L;                   // entries a lane loads
+    constexpr int kWaves = kMultiThreads / kWave;
+    typedef VecOf<float, Q> XV;
+    typedef VecOf<float, QP> PV;
+    struct WaveLds {
+        float acc[kWave * AS];
+        float head[NU * KB];
+        int rp[kWave + 4];
+    };
+    __shared__ __attribute__((aligned(16))) union {
+        WaveLds w[kWaves];
+        float part[kWaves][launch::kMultiMax];
+        double part64[kWaves][launch::kMultiMax];
+    } lds;
+    if ((int)blockIdx.x < nlong) {  // the longest work first
+        const int r = longs[blockIdx.x], j0 = rp[r], j1 = rp[r + 1];
+        if (j1 - j0 > launch::kLongRowF64)
+            csr_multi_long<V, double>(val, col, r, j0, j1, X, k, vec, Y, ldy, lds.part64);
         else
-            csr_multi_long<KB, V, float>(val, col, r0, rp[r0], rp[r1], X, k, vec, Y, ldy, part);
+            csr_multi_long<V, float>(val, col, r, j0, j1, X, k, vec, Y, ldy, lds.part);
         return;
     }
-    const int s = rp[r0];
-    const int n = rp[r1] - s;  // at most kAdaptiveNnz
-    for (int i = t; i <= nrows; i += kBlock) srp[i] = rp[r0 + i] - s;
-    __syncthreads();
-    if (n == 0) return;  // only empty rows (the whole work-group)
-    const int gi = t / L;
-    const int C = (n + G - 1) / G;  // <= CM
-    const int c0 = min(n, gi * C), c1 = min(n, c0 + C);
-    // Every load of the chunk before its first product (slots past the
-    // chunk read nonzero s and are never used).
-    int cc[CM];
-    float vv[CM], xv[CM][Q];
-#pragma unroll
-    for (int u = 0; u < CM; ++u) {
-        const int j = c0 + u < c1 ? s + c0 + u : s;
-        cc[u] = ld_stream(col + j);
-        vv[u] = V::ld(val + j);
-    }
-#pragma unroll
-    for (int u = 0; u < CM; ++u) load_xq<Q>(X, cc[u], k, qb, vec, xv[u]);
-    float acc[Q];
-#pragma unroll
-    for (int q = 0; q < Q; ++q) acc[q] = 0.0f;
-    auto add_y = [&](int r) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q)
-            if (qb + q < k) Y[(size_t)(qb + q) * ldy + r0 + r] += acc[q];
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int b = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x - nlong, gridDim.x - nlong) * kWaves + wave);
+    if (b >= nblk) return;  // the whole wave
+    const int4 B = blk[b];  // {first row, rows, first entry, entries}
+    const int r0 = B.x, nrows = B.y, s = B.z, n = B.w;
+    WaveLds& W = lds.w[wave];
+    const int gi = lane / L, p = lane % L;
+    const int q0 = p * Q, qs = min(q0, k - Q);  // the last piece ends at k
+    const bool act = q0 < k;
+    const float* Xq = X + qs;
+    typedef VecOf<int, NE> CV;
+    typedef VecOf<T, NE> TV;
+    typename CV::type cn;
+    typename TV::type vn;
+    auto load = [&](int u) {  // unit u's columns and values; the arrays are padded past the last entry
+        const int at = u * kUnit + p * NE;
+        cn = __builtin_nontemporal_load(reinterpret_cast<const typename UVec<int, NE>::type*>(col + s + at));
+        vn = __builtin_nontemporal_load(reinterpret_cast<const typename UVec<T, NE>::type*>(val + s + at));
     };
-    int r = 0, rend = 0;
-    bool in_head = false;  // the current row began before this chunk
-    if (c0 < c1) {
-        // The row holding nonzero c0: the last row starting at or before it
-        // (empty rows before it start at the same place and are passed).
-        int lo = 0, hi = nrows - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (srp[mid] <= c0) lo = mid;
-            else hi = mid - 1;
-        }
-        r = lo;
-        rend = srp[r + 1];
-        in_head = srp[r] < c0;
+    const int nunits = (n + kUnit - 1) / kUnit;
+    if (nunits > 0) load(min(gi, nunits - 1));
+    const int myrp = rp[r0 + min(lane, nrows)] - s;
+    W.rp[lane] = myrp;  // entries past nrows repeat the end
+    if (lane == 0) W.rp[kWave] = n;
+    wave_lds_order();
+    for (int u0 = 0; u0 < nunits; u0 += G) {
+        const int u = u0 + gi;
+        int c[kUnit];
+        float v[kUnit];
 #pragma unroll
-        for (int u = 0; u < CM; ++u) {
-            const int j = c0 + u;
-            if (j < c1) {
-                if (j >= rend) {  // row r ended inside the chunk
-                    if (in_head) {
-#pragma unroll
-                        for (int q = 0; q < Q; ++q) head[gi][qb + q] = acc[q];
-                    } else {
-                        add_y(r);
-                    }
-                    in_head = false;
-                    do {
-                        ++r;
-                        rend = srp[r + 1];
-                    } while (j >= rend);  // empty rows
-#pragma unroll
-                    for (int q = 0; q < Q; ++q) acc[q] = 0.0f;
-                }
-#pragma unroll
-                for (int q = 0; q < Q; ++q) acc[q] = fmaf(vv[u], xv[u][q], acc[q]);
+        for (int e = 0; e < NE; ++e) {
+            const int ce = CV::get(cn, e);
+            const float ve = V::cvt(TV::get(vn, e));
+            c[e] = group_lane<L, 0>(ce);
+            v[e] = group_lane<L, 0>(ve);
+            if constexpr (L >= 2) {
+                c[NE + e] = group_lane<L, 1>(ce);
+                v[NE + e] = group_lane<L, 1>(ve);
+            }
+            if constexpr (L == 4) {
+                c[2 * NE + e] = group_lane<L, 2>(ce);
+                v[2 * NE + e] = group_lane<L, 2>(ve);
+                c[3 * NE + e] = group_lane<L, 3>(ce);
+                v[3 * NE + e] = group_lane<L, 3>(ve);
             }
         }
-        if (in_head) {
+        typename XV::type xv[kUnit];
+        const bool on = u < nunits && act;
+        if (on) {
 #pragma unroll
-            for (int q = 0; q < Q; ++q) head[gi][qb + q] = acc[q];
-        } else if (rend <= c1) {
-            add_y(r);
+            for (int e = 0; e < kUnit; ++e)
+                xv[e] = *reinterpret_cast<const typename UVec<float, Q>::type*>(Xq + (size_t)c[e] * k);
+        }
+        if (u0 + G < nunits) load(min(u + G, nunits - 1));
+        if (on) {
+            const int j0 = u * kUnit, j1 = min(n, j0 + kUnit);
+            // The row of the unit's first entry: the last one starting at or
+            // before it.
+            int r = 0;
+#pragma unroll
+            for (int m = kWave / 2; m >= 1; m >>= 1)
+                if (r + m < nrows && W.rp[r + m] <= j0) r += m;
+            int rend = W.rp[r + 1];
+            bool head = W.rp[r] < j0;
+            float a[QP];
+#pragma unroll
+            for (int q = 0; q < QP; ++q) a[q] = 0.0f;
+            auto flush = [&]() {
+                float* to = head ? W.head + u * KB + p * QP : W.acc + r * AS + p * QP;
+                typename PV::type t;
+#pragma unroll
+                for (int q = 0; q < QP; ++q) PV::set(t, q, a[q]);
+                *reinterpret_cast<typename PV::type*>(to) = t;
+            };
+#pragma unroll
+            for (int e = 0; e < kUnit; ++e) {
+                const int j = j0 + e;
+                if (j < j1) {
+                    if (j >= rend) {  // row r ended in the unit
+                        flush();
+                        head = false;
+                        do rend = W.rp[++r + 1];
+                        while (j >= rend);  // empty rows
+#pragma unroll
+                        for (int q = 0; q < QP; ++q) a[q] = 0.0f;
+                    }
+#pragma unroll
+                    for (int q = 0; q < Q; ++q) a[q] = fmaf(v[e], XV::get(xv[e], q), a[q]);
+                }
+            }
+            flush();
         }
     }
-    __syncthreads();
-    // The row this chunk ends inside of and began: its tail, then the heads
-    // of the later chunks it runs through, in order.
-    if (c0 < c1 && !in_head && rend > c1) {
-        const int last = (rend - 1) / C;  // the chunk holding the row's last nonzero
-        for (int g2 = gi + 1; g2 <= last; ++g2)
+    wave_lds_order();
+    // Rows that run through several units add the later ones' heads.
+    for (int rr = gi; rr < nrows; rr += G) {
+        const int e0 = W.rp[rr], e1 = W.rp[rr + 1];
+        const int ua = e0 / kUnit, uz = (e1 - 1) / kUnit;
+        if (e1 == e0 || uz == ua || !act) continue;
+        float* at = W.acc + rr * AS + p * QP;
+        typename PV::type t = *reinterpret_cast<typename PV::type*>(at);
+        for (int u = ua + 1; u <= uz; ++u)
+            t += *reinterpret_cast<const typename PV::type*>(W.head + u * KB + p * QP);
+        *reinterpret_cast<typename PV::type*>(at) = t;
+    }
+    wave_lds_order();
+    if (lane < nrows && W.rp[lane + 1] > W.rp[lane]) {  // empty rows leave Y as it is
+        float* yp = Y + r0 + lane;
+        const float* ap = W.acc + lane * AS;
+        const int full = (k - 1) / Q * Q, shift = full + Q - k;  // columns before the last piece, its overlap
+        constexpr int KM = Q * L;
+        float y[KM];
 #pragma unroll
-            for (int q = 0; q < Q; ++q) acc[q] += head[g2][qb + q];
-        add_y(r);
+        for (int q = 0; q < KM; ++q)
+            if (q < k) y[q] = yp[(size_t)q * ldy];
+#pragma unroll
+        for (int q = 0; q < KM; ++q)
+            if (q < k) yp[(size_t)q * ldy] = y[q] + ap[q < full ? q : q + shift];
     }
 }
 
@@ -483,34 +544,29 @@ hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int nseg, int
 #undef CLSPMV_DIA_MULTI
 }
 
-template <int KB, class V>
-hipError_t csr_multi_kb(hipStream_t s, int nblocks, const int* blocks, const int* rp, const int* col,
-                        const void* val, int k, const float* X, float* Y, int ldy) {
-    constexpr int Q = KB < 4 ? KB : 4;
-    const bool vec = Q > 1 && k % Q == 0 && ((uintptr_t)X % (Q * sizeof(float))) == 0;
-    hipLaunchKernelGGL((csr_multi_kernel<KB, V>), dim3(nblocks), dim3(kBlock), 0, s, blocks, rp, col,
-                       static_cast<const typename V::T*>(val), k, X, vec, Y, ldy);
+template <int Q, int L, class V>
+hipError_t csr_multi_tile(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
+                          int k, const float* X, float* Y, int ldy) {
+    const bool vec = k % 4 == 0 && ((uintptr_t)X % 16) == 0;  // long rows: aligned 16-byte pieces
+    hipLaunchKernelGGL((csr_multi_kernel<Q, L, V>), dim3(W.nlong + ceil_div(W.nblk, kMultiThreads / kWave)),
+                       dim3(kMultiThreads), 0, s,
+                       W.nlong, W.longs, W.nblk, W.blk, rp, col, static_cast<const typename V::T*>(val), k, X, vec, Y,
+                       ldy);
     return hipGetLastError();
 }
 
 template <class V>
-hipError_t csr_multi_v(hipStream_t s, int nblocks, const int* blocks, const int* rp, const int* col,
-                       const void* val, int k, const float* X, float* Y, int ldy, int kb) {
-    if (kb > 0) {  // a fixed width: the summation order of each right-hand side does not depend on k
-        switch (kb) {
-            case 1: return csr_multi_kb<1, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-            case 2: return csr_multi_kb<2, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-            case 4: return csr_multi_kb<4, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-            case 8: return csr_multi_kb<8, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-            case 16: return csr_multi_kb<16, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-            default: return hipErrorInvalidValue;
-        }
+hipError_t csr_multi_v(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val, int k,
+                       const float* X, float* Y, int ldy) {
+    switch (k) {
+        case 1: return csr_multi_tile<1, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
+        case 2: return csr_multi_tile<2, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
+        case 3: return csr_multi_tile<3, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
+        case 4: return csr_multi_tile<4, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
+        default: break;
     }
-    if (k <= 1) return csr_multi_kb<1, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-    if (k <= 2) return csr_multi_kb<2, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-    if (k <= 4) return csr_multi_kb<4, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-    if (k <= 8) return csr_multi_kb<8, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
-    return csr_multi_kb<16, V>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy);
+    return k <= 8 ? csr_multi_tile<4, 2, V>(s, W, rp, col, val, k, X, Y, ldy)
+                  : csr_multi_tile<4, 4, V>(s, W, rp, col, val, k, X, Y, ldy);
 }
 
 }  // namespace
@@ -529,14 +585,14 @@ hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w
     }
 }
 
-hipError_t csr_multi(hipStream_t s, int nblocks, const int* blocks, const int* rp, const int* col,
-                     int dtype, const void* val, int k, const float* X, float* Y, int ldy, int kb) {
-    if (nblocks <= 0 || k <= 0) return hipSuccess;
-    if (k > kMultiMax || (kb > 0 && k > kb)) return hipErrorInvalidValue;
+hipError_t csr_multi(hipStream_t s, const CsrWave& W, const int* rp, const int* col,
+                     int dtype, const void* val, int k, const float* X, float* Y, int ldy) {
+    if (W.nblk + W.nlong <= 0 || k <= 0) return hipSuccess;
+    if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return csr_multi_v<ValF32>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy, kb);
-        case 1: return csr_multi_v<ValBF16>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy, kb);
-        case 2: return csr_multi_v<ValF16>(s, nblocks, blocks, rp, col, val, k, X, Y, ldy, kb);
+        case 0: return csr_multi_v<ValF32>(s, W, rp, col, val, k, X, Y, ldy);
+        case 1: return csr_multi_v<ValBF16>(s, W, rp, col, val, k, X, Y, ldy);
+        case 2: return csr_multi_v<ValF16>(s, W, rp, col, val, k, X, Y, ldy);
         default: return hipErrorInvalidValue;
     }
 }

@@ -12,7 +12,7 @@ namespace launch {
 // Vector kernel: `lanes` (power of two, 1..64) lanes cooperate on one row.
 hipError_t csr_vector(hipStream_t s, int rows, int lanes, const int* rp,
                       const int* col, const float* val, const float* x, float* y);
-// Row blocks of the multi-vector and verification kernels: a block is a run
+// Row blocks of the verification kernel: a block is a run
 // of at most kAdaptiveRows rows whose entries fit kAdaptiveNnz, or one
 // longer row.
 constexpr int kAdaptiveNnz = 1024;
@@ -166,12 +166,10 @@ constexpr int kMultiMax = 16;
 constexpr int kDiaRun = 3;
 hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy);
-// CSR over the row blocks above.  kb > 0 runs
-// the kernel built for kb right-hand sides (k <= kb; 1, 2, 4, 8 or 16)
-// whatever k is, so that each right-hand side's summation order stays that
-// of kb; kb = 0 picks the smallest width that holds k.
-hipError_t csr_multi(hipStream_t s, int nblocks, const int* blocks, const int* rp, const int* col,
-                     int dtype, const void* val, int k, const float* X, float* Y, int ldy, int kb = 0);
+// CSR over the wave kernel's blocks and long rows.  A right-hand side's
+// result does not depend on k, nor does DIA's.
+hipError_t csr_multi(hipStream_t s, const CsrWave& W, const int* rp, const int* col,
+                     int dtype, const void* val, int k, const float* X, float* Y, int ldy);
 
 // ---- mixed-precision 4x4-block SpMM (MFMA) -------------------------------------
 // Y[:, 0:k] += A X[:, 0:k]; A in slices of kSpmmSlice block rows: sptr[s] is

@@ -60,7 +60,7 @@ clspmv_dmat* new_dmat(int format, const clspmv_matinfo& mi) {
     return m;
 }
 
-// Row blocks of the multi-vector and verification CSR kernels: a block is a maximal run of at most
+// Row blocks of the verification kernel: a block is a maximal run of at most
 // kAdaptiveRows rows whose entries fit kAdaptiveNnz, or a single longer row.
 std::vector<int> csr_row_blocks(const int* rp, int rows) {
     std::vector<int> b{0};
@@ -98,17 +98,33 @@ std::vector<int4> dia_segments(const int* off, int ndiag, int rows, int cols, in
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
-// x windows (launch::CsrWave, launch::EllWindows) for `groups` work-groups,
-// where neighbouring rows' columns are near each other but scattered over the
-// 128-byte lines of x: a gather instruction then touches many lines and L1's
-// tag rate bounds the kernel, while the window costs one coalesced pass.
-// sample(g, cols) gives the 64 columns of one gather instruction of group g
-// (false: none); they are looked at on up to 256 groups and must touch 24
-// lines on average.  range(g, lo, hi) widens [*lo, *hi] by the group's columns; a
-// group wider than `limit` gathers from memory, and with more than one in
-// ten of those the matrix gets no windows.
-template <class Sample, class Range>
-int add_windows(clspmv_dmat* d, size_t groups, int limit, Sample&& sample, Range&& range) {
+// The columns of a run of entries: [lo, hi], empty as hi < lo.
+struct ColRange {
+    int lo = INT_MAX, hi = -1;
+    void widen(const int* c, size_t n) {
+        int l = lo, h = hi;
+        for (size_t i = 0; i < n; ++i) {
+            l = std::min(l, c[i]);
+            h = std::max(h, c[i]);
+        }
+        lo = l;
+        hi = h;
+    }
+    bool within(int cols) const { return lo >= 0 && hi < cols; }
+};
+
+// x windows (launch::CsrWave, launch::EllWindows) for the work-groups whose
+// columns are `range`, where neighbouring rows' columns are near each other
+// but scattered over the 128-byte lines of x: a gather instruction then
+// touches many lines and L1's tag rate bounds the kernel, while the window
+// costs one coalesced pass.  sample(g, cols) gives the 64 columns of one gather
+// instruction of group g (false: none); they are looked at on up to 256 groups
+// and must touch 24 lines on average.  A group wider than `limit` gathers
+// from memory, and with more than one in ten of those the matrix gets no
+// windows.
+template <class Sample>
+int add_windows(clspmv_dmat* d, const std::vector<ColRange>& range, int limit, Sample&& sample) {
+    const size_t groups = range.size();
     long long lines = 0, samples = 0;
     for (size_t g = 0, step = std::max<size_t>(1, groups / 256); g < groups; g += step) {
         int line[64];
@@ -123,14 +139,12 @@ int add_windows(clspmv_dmat* d, size_t groups, int limit, Sample&& sample, Range
     size_t wide = 0;
     int wmax = 0;
     for (size_t g = 0; g < groups; ++g) {
-        int lo = INT_MAX, hi = -1;
-        range(g, &lo, &hi);
-        const int n = hi < 0 ? 0 : hi - lo + 1;
-        win[g] = n > 0 && n <= limit ? make_int2(lo, n) : make_int2(0, 0);
+        const int n = range[g].hi < 0 ? 0 : range[g].hi - range[g].lo + 1;
+        win[g] = n > 0 && n <= limit ? make_int2(range[g].lo, n) : make_int2(0, 0);
         wide += n > limit;
         wmax = std::max(wmax, win[g].y);
-        if (wide * 10 > groups) return CLSPMV_OK;
     }
+    if (wide * 10 > groups) return CLSPMV_OK;
     d->wwin_max = round_up(wmax, 4);
     return upload_array(d, win.data(), win.size(), &d->wwin);
 }
@@ -154,25 +168,22 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
     d->nwlong = (int)longs.size();
     int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
     if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
-    if (st || !col || blk.empty()) return st;
+    if (st || !col) return st;
     // x windows where they pay: mesh of 500,009 rows (a gather instruction
     // touches 52 lines, windows of 4.5 K columns) 22 us against 32; 27-point
     // stencil 47^3 (16 lines, 4.6 K columns) 10.2 against 8.0 us.
     constexpr int W = launch::kCsrWaves;
-    return add_windows(
-        d, (blk.size() + W - 1) / W, launch::kCsrWinMax,
-        [&](size_t g, int* line) {
-            const int4 b = blk[g * W];
-            for (int i = 0; i < 64 && b.w >= 256; ++i) line[i] = col[b.z + 4 * i];
-            return b.w >= 256;
-        },
-        [&](size_t g, int* lo, int* hi) {
-            for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
-                for (int k = blk[b].z; k < blk[b].z + blk[b].w; ++k) {
-                    *lo = std::min(*lo, col[k]);
-                    *hi = std::max(*hi, col[k]);
-                }
-        });
+    std::vector<ColRange> range((blk.size() + W - 1) / W);
+    for (size_t b = 0; b < blk.size(); ++b) range[b / W].widen(col + blk[b].z, blk[b].w);
+    ColRange all;  // of the long rows, then of all entries
+    for (int r : longs) all.widen(col + rp[r], rp[r + 1] - rp[r]);
+    for (const ColRange& g : range) all.lo = std::min(all.lo, g.lo), all.hi = std::max(all.hi, g.hi);
+    if (rp[rows] > 0 && !all.within(d->info.cols)) return check_cols(col, rp[rows], d->info.cols, 1, "csr");
+    return add_windows(d, range, launch::kCsrWinMax, [&](size_t g, int* line) {
+        const int4 b = blk[g * W];
+        for (int i = 0; i < 64 && b.w >= 256; ++i) line[i] = col[b.z + 4 * i];
+        return b.w >= 256;
+    });
 }
 
 int auto_method(const clspmv_dmat* A) {
@@ -221,6 +232,10 @@ int dmat_prepass(hipStream_t s, const clspmv_dmat* A, const float* x, const clsp
 }
 
 namespace {
+launch::CsrWave csr_wave_of(const clspmv_dmat* A) {
+    return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->wwin, A->wwin_max};
+}
+
 int resolve_method(const clspmv_dmat* A, int* method) {
     if (*method == CLSPMV_METHOD_AUTO) *method = auto_method(A);
     if (*method < 0 || *method >= clspmv_method_count(A->info.format))
@@ -261,9 +276,8 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
             if (method == 0 && !A->dtype)
                 e = launch::csr_vector(s, I.rows, A->lanes, A->rp, A->col, A->val, x, y);
             else
-                e = launch::csr_wave(
-                    s, launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->wwin, A->wwin_max}, A->rp, A->col,
-                    A->dtype, A->dtype ? (const void*)A->lpval : (const void*)A->val, x, y);
+                e = launch::csr_wave(s, csr_wave_of(A), A->rp, A->col, A->dtype,
+                                     A->dtype ? (const void*)A->lpval : (const void*)A->val, x, y);
             break;
         case CLSPMV_FMT_COO:
             e = launch::coo_segreduce(s, I.nnz, A->row, A->col, A->val, x, y,
@@ -335,15 +349,15 @@ bool has_multi(const clspmv_dmat* A) {
     return A->info.format == CLSPMV_FMT_DIA || (A->info.format == CLSPMV_FMT_CSR && A->plain);
 }
 
-int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy, int kb) {
+int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy) {
     const clspmv_dmat_info& I = A->info;
     hipError_t e;
     if (I.format == CLSPMV_FMT_DIA) {
         e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, A->ndseg, A->seg_w, A->dseg, A->dtype,
                               A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy);
     } else if (I.format == CLSPMV_FMT_CSR && A->plain) {
-        e = launch::csr_multi(s, A->nblocks, A->blocks, A->rp, A->col, A->dtype,
-                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy, kb);
+        e = launch::csr_multi(s, csr_wave_of(A), A->rp, A->col, A->dtype,
+                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy);
     } else {
         return fail(CLSPMV_ERR_UNSUPPORTED, "multi-vector SpMV exists for DIA and CSR (own arrays) only");
     }
@@ -559,11 +573,11 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
         if (len < 0) UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "CSR row pointer decreases at %d", r));
         max_row = std::max(max_row, len);
     }
-    UPLOAD_CHECK(check_cols(m->csr_col_id, nnz, m->matinfo.width, 1, "csr"));
     d->info.stored = nnz;
     d->max_row = max_row;
     double avg = rows ? (double)nnz / rows : 0.0;
     d->lanes = pow2_at_least((int)std::ceil(avg), 64);
+    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, m->csr_col_id));  // checks the columns
     UPLOAD_CHECK(upload_array(d, m->csr_row_ptr, (size_t)rows + 1, &d->rp));
     UPLOAD_CHECK(upload_padded(d, m->csr_col_id, nnz, launch::kWaveNnz, &d->col));
     if (o.dtype != CLSPMV_DT_F32) {
@@ -575,7 +589,6 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     } else {
         UPLOAD_CHECK(upload_padded(d, m->csr_data, nnz, launch::kWaveNnz, &d->val));
     }
-    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, m->csr_col_id));
     std::vector<int> blocks = csr_row_blocks(m->csr_row_ptr, rows);
     d->nblocks = (int)blocks.size() - 1;
     UPLOAD_CHECK(upload_array(d, blocks.data(), blocks.size(), &d->blocks));
@@ -631,30 +644,27 @@ int clspmv_upload_ell(clspmv_ctx* ctx, const clspmv_ell_matrix* m, clspmv_dmat**
     const size_t total = (size_t)m->ell_height_aligned * m->ell_num;
     if (m->ell_height_aligned < m->matinfo.height || m->ell_num < 0)
         UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "malformed ELL matrix"));
-    UPLOAD_CHECK(check_cols(m->ell_col_id, total, std::max(m->matinfo.width, 1), 1, "ell"));
+    const int rows = m->matinfo.height, hal = m->ell_height_aligned, cols = std::max(m->matinfo.width, 1);
+    constexpr int R = launch::kEllRows;
+    std::vector<ColRange> range((rows + R - 1) / R);
+    ColRange all;  // of the padding rows, then of all slots
+    for (int s = 0; s < m->ell_num; ++s) {
+        const int* c = m->ell_col_id + (size_t)s * hal;
+        for (int r = 0; r < rows; r += R) range[r / R].widen(c + r, std::min(R, rows - r));
+        all.widen(c + rows, hal - rows);
+    }
+    for (const ColRange& g : range) all.lo = std::min(all.lo, g.lo), all.hi = std::max(all.hi, g.hi);
+    if (total > 0 && !all.within(cols)) UPLOAD_CHECK(check_cols(m->ell_col_id, total, cols, 1, "ell"));
     d->hal = m->ell_height_aligned;
     d->ellnum = m->ell_num;
     d->info.stored = (long long)total;
     UPLOAD_CHECK(upload_array(d, m->ell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->ell_data, total, &d->val));
-    if (m->ell_num > 0) {
-        const int rows = m->matinfo.height, hal = m->ell_height_aligned;
-        constexpr int R = launch::kEllRows;
-        UPLOAD_CHECK(add_windows(
-            d, (rows + R - 1) / R, launch::kEllWinMax,
-            [&](size_t g, int* line) {
-                if ((int)g * R + 64 > rows) return false;
-                std::copy_n(m->ell_col_id + (size_t)(m->ell_num / 2) * hal + g * R, 64, line);
-                return true;
-            },
-            [&](size_t g, int* lo, int* hi) {
-                for (int s = 0; s < m->ell_num; ++s)
-                    for (int r = (int)g * R; r < std::min(rows, ((int)g + 1) * R); ++r) {
-                        *lo = std::min(*lo, m->ell_col_id[(size_t)s * hal + r]);
-                        *hi = std::max(*hi, m->ell_col_id[(size_t)s * hal + r]);
-                    }
-            }));
-    }
+    UPLOAD_CHECK(add_windows(d, range, launch::kEllWinMax, [&](size_t g, int* line) {
+        if (m->ell_num == 0 || (int)g * R + 64 > rows) return false;
+        std::copy_n(m->ell_col_id + (size_t)(m->ell_num / 2) * hal + g * R, 64, line);
+        return true;
+    }));
     *out = d;
     return CLSPMV_OK;
 }
@@ -662,47 +672,45 @@ int clspmv_upload_ell(clspmv_ctx* ctx, const clspmv_ell_matrix* m, clspmv_dmat**
 int clspmv_upload_sell(clspmv_ctx* ctx, const clspmv_sell_matrix* m, clspmv_dmat** out) {
     UPLOAD_PROLOGUE(m, CLSPMV_FMT_SELL)
     const int h = (int)m->sell_slice_height, ns = m->sell_slice_num;
-    if (h <= 0 || ns < 0 || (long long)ns * h < m->matinfo.height || !m->sell_slice_ptr)
+    if (h <= 0 || ns < 0 || (long long)ns * h < m->matinfo.height || !m->sell_slice_ptr || m->sell_slice_ptr[0] < 0)
         UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "malformed SELL matrix"));
     for (int s = 0; s < ns; ++s) {
         int w = m->sell_slice_ptr[s + 1] - m->sell_slice_ptr[s];
         if (w < 0 || w % h) UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "SELL slice %d size %d", s, w));
     }
     const size_t total = (size_t)m->sell_slice_ptr[ns];
-    UPLOAD_CHECK(check_cols(m->sell_col_id, total, std::max(m->matinfo.width, 1), 1, "sell"));
+    // Column ranges of the kernel's work-groups; a slice that reaches into
+    // several counts for each.
+    const int rows = m->matinfo.height, cols = std::max(m->matinfo.width, 1);
+    const int* sp = m->sell_slice_ptr;
+    constexpr int R = launch::kEllRows;
+    std::vector<ColRange> range((rows + R - 1) / R);
+    ColRange all;
+    all.widen(m->sell_col_id, sp[0]);
+    for (int s = 0; s < ns; ++s) {
+        ColRange one;
+        one.widen(m->sell_col_id + sp[s], sp[s + 1] - sp[s]);
+        all.lo = std::min(all.lo, one.lo), all.hi = std::max(all.hi, one.hi);
+        const long long r0 = (long long)s * h, r1 = std::min<long long>(rows, r0 + h);
+        for (long long g = r0 / R; g * R < r1; ++g) {
+            range[g].lo = std::min(range[g].lo, one.lo);
+            range[g].hi = std::max(range[g].hi, one.hi);
+        }
+    }
+    if (total > 0 && !all.within(cols)) UPLOAD_CHECK(check_cols(m->sell_col_id, total, cols, 1, "sell"));
     d->info.slice_height = h;
     d->info.stored = (long long)total;
     UPLOAD_CHECK(upload_array(d, m->sell_slice_ptr, (size_t)ns + 1, &d->sptr));
     UPLOAD_CHECK(upload_array(d, m->sell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->sell_data, total, &d->val));
-    {
-        const int rows = m->matinfo.height;
-        const int* sp = m->sell_slice_ptr;
-        constexpr int R = launch::kEllRows;
-        UPLOAD_CHECK(add_windows(
-            d, (rows + R - 1) / R, launch::kEllWinMax,
-            [&](size_t g, int* line) {
-                // The middle slot of each of 64 rows.
-                for (int i = 0; i < 64; ++i) {
-                    const int r = (int)g * R + i, s = r / h;
-                    if (r >= rows || sp[s + 1] == sp[s]) return false;
-                    line[i] = m->sell_col_id[sp[s] + (sp[s + 1] - sp[s]) / h / 2 * h + r % h];
-                }
-                return true;
-            },
-            [&](size_t g, int* lo, int* hi) {
-                const int r1 = std::min(rows, ((int)g + 1) * R);
-                for (int r = (int)g * R; r < r1;) {  // the group's rows of each slice
-                    const int s = r / h, i0 = r % h, i1 = std::min(h, i0 + r1 - r);
-                    for (int k = sp[s]; k < sp[s + 1]; k += h)
-                        for (int i = i0; i < i1; ++i) {
-                            *lo = std::min(*lo, m->sell_col_id[k + i]);
-                            *hi = std::max(*hi, m->sell_col_id[k + i]);
-                        }
-                    r += i1 - i0;
-                }
-            }));
-    }
+    UPLOAD_CHECK(add_windows(d, range, launch::kEllWinMax, [&](size_t g, int* line) {
+        for (int i = 0; i < 64; ++i) {  // the middle slot of each of 64 rows
+            const int r = (int)g * R + i, s = r / h;
+            if (r >= rows || sp[s + 1] == sp[s]) return false;
+            line[i] = m->sell_col_id[sp[s] + (sp[s + 1] - sp[s]) / h / 2 * h + r % h];
+        }
+        return true;
+    }));
     *out = d;
     return CLSPMV_OK;
 }

@@ -21,9 +21,9 @@ struct clspmv_dmat {
     std::vector<std::pair<void*, size_t>> bufs;  // device allocations owned by the matrix
 
     // CSR: rp/col/val (col and val padded by launch::kWaveNnz entries);
-    // row blocks of the multi-vector and verification kernels; blocks, long
-    // rows and x windows of the wave kernel (launch::CsrWave); lanes per row
-    // of the vector kernel.
+    // row blocks of the verification kernel; blocks, long rows and x windows
+    // of the wave and multi-vector kernels (launch::CsrWave); lanes per row of
+    // the vector kernel.
     int* rp = nullptr;
     int* col = nullptr;
     float* val = nullptr;
@@ -206,12 +206,10 @@ int dmat_launch_rest(hipStream_t stream, const clspmv_dmat* A, int method,
                      const float* x, float* y);
 
 // Multi-vector SpMV (DIA, CSR with its own arrays): Y[:, q] += A X[:, q],
-// X row-major, Y column-major; no argument checks.  kb > 0: CSR runs the
-// kernel built for kb right-hand sides whatever k is (launch::csr_multi);
-// each right-hand side's result then does not depend on k.  DIA's never
-// does.
+// X row-major, Y column-major; no argument checks.  Each right-hand side's
+// result does not depend on k.
 bool has_multi(const clspmv_dmat* A);
-int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy, int kb = 0);
+int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy);
 
 // Method chosen for CLSPMV_METHOD_AUTO.
 int auto_method(const clspmv_dmat* A);

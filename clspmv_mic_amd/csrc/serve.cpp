@@ -16,8 +16,8 @@
 // Bit-for-bit independence from the mix: the kernels of a matrix are fixed
 // at registration, and in each of them a column's arithmetic does not
 // depend on the other columns: DIA's multi-vector kernel sums each column
-// alone in diagonal order; CSR's runs at the fixed 16-column width
-// (launch::csr_multi with kb = 16); the SpMM's MFMA output columns depend
+// alone in diagonal order; CSR's in units of 8 entries fixed by the matrix's
+// row blocks; the SpMM's MFMA output columns depend
 // only on their own X column, in block order; per-column SpMVs are
 // independent launches.
 
@@ -271,11 +271,10 @@ int enqueue_pass(hipStream_t s, const SMatrix& M, int K) {
     hipLaunchKernelGGL(zero_kernel, dim3(grid_for(ny)), dim3(256), 0, s, ny, M.Y);
     CLSPMV_HIP(hipGetLastError());
     if (M.path == kMulti) {
-        const int kb = M.A->info.format == CLSPMV_FMT_CSR ? kMultiCols : 0;
         for (int c = 0; c * kMultiCols < K; ++c) {
             const int kc = std::min(kMultiCols, K - c * kMultiCols);
             int st = multi_launch(s, M.A, kc, static_cast<const float*>(M.X) + (size_t)c * kMultiCols * M.ldx,
-                                  M.Y + (size_t)c * kMultiCols * M.ldy, M.ldy, kb);
+                                  M.Y + (size_t)c * kMultiCols * M.ldy, M.ldy);
             if (st) return st;
         }
         return CLSPMV_OK;

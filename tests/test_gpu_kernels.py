@@ -490,6 +490,38 @@ def test_ell_slot_groups(ctx, oracle, width, rows):
     _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
     _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
 
+@pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16])
+@pytest.mark.parametrize("x_offset", [0, 1])
+def test_csr_multi_units(ctx, dtype, x_offset):
+    """The multi-vector CSR kernel on rows around its blocks and units (empty
+    rows, rows of 7..17, 511..513, 4096, 4097 and 5000 entries) for every k:
+    dyadic inputs, so Y equals the FP64 product, and each right-hand side's
+    bits on random inputs do not depend on k."""
+    A = _csr_wave_case("row_lengths")
+    dA = cs.DeviceMatrix(ctx, cs.coo2csr(A.copy()), panel=0, dtype=dtype)
+    R = cs.Coo(A.row, A.col, np.random.default_rng(3).standard_normal(A.nnz).astype(np.float32), A.height, A.width)
+    dR = cs.DeviceMatrix(ctx, cs.coo2csr(R.copy()), panel=0, dtype=dtype)
+    rng = np.random.default_rng(5)
+    Xd = (rng.integers(-64, 65, size=(A.width, 16)) / 64.0).astype(np.float32)
+    Xr = rng.uniform(-1, 1, size=(A.width, 16)).astype(np.float32)
+    Y0 = (rng.integers(-64, 65, size=(16, A.height)) / 64.0).astype(np.float32)
+    ref = Y0.astype(np.float64)
+    for q in range(16):
+        np.add.at(ref[q], A.row, A.val.astype(np.float64) * Xd[A.col, q])
+
+    def run(m, X, k):
+        pad = np.zeros(x_offset, np.float32)
+        dX = cs.DeviceVector(ctx, X[:, :k].size + x_offset, np.concatenate([pad, X[:, :k].reshape(-1)])).view(x_offset)
+        dY = cs.DeviceVector(ctx, k * A.height, Y0[:k].reshape(-1))
+        m.spmv_multi(k, dX, dY, A.height)
+        ctx.sync()
+        return dY.download().reshape(k, A.height)
+
+    wide = run(dR, Xr, 16)
+    for k in range(1, 17):
+        np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
+        np.testing.assert_array_equal(run(dR, Xr, k), wide[:k])
+
 
 @pytest.mark.parametrize("name", ["rand_small", "rand_dyadic", "rand_long_rows"])
 @pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
