@@ -76,7 +76,7 @@ template <int Q, int L, int R, int W, class V>
 __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
     int rows, int cols, int len, int nseg, const int4* __restrict__ seg,
     const typename V::T* __restrict__ data, int k, const float* __restrict__ X, float* __restrict__ Y,
-    int ldy) {
+    int ldy, bool accumulate) {
     typedef typename V::T T;
     constexpr int NR = kWave / L * R;                    // rows per wave
     constexpr int RW = kWave / L;                        // X rows per load instruction
@@ -224,14 +224,15 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
         float* yp = Y + (size_t)(qs + q) * ldy + r0;
         if (r0 + R <= rows) {
             typedef typename UVec<float, R>::type YU;
-            typename RV::type v = *reinterpret_cast<const YU*>(yp);
+            typename RV::type v{};
+            if (accumulate) v = *reinterpret_cast<const YU*>(yp);
 #pragma unroll
             for (int r = 0; r < R; ++r) RV::set(v, r, RV::get(v, r) + acc[r][q]);
             *reinterpret_cast<YU*>(yp) = v;
         } else {
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                if (r0 + r < rows) yp[r] += acc[r][q];
+                if (r0 + r < rows) yp[r] = (accumulate ? yp[r] : 0.0f) + acc[r][q];
         }
     }
 }
@@ -286,7 +287,8 @@ template <class V, class Acc>
 __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__ val,
                                                const int* __restrict__ col, int r, int j0, int j1,
                                                const float* __restrict__ X, int k, bool vec,
-                                               float* __restrict__ Y, int ldy, Acc (*part)[launch::kMultiMax]) {
+                                               float* __restrict__ Y, int ldy, bool accumulate,
+                                               Acc (*part)[launch::kMultiMax]) {
     constexpr int Q = 4, L = launch::kMultiMax / Q;
     const int t = threadIdx.x;
     const int qb = (t % L) * Q;
@@ -307,10 +309,11 @@ __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__
 #pragma unroll
         for (int w = 0; w < kMultiThreads / kWave; ++w) tot += part[w][t];
         float* yp = Y + (size_t)t * ldy + r;
+        const float y0 = accumulate ? *yp : 0.0f;
         if constexpr (sizeof(Acc) == sizeof(double))
-            *yp = (float)((double)*yp + tot);  // one rounding of the whole row
+            *yp = (float)((double)y0 + tot);  // one rounding of the whole row
         else
-            *yp += tot;
+            *yp = y0 + tot;
     }
 }
 
@@ -352,7 +355,7 @@ template <int Q, int L, class V>
 __global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
     int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
     const int* __restrict__ rp, const int* __restrict__ col, const typename V::T* __restrict__ val, int k,
-    const float* __restrict__ X, bool vec, float* __restrict__ Y, int ldy) {
+    const float* __restrict__ X, bool vec, float* __restrict__ Y, int ldy, bool accumulate) {
     typedef typename V::T T;
     constexpr int QP = Q == 3 ? 4 : Q;              // LDS floats per piece
     constexpr int KB = QP * L;                      // and per row or unit
@@ -376,9 +379,9 @@ __global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
     if ((int)blockIdx.x < nlong) {  // the longest work first
         const int r = longs[blockIdx.x], j0 = rp[r], j1 = rp[r + 1];
         if (j1 - j0 > launch::kLongRowF64)
-            csr_multi_long<V, double>(val, col, r, j0, j1, X, k, vec, Y, ldy, lds.part64);
+            csr_multi_long<V, double>(val, col, r, j0, j1, X, k, vec, Y, ldy, accumulate, lds.part64);
         else
-            csr_multi_long<V, float>(val, col, r, j0, j1, X, k, vec, Y, ldy, lds.part);
+            csr_multi_long<V, float>(val, col, r, j0, j1, X, k, vec, Y, ldy, accumulate, lds.part);
         return;
     }
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -487,7 +490,8 @@ __global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
         *reinterpret_cast<typename PV::type*>(at) = t;
     }
     wave_lds_order();
-    if (lane < nrows && W.rp[lane + 1] > W.rp[lane]) {  // empty rows leave Y as it is
+    const bool empty = lane < nrows && W.rp[lane + 1] == W.rp[lane];
+    if (lane < nrows && !(empty && accumulate)) {  // empty rows leave Y as it is
         float* yp = Y + r0 + lane;
         const float* ap = W.acc + lane * AS;
         const int full = (k - 1) / Q * Q, shift = full + Q - k;  // columns before the last piece, its overlap
@@ -495,10 +499,10 @@ __global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
         float y[KM];
 #pragma unroll
         for (int q = 0; q < KM; ++q)
-            if (q < k) y[q] = yp[(size_t)q * ldy];
+            if (q < k) y[q] = accumulate ? yp[(size_t)q * ldy] : 0.0f;
 #pragma unroll
         for (int q = 0; q < KM; ++q)
-            if (q < k) yp[(size_t)q * ldy] = y[q] + ap[q < full ? q : q + shift];
+            if (q < k) yp[(size_t)q * ldy] = y[q] + (empty ? 0.0f : ap[q < full ? q : q + shift]);
     }
 }
 
@@ -506,15 +510,15 @@ int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 
 template <int Q, int L, int R, class V>
 hipError_t dia_multi_tile(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
-                          const void* data, int k, const float* X, float* Y, int ldy) {
+                          const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
     const dim3 grid(ceil_div(rows, kBlock / L * R)), block(kBlock);
     const typename V::T* d = static_cast<const typename V::T*>(data);
     if (w == 1)
         hipLaunchKernelGGL((dia_multi_kernel<Q, L, R, 1, V>), grid, block, 0, s, rows, cols, len, nseg, seg, d, k, X,
-                           Y, ldy);
+                           Y, ldy, accumulate);
     else
         hipLaunchKernelGGL((dia_multi_kernel<Q, L, R, kDiaRun, V>), grid, block, 0, s, rows, cols, len, nseg, seg, d,
-                           k, X, Y, ldy);
+                           k, X, Y, ldy, accumulate);
     return hipGetLastError();
 }
 
@@ -528,10 +532,10 @@ hipError_t dia_multi_tile(hipStream_t s, int rows, int cols, int len, int nseg, 
 // (32^3: 9.8 us, 22^3: 10.3 against 7.9 us).
 template <class V>
 hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
-                       const void* data, int k, const float* X, float* Y, int ldy) {
+                       const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
     const bool large = rows >= (1 << 19);
     const bool deep = large && nseg >= 6;
-#define CLSPMV_DIA_MULTI(Q, L, R) dia_multi_tile<Q, L, R, V>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy)
+#define CLSPMV_DIA_MULTI(Q, L, R) dia_multi_tile<Q, L, R, V>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate)
     switch (k) {
         case 1: return large ? CLSPMV_DIA_MULTI(1, 1, 4) : CLSPMV_DIA_MULTI(1, 1, 1);
         case 2: return deep ? CLSPMV_DIA_MULTI(2, 1, 2) : CLSPMV_DIA_MULTI(2, 1, 1);
@@ -546,27 +550,27 @@ hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int nseg, int
 
 template <int Q, int L, class V>
 hipError_t csr_multi_tile(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
-                          int k, const float* X, float* Y, int ldy) {
+                          int k, const float* X, float* Y, int ldy, bool accumulate) {
     const bool vec = k % 4 == 0 && ((uintptr_t)X % 16) == 0;  // long rows: aligned 16-byte pieces
     hipLaunchKernelGGL((csr_multi_kernel<Q, L, V>), dim3(W.nlong + ceil_div(W.nblk, kMultiThreads / kWave)),
                        dim3(kMultiThreads), 0, s,
                        W.nlong, W.longs, W.nblk, W.blk, rp, col, static_cast<const typename V::T*>(val), k, X, vec, Y,
-                       ldy);
+                       ldy, accumulate);
     return hipGetLastError();
 }
 
 template <class V>
 hipError_t csr_multi_v(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val, int k,
-                       const float* X, float* Y, int ldy) {
+                       const float* X, float* Y, int ldy, bool accumulate) {
     switch (k) {
-        case 1: return csr_multi_tile<1, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
-        case 2: return csr_multi_tile<2, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
-        case 3: return csr_multi_tile<3, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
-        case 4: return csr_multi_tile<4, 1, V>(s, W, rp, col, val, k, X, Y, ldy);
+        case 1: return csr_multi_tile<1, 1, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
+        case 2: return csr_multi_tile<2, 1, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
+        case 3: return csr_multi_tile<3, 1, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
+        case 4: return csr_multi_tile<4, 1, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
         default: break;
     }
-    return k <= 8 ? csr_multi_tile<4, 2, V>(s, W, rp, col, val, k, X, Y, ldy)
-                  : csr_multi_tile<4, 4, V>(s, W, rp, col, val, k, X, Y, ldy);
+    return k <= 8 ? csr_multi_tile<4, 2, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate)
+                  : csr_multi_tile<4, 4, V>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
 }
 
 }  // namespace
@@ -574,25 +578,25 @@ hipError_t csr_multi_v(hipStream_t s, const launch::CsrWave& W, const int* rp, c
 namespace launch {
 
 hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
-                     int dtype, const void* data, int k, const float* X, float* Y, int ldy) {
+                     int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
     if (rows <= 0 || cols <= 0 || nseg <= 0 || k <= 0) return hipSuccess;
     if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
-        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
-        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy);
+        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
+        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
+        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
         default: return hipErrorInvalidValue;
     }
 }
 
 hipError_t csr_multi(hipStream_t s, const CsrWave& W, const int* rp, const int* col,
-                     int dtype, const void* val, int k, const float* X, float* Y, int ldy) {
+                     int dtype, const void* val, int k, const float* X, float* Y, int ldy, bool accumulate) {
     if (W.nblk + W.nlong <= 0 || k <= 0) return hipSuccess;
     if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return csr_multi_v<ValF32>(s, W, rp, col, val, k, X, Y, ldy);
-        case 1: return csr_multi_v<ValBF16>(s, W, rp, col, val, k, X, Y, ldy);
-        case 2: return csr_multi_v<ValF16>(s, W, rp, col, val, k, X, Y, ldy);
+        case 0: return csr_multi_v<ValF32>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
+        case 1: return csr_multi_v<ValBF16>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
+        case 2: return csr_multi_v<ValF16>(s, W, rp, col, val, k, X, Y, ldy, accumulate);
         default: return hipErrorInvalidValue;
     }
 }

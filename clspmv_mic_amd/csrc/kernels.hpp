@@ -158,18 +158,19 @@ hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
                  const float* data, const float* x, bool x_aligned, float* y);
 
 // ---- multi-right-hand-side SpMV (k <= kMultiMax) --------------------------------
-// Y[:, q] += A X[:, q]; X row-major (X[c*k + q]), Y column-major (ldy).
+// Y[:, q] += A X[:, q], or without `accumulate` Y[:, q] = 0 + A X[:, q], Y not
+// read; X row-major (X[c*k + q]), Y column-major (ldy).
 constexpr int kMultiMax = 16;
 // DIA: the diagonals as nseg segments {first diagonal, its offset, how many
 // consecutive offsets follow each other (at most w), 0} in diagonal order;
 // w is 1 or kDiaRun.
 constexpr int kDiaRun = 3;
 hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
-                     int dtype, const void* data, int k, const float* X, float* Y, int ldy);
+                     int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate);
 // CSR over the wave kernel's blocks and long rows.  A right-hand side's
 // result does not depend on k, nor does DIA's.
 hipError_t csr_multi(hipStream_t s, const CsrWave& W, const int* rp, const int* col,
-                     int dtype, const void* val, int k, const float* X, float* Y, int ldy);
+                     int dtype, const void* val, int k, const float* X, float* Y, int ldy, bool accumulate);
 
 // ---- mixed-precision 4x4-block SpMM (MFMA) -------------------------------------
 // Y[:, 0:k] += A X[:, 0:k]; A in slices of kSpmmSlice block rows: sptr[s] is

@@ -349,15 +349,23 @@ bool has_multi(const clspmv_dmat* A) {
     return A->info.format == CLSPMV_FMT_DIA || (A->info.format == CLSPMV_FMT_CSR && A->plain);
 }
 
-int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy) {
+bool multi_overwrites(const clspmv_dmat* A) {
+    // Every row is written: DIA's when the diagonals are as long as the matrix
+    // is high and some meet it, CSR's always.
+    if (A->info.format == CLSPMV_FMT_DIA) return A->ndseg > 0 && A->info.cols > 0 && A->len >= A->info.rows;
+    return A->info.format == CLSPMV_FMT_CSR && A->plain;
+}
+
+int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy, bool accumulate) {
     const clspmv_dmat_info& I = A->info;
     hipError_t e;
     if (I.format == CLSPMV_FMT_DIA) {
         e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, A->ndseg, A->seg_w, A->dseg, A->dtype,
-                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy);
+                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy, accumulate);
     } else if (I.format == CLSPMV_FMT_CSR && A->plain) {
         e = launch::csr_multi(s, csr_wave_of(A), A->rp, A->col, A->dtype,
-                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy);
+                              A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy,
+                              accumulate);
     } else {
         return fail(CLSPMV_ERR_UNSUPPORTED, "multi-vector SpMV exists for DIA and CSR (own arrays) only");
     }

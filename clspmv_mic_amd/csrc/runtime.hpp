@@ -207,9 +207,12 @@ int dmat_launch_rest(hipStream_t stream, const clspmv_dmat* A, int method,
 
 // Multi-vector SpMV (DIA, CSR with its own arrays): Y[:, q] += A X[:, q],
 // X row-major, Y column-major; no argument checks.  Each right-hand side's
-// result does not depend on k.
+// result does not depend on k.  accumulate = false (only where
+// multi_overwrites): Y = 0 + A X, Y not read.
+bool multi_overwrites(const clspmv_dmat* A);
 bool has_multi(const clspmv_dmat* A);
-int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy);
+int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, float* Y, int ldy,
+                 bool accumulate = true);
 
 // Method chosen for CLSPMV_METHOD_AUTO.
 int auto_method(const clspmv_dmat* A);

@@ -8,9 +8,9 @@
 // takes the matrix's claim (one pass per device matrix across servers),
 // coalesces its waiting requests into one batch, and (3) launches the batch
 // on the matrix's stream: stage each request's x into its columns of the
-// matrix's X, replay the captured (matrix, K) graph (one MFMA SpMM writing
-// y, or zero y, then one multi-vector pass per 16 columns or one SpMV per
-// column),
+// matrix's X, run the pass (one MFMA SpMM or one multi-vector pass per 16
+// columns writing y; or zero y, then one SpMV per column) as plain launches
+// where it has few, else by replaying the captured (matrix, K) graph, and
 // copy each request's y out.  Callers only touch the queue.
 //
 // Bit-for-bit independence from the mix: the kernels of a matrix are fixed
@@ -63,6 +63,7 @@ enum Layout {
 // SpMM reads whole 4-row pieces).
 __global__ void stage_x_kernel(unsigned long long seed, const float* __restrict__ src, int src_ld, int k,
                                int cols, int layout, int dtype, int K, int g0, int ldx, void* __restrict__ X) {
+    // (kChunkF32: stage_rows_kernel.)
     const int cpad = layout >= kTile16 ? (cols + 3) / 4 * 4 : cols;
     const long long n = (long long)k * cpad;
     for (long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x; t < n;
@@ -75,11 +76,6 @@ __global__ void stage_x_kernel(unsigned long long seed, const float* __restrict_
             case kColF32:
                 static_cast<float*>(X)[(size_t)g * ldx + i] = v;
                 break;
-            case kChunkF32: {
-                const int c = g / kMultiCols, kc = min(kMultiCols, K - c * kMultiCols);
-                static_cast<float*>(X)[(size_t)c * kMultiCols * ldx + (size_t)i * kc + g % kMultiCols] = v;
-                break;
-            }
             case kTile16:
                 static_cast<unsigned short*>(X)[((size_t)(i >> 2) * K + g) * 4 + (i & 3)] =
                     dtype == CLSPMV_DT_BF16 ? to_bf16(v) : to_f16(v);
@@ -90,6 +86,47 @@ __global__ void stage_x_kernel(unsigned long long seed, const float* __restrict_
                 break;
         }
     }
+}
+
+// x of k columns of one request (as above) into columns [off, off + k) of a
+// row-major chunk of kc: X[i * kc + off + j].  A work-group reads kStageRows
+// rows of each column as contiguous runs into LDS and writes them out row by
+// row; writing each value from the thread that read it touched a line per
+// value (average over a burst of 48 requests, other passes running: 14.2 ->
+// 10.1 us).
+constexpr int kStageRows = 256;
+__global__ __launch_bounds__(kStageRows) void stage_rows_kernel(unsigned long long seed, int j0,
+                                                                const float* __restrict__ src, int src_ld, int k,
+                                                                int cols, int kc, int off, float* __restrict__ X) {
+    __shared__ float tile[kStageRows * (kMultiCols + 1)];
+    const int i0 = blockIdx.x * kStageRows, t = threadIdx.x, ld = k | 1;
+    const int nr = min(kStageRows, cols - i0);
+    if (t < nr) {
+        float v[kMultiCols];
+        if (src) {  // every column's load in flight at once
+#pragma unroll
+            for (int j = 0; j < kMultiCols; ++j)
+                if (j < k) v[j] = src[(size_t)j * src_ld + i0 + t];
+        } else {
+#pragma unroll
+            for (int j = 0; j < kMultiCols; ++j)
+                if (j < k) v[j] = uniform_at(seed, j0 + j, i0 + t);
+        }
+#pragma unroll
+        for (int j = 0; j < kMultiCols; ++j)
+            if (j < k) tile[t * ld + j] = v[j];
+    }
+    __syncthreads();
+    for (int e = t; e < nr * k; e += kStageRows) {
+        const int r = e / k, j = e - r * k;
+        X[(size_t)(i0 + r) * kc + off + j] = tile[r * ld + j];
+    }
+}
+
+// Columns of y (leading dimension ldy) to the caller's (rows floats each).
+__global__ void copy_y_kernel(int rows, int ldy, const float* __restrict__ y, float* __restrict__ out) {
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += gridDim.x * blockDim.x)
+        out[(size_t)blockIdx.y * rows + i] = y[(size_t)blockIdx.y * ldy + i];
 }
 
 __global__ void zero_kernel(long long n, float* y) {
@@ -255,33 +292,48 @@ bool ensure_slot(clspmv_server* S, SMatrix& M) {
     return true;
 }
 
-// The products of K right-hand sides into y: the SpMM writes Y = A X
-// (the bits a zeroed Y plus A X gives); the other paths add into a zeroed
-// y.  Runs on `s` (captured or not).
-int enqueue_pass(hipStream_t s, const SMatrix& M, int K) {
+// Kernel launches of a pass over K columns.
+int pass_launches(const SMatrix& M, int K) {
+    if (M.path == kSpmm) return 1;
+    if (M.path == kMulti) return (K + kMultiCols - 1) / kMultiCols + !multi_overwrites(M.A);
+    return 1 + K * (M.A->info.format == CLSPMV_FMT_COO || dmat_has_prepass(M.A) ? 2 : 1);
+}
+
+// Passes of at most this many launches go out as plain launches: replaying a
+// graph costs the scheduler about 14 us, a kernel launch about 3.5 us.
+constexpr int kPlainLaunches = 4;
+
+// The products of K right-hand sides into Y (leading dimension ldy): the SpMM
+// and the multi-vector kernels write Y = A X (the bits a zeroed Y plus A X
+// gives); the other paths add into a zeroed y.  Runs on `s` (captured or
+// not).
+int enqueue_pass(hipStream_t s, const SMatrix& M, int K, float* Y, int ldy) {
     if (M.path == kSpmm) {
         const clspmv_dmat* A = M.A;
         CLSPMV_HIP(launch::bspmm4(s, A->dtype == CLSPMV_DT_BF16, A->long_brows, A->brows, M.rows, M.cols, K, A->rp,
-                                  A->col, A->lpval, static_cast<const unsigned short*>(M.X), K, M.Y, M.ldy,
+                                  A->col, A->lpval, static_cast<const unsigned short*>(M.X), K, Y, ldy,
                                   /*tiled=*/true, /*accumulate=*/false,
                                   launch::SpmmWindows{A->wtile, A->widx, A->win_max}));
         return CLSPMV_OK;
     }
-    const long long ny = (long long)M.ldy * K;
-    hipLaunchKernelGGL(zero_kernel, dim3(grid_for(ny)), dim3(256), 0, s, ny, M.Y);
-    CLSPMV_HIP(hipGetLastError());
+    const bool overwrite = M.path == kMulti && multi_overwrites(M.A);
+    if (!overwrite) {
+        const long long ny = (long long)ldy * K;
+        hipLaunchKernelGGL(zero_kernel, dim3(grid_for(ny)), dim3(256), 0, s, ny, Y);
+        CLSPMV_HIP(hipGetLastError());
+    }
     if (M.path == kMulti) {
         for (int c = 0; c * kMultiCols < K; ++c) {
             const int kc = std::min(kMultiCols, K - c * kMultiCols);
             int st = multi_launch(s, M.A, kc, static_cast<const float*>(M.X) + (size_t)c * kMultiCols * M.ldx,
-                                  M.Y + (size_t)c * kMultiCols * M.ldy, M.ldy);
+                                  Y + (size_t)c * kMultiCols * ldy, ldy, !overwrite);
             if (st) return st;
         }
         return CLSPMV_OK;
     }
     for (int j = 0; j < K; ++j) {
         int st = dmat_launch(s, M.A, M.method, static_cast<const float*>(M.X) + (size_t)j * M.ldx,
-                             M.Y + (size_t)j * M.ldy);
+                             Y + (size_t)j * ldy);
         if (st) return st;
     }
     return CLSPMV_OK;
@@ -297,26 +349,35 @@ int layout_of(const SMatrix& M, bool plain) {
 int stage_x(hipStream_t s, const SMatrix& M, const clspmv_request& r, int K, int g0, bool plain) {
     const int layout = layout_of(M, plain);
     const float* src = nullptr;
-    if (r.x) {
-        if (r.x_on_device) {
-            src = r.x;
-        } else if (layout == kColF32) {  // straight into X
-            CLSPMV_HIP(hipMemcpy2DAsync(static_cast<float*>(M.X) + (size_t)g0 * M.ldx, sizeof(float) * M.ldx, r.x,
-                                        sizeof(float) * M.cols, sizeof(float) * M.cols, r.k,
-                                        hipMemcpyHostToDevice, s));
-            return CLSPMV_OK;
-        } else {  // through the staging columns, then converted
-            CLSPMV_HIP(hipMemcpy2DAsync(M.S + (size_t)g0 * M.ldx, sizeof(float) * M.ldx, r.x, sizeof(float) * M.cols,
-                                        sizeof(float) * M.cols, r.k, hipMemcpyHostToDevice, s));
-            src = M.S + (size_t)g0 * M.ldx;
-            hipLaunchKernelGGL(stage_x_kernel, dim3(grid_for((long long)r.k * (M.cols + 3))), dim3(256), 0, s,
-                               r.seed, src, M.ldx, r.k, M.cols, layout, M.A->dtype, K, g0, M.ldx, M.X);
+    int src_ld = M.cols;
+    if (r.x && r.x_on_device) {
+        src = r.x;
+    } else if (r.x && layout == kColF32) {  // straight into X
+        CLSPMV_HIP(hipMemcpy2DAsync(static_cast<float*>(M.X) + (size_t)g0 * M.ldx, sizeof(float) * M.ldx, r.x,
+                                    sizeof(float) * M.cols, sizeof(float) * M.cols, r.k, hipMemcpyHostToDevice, s));
+        return CLSPMV_OK;
+    } else if (r.x) {  // through the staging columns, then converted
+        CLSPMV_HIP(hipMemcpy2DAsync(M.S + (size_t)g0 * M.ldx, sizeof(float) * M.ldx, r.x, sizeof(float) * M.cols,
+                                    sizeof(float) * M.cols, r.k, hipMemcpyHostToDevice, s));
+        src = M.S + (size_t)g0 * M.ldx;
+        src_ld = M.ldx;
+    }
+    if (layout == kChunkF32) {
+        if (M.cols <= 0) return CLSPMV_OK;
+        for (int j = 0; j < r.k;) {  // the request's columns of each chunk
+            const int c = (g0 + j) / kMultiCols, off = (g0 + j) % kMultiCols;
+            const int n = std::min(r.k - j, kMultiCols - off);
+            hipLaunchKernelGGL(stage_rows_kernel, dim3((M.cols + kStageRows - 1) / kStageRows), dim3(kStageRows), 0, s,
+                               r.seed, j, src ? src + (size_t)j * src_ld : nullptr, src_ld, n, M.cols,
+                               std::min(kMultiCols, K - c * kMultiCols), off,
+                               static_cast<float*>(M.X) + (size_t)c * kMultiCols * M.ldx);
             CLSPMV_HIP(hipGetLastError());
-            return CLSPMV_OK;
+            j += n;
         }
+        return CLSPMV_OK;
     }
     hipLaunchKernelGGL(stage_x_kernel, dim3(grid_for((long long)r.k * (M.cols + 3))), dim3(256), 0, s, r.seed, src,
-                       M.cols, r.k, M.cols, layout, M.A->dtype, K, g0, M.ldx, M.X);
+                       src_ld, r.k, M.cols, layout, M.A->dtype, K, g0, M.ldx, M.X);
     CLSPMV_HIP(hipGetLastError());
     return CLSPMV_OK;
 }
@@ -325,9 +386,14 @@ int stage_x(hipStream_t s, const SMatrix& M, const clspmv_request& r, int K, int
 int copy_y(hipStream_t s, const SMatrix& M, const clspmv_request& r, int g0, float* pinned) {
     const float* y = M.Y + (size_t)g0 * M.ldy;
     const size_t row_bytes = sizeof(float) * M.rows;
-    if (r.device_y)
+    if (r.device_y && M.rows > 0 && r.k <= 65535) {  // the grid's y limit
+        hipLaunchKernelGGL(copy_y_kernel, dim3(std::min((M.rows + 255) / 256, 2048), r.k), dim3(256), 0, s, M.rows,
+                           M.ldy, y, r.device_y);
+        CLSPMV_HIP(hipGetLastError());
+    } else if (r.device_y) {
         CLSPMV_HIP(hipMemcpy2DAsync(r.device_y, row_bytes, y, sizeof(float) * M.ldy, row_bytes, r.k,
                                     hipMemcpyDeviceToDevice, s));
+    }
     if (r.host_y && pinned)
         CLSPMV_HIP(hipMemcpy2DAsync(pinned, row_bytes, y, sizeof(float) * M.ldy, row_bytes, r.k,
                                     hipMemcpyDeviceToHost, s));
@@ -338,7 +404,7 @@ int graph_for(clspmv_server* S, SMatrix& M, int K, hipGraphExec_t* out) {
     if (!M.exec[K]) {
         hipStream_t s = S->streams[M.stream];
         CLSPMV_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        int st = enqueue_pass(s, M, K);
+        int st = enqueue_pass(s, M, K, M.Y, M.ldy);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(s, &g);
         if (st) {
@@ -367,16 +433,25 @@ int launch_batch(clspmv_server* S, SMatrix& M, SBatch& b) {
         if (st) return st;
         g += q.r.k;
     }
-    if (S->cfg.use_graphs) {
+    // One request with its y on the device alone: the multi-vector pass writes
+    // there, without the copy.
+    const clspmv_request& r0 = S->reqs[b.tickets[0]].r;
+    const bool direct = M.path == kMulti && b.tickets.size() == 1 && r0.device_y && !r0.host_y &&
+                        pass_launches(M, K) <= kPlainLaunches;
+    if (direct) {
+        int st = enqueue_pass(s, M, K, r0.device_y, M.rows);
+        if (st) return st;
+    } else if (S->cfg.use_graphs && pass_launches(M, K) > kPlainLaunches) {
         hipGraphExec_t ex = nullptr;
         int st = graph_for(S, M, K, &ex);
         if (st) return st;
         CLSPMV_HIP(hipGraphLaunch(ex, s));
     } else {
-        int st = enqueue_pass(s, M, K);
+        int st = enqueue_pass(s, M, K, M.Y, M.ldy);
         if (st) return st;
     }
     for (long long t : b.tickets) {
+        if (direct) break;
         SRequest& q = S->reqs[t];
         int st = copy_y(s, M, q.r, q.col, q.pin != kNone ? S->pinned + q.pin / sizeof(float) : nullptr);
         if (st) return st;
@@ -561,9 +636,9 @@ int calibrate(SMatrix M) {
         hipLaunchKernelGGL(zero_kernel, dim3(grid_for(n)), dim3(256), 0, s, n, static_cast<float*>(M.X));
         st = hipGetLastError() == hipSuccess ? CLSPMV_OK : fail(CLSPMV_ERR_HIP, "zero launch failed");
         M.path = kSingle;
-        if (!st) st = time_pass(s, e0, e1, [&] { return enqueue_pass(s, M, k); }, &t_single);
+        if (!st) st = time_pass(s, e0, e1, [&] { return enqueue_pass(s, M, k, M.Y, M.ldy); }, &t_single);
         M.path = kMulti;
-        if (!st) st = time_pass(s, e0, e1, [&] { return enqueue_pass(s, M, k); }, &t_multi);
+        if (!st) st = time_pass(s, e0, e1, [&] { return enqueue_pass(s, M, k, M.Y, M.ldy); }, &t_multi);
     }
     (void)hipStreamSynchronize(s);
     if (e0) (void)hipEventDestroy(e0);

@@ -19,10 +19,10 @@
  *     not fit waits until idle matrices' buffers are evicted (least
  *     recently used first).  Copies to host_y go through a pinned staging
  *     area of host_staging bytes, taken per request;
- *   - each (matrix, right-hand-side count) pass is captured once into a HIP
- *     graph against the matrix's buffers (zero y, then the products) and
- *     replayed for every later batch of that size, until the buffers are
- *     evicted;
+ *   - passes of more than four kernel launches are captured once per
+ *     (matrix, right-hand-side count) into a HIP graph against the matrix's
+ *     buffers and replayed for every later batch of that size, until the
+ *     buffers are evicted; shorter ones are launched plainly;
  *   - results do not depend on the mix: the kernels a matrix runs are fixed
  *     when it is registered, each right-hand side's arithmetic in them does
  *     not depend on the other columns of the pass, and every kernel has a

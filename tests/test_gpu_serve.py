@@ -192,3 +192,33 @@ def test_submit_and_wait(ctx, resident):
     with pytest.raises(cs.ClspmvError):
         s.submit(ids[0], 9, 1)          # k above kmax
     s.close()
+
+
+@pytest.mark.parametrize("fmt", ["dia", "csr"])
+def test_device_y_direct_and_batched(ctx, oracle, fmt):
+    """A lone request whose y stays on the device gets it straight from the
+    pass, one with host_y through the working buffers: the same bits, every
+    row written (empty rows as zeros over what was there), for right-hand-side
+    counts within, at and across the 16-column chunks."""
+    if fmt == "dia":
+        A = matrices.laplacian_2d(301)
+        dm = cs.DeviceMatrix(ctx, cs.coo2dia(A.copy()))
+    else:
+        A = matrices.random_sparse(30_001, 29_000, 0.0004, seed=21, empty_rows=0.3, long_rows=3, long_len=3000)
+        dm = cs.DeviceMatrix(ctx, cs.coo2csr(A.copy()), panel=0)
+    s = cs.Server(streams=2, max_batch=4, hbm_budget=256 << 20)
+    i = s.add(dm, kmax=40)
+    for k in (1, 3, 5, 16, 17, 40):
+        seed = 900 + k
+        host = np.zeros(A.height * k, np.float32)
+        s.wait(s.submit(i, k, seed, host))
+        x = np.concatenate([cs.request_x(seed, j, A.width) for j in range(k)])
+        dx = cs.DeviceVector(ctx, x.size, x)
+        dy = cs.DeviceVector(ctx, A.height * k, np.full(A.height * k, np.nan, np.float32))
+        s.wait(s.submit(i, k, 0, x=dx, device_y=dy))
+        np.testing.assert_array_equal(dy.download(), host)
+        for j in (0, k - 1):
+            y64, bound = oracle.spmv_f64(A.row, A.col, A.val, x[j * A.width:(j + 1) * A.width].copy(), A.height)
+            err, worst = oracle.scaled_error(host[j * A.height:(j + 1) * A.height].copy(), y64, bound)
+            assert err <= TOL, f"k {k} rhs {j}: {err:.3e} at row {worst}"
+    s.close()
