@@ -85,6 +85,84 @@ __global__ __launch_bounds__(kBlock) void dia_row_kernel(
     y[r] += a;
 }
 
+// Four consecutive rows per lane over the segments of consecutive offsets
+// (launch::dia_multi's; at most W diagonals each), S segments' loads in flight:
+// a diagonal's four values are one load and the W + 3 x values that a
+// segment's rows need are two, where dia_row_kernel issues 2 W loads per row.
+// The sums are dia_row_kernel's, in diagonal order, bit for bit; x reads zero
+// outside the matrix.  len must be a multiple of 4.
+//
+// 16-bit values only, from 3 << 18 rows and 8 M values on: 27-point stencil 93^3 /
+// 101^3 / 128^3 14.0 / 17.1 / 31.4 -> 13.6 / 14.4 / 28.9 us, 5-point Laplacian
+// 1400^2 11.6 -> 10.6; below, the waves are too few (80^3 8.6 -> 9.6 us, 900^2
+// 5.9 -> 6.9).  FP32 values already set dia_row_kernel's pace (128^3 42.3 against
+// 42.7 us, 1400^2 12.4 against 13.1).
+constexpr int kQuadRows = 3 << 18;
+constexpr long long kQuadValues = 8 << 20;
+template <int W, int S, class V>
+__global__ __launch_bounds__(kBlock) void dia_quad_kernel(
+    int rows, int cols, int len, int nseg, const int4* __restrict__ seg,
+    const typename V::T* __restrict__ data, const float* __restrict__ x, float* __restrict__ y) {
+    constexpr int R = 4, NX = R + W - 1;
+    typedef typename V::T T;
+    const int r0 = (xcd_tile(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) * R;
+    const int w0 = __builtin_amdgcn_readfirstlane(r0);
+    if (w0 >= rows) return;  // the whole wave
+    const int dl = min(r0, len - R) - w0, xl = r0 - w0;
+    float acc[R] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s = 0; s < nseg; s += S) {
+        float xv[S][NX];
+        typename VecOf<T, R>::type d[S][W];
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const int4 sg = seg[min(s + i, nseg - 1)];
+            const long long c0 = (long long)w0 + sg.y;
+            if (c0 >= 0 && c0 + kWave * R + W - 1 <= cols) {
+                const float* xp = x + c0;
+                const f32x4 a = *reinterpret_cast<const UVec<float, 4>::type*>(xp + xl);
+#pragma unroll
+                for (int e = 0; e < R; ++e) xv[i][e] = a[e];
+                if constexpr (W > 1) {
+                    typedef VecOf<float, W - 1> XV;
+                    const typename XV::type b =
+                        *reinterpret_cast<const typename UVec<float, W - 1>::type*>(xp + xl + R);
+#pragma unroll
+                    for (int e = 0; e < W - 1; ++e) xv[i][R + e] = XV::get(b, e);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < NX; ++e) xv[i][e] = x_at(x, r0 + sg.y + e, cols);
+            }
+            // Diagonals past the segment's re-read its last one and are not added.
+            const T* dp = data + (size_t)sg.x * len + w0;
+#pragma unroll
+            for (int n = 0; n < W; ++n)
+                d[i][n] = __builtin_nontemporal_load(
+                    reinterpret_cast<const typename UVec<T, R>::type*>(dp + (size_t)min(n, sg.z - 1) * len + dl));
+        }
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            const int z = s + i < nseg ? seg[s + i].z : 0;
+#pragma unroll
+            for (int n = 0; n < W; ++n)
+                if (n < z)
+#pragma unroll
+                    for (int r = 0; r < R; ++r) acc[r] = fmaf(V::cvt(d[i][n][r]), xv[i][n + r], acc[r]);
+        }
+    }
+    if (r0 + R <= rows) {
+        typedef UVec<float, R>::type YU;
+        f32x4 v = *reinterpret_cast<const YU*>(y + r0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) v[r] += acc[r];
+        *reinterpret_cast<YU*>(y + r0) = v;
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            if (r0 + r < rows) y[r0 + r] += acc[r];
+    }
+}
+
 // Two consecutive rows per lane (64-bit data loads, len % 2 == 0), U
 // diagonals per iteration.
 template <int U, class V>
@@ -214,7 +292,7 @@ namespace launch {
 
 template <class V>
 hipError_t dia_typed(hipStream_t s, int rows, int cols, int len, int ndiag,
-                     const int* offsets, int min_off, int max_off, int method,
+                     const int* offsets, int min_off, int max_off, DiaSegments S, int method,
                      const typename V::T* data, const float* x, float* y) {
     const int span = max_off - min_off;
     switch (method) {
@@ -222,6 +300,19 @@ hipError_t dia_typed(hipStream_t s, int rows, int cols, int len, int ndiag,
             // Up to 32 diagonals: all in flight (the smallest multiple of 4
             // slots that holds them); more: 8 at a time.
             const dim3 g(ceil_div(rows, kBlock)), b(kBlock);
+            if constexpr (sizeof(typename V::T) == 2) {
+                if (ndiag <= 32 && S.count > 0 && rows >= kQuadRows && rows * (long long)ndiag >= kQuadValues &&
+                    len % 4 == 0) {
+                    const dim3 q(ceil_div(rows, 4 * kBlock));
+                    if (S.width == 1)
+                        hipLaunchKernelGGL((dia_quad_kernel<1, 5, V>), q, b, 0, s, rows, cols, len, S.count, S.seg,
+                                           data, x, y);
+                    else
+                        hipLaunchKernelGGL((dia_quad_kernel<kDiaRun, 1, V>), q, b, 0, s, rows, cols, len, S.count,
+                                           S.seg, data, x, y);
+                    break;
+                }
+            }
             switch ((ndiag + 3) / 4) {
 #define CLSPMV_DIA_ROW(Q)                                                                              \
     case Q:                                                                                           \
@@ -263,18 +354,18 @@ hipError_t dia_typed(hipStream_t s, int rows, int cols, int len, int ndiag,
 }
 
 hipError_t dia(hipStream_t s, int rows, int cols, int len, int ndiag,
-               const int* offsets, int min_off, int max_off, int method, int dtype,
+               const int* offsets, int min_off, int max_off, DiaSegments S, int method, int dtype,
                const void* data, const float* x, float* y) {
     if (rows <= 0 || ndiag <= 0) return hipSuccess;
     switch (dtype) {
         case 0:
-            return dia_typed<ValF32>(s, rows, cols, len, ndiag, offsets, min_off, max_off, method,
+            return dia_typed<ValF32>(s, rows, cols, len, ndiag, offsets, min_off, max_off, S, method,
                                      static_cast<const float*>(data), x, y);
         case 1:
-            return dia_typed<ValBF16>(s, rows, cols, len, ndiag, offsets, min_off, max_off, method,
+            return dia_typed<ValBF16>(s, rows, cols, len, ndiag, offsets, min_off, max_off, S, method,
                                       static_cast<const unsigned short*>(data), x, y);
         case 2:
-            return dia_typed<ValF16>(s, rows, cols, len, ndiag, offsets, min_off, max_off, method,
+            return dia_typed<ValF16>(s, rows, cols, len, ndiag, offsets, min_off, max_off, S, method,
                                      static_cast<const unsigned short*>(data), x, y);
         default:
             return hipErrorInvalidValue;

@@ -577,14 +577,14 @@ hipError_t csr_multi_v(hipStream_t s, const launch::CsrWave& W, const int* rp, c
 
 namespace launch {
 
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, DiaSegments S,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
-    if (rows <= 0 || cols <= 0 || nseg <= 0 || k <= 0) return hipSuccess;
+    if (rows <= 0 || cols <= 0 || S.count <= 0 || k <= 0) return hipSuccess;
     if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
-        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
-        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate);
+        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
+        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
+        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
         default: return hipErrorInvalidValue;
     }
 }

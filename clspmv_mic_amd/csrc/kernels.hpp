@@ -129,8 +129,16 @@ hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, EllWi
 // Methods: 0 one row per lane, 1 two rows per lane (len % 2 == 0),
 // 2 / 3 one / four rows per lane with an LDS x window.
 // dtype: 0 FP32 values, 1 BF16, 2 FP16 (data holds 16-bit bits).
+// S: the diagonals as `count` segments {first diagonal, its offset, how many
+// consecutive offsets follow each other (at most width), 0} in diagonal
+// order, those that meet no column left out; width is 1 or kDiaRun.
+constexpr int kDiaRun = 3;
+struct DiaSegments {
+    const int4* seg = nullptr;
+    int count = 0, width = 1;
+};
 hipError_t dia(hipStream_t s, int rows, int cols, int len, int ndiag,
-               const int* offsets, int min_off, int max_off, int method, int dtype,
+               const int* offsets, int min_off, int max_off, DiaSegments S, int method, int dtype,
                const void* data, const float* x, float* y);
 // Largest x window (floats) a work-group stages in LDS.
 constexpr int kLdsWindow = 8192;
@@ -161,11 +169,7 @@ hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
 // Y[:, q] += A X[:, q], or without `accumulate` Y[:, q] = 0 + A X[:, q], Y not
 // read; X row-major (X[c*k + q]), Y column-major (ldy).
 constexpr int kMultiMax = 16;
-// DIA: the diagonals as nseg segments {first diagonal, its offset, how many
-// consecutive offsets follow each other (at most w), 0} in diagonal order;
-// w is 1 or kDiaRun.
-constexpr int kDiaRun = 3;
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, DiaSegments S,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate);
 // CSR over the wave kernel's blocks and long rows.  A right-hand side's
 // result does not depend on k, nor does DIA's.

@@ -96,6 +96,22 @@ std::vector<int4> dia_segments(const int* off, int ndiag, int rows, int cols, in
     return seg;
 }
 
+// Uploads them.  Runs of consecutive offsets share the x values that the DIA
+// kernels load (and the X rows that the multi-vector kernel stages); a run's
+// window is two rows longer than a lone diagonal's and its values load in
+// threes, which pays while runs save a good part of the windows (multi-vector,
+// 5-point Laplacian, 3 of 5, k = 16: 42 against 47 us; lone diagonals as runs
+// of one, k = 8: 21.2 against 18.3 us).
+int upload_segments(clspmv_dmat* d, const int* off, int ndiag) {
+    std::vector<int4> seg = dia_segments(off, ndiag, d->info.rows, d->info.cols, 1);
+    std::vector<int4> run = dia_segments(off, ndiag, d->info.rows, d->info.cols, launch::kDiaRun);
+    const bool runs = run.size() * 10 <= seg.size() * 7;
+    if (runs) seg.swap(run);
+    d->seg_w = runs ? launch::kDiaRun : 1;
+    d->ndseg = (int)seg.size();
+    return upload_array(d, seg.data(), seg.size(), &d->dseg);
+}
+
 bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
 
 // The columns of a run of entries: [lo, hi], empty as hi < lo.
@@ -232,6 +248,8 @@ int dmat_prepass(hipStream_t s, const clspmv_dmat* A, const float* x, const clsp
 }
 
 namespace {
+launch::DiaSegments segments_of(const clspmv_dmat* A) { return launch::DiaSegments{A->dseg, A->ndseg, A->seg_w}; }
+
 launch::CsrWave csr_wave_of(const clspmv_dmat* A) {
     return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->wwin, A->wwin_max};
 }
@@ -300,7 +318,7 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
             if (method >= 2 && (method == 3 ? 4 : 1) * 256 + span > launch::kLdsWindow)
                 return fail(CLSPMV_ERR_UNSUPPORTED, "DIA method %d: offset span %d too wide for LDS", method, span);
             e = launch::dia(s, std::min(I.rows, A->len), I.cols, A->len, A->ndiag, A->offs,
-                            A->min_off, A->max_off, method, A->dtype,
+                            A->min_off, A->max_off, segments_of(A), method, A->dtype,
                             A->dtype ? (const void*)A->lpval : (const void*)A->val, x, y);
             break;
         }
@@ -313,7 +331,7 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
                 if (method == 3 && A->len % 2)
                     return fail(CLSPMV_ERR_UNSUPPORTED, "BDIA method 3 needs an even aligned length");
                 e = launch::dia(s, std::min(I.rows, A->len), I.cols, A->len, A->ndiag, A->offs_exp,
-                                A->min_off, A->max_off, method == 0 ? 0 : 1, 0, A->val, x, y);
+                                A->min_off, A->max_off, segments_of(A), method == 0 ? 0 : 1, 0, A->val, x, y);
                 break;
             }
             e = launch::bdia(s, std::min(I.rows, A->len), I.cols, A->len, A->nband, A->offs,
@@ -360,7 +378,7 @@ int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, flo
     const clspmv_dmat_info& I = A->info;
     hipError_t e;
     if (I.format == CLSPMV_FMT_DIA) {
-        e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, A->ndseg, A->seg_w, A->dseg, A->dtype,
+        e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, segments_of(A), A->dtype,
                               A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy, accumulate);
     } else if (I.format == CLSPMV_FMT_CSR && A->plain) {
         e = launch::csr_multi(s, csr_wave_of(A), A->rp, A->col, A->dtype,
@@ -744,21 +762,7 @@ int clspmv_upload_dia_ex(clspmv_ctx* ctx, const clspmv_dia_matrix* m, const clsp
     }
     d->info.stored = (long long)m->dia_num * m->dia_length_aligned;
     UPLOAD_CHECK(upload_array(d, m->dia_offsets, (size_t)m->dia_num, &d->offs));
-    // Runs of consecutive offsets share the X rows the multi-vector kernel
-    // stages; a run's window is two rows longer than a lone diagonal's and
-    // its values load in threes, which pays while runs save a good part of
-    // the windows (5-point Laplacian, 3 of 5, k = 16: 42 against 47 us; lone
-    // diagonals as runs of one, k = 8: 21.2 against 18.3 us).
-    {
-        std::vector<int4> seg = dia_segments(m->dia_offsets, m->dia_num, m->matinfo.height, m->matinfo.width, 1);
-        std::vector<int4> run =
-            dia_segments(m->dia_offsets, m->dia_num, m->matinfo.height, m->matinfo.width, launch::kDiaRun);
-        const bool runs = run.size() * 10 <= seg.size() * 7;
-        if (runs) seg.swap(run);
-        d->seg_w = runs ? launch::kDiaRun : 1;
-        d->ndseg = (int)seg.size();
-        UPLOAD_CHECK(upload_array(d, seg.data(), seg.size(), &d->dseg));
-    }
+    UPLOAD_CHECK(upload_segments(d, m->dia_offsets, m->dia_num));
     const size_t total = (size_t)m->dia_num * m->dia_length_aligned;
     if (dtype == CLSPMV_DT_F32) {
         UPLOAD_CHECK(upload_array(d, m->dia_data, total, &d->val));

@@ -50,8 +50,8 @@ struct clspmv_dmat {
     int* bptr = nullptr;
     int* offs_exp = nullptr;  // BDIA: one offset per diagonal
     int len = 0, ndiag = 0, nband = 0, min_off = 0, max_off = 0, max_band = 0;
-    // DIA: the diagonals as segments of at most seg_w consecutive offsets
-    // (launch::dia_multi), those that meet no column left out.
+    // DIA: the diagonals as segments of at most seg_w consecutive
+    // offsets (launch::DiaSegments).
     int4* dseg = nullptr;
     int ndseg = 0, seg_w = 1;
     // Block formats: block rows, aligned sizes, group lanes.

@@ -522,6 +522,33 @@ def test_csr_multi_units(ctx, dtype, x_offset):
         np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
         np.testing.assert_array_equal(run(dR, Xr, k), wide[:k])
 
+@pytest.mark.parametrize("offsets", sorted(DIA_TILE_OFFSETS))
+@pytest.mark.parametrize("n,align", [((3 << 18) - 1, 32), ((3 << 18) + 37, 32), ((3 << 18) + 37, 1),
+                                     ((1 << 21) + 5, 32)])
+@pytest.mark.parametrize("dtype", [cs.DT_F16, cs.DT_BF16])
+def test_dia_quad(ctx, offsets, n, align, dtype):
+    """DIA method 0 at and around the row count from which a lane takes four
+    rows, and with a stored length that is no multiple of 4; dyadic inputs on
+    vectors aligned to one float only: y equals the FP64 product."""
+    off = DIA_TILE_OFFSETS[offsets]
+    A = matrices.banded(n, off, seed=7, dyadic=True)
+    length = cs.lib.clspmv_aligned_length(n, align)
+    data, o32 = np.zeros((len(off), length), np.float32), np.array(off, np.int32)
+    diff = A.col.astype(np.int64) - A.row
+    x, y0 = matrices.dyadic_vector(n, seed=11), matrices.dyadic_vector(n, seed=12)
+    ref = y0.astype(np.float64)
+    for j, o in enumerate(off):
+        at = diff == o
+        data[j, A.row[at]] = A.val[at]
+        ref[A.row[at]] += A.val[at].astype(np.float64) * x[A.col[at]]
+    m = cs.DiaMatrix(cs.MatInfo(n, n, A.nnz), len(off), n, length, cs._ip(o32), cs._fp(data))
+    dA = cs.DeviceMatrix(ctx, m, dtype=dtype)
+    dx = cs.DeviceVector(ctx, n + 1, np.concatenate([[0], x]).astype(np.float32))
+    dy = cs.DeviceVector(ctx, n + 1, np.concatenate([[0], y0]).astype(np.float32))
+    dA.spmv(dx.view(1), dy.view(1), 0)
+    ctx.sync()
+    np.testing.assert_array_equal(dy.download()[1:], ref.astype(np.float32))
+
 
 @pytest.mark.parametrize("name", ["rand_small", "rand_dyadic", "rand_long_rows"])
 @pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
