@@ -43,8 +43,9 @@ __global__ __launch_bounds__(kBlock) void csr_vector_kernel(
 }
 
 // One row longer than kWaveNnz by the whole work-group: it strides over the
-// row, U entries' loads in flight per thread (each thread's sum in index
-// order), the waves' sums are added in order.  Acc is double for rows longer
+// row, U entries' loads in flight per thread also in the last round (a row of
+// up to 2,048 entries is one round), each thread's sum in index order; the
+// waves' sums are added in order.  Acc is double for rows longer
 // than kLongRowF64 of 16-bit values: their products are exact and the row is
 // rounded once, into y.
 template <class V, class Acc>
@@ -55,21 +56,21 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
     constexpr int U = 4, kThreads = kWave * launch::kCsrWaves;
     const int t = threadIdx.x;
     Acc acc = 0;
-    int k = s + t;
-    for (; k + (U - 1) * kThreads < e; k += U * kThreads) {
+    for (int k = s + t; k < e; k += U * kThreads) {
         int c[U];
         float v[U], xv[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            c[u] = ld_stream(col + k + u * kThreads);
-            v[u] = V::ld(val + k + u * kThreads);
+        for (int u = 0; u < U; ++u) {  // past the end: the last entry again, not added
+            const int at = min(k + u * kThreads, e - 1);
+            c[u] = ld_stream(col + at);
+            v[u] = V::ld(val + at);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
 #pragma unroll
-        for (int u = 0; u < U; ++u) acc = fma((Acc)v[u], (Acc)xv[u], acc);
+        for (int u = 0; u < U; ++u)
+            if (k + u * kThreads < e) acc = fma((Acc)v[u], (Acc)xv[u], acc);
     }
-    for (; k < e; k += kThreads) acc = fma((Acc)V::ld(val + k), (Acc)x[ld_stream(col + k)], acc);
     for (int m = kWave >> 1; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, kWave);
     if (t % kWave == 0) part[t / kWave] = acc;
     __syncthreads();

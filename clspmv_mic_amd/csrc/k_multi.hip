@@ -238,38 +238,32 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
 }
 
 // Accumulates a[q] += val[j] * X[col[j]][qb + q] over j = j0, j0 + step, ...
-// below j1 in that order, U nonzeros in flight per lane.  Acc is float, or
-// double for rows longer than kLongRowF64 (the products are exact in
+// below j1 in that order, U nonzeros in flight per lane also in the last round
+// (slots past the end re-read the last one and are not added).  Acc is float,
+// or double for rows longer than kLongRowF64 (the products are exact in
 // double).
 template <int Q, class V, class Acc, int U>
 __device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
                                               const typename V::T* __restrict__ val, int j0, int j1,
                                               int step, const float* __restrict__ X, int k, int qb,
                                               bool vec, Acc* a) {
-    int j = j0;
-    for (; j + (U - 1) * step < j1; j += U * step) {
+    for (int j = j0; j < j1; j += U * step) {
         int c[U];
         float v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            c[u] = ld_stream(col + j + u * step);
-            v[u] = V::ld(val + j + u * step);
+            const int at = min(j + u * step, j1 - 1);
+            c[u] = ld_stream(col + at);
+            v[u] = V::ld(val + at);
         }
         float xv[U][Q];
 #pragma unroll
         for (int u = 0; u < U; ++u) load_xq<Q>(X, c[u], k, qb, vec, xv[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
+            if (j + u * step < j1)
 #pragma unroll
-            for (int q = 0; q < Q; ++q) a[q] = fma((Acc)v[u], (Acc)xv[u][q], a[q]);
-    }
-    for (; j < j1; j += step) {
-        const int c = ld_stream(col + j);
-        const float v = V::ld(val + j);
-        float xv[Q];
-        load_xq<Q>(X, c, k, qb, vec, xv);
-#pragma unroll
-        for (int q = 0; q < Q; ++q) a[q] = fma((Acc)v, (Acc)xv[q], a[q]);
+                for (int q = 0; q < Q; ++q) a[q] = fma((Acc)v[u], (Acc)xv[u][q], a[q]);
     }
 }
 
