@@ -11,7 +11,7 @@
 // (kernels/spmv_bcsr.cl:4-40); here a group of G lanes (G from the average
 // number of blocks per block row) shares a block row, strides over its
 // blocks and combines its bh partial sums with lane shuffles.
-// BELL/SBELL: one lane per block row walks its block slots.
+// BELL/SBELL and slot-major BCSR: a lane per row of a block row walks the slots.
 
 #include "device_common.hpp"
 #include "kernels.hpp"
@@ -57,126 +57,148 @@ __global__ __launch_bounds__(kBlock) void bcsr_kernel(
     }
 }
 
-// BCSR in the slot-major encoding: one lane per block row walks its slots,
-// each slot's block columns and value planes contiguous across the wave
-// (BELL's pattern).  Padding slots (column -1) hold zero values; their loads
-// go to block column 0 and their products are not added, so the sum is the
-// row's blocks' in block order, one float4 dot per (w4, h).
-template <int BH, int BW4>
-__global__ __launch_bounds__(kBlock) void bcsr_slots_kernel(
-    int brows, int rows, int cols, int hal, int nslots, const int* __restrict__ col4,
-    const float* __restrict__ data, const float* __restrict__ x, bool x_aligned, float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= brows) return;
-    float acc[BH];
-#pragma unroll
-    for (int h = 0; h < BH; ++h) acc[h] = 0.0f;
-    const size_t plane = (size_t)hal * 4;  // floats per (slot, w4, h) plane
-    for (int sl = 0; sl < nslots; ++sl) {
-        const int c4 = ld_stream(col4 + (size_t)sl * hal + r);
-        const bool live = c4 >= 0;
-        const float* base = data + (size_t)sl * BW4 * BH * plane + (size_t)r * 4;
-#pragma unroll
-        for (int w4 = 0; w4 < BW4; ++w4) {
-            const float4 xv = ld_x4(x, ((live ? c4 : 0) + w4) * 4, cols, x_aligned);
-#pragma unroll
-            for (int h = 0; h < BH; ++h) {
-                const float4 d = ld_stream(reinterpret_cast<const float4*>(base + (w4 * BH + h) * plane));
-                const float a = dot4(d, xv, acc[h]);
-                acc[h] = live ? a : acc[h];
-            }
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < BH; ++h) {
-        const int row = r * BH + h;
-        if (row < rows) y[row] += acc[h];
-    }
-}
+// BELL, SBELL and BCSR in the slot-major encoding: block row r's slot s has its
+// block column at col[s * cs] and the float4 of (w4, h) at data[((s * BW4 + w4)
+// * BH + h) * 4 cs], both from the row's own base: the layouts differ in the
+// bases, the stride cs between slots and the slot count (SBELL's differs by
+// slice).  A float4 load of 64 block rows is one contiguous run.
+//
+// What bounds it: HBM on large matrices, the chain of slots (block column, then
+// x) on small ones.  The rows of a block go to different waves (kHWaves of
+// them share the block rows and find the columns and x in L1), which gives
+// four times the waves of a lane per block row, and U slots' columns and
+// values load at once, the next U's in flight while the present ones' x is
+// fetched (two register sets taking turns; the last group loads no more than
+// its slots).  12 4x4 blocks per block row, BCSR / BELL / SBELL: 20,000 block
+// rows 14.7 / 14.7 / 15.5 -> 6.5 / 6.2 / 6.7 us, 131,072 21.7 / 21.3 / 22.9 ->
+// 21.1 / 21.0 / 21.0 us (6.76 TB/s would be 16.8).
+//
+// Padding slots of BCSR (column -1) and slots past a lane's last load what is
+// there for another and are not added, so the sum is the row's blocks' in slot
+// order, one float4 dot per w4.  F4ACC = true (BELL method 1, the reference's
+// "_mad" variant, kernels/spmv_bell.cl:24-42): float4 accumulators reduced at
+// the end.
+enum Layout { kBcsrSlots, kBell, kSbell };
+constexpr int kHWaves = kBlock / kWave;  // waves of a work-group
 
-// F4ACC = false: one scalar accumulator per block row row (method 0);
-// true: float4 accumulators reduced at the end (method 1, the reference's
-// "_mad" variant, kernels/spmv_bell.cl:24-42).
-template <int BH, int BW4, bool F4ACC>
-__global__ __launch_bounds__(kBlock) void bell_kernel(
-    int brows, int rows, int cols, int hal, int f4, int ellnum,
-    const int* __restrict__ col4, const float* __restrict__ data,
-    const float* __restrict__ x, bool x_aligned, float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= brows) return;
-    float acc[BH];
-    float4 acc4[BH];
+template <int BH, int BW4, Layout LAY, bool F4ACC>
+__global__ __launch_bounds__(kBlock) void block_rows_kernel(
+    int brows, int rows, int cols, int cs, int f4, int nslots, const int* __restrict__ sptr,
+    const int* __restrict__ col4, const float* __restrict__ data, const float* __restrict__ x,
+    bool x_aligned, float* __restrict__ y) {
+    constexpr int HW = BH < kHWaves ? BH : kHWaves;  // waves sharing block rows
+    constexpr int HN = BH / HW;                      // rows of a block per wave
+    constexpr int U = BW4 * HN == 1 ? 4 : BW4 * HN == 2 ? 3 : 2;  // slots in flight
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int h0 = wave % HW * HN;
+    const int row = (xcd_tile(blockIdx.x, gridDim.x) * (kHWaves / HW) + wave / HW) * kWave + lane;
+    const int r = min(row, brows - 1);  // lanes past the end shadow the last block row
+    int w = nslots;
+    const int* cp = col4 + r;
+    const float* dp = data + (size_t)r * 4;
+    int P = f4;  // floats per (slot, w4, h) plane
+    if constexpr (LAY == kSbell) {  // cs: the slice height
+        const int sl = r / cs, p0 = sptr[sl];
+        w = (sptr[sl + 1] - p0) / cs;
+        P = cs * 4;
+        // A lane whose slice is empty reads entry 0 beside its neighbours.
+        const int at = w > 0 ? p0 + (r - sl * cs) : 0;
+        cp = col4 + at;
+        dp = data + (w > 0 ? (size_t)p0 * BH * BW4 * 4 + (size_t)(r - sl * cs) * 4 : 0);
+    }
+    int wm = w;  // the most slots of the wave's block rows
+    if constexpr (LAY == kSbell)
+        for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    wm = __builtin_amdgcn_readfirstlane(wm);
+    dp += (size_t)h0 * P;
+    float acc[HN];
+    float4 acc4[HN];
 #pragma unroll
-    for (int h = 0; h < BH; ++h) {
+    for (int h = 0; h < HN; ++h) {
         acc[h] = 0.0f;
         acc4[h] = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    const size_t slot_stride = (size_t)f4 * BW4 * BH;
-    const size_t w4_stride = (size_t)f4 * BH;
-    for (int sl = 0; sl < ellnum; ++sl) {
-        const int c4 = ld_stream(col4 + r + (size_t)sl * hal);
-        const float* base = data + sl * slot_stride + (size_t)r * 4;
+    int c[2][U];
+    float4 d[2][U][BW4][HN];
+    auto load_slot = [&](int s, int& cc, float4 (*dd)[HN]) {
+        const size_t at = LAY == kSbell ? (size_t)max(min(s, w - 1), 0) : (size_t)s;
+        cc = ld_stream(cp + at * cs);
 #pragma unroll
-        for (int w4 = 0; w4 < BW4; ++w4) {
-            const float4 xv = ld_x4(x, (c4 + w4) * 4, cols, x_aligned);
+        for (int w4 = 0; w4 < BW4; ++w4)
 #pragma unroll
-            for (int h = 0; h < BH; ++h) {
-                const float4 d = ld_stream(reinterpret_cast<const float4*>(
-                    base + (size_t)h * f4 + w4 * w4_stride));
-                if (F4ACC) {
-                    acc4[h].x = fmaf(d.x, xv.x, acc4[h].x);
-                    acc4[h].y = fmaf(d.y, xv.y, acc4[h].y);
-                    acc4[h].z = fmaf(d.z, xv.z, acc4[h].z);
-                    acc4[h].w = fmaf(d.w, xv.w, acc4[h].w);
-                } else {
-                    acc[h] = dot4(d, xv, acc[h]);
-                }
-            }
+            for (int h = 0; h < HN; ++h)
+                dd[w4][h] = ld_stream(reinterpret_cast<const float4*>(dp + ((at * BW4 + w4) * BH + h) * P));
+    };
+    auto load = [&](int s, int b) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_slot(s + u, c[b][u], d[b][u]);
+    };
+    auto load_part = [&](int s, int b) {  // slots below wm
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s + u >= wm) break;
+            load_slot(s + u, c[b][u], d[b][u]);
         }
-    }
+    };
+    auto add = [&](int s, int b) {
+        float4 xv[U][BW4];
 #pragma unroll
-    for (int h = 0; h < BH; ++h) {
-        const int row = r * BH + h;
+        for (int u = 0; u < U; ++u) {
+            if (s + u >= wm) break;
+            const int cc = LAY == kBcsrSlots ? max(c[b][u], 0) : c[b][u];
+#pragma unroll
+            for (int w4 = 0; w4 < BW4; ++w4) xv[u][w4] = ld_x4(x, (cc + w4) * 4, cols, x_aligned);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s + u >= wm) break;
+            const bool live = LAY == kBcsrSlots ? c[b][u] >= 0 : LAY == kSbell ? s + u < w : true;
+#pragma unroll
+            for (int w4 = 0; w4 < BW4; ++w4)
+#pragma unroll
+                for (int h = 0; h < HN; ++h) {
+                    const float4 dv = d[b][u][w4][h], xx = xv[u][w4];
+                    if (F4ACC) {
+                        acc4[h].x = live ? fmaf(dv.x, xx.x, acc4[h].x) : acc4[h].x;
+                        acc4[h].y = live ? fmaf(dv.y, xx.y, acc4[h].y) : acc4[h].y;
+                        acc4[h].z = live ? fmaf(dv.z, xx.z, acc4[h].z) : acc4[h].z;
+                        acc4[h].w = live ? fmaf(dv.w, xx.w, acc4[h].w) : acc4[h].w;
+                    } else {
+                        const float a = dot4(dv, xx, acc[h]);
+                        acc[h] = live ? a : acc[h];
+                    }
+                }
+        }
+    };
+    if (U <= wm) load(0, 0);
+    else load_part(0, 0);
+    int s = 0;
+    for (; s + 3 * U <= wm; s += 2 * U) {
+        load(s + U, 1);
+        add(s, 0);
+        load(s + 2 * U, 0);
+        add(s + U, 1);
+    }
+    if (s + U < wm) load_part(s + U, 1);
+    add(s, 0);
+    if (s + 2 * U < wm) load_part(s + 2 * U, 0);
+    if (s + U < wm) add(s + U, 1);
+    if (s + 2 * U < wm) add(s + 2 * U, 0);
+#pragma unroll
+    for (int h = 0; h < HN; ++h) {
+        const int at = r * BH + h0 + h;
         const float v = F4ACC ? (acc4[h].x + acc4[h].y) + (acc4[h].z + acc4[h].w) : acc[h];
-        if (row < rows) y[row] += v;
+        if (row < brows && at < rows) y[at] += v;
     }
 }
 
-template <int BH, int BW4>
-__global__ __launch_bounds__(kBlock) void sbell_kernel(
-    int brows, int rows, int cols, int sh, const int* __restrict__ sptr,
-    const int* __restrict__ col4, const float* __restrict__ data,
-    const float* __restrict__ x, bool x_aligned, float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= brows) return;
-    const int sl = r / sh, i = r - sl * sh;
-    const int p0 = sptr[sl];
-    const int w = (sptr[sl + 1] - p0) / sh;
-    const float* base = data + (size_t)p0 * BH * BW4 * 4 + (size_t)i * 4;
-    const size_t slot_stride = (size_t)sh * BW4 * BH * 4;
-    const size_t h_stride = (size_t)sh * 4;
-    const size_t w4_stride = (size_t)sh * BH * 4;
-    float acc[BH];
-#pragma unroll
-    for (int h = 0; h < BH; ++h) acc[h] = 0.0f;
-    for (int k = 0; k < w; ++k) {
-        const int c4 = ld_stream(col4 + p0 + i + (size_t)k * sh);
-#pragma unroll
-        for (int w4 = 0; w4 < BW4; ++w4) {
-            const float4 xv = ld_x4(x, (c4 + w4) * 4, cols, x_aligned);
-#pragma unroll
-            for (int h = 0; h < BH; ++h) {
-                const float4 d = ld_stream(reinterpret_cast<const float4*>(
-                    base + k * slot_stride + h * h_stride + w4 * w4_stride));
-                acc[h] = dot4(d, xv, acc[h]);
-            }
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < BH; ++h) {
-        const int row = r * BH + h;
-        if (row < rows) y[row] += acc[h];
-    }
+template <int BH, int BW4, Layout LAY, bool F4ACC>
+hipError_t block_rows(hipStream_t s, int brows, int rows, int cols, int cs, int f4, int nslots, const int* sptr,
+                      const int* col4, const float* data, const float* x, bool xa, float* y) {
+    constexpr int per = kWave * kHWaves / (BH < kHWaves ? BH : kHWaves);  // block rows per work-group
+    hipLaunchKernelGGL((block_rows_kernel<BH, BW4, LAY, F4ACC>), dim3(((long long)brows + per - 1) / per), dim3(kBlock), 0, s,
+                       brows, rows, cols, cs, f4, nslots, sptr, col4, data, x, xa, y);
+    return hipGetLastError();
 }
 
 int grid_for(long long threads) { return (int)((threads + kBlock - 1) / kBlock); }
@@ -203,72 +225,46 @@ hipError_t bcsr_shape(hipStream_t s, int brows, int rows, int cols, int lanes,
 
 namespace launch {
 
-#define SHAPE_DISPATCH(FN, ...)                                   \
+#define SHAPE_DISPATCH(FN, OPT, ...)                              \
     switch (bh * 10 + bw) {                                       \
-        case 14: return FN<1, 1>(__VA_ARGS__);                    \
-        case 24: return FN<2, 1>(__VA_ARGS__);                    \
-        case 44: return FN<4, 1>(__VA_ARGS__);                    \
-        case 84: return FN<8, 1>(__VA_ARGS__);                    \
-        case 18: return FN<1, 2>(__VA_ARGS__);                    \
-        case 28: return FN<2, 2>(__VA_ARGS__);                    \
-        case 48: return FN<4, 2>(__VA_ARGS__);                    \
-        case 88: return FN<8, 2>(__VA_ARGS__);                    \
+        case 14: return FN<1, 1 OPT>(__VA_ARGS__);                \
+        case 24: return FN<2, 1 OPT>(__VA_ARGS__);                \
+        case 44: return FN<4, 1 OPT>(__VA_ARGS__);                \
+        case 84: return FN<8, 1 OPT>(__VA_ARGS__);                \
+        case 18: return FN<1, 2 OPT>(__VA_ARGS__);                \
+        case 28: return FN<2, 2 OPT>(__VA_ARGS__);                \
+        case 48: return FN<4, 2 OPT>(__VA_ARGS__);                \
+        case 88: return FN<8, 2 OPT>(__VA_ARGS__);                \
         default: return hipErrorInvalidValue;                     \
     }
+// The template arguments after the block shape (a macro argument with commas).
+#define LAYOUT(L, F4) , L, F4
 
 hipError_t bcsr(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
                 int lanes, int aligned, const int* rp, const int* col4,
                 const float* data, const float* x, bool x_aligned, float* y) {
     if (brows <= 0) return hipSuccess;
-    SHAPE_DISPATCH(bcsr_shape, s, brows, rows, cols, lanes, aligned, rp, col4,
+    SHAPE_DISPATCH(bcsr_shape, , s, brows, rows, cols, lanes, aligned, rp, col4,
                    data, x, x_aligned, y)
-}
-
-template <int BH, int BW4>
-static hipError_t bcsr_slots_shape(hipStream_t s, int brows, int rows, int cols, int hal, int nslots,
-                                   const int* col4, const float* data, const float* x, bool xa, float* y) {
-    hipLaunchKernelGGL((bcsr_slots_kernel<BH, BW4>), dim3(grid_for(brows)), dim3(kBlock), 0, s, brows, rows, cols,
-                       hal, nslots, col4, data, x, xa, y);
-    return hipGetLastError();
 }
 
 hipError_t bcsr_slots(hipStream_t s, int brows, int rows, int cols, int bh, int bw, int hal, int nslots,
                       const int* col4, const float* data, const float* x, bool x_aligned, float* y) {
     if (brows <= 0 || nslots <= 0) return hipSuccess;
     if (hal < brows || nslots > kBcsrSlotsMax) return hipErrorInvalidValue;
-    SHAPE_DISPATCH(bcsr_slots_shape, s, brows, rows, cols, hal, nslots, col4, data, x, x_aligned, y)
-}
-
-template <int BH, int BW4>
-static hipError_t bell_shape(hipStream_t s, int brows, int rows, int cols,
-                             int method, int hal, int f4, int ellnum,
-                             const int* col4, const float* data, const float* x,
-                             bool xa, float* y) {
-    const int grid = grid_for(brows);
-    if (method == 1)
-        hipLaunchKernelGGL((bell_kernel<BH, BW4, true>), dim3(grid), dim3(kBlock), 0, s,
-                           brows, rows, cols, hal, f4, ellnum, col4, data, x, xa, y);
-    else
-        hipLaunchKernelGGL((bell_kernel<BH, BW4, false>), dim3(grid), dim3(kBlock), 0, s,
-                           brows, rows, cols, hal, f4, ellnum, col4, data, x, xa, y);
-    return hipGetLastError();
+    SHAPE_DISPATCH(block_rows, LAYOUT(kBcsrSlots, false), s, brows, rows, cols, hal, 4 * hal, nslots, nullptr, col4,
+                   data, x, x_aligned, y)
 }
 
 hipError_t bell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
                 int method, int hal, int f4, int ellnum, const int* col4,
                 const float* data, const float* x, bool x_aligned, float* y) {
     if (brows <= 0 || ellnum <= 0) return hipSuccess;
-    SHAPE_DISPATCH(bell_shape, s, brows, rows, cols, method, hal, f4, ellnum,
-                   col4, data, x, x_aligned, y)
-}
-
-template <int BH, int BW4>
-static hipError_t sbell_shape(hipStream_t s, int brows, int rows, int cols,
-                              int sh, const int* sptr, const int* col4,
-                              const float* data, const float* x, bool xa, float* y) {
-    hipLaunchKernelGGL((sbell_kernel<BH, BW4>), dim3(grid_for(brows)), dim3(kBlock), 0, s,
-                       brows, rows, cols, sh, sptr, col4, data, x, xa, y);
-    return hipGetLastError();
+    if (method == 1)
+        SHAPE_DISPATCH(block_rows, LAYOUT(kBell, true), s, brows, rows, cols, hal, f4, ellnum, nullptr, col4, data, x,
+                       x_aligned, y)
+    SHAPE_DISPATCH(block_rows, LAYOUT(kBell, false), s, brows, rows, cols, hal, f4, ellnum, nullptr, col4, data, x,
+                   x_aligned, y)
 }
 
 hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
@@ -276,10 +272,11 @@ hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
                  const float* data, const float* x, bool x_aligned, float* y) {
     if (brows <= 0) return hipSuccess;
     if (slice_height <= 0) return hipErrorInvalidValue;
-    SHAPE_DISPATCH(sbell_shape, s, brows, rows, cols, slice_height, sptr, col4,
-                   data, x, x_aligned, y)
+    SHAPE_DISPATCH(block_rows, LAYOUT(kSbell, false), s, brows, rows, cols, slice_height, 0, 0, sptr, col4, data, x,
+                   x_aligned, y)
 }
 
+#undef LAYOUT
 #undef SHAPE_DISPATCH
 
 }  // namespace launch

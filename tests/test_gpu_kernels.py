@@ -490,6 +490,35 @@ def test_ell_slot_groups(ctx, oracle, width, rows):
     _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
     _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
 
+@pytest.mark.parametrize("shape", [(4, 1), (4, 2), (4, 4), (4, 8), (8, 1), (8, 4), (8, 8)])
+@pytest.mark.parametrize("width", [1, 2, 3, 4, 5, 7, 8, 9, 12, 13])
+def test_block_slot_groups(ctx, oracle, shape, width):
+    """Block rows of width and width - 1 blocks around the groups of slots in
+    flight, SBELL slices of different widths (one empty) in one wave, rows and
+    columns that are no multiple of the block; dyadic inputs, exact sums."""
+    bw, bh = shape
+    rng = np.random.default_rng(width)
+    nbr = 131
+    lens = np.where(np.arange(nbr) % 12 == 5, width - 1, width)
+    br = np.repeat(np.arange(nbr), lens)
+    bc = br + np.arange(br.size) - (np.cumsum(lens) - lens)[br]  # consecutive block columns
+    r = (br[:, None, None] * bh + np.arange(bh)[:, None] + np.zeros(bw, int)).reshape(-1)
+    c = (bc[:, None, None] * bw + np.zeros((bh, 1), int) + np.arange(bw)).reshape(-1)
+    o = np.lexsort((c, r))
+    rows, cols = nbr * bh - bh // 2, (nbr + width - 1) * bw - 3
+    o = o[(r[o] < rows) & (c[o] < cols)]
+    A = cs.Coo(r[o].astype(np.int32), c[o].astype(np.int32), (rng.integers(-64, 65, o.size) / 64.0).astype(np.float32),
+               rows, cols)
+    b = cs.coo2b4csr(A.copy(), bw, bh)
+    assert _bcsr_slots(b) == width
+    _run(ctx, oracle, A, b, 0)
+    for m in (0, 1):
+        _run(ctx, oracle, A, cs.coo2b4ell(A.copy(), bw, bh), m)
+    keep = (r[o] // bh) // 32 != 1  # block rows 32..63 empty: an empty slice beside a full one
+    E = cs.Coo(A.row[keep], A.col[keep], A.val[keep], rows, cols)
+    _run(ctx, oracle, E, cs.coo2sbell(E.copy(), bw, bh), 0)
+
+
 @pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16])
 @pytest.mark.parametrize("x_offset", [0, 1])
 def test_csr_multi_units(ctx, dtype, x_offset):
