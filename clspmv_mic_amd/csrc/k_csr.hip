@@ -100,6 +100,13 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
 // rows, 12.5 M entries, windows of 4.5 K floats: 32 -> 22 us (75 us with
 // csr_vector).  A work-group whose window is too wide (count 0) gathers from
 // memory.
+// A skewed block (a row of 400 entries among 50 of a few) would leave the long
+// row's sum to the one or two lanes its row count gives each row; rows of more
+// than kWideRow entries per lane go to the whole wave instead: power-law rows,
+// 30,000: 9.7 -> 5.5 us, 270,342: 36 -> 32.7 us (16 per lane: mesh of 50,009
+// rows 5.8 -> 7.9 us; 32 no different; 128: 6.4 us on the 30,000 rows).
+constexpr int kWideRow = 64;
+
 template <class V, bool WIN>
 __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
     int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
@@ -171,7 +178,18 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
     }
     wave_lds_order();
     float acc = 0.0f;
-    if (live) {
+    // Rows much longer than the others of their block, one after the other by
+    // the whole wave.
+    const bool wide = k1 - k0 > kWideRow * g;
+    for (unsigned long long m = __ballot(live && wide && gl == 0); m; m &= m - 1) {
+        const int l = __builtin_ctzll(m);
+        const int e = __builtin_amdgcn_readlane(k1, l);
+        float a = 0.0f;
+        for (int k = __builtin_amdgcn_readlane(k0, l) + lane; k < e; k += kWave) a += prod[k];
+        a = group_sum<kWave>(a);
+        if (lane == l) acc = a;
+    }
+    if (live && !wide) {
         float a1 = 0.0f, a2 = 0.0f, a3 = 0.0f;
         int k = k0 + gl;
         for (; k + 3 * g < k1; k += 4 * g) {

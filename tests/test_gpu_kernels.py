@@ -490,6 +490,25 @@ def test_ell_slot_groups(ctx, oracle, width, rows):
     _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
     _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
 
+@pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16])
+@pytest.mark.parametrize("others", [0, 1, 2, 15, 31, 32, 62, 63])
+def test_csr_wide_rows(ctx, oracle, others, dtype):
+    """Rows around the wave kernel's bound for rows summed by the whole wave
+    (64, 65, 128, ... entries beside `others` rows of up to two, in front of
+    and behind them; several in a block), longer ones of mixed lengths among
+    them; dyadic inputs, exact sums."""
+    lens = []
+    for wide in (63, 64, 65, 127, 128, 129, 256, 257, 300, 511, 512, 513, 700, 600):
+        lens += [wide] + [j % 3 for j in range(others)] + [wide]
+    lens += [65, 70, 0, 66, 100, 1, 3, 65]
+    rng = np.random.default_rng(others)
+    r = np.repeat(np.arange(len(lens)), lens)
+    c = np.concatenate([np.sort(rng.choice(900, n, replace=False)) for n in lens])
+    A = cs.Coo(r.astype(np.int32), c.astype(np.int32), (rng.integers(-64, 65, r.size) / 64.0).astype(np.float32),
+               len(lens), 900)
+    _run(ctx, oracle, A, cs.coo2csr(A.copy()), cs.METHOD_AUTO, panel=0, dtype=dtype)
+
+
 @pytest.mark.parametrize("shape", [(4, 1), (4, 2), (4, 4), (4, 8), (8, 1), (8, 4), (8, 8)])
 @pytest.mark.parametrize("width", [1, 2, 3, 4, 5, 7, 8, 9, 12, 13])
 def test_block_slot_groups(ctx, oracle, shape, width):
