@@ -201,7 +201,7 @@ int make_flat(hipStream_t s, int format, int dim, int width, int slice_h, clspmv
             if (!st) st = fillf(s, m->val, nnz + launch::kWaveNnz, 1.0f);
             std::vector<int> rp(dim + 1);
             for (int r = 0; r <= dim; ++r) rp[r] = r * width;
-            if (!st) st = build_csr_wave(m, rp.data(), dim, nullptr);
+            if (!st) st = build_csr_wave(m, rp.data(), dim);
             // Row blocks for constant row length.
             std::vector<int> blocks{0};
             if (width > launch::kAdaptiveNnz) {

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kernels.hpp"
+
 namespace clspmv {
 namespace dev {
 
@@ -117,6 +119,45 @@ struct VecOf<T, 1> {
 template <class T, int N>
 struct UVec {
     typedef typename VecOf<T, N>::type type __attribute__((aligned(sizeof(T))));
+};
+
+// x chunks of a work-group of kThreads threads (launch::XStage): ids() loads
+// the list, to be called before the work-group's streams so that waiting for
+// it does not wait for them; fetch() loads the chunks into xs, four threads
+// each (columns at or past `cols` as zeros), and ends with the work-group's
+// barrier.
+template <int kThreads>
+struct StageX {
+    static constexpr int kPer = kThreads * 4 / launch::kXChunk;  // chunks per round
+    static constexpr int kRounds = launch::kXChunksMax / kPer;
+    int ch[kRounds];
+    __device__ __forceinline__ void ids(const int* __restrict__ list, int stride) {
+        const int i = threadIdx.x / (launch::kXChunk / 4);
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            ch[j] = -1;
+            if (j * kPer < stride && j * kPer + i < stride) ch[j] = list[j * kPer + i];
+        }
+    }
+    __device__ __forceinline__ void fetch(int stride, int cols, const float* __restrict__ x, float* xs) {
+        constexpr int L = launch::kXChunk / 4;
+        f32x4 v[kRounds];
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j) {
+            if (ch[j] < 0) continue;
+            const int e = ch[j] * launch::kXChunk + threadIdx.x % L * 4;
+            if (e + 4 <= cols) {
+                v[j] = *reinterpret_cast<const typename UVec<float, 4>::type*>(x + e);
+            } else {
+#pragma unroll
+                for (int h = 0; h < 4; ++h) v[j][h] = e + h < cols ? x[e + h] : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kRounds; ++j)
+            if (ch[j] >= 0) *reinterpret_cast<f32x4*>(xs + j * kPer * launch::kXChunk + threadIdx.x * 4) = v[j];
+        __syncthreads();
+    }
 };
 
 // The lane's value from another lane of its 16-lane row, by DPP (no LDS

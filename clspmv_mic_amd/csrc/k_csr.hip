@@ -92,14 +92,15 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
 // with a barrier: 27-point stencil 77^3 52 / 31 -> 24 us, 5-point Laplacian
 // 701^2 15 / 10.5 -> 8 us.
 //
-// WIN: the columns of neighbouring rows are near each other but scattered
-// within the lines (meshes): a gather instruction then touches up to 64
-// lines and L1's tag rate bounds the kernel.  The work-group stages the
-// x window of its waves' columns ({first column, count} in `win`) in LDS
-// while the waves' entries are in flight and gathers there: mesh of 500,009
-// rows, 12.5 M entries, windows of 4.5 K floats: 32 -> 22 us (75 us with
-// csr_vector).  A work-group whose window is too wide (count 0) gathers from
-// memory.
+// WIN: gathers through L1 return in order behind the streams; without them
+// the 27-point stencil 97^3 (24.6 M entries) ran in 31.8 us instead of 47.7.
+// Where the rows of a work-group share x, it stages their chunks of x in LDS
+// (launch::XStage) while the entries are in flight and gathers there, by
+// 16-bit places instead of 32-bit columns (6 bytes an entry): 77^3 23.9 -> 16.5
+// us, 97^3 48.1 -> 33.2, 5-point Laplacian 1300^2 20.9 -> 16.9, mesh of 700,000
+// rows 34.9 -> 28.6 us (with one window of consecutive columns staged and
+// 32-bit columns), the stencil 30^3 4.8 -> 4.2 us.
+//
 // A skewed block (a row of 400 entries among 50 of a few) would leave the long
 // row's sum to the one or two lanes its row count gives each row; rows of more
 // than kWideRow entries per lane go to the whole wave instead: power-law rows,
@@ -110,12 +111,14 @@ constexpr int kWideRow = 64;
 template <class V, bool WIN>
 __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
     int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
-    const int2* __restrict__ win, int wmax, const int* __restrict__ rp, const int* __restrict__ col,
+    const int* __restrict__ list, const unsigned short* __restrict__ idx, int stride, int cols,
+    const int* __restrict__ rp, const int* __restrict__ col,
     const typename V::T* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
     constexpr int U = launch::kWaveNnz / kWave, P4 = kWave * 4;
     typedef typename V::T T;
     typedef typename UVec<T, 4>::type T4U;
-    extern __shared__ __attribute__((aligned(16))) float sm[];  // x window, then the products of each wave
+    typedef VecOf<unsigned short, 4> I4;
+    extern __shared__ __attribute__((aligned(16))) float sm[];  // x chunks, then the products of each wave
     if ((int)blockIdx.x < nlong) {  // the longest work first
         const int r = longs[blockIdx.x], s = rp[r], e = rp[r + 1];
         double* part = reinterpret_cast<double*>(sm);
@@ -129,15 +132,22 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
     const int wg = xcd_tile(blockIdx.x - nlong, gridDim.x - nlong);
     const int b = __builtin_amdgcn_readfirstlane(wg * launch::kCsrWaves + wave);
     if (!WIN && b >= nblk) return;
+    StageX<kWave * launch::kCsrWaves> stage;
+    if constexpr (WIN) stage.ids(list + (size_t)wg * stride, stride);
     int4 B = blk[min(b, nblk - 1)];  // {first row, rows, first entry, entries}
     if (WIN && b >= nblk) B.y = B.w = 0;
     const int nrows = B.y, s = B.z, n = B.w;
     i32x4 c[U / 4];
+    typename I4::type ix[U / 4];
     typename VecOf<T, 4>::type v[U / 4];
 #pragma unroll
     for (int u = 0; u < U / 4; ++u) {
-        c[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<int, 4>::type*>(col + s + u * P4 + lane * 4));
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const T4U*>(val + s + u * P4 + lane * 4));
+        const int at = s + u * P4 + lane * 4;
+        if constexpr (WIN)
+            ix[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<unsigned short, 4>::type*>(idx + at));
+        else
+            c[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<int, 4>::type*>(col + at));
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const T4U*>(val + at));
     }
     // Lane groups for the sums: the largest power of two with nrows groups in
     // the wave (a block holds at most kWave rows).
@@ -147,26 +157,16 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
     const int r = B.x + (live ? lane >> sh : 0);
     const int k0 = rp[r] - s, k1 = rp[r + 1] - s;
     const float yv = y[r];
-    float* prod = sm + (WIN ? wmax : 0) + wave * launch::kWaveNnz;
-    int2 w = make_int2(0, 0);
-    if constexpr (WIN) {
-        w = win[wg];
-        for (int i = threadIdx.x * 4; i < w.y; i += kWave * launch::kCsrWaves * 4) {
-            if (i + 4 <= w.y)
-                *reinterpret_cast<f32x4*>(sm + i) = *reinterpret_cast<const UVec<float, 4>::type*>(x + w.x + i);
-            else
-                for (int h = i; h < w.y; ++h) sm[h] = x[w.x + h];
-        }
-        __syncthreads();
-    }
+    float* prod = sm + (WIN ? stride * launch::kXChunk : 0) + wave * launch::kWaveNnz;
+    if constexpr (WIN) stage.fetch(stride, cols, x, sm);
+    const unsigned last = (unsigned)stride * launch::kXChunk - 1u;
 #pragma unroll
     for (int u = 0; u < U / 4; ++u) {
         if (u * P4 + lane * 4 >= n) continue;
         f32x4 p;
-        if (WIN && w.y > 0) {  // uniform; entries past the block clamp into the window
+        if constexpr (WIN) {  // entries past the block are another work-group's: clamped, not read
 #pragma unroll
-            for (int h = 0; h < 4; ++h)
-                p[h] = V::cvt(v[u][h]) * sm[min((unsigned)(c[u][h] - w.x), (unsigned)w.y - 1u)];
+            for (int h = 0; h < 4; ++h) p[h] = V::cvt(v[u][h]) * sm[min((unsigned)I4::get(ix[u], h), last)];
         } else {
             float xv[4];
 #pragma unroll
@@ -207,16 +207,17 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
 
 template <class V>
 hipError_t csr_wave_v(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
-                      const float* x, float* y) {
+                      int cols, const float* x, float* y) {
     const dim3 grid(W.nlong + (W.nblk + launch::kCsrWaves - 1) / launch::kCsrWaves), block(kWave * launch::kCsrWaves);
     const size_t lds = sizeof(float) * launch::kWaveNnz * launch::kCsrWaves;
     const typename V::T* v = static_cast<const typename V::T*>(val);
-    if (W.win)
-        hipLaunchKernelGGL((csr_wave_kernel<V, true>), grid, block, lds + sizeof(float) * W.wmax, s, W.nlong, W.longs,
-                           W.nblk, W.blk, W.win, W.wmax, rp, col, v, x, y);
+    if (W.stage.list)
+        hipLaunchKernelGGL((csr_wave_kernel<V, true>), grid, block,
+                           lds + sizeof(float) * launch::kXChunk * W.stage.stride, s, W.nlong, W.longs, W.nblk, W.blk,
+                           W.stage.list, W.stage.idx, W.stage.stride, cols, rp, col, v, x, y);
     else
-        hipLaunchKernelGGL((csr_wave_kernel<V, false>), grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, W.win,
-                           0, rp, col, v, x, y);
+        hipLaunchKernelGGL((csr_wave_kernel<V, false>), grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, nullptr,
+                           nullptr, 0, cols, rp, col, v, x, y);
     return hipGetLastError();
 }
 
@@ -243,12 +244,12 @@ hipError_t csr_vector(hipStream_t s, int rows, int lanes, const int* rp,
 }
 
 hipError_t csr_wave(hipStream_t s, const CsrWave& W, const int* rp, const int* col, int dtype, const void* val,
-                    const float* x, float* y) {
+                    int cols, const float* x, float* y) {
     if (W.nblk + W.nlong <= 0) return hipSuccess;
     switch (dtype) {
-        case 0: return csr_wave_v<ValF32>(s, W, rp, col, val, x, y);
-        case 1: return csr_wave_v<ValBF16>(s, W, rp, col, val, x, y);
-        case 2: return csr_wave_v<ValF16>(s, W, rp, col, val, x, y);
+        case 0: return csr_wave_v<ValF32>(s, W, rp, col, val, cols, x, y);
+        case 1: return csr_wave_v<ValBF16>(s, W, rp, col, val, cols, x, y);
+        case 2: return csr_wave_v<ValF16>(s, W, rp, col, val, cols, x, y);
         default: return hipErrorInvalidValue;
     }
 }

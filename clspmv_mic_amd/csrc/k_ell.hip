@@ -26,30 +26,40 @@ using namespace dev;
 // 14.4 / 15.2 us on a mesh of 40,000 rows; this takes 6.5 / 7.1 and 10.2 /
 // 11.1 us.
 //
-// WIN: where neighbouring rows' columns are near each other but scattered
-// over lines (meshes) the work-group stages the x window of its rows
-// ({first column, count} in `win`; 0: gather from memory) in LDS and gathers
-// there, past L1's tag rate: mesh of 500,009 rows 60 / 63 -> 29 / 29 us, of
-// which reading the padded slots takes 23 us.
+// WIN: the work-group stages the chunks of x that its rows touch in LDS and
+// gathers there, by 16-bit places instead of 32-bit columns (launch::XStage;
+// two slots to a word, so that a word is loaded as it is used: single 16-bit
+// loads were widened behind a wait for the next slots').  ELL / SELL, against
+// gathering from memory, for meshes against one window of consecutive columns
+// in LDS: 27-point stencil 30^3 5.6 / 8.8 -> 4.5 / 6.1 us, 97^3 37.0 / 39.2 ->
+// 29.0 / 30.4, mesh of 20,000 rows 9.7 / 10.5 -> 6.2 / 6.9, 700,000 40.1 / 43.3
+// -> 32.0 / 33.7 us.
 template <bool SELL, bool WIN, int kSlots>
 __global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
-    int rows, int h, int w0, const int* __restrict__ ptr, const int2* __restrict__ win,
-    const int* __restrict__ col, const float* __restrict__ val, const float* __restrict__ x,
+    int rows, int h, int w0, const int* __restrict__ ptr, const int* __restrict__ list, const unsigned short* __restrict__ idx,
+    int stride, int cols, const int* __restrict__ col, const float* __restrict__ val, const float* __restrict__ x,
     float* __restrict__ y) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     const int wg = xcd_tile(blockIdx.x, gridDim.x);
     const int row = wg * launch::kEllRows + (int)threadIdx.x;
     const int r = min(row, rows - 1);  // lanes past the end shadow the last row
     int w = w0;
-    const int* cp = col + r;
-    const float* vp = val + r;
+    constexpr int kPer = WIN ? 2 : 1;  // slots per column word
+    const int* cp = WIN ? reinterpret_cast<const int*>(idx) : col;
+    const float* vp = val;
+    StageX<launch::kEllRows> stage;
+    if constexpr (WIN) stage.ids(list + (size_t)wg * stride, stride);
     if constexpr (SELL) {
-        const int sl = r / h, p0 = ptr[sl];
-        w = (ptr[sl + 1] - p0) / h;
+        const int sl = r / h, p0 = ptr[sl], q0 = p0 / h;
+        w = ptr[sl + 1] / h - q0;
         // A lane whose slice is empty reads entry 0 beside its neighbours (the
         // matrix has entries when they have any): at p0 there may be none.
-        cp = w > 0 ? col + p0 + (r - sl * h) : col;
-        vp = w > 0 ? val + p0 + (r - sl * h) : val;
+        const int i = r - sl * h;
+        cp += w > 0 ? (WIN ? (size_t)((q0 + sl) >> 1) * h + i : (size_t)p0 + i) : 0;
+        vp += w > 0 ? p0 + i : 0;
+    } else {
+        cp += r;
+        vp += r;
     }
     // The widest row of the wave: its slots are walked, and slots past the
     // lane's own last one re-read that one and are not added.
@@ -57,45 +67,37 @@ __global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
     if constexpr (SELL)
         for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
     wm = __builtin_amdgcn_readfirstlane(wm);
-    int c[2][kSlots];
+    int c[2][kSlots / kPer];
     float v[2][kSlots];
+    auto load_slot = [&](int s, int u, int* cc, float* vv) {
+        const int at = SELL ? max(min(s + u, w - 1), 0) : s + u;
+        if (u % kPer == 0) cc[u / kPer] = ld_stream(cp + (size_t)(at / kPer) * h);
+        vv[u] = ld_stream(vp + (size_t)at * h);
+    };
     auto load = [&](int s, int* cc, float* vv) {
 #pragma unroll
-        for (int u = 0; u < kSlots; ++u) {
-            const size_t at = (size_t)(SELL ? max(min(s + u, w - 1), 0) : s + u) * h;
-            cc[u] = ld_stream(cp + at);
-            vv[u] = ld_stream(vp + at);
-        }
+        for (int u = 0; u < kSlots; ++u) load_slot(s, u, cc, vv);
     };
     auto load_part = [&](int s, int* cc, float* vv) {  // slots below wm
 #pragma unroll
         for (int u = 0; u < kSlots; ++u) {
             if (s + u >= wm) break;
-            const size_t at = (size_t)(SELL ? max(min(s + u, w - 1), 0) : s + u) * h;
-            cc[u] = ld_stream(cp + at);
-            vv[u] = ld_stream(vp + at);
+            load_slot(s, u, cc, vv);
         }
     };
     if (kSlots <= wm) load(0, c[0], v[0]);
     else load_part(0, c[0], v[0]);
-    int2 wn = make_int2(0, 0);
-    if constexpr (WIN) {
-        wn = win[wg];
-        for (int i = threadIdx.x * 4; i < wn.y; i += launch::kEllRows * 4) {
-            if (i + 4 <= wn.y)
-                *reinterpret_cast<f32x4*>(xs + i) = *reinterpret_cast<const UVec<float, 4>::type*>(x + wn.x + i);
-            else
-                for (int e = i; e < wn.y; ++e) xs[e] = x[wn.x + e];
-        }
-        __syncthreads();
-    }
+    if constexpr (WIN) stage.fetch(stride, cols, x, xs);
+    const unsigned last = (unsigned)stride * launch::kXChunk - 1u;
     float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     auto add = [&](int s, const int* cc, const float* vv) {
         float xv[kSlots];
-        if (WIN && wn.y > 0) {
+        if constexpr (WIN) {  // entry 0 may be another work-group's: clamped, not added
 #pragma unroll
-            for (int u = 0; u < kSlots; ++u)
-                if (s + u < wm) xv[u] = xs[min((unsigned)(cc[u] - wn.x), (unsigned)wn.y - 1u)];
+            for (int u = 0; u < kSlots; ++u) {
+                const unsigned i = u % 2 ? (unsigned)cc[u / 2] >> 16 : cc[u / 2] & 0xFFFFu;
+                if (s + u < wm) xv[u] = xs[SELL ? min(i, last) : i];
+            }
         } else {
 #pragma unroll
             for (int u = 0; u < kSlots; ++u)
@@ -149,33 +151,33 @@ __global__ __launch_bounds__(kBlock) void ell4_kernel(
 // matters (stencil 77^3 19 against 22 us, 5-point Laplacian 701^2 5.9 against
 // 6.6 us).
 template <bool SELL, int kSlots>
-hipError_t ell_rows_k(hipStream_t s, int rows, int h, int w, const int* ptr, launch::EllWindows W, const int* col,
-                      const float* val, const float* x, float* y) {
+hipError_t ell_rows_k(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
+                      const float* val, int cols, const float* x, float* y) {
     const dim3 grid((rows + launch::kEllRows - 1) / launch::kEllRows), block(launch::kEllRows);
-    if (W.win)
-        hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots>), grid, block, sizeof(float) * W.max, s, rows, h, w, ptr,
-                           W.win, col, val, x, y);
+    if (W.list)
+        hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots>), grid, block, sizeof(float) * launch::kXChunk * W.stride,
+                           s, rows, h, w, ptr, W.list, W.idx, W.stride, cols, col, val, x, y);
     else
-        hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots>), grid, block, 0, s, rows, h, w, ptr, W.win, col, val,
-                           x, y);
+        hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots>), grid, block, 0, s, rows, h, w, ptr, nullptr, nullptr,
+                           0, cols, col, val, x, y);
     return hipGetLastError();
 }
 
 template <bool SELL>
-hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, launch::EllWindows W, const int* col,
-                    const float* val, const float* x, float* y) {
-    return rows < (1 << 17) ? ell_rows_k<SELL, 8>(s, rows, h, w, ptr, W, col, val, x, y)
-                            : ell_rows_k<SELL, 4>(s, rows, h, w, ptr, W, col, val, x, y);
+hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
+                    const float* val, int cols, const float* x, float* y) {
+    return rows < (1 << 17) ? ell_rows_k<SELL, 8>(s, rows, h, w, ptr, W, col, val, cols, x, y)
+                            : ell_rows_k<SELL, 4>(s, rows, h, w, ptr, W, col, val, cols, x, y);
 }
 
 }  // namespace
 
 namespace launch {
 
-hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, EllWindows W,
-               const int* col, const float* val, const float* x, float* y) {
+hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, XStage W,
+               const int* col, const float* val, int cols, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
-    if (rows_per_lane != 4) return ell_rows<false>(s, rows, hal, ellnum, nullptr, W, col, val, x, y);
+    if (rows_per_lane != 4) return ell_rows<false>(s, rows, hal, ellnum, nullptr, W, col, val, cols, x, y);
     if (hal % 4 != 0) return hipErrorInvalidValue;
     const int lanes = (rows + 3) / 4;
     hipLaunchKernelGGL(ell4_kernel, dim3((lanes + kBlock - 1) / kBlock),
@@ -183,11 +185,11 @@ hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, 
     return hipGetLastError();
 }
 
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, EllWindows W,
-                const int* col, const float* val, const float* x, float* y) {
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, XStage W,
+                const int* col, const float* val, int cols, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
     if (slice_height <= 0) return hipErrorInvalidValue;
-    return ell_rows<true>(s, rows, slice_height, 0, ptr, W, col, val, x, y);
+    return ell_rows<true>(s, rows, slice_height, 0, ptr, W, col, val, cols, x, y);
 }
 
 }  // namespace launch

@@ -20,26 +20,37 @@ constexpr int kAdaptiveRows = 256;
 // Rows longer than this are accumulated in FP64 by the 16-bit-value and
 // multi-vector CSR paths, the panel row sums and the block SpMM.
 constexpr int kLongRowF64 = 4096;
+// Staged x (null list: absent), for matrices whose neighbouring rows share
+// x: the aligned runs of kXChunk columns ("chunks") that the entries of each
+// work-group touch, at list[group * stride ..] (-1 past the last one, at most
+// kXChunksMax), and for every entry its column's place in the work-group's
+// staged chunks, position in the list * kXChunk + column % kXChunk: for CSR in
+// the order of the columns, for ELL and SELL two slots of a row to a 32-bit
+// word, the words laid out like the columns of (slots + 1) / 2 slots (SELL:
+// slice s's from word ((slots of the slices before it) + s) / 2 * height).
+constexpr int kXChunk = 16;
+constexpr int kXChunksMax = 512;
+struct XStage {
+    const int* list = nullptr;
+    const unsigned short* idx = nullptr;
+    int stride = 0;
+};
 // Wave kernel: blk holds {first row, rows (at most 64), first entry, entries
 // (at most kWaveNnz)} per wave, longs the rows with more entries; col and val
-// carry kWaveNnz entries of padding (column 0) after the last one.  win
-// (or null): {first column, columns} of x staged for each run of kCsrWaves
-// blocks, columns 0 where it gathers from memory; wmax the most columns of
-// one, at most kCsrWinMax, rounded up to a multiple of 4.
+// (and stage.idx) carry kWaveNnz entries of padding (column 0) after the last
+// one.  A work-group takes kCsrWaves blocks.
 constexpr int kWaveNnz = 512;
 constexpr int kCsrWaves = 8;
-constexpr int kCsrWinMax = 8192;
-static_assert(4 * (kWaveNnz * kCsrWaves + kCsrWinMax) <= 64 * 1024, "within the default LDS limit");
+static_assert(4 * (kWaveNnz * kCsrWaves + kXChunk * kXChunksMax) <= 64 * 1024, "within the default LDS limit");
 struct CsrWave {
     const int4* blk = nullptr;
     int nblk = 0;
     const int* longs = nullptr;
     int nlong = 0;
-    const int2* win = nullptr;
-    int wmax = 0;
+    XStage stage;
 };
 hipError_t csr_wave(hipStream_t s, const CsrWave& W, const int* rp, const int* col, int dtype, const void* val,
-                    const float* x, float* y);
+                    int cols, const float* x, float* y);
 
 // ---- COO ------------------------------------------------------------------
 // Row-sorted COO in chunks of kCooChunk entries; 2 carry slots per chunk.
@@ -110,19 +121,12 @@ hipError_t panel_pass2(hipStream_t s, const float* seg_val, int nblocks, const i
                        const int* longs, float* y);
 
 // ---- ELL / SELL --------------------------------------------------------------
-// win (or null): {first column, columns} of x for each kEllRows rows, staged
-// in LDS by their work-group; columns 0 where it gathers from memory; max the
-// most columns of one, at most kEllWinMax.
+// A work-group takes kEllRows rows.
 constexpr int kEllRows = 512;
-constexpr int kEllWinMax = 8192;
-struct EllWindows {
-    const int2* win = nullptr;
-    int max = 0;
-};
-hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, EllWindows W,
-               const int* col, const float* val, const float* x, float* y);
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, EllWindows W,
-                const int* col, const float* val, const float* x, float* y);
+hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, XStage W,
+               const int* col, const float* val, int cols, const float* x, float* y);
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, XStage W,
+                const int* col, const float* val, int cols, const float* x, float* y);
 
 // ---- DIA / BDIA -------------------------------------------------------------
 // rows = number of rows computed (min(height, dia_length_aligned)).

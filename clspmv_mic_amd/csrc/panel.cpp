@@ -368,7 +368,8 @@ void drop_encoding(clspmv_dmat* d, bool panel) {
     release_array(d, &d->blocks);
     release_array(d, &d->wblk);
     release_array(d, &d->wlong);
-    release_array(d, &d->wwin);
+    release_array(d, &d->xlist);
+    release_array(d, &d->xidx);
     d->plain = false;
     d->use_panel = true;
 }

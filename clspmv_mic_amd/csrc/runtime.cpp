@@ -14,7 +14,10 @@
 #include <climits>
 #include <cmath>
 #include <cstdint>
+#include <exception>
+#include <memory>
 #include <numeric>
+#include <thread>
 
 #include "kernels.hpp"
 #include "runtime.hpp"
@@ -129,45 +132,155 @@ struct ColRange {
     bool within(int cols) const { return lo >= 0 && hi < cols; }
 };
 
-// x windows (launch::CsrWave, launch::EllWindows) for the work-groups whose
-// columns are `range`, where neighbouring rows' columns are near each other
-// but scattered over the 128-byte lines of x: a gather instruction then
-// touches many lines and L1's tag rate bounds the kernel, while the window
-// costs one coalesced pass.  sample(g, cols) gives the 64 columns of one gather
-// instruction of group g (false: none); they are looked at on up to 256 groups
-// and must touch 24 lines on average.  A group wider than `limit` gathers
-// from memory, and with more than one in ten of those the matrix gets no
-// windows.
-template <class Sample>
-int add_windows(clspmv_dmat* d, const std::vector<ColRange>& range, int limit, Sample&& sample) {
-    const size_t groups = range.size();
-    long long lines = 0, samples = 0;
-    for (size_t g = 0, step = std::max<size_t>(1, groups / 256); g < groups; g += step) {
-        int line[64];
-        if (!sample(g, line)) continue;
-        for (int& l : line) l /= 32;
-        std::sort(line, line + 64);
-        lines += std::unique(line, line + 64) - line;
-        ++samples;
+// x is staged from this many entries per chunk, and per work-group, on
+// (random columns in a band, staged against gathered, us; 1 M rows of 4: 5
+// entries per chunk CSR 13.6 / 18.7, ELL 10.1 / 14.8, 9 per chunk 11.5 / 14.7
+// and 8.8 / 10.9; rows of 2 and 1 entries, ELL: 6.7 / 6.6 and 6.3 / 5.2).
+// Matrices of few work-groups wait for the list and the chunks: 60,000 rows
+// of 4, 5 entries per chunk, CSR 6.2 / 5.8, ELL 6.0 / 5.4; the 27-point stencil
+// 30^3, 40 per chunk, gains: CSR 4.2 / 4.8, ELL 4.5 / 5.6.
+constexpr int kEntriesPerChunk = 4, kFewGroups = 256, kEntriesPerChunkFew = 8, kEntriesPerGroup = 1536;
+
+// A work-group's chunks and its entries' places in them.  runs(g, f) calls
+// f(first entry, count, to, step) for the entries of group g: entry first + i's
+// place goes to idx[to + i * step].
+struct ChunkMap {
+    std::vector<long long> seen;  // per chunk: the last group that touched it, + 1
+    std::vector<int> place;       // and its place in that group's list
+    explicit ChunkMap(int cols) : seen((size_t)cols / launch::kXChunk + 1), place(seen.size()) {}
+    // idx null: only counts.  Returns the chunks (more than kXChunksMax: idx is
+    // not complete), adds the entries.
+    template <class Runs>
+    int group(size_t g, const int* col, const Runs& runs, unsigned short* idx, std::vector<int>* list,
+              long long* entries) {
+        int n = 0;
+        long long total = 0;
+        runs(g, [&](size_t first, size_t count, size_t to, size_t step) {
+            total += (long long)count;
+            for (size_t e = first; e < first + count && n <= launch::kXChunksMax; ++e, to += step) {
+                const size_t c = (size_t)(col[e] / launch::kXChunk);
+                if (seen[c] != (long long)g + 1) {
+                    seen[c] = (long long)g + 1;
+                    place[c] = n++;
+                    if (list) list->push_back((int)c);
+                }
+                if (idx) idx[to] = (unsigned short)(place[c] * launch::kXChunk + col[e] % launch::kXChunk);
+            }
+        });
+        *entries += total;
+        return n;
     }
-    if (samples == 0 || lines < 24 * samples) return CLSPMV_OK;
-    std::vector<int2> win(groups);
-    size_t wide = 0;
-    int wmax = 0;
-    for (size_t g = 0; g < groups; ++g) {
-        const int n = range[g].hi < 0 ? 0 : range[g].hi - range[g].lo + 1;
-        win[g] = n > 0 && n <= limit ? make_int2(range[g].lo, n) : make_int2(0, 0);
-        wide += n > limit;
-        wmax = std::max(wmax, win[g].y);
+};
+
+// Staged x (launch::XStage) of a matrix with `total` entries (columns checked)
+// in `groups` work-groups, when every group's chunks fit and the entries per
+// chunk pay for the staging.  start() builds it on threads of its own while
+// the caller uploads the matrix (col and what `runs` refers to must outlive
+// the object); finish() uploads it.  places: 16-bit words of idx.  Without the
+// host or device memory for it the matrix goes without.
+class StageBuild {
+public:
+    ~StageBuild() {
+        if (main_.joinable()) main_.join();
     }
-    if (wide * 10 > groups) return CLSPMV_OK;
-    d->wwin_max = round_up(wmax, 4);
-    return upload_array(d, win.data(), win.size(), &d->wwin);
-}
+    template <class Runs>
+    void start(int cols, size_t groups, const int* col, size_t total, size_t places, Runs runs) {
+        if (groups == 0 || total == 0) return;
+        if (total >= (1u << 18)) {
+            try {
+                main_ = std::thread([=] { build(cols, groups, col, total, places, runs); });
+                return;
+            } catch (const std::exception&) {  // no thread: here
+            }
+        }
+        build(cols, groups, col, total, places, runs);
+    }
+    int finish(clspmv_dmat* d) {
+        if (main_.joinable()) main_.join();
+        if (stride_ == 0) return CLSPMV_OK;
+        if (upload_array(d, list_.data(), list_.size(), &d->xlist) || upload_array(d, idx_.get(), places_, &d->xidx)) {
+            release_array(d, &d->xlist);
+            release_array(d, &d->xidx);
+            (void)hipGetLastError();
+            return CLSPMV_OK;
+        }
+        d->xstride = stride_;
+        return CLSPMV_OK;
+    }
+
+private:
+    template <class Runs>
+    void build(int cols, size_t groups, const int* col, size_t total, size_t places, const Runs& runs) {
+        try {
+            {  // a look at up to 64 groups
+                ChunkMap map(cols);
+                long long chunks = 0, entries = 0, looked = 0;
+                for (size_t g = 0, step = std::max<size_t>(1, groups / 64); g < groups; g += step) {
+                    const int n = map.group(g, col, runs, nullptr, nullptr, &entries);
+                    if (n > launch::kXChunksMax) return;
+                    chunks += n;
+                    ++looked;
+                }
+                const int per_chunk = groups < kFewGroups ? kEntriesPerChunkFew : kEntriesPerChunk;
+                if (entries < per_chunk * chunks || entries < kEntriesPerGroup * looked) return;
+            }
+            // The groups in `parts` runs of about as many, a thread each.
+            const size_t parts = std::min<size_t>(total < (1u << 20) ? 1 : 8, groups);
+            idx_.reset(new unsigned short[places]);  // the threads' pages are theirs to touch first
+            const size_t pad = std::min<size_t>(places, launch::kWaveNnz);
+            std::fill_n(idx_.get() + places - pad, pad, (unsigned short)0);
+            std::vector<int> count(groups);
+            std::vector<std::vector<int>> lists(parts);
+            std::vector<char> ok(parts, 0);
+            auto part = [&](size_t p) {
+                try {
+                    ChunkMap map(cols);
+                    long long entries = 0;
+                    for (size_t g = groups * p / parts; g < groups * (p + 1) / parts; ++g) {
+                        count[g] = map.group(g, col, runs, idx_.get(), &lists[p], &entries);
+                        if (count[g] > launch::kXChunksMax) return;
+                    }
+                    ok[p] = 1;
+                } catch (const std::exception&) {  // not complete
+                }
+            };
+            std::vector<std::thread> threads;
+            threads.reserve(parts);
+            for (size_t p = 1; p < parts; ++p) {
+                try {
+                    threads.emplace_back(part, p);
+                } catch (const std::exception&) {
+                    part(p);
+                }
+            }
+            part(0);
+            for (std::thread& t : threads) t.join();
+            if (std::count(ok.begin(), ok.end(), 1) != (long)parts) return;
+            const int stride = *std::max_element(count.begin(), count.end());
+            list_.assign(groups * (size_t)stride, -1);
+            for (size_t p = 0; p < parts; ++p) {
+                const int* from = lists[p].data();
+                for (size_t g = groups * p / parts; g < groups * (p + 1) / parts; ++g) {
+                    std::copy_n(from, count[g], list_.begin() + g * stride);
+                    from += count[g];
+                }
+            }
+            places_ = places;
+            stride_ = stride;
+        } catch (const std::exception&) {  // no host memory for it
+        }
+    }
+
+    std::thread main_;
+    std::vector<int> list_;
+    std::unique_ptr<unsigned short[]> idx_;
+    size_t places_ = 0;
+    int stride_ = 0;
+};
 
 }  // namespace
 
-int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
+int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks) {
     std::vector<int4> blk;
     std::vector<int> longs;
     for (int r = 0; r < rows;) {
@@ -187,22 +300,8 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col) {
     d->nwlong = (int)longs.size();
     int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
     if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
-    if (st || !col) return st;
-    // x windows where they pay: mesh of 500,009 rows (a gather instruction
-    // touches 52 lines, windows of 4.5 K columns) 22 us against 32; 27-point
-    // stencil 47^3 (16 lines, 4.6 K columns) 10.2 against 8.0 us.
-    constexpr int W = launch::kCsrWaves;
-    std::vector<ColRange> range((blk.size() + W - 1) / W);
-    for (size_t b = 0; b < blk.size(); ++b) range[b / W].widen(col + blk[b].z, blk[b].w);
-    ColRange all;  // of the long rows, then of all entries
-    for (int r : longs) all.widen(col + rp[r], rp[r + 1] - rp[r]);
-    for (const ColRange& g : range) all.lo = std::min(all.lo, g.lo), all.hi = std::max(all.hi, g.hi);
-    if (rp[rows] > 0 && !all.within(d->info.cols)) return check_cols(col, rp[rows], d->info.cols, 1, "csr");
-    return add_windows(d, range, launch::kCsrWinMax, [&](size_t g, int* line) {
-        const int4 b = blk[g * W];
-        for (int i = 0; i < 64 && b.w >= 256; ++i) line[i] = col[b.z + 4 * i];
-        return b.w >= 256;
-    });
+    if (blocks) *blocks = std::move(blk);
+    return st;
 }
 
 int auto_method(const clspmv_dmat* A) {
@@ -253,8 +352,10 @@ int dmat_prepass(hipStream_t s, const clspmv_dmat* A, const float* x, const clsp
 namespace {
 launch::DiaSegments segments_of(const clspmv_dmat* A) { return launch::DiaSegments{A->dseg, A->ndseg, A->seg_w}; }
 
+launch::XStage stage_of(const clspmv_dmat* A) { return launch::XStage{A->xlist, A->xidx, A->xstride}; }
+
 launch::CsrWave csr_wave_of(const clspmv_dmat* A) {
-    return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->wwin, A->wwin_max};
+    return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, stage_of(A)};
 }
 
 int resolve_method(const clspmv_dmat* A, int* method) {
@@ -298,7 +399,7 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
                 e = launch::csr_vector(s, I.rows, A->lanes, A->rp, A->col, A->val, x, y);
             else
                 e = launch::csr_wave(s, csr_wave_of(A), A->rp, A->col, A->dtype,
-                                     A->dtype ? (const void*)A->lpval : (const void*)A->val, x, y);
+                                     A->dtype ? (const void*)A->lpval : (const void*)A->val, I.cols, x, y);
             break;
         case CLSPMV_FMT_COO:
             e = launch::coo_segreduce(s, I.nnz, A->row, A->col, A->val, x, y,
@@ -307,12 +408,12 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
         case CLSPMV_FMT_ELL:
             if (method == 1 && A->hal % 4 != 0)
                 return fail(CLSPMV_ERR_UNSUPPORTED, "ELL method 1 needs height_aligned %% 4 == 0");
-            e = launch::ell(s, I.rows, A->hal, A->ellnum, method == 1 ? 4 : 1, launch::EllWindows{A->wwin, A->wwin_max},
-                            A->col, A->val, x, y);
+            e = launch::ell(s, I.rows, A->hal, A->ellnum, method == 1 ? 4 : 1, stage_of(A),
+                            A->col, A->val, I.cols, x, y);
             break;
         case CLSPMV_FMT_SELL:
-            e = launch::sell(s, I.rows, I.slice_height, A->sptr, launch::EllWindows{A->wwin, A->wwin_max}, A->col,
-                             A->val, x, y);
+            e = launch::sell(s, I.rows, I.slice_height, A->sptr, stage_of(A), A->col,
+                             A->val, I.cols, x, y);
             break;
         case CLSPMV_FMT_DIA: {
             const int span = A->max_off - A->min_off;
@@ -606,7 +707,19 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     d->max_row = max_row;
     double avg = rows ? (double)nnz / rows : 0.0;
     d->lanes = pow2_at_least((int)std::ceil(avg), 64);
-    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, m->csr_col_id));  // checks the columns
+    ColRange all;
+    all.widen(m->csr_col_id, nnz);
+    if (nnz > 0 && !all.within(m->matinfo.width))
+        UPLOAD_CHECK(check_cols(m->csr_col_id, nnz, m->matinfo.width, 1, "csr"));
+    std::vector<int4> blk;
+    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, &blk));
+    constexpr size_t W = launch::kCsrWaves;
+    StageBuild stage;
+    stage.start(m->matinfo.width, (blk.size() + W - 1) / W, m->csr_col_id, nnz, (size_t)nnz + launch::kWaveNnz,
+                [&blk](size_t g, auto&& f) {
+                    for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
+                        f(blk[b].z, blk[b].w, blk[b].z, 1);
+                });
     UPLOAD_CHECK(upload_array(d, m->csr_row_ptr, (size_t)rows + 1, &d->rp));
     UPLOAD_CHECK(upload_padded(d, m->csr_col_id, nnz, launch::kWaveNnz, &d->col));
     if (o.dtype != CLSPMV_DT_F32) {
@@ -618,6 +731,7 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     } else {
         UPLOAD_CHECK(upload_padded(d, m->csr_data, nnz, launch::kWaveNnz, &d->val));
     }
+    UPLOAD_CHECK(stage.finish(d));
     std::vector<int> blocks = csr_row_blocks(m->csr_row_ptr, rows);
     d->nblocks = (int)blocks.size() - 1;
     UPLOAD_CHECK(upload_array(d, blocks.data(), blocks.size(), &d->blocks));
@@ -674,26 +788,22 @@ int clspmv_upload_ell(clspmv_ctx* ctx, const clspmv_ell_matrix* m, clspmv_dmat**
     if (m->ell_height_aligned < m->matinfo.height || m->ell_num < 0)
         UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "malformed ELL matrix"));
     const int rows = m->matinfo.height, hal = m->ell_height_aligned, cols = std::max(m->matinfo.width, 1);
-    constexpr int R = launch::kEllRows;
-    std::vector<ColRange> range((rows + R - 1) / R);
-    ColRange all;  // of the padding rows, then of all slots
-    for (int s = 0; s < m->ell_num; ++s) {
-        const int* c = m->ell_col_id + (size_t)s * hal;
-        for (int r = 0; r < rows; r += R) range[r / R].widen(c + r, std::min(R, rows - r));
-        all.widen(c + rows, hal - rows);
-    }
-    for (const ColRange& g : range) all.lo = std::min(all.lo, g.lo), all.hi = std::max(all.hi, g.hi);
+    ColRange all;
+    all.widen(m->ell_col_id, total);
     if (total > 0 && !all.within(cols)) UPLOAD_CHECK(check_cols(m->ell_col_id, total, cols, 1, "ell"));
+    constexpr size_t R = launch::kEllRows;
+    const size_t words = (size_t)(m->ell_num + 1) / 2 * hal;
+    StageBuild stage;
+    stage.start(m->matinfo.width, (rows + R - 1) / R, m->ell_col_id, total, 2 * words, [=](size_t g, auto&& f) {
+        for (size_t s = 0; s < (size_t)m->ell_num; ++s)
+            f(s * hal + g * R, std::min(R, rows - g * R), 2 * (s / 2 * hal + g * R) + s % 2, 2);
+    });
     d->hal = m->ell_height_aligned;
     d->ellnum = m->ell_num;
     d->info.stored = (long long)total;
     UPLOAD_CHECK(upload_array(d, m->ell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->ell_data, total, &d->val));
-    UPLOAD_CHECK(add_windows(d, range, launch::kEllWinMax, [&](size_t g, int* line) {
-        if (m->ell_num == 0 || (int)g * R + 64 > rows) return false;
-        std::copy_n(m->ell_col_id + (size_t)(m->ell_num / 2) * hal + g * R, 64, line);
-        return true;
-    }));
+    UPLOAD_CHECK(stage.finish(d));
     *out = d;
     return CLSPMV_OK;
 }
@@ -708,38 +818,29 @@ int clspmv_upload_sell(clspmv_ctx* ctx, const clspmv_sell_matrix* m, clspmv_dmat
         if (w < 0 || w % h) UPLOAD_CHECK(fail(CLSPMV_ERR_INVALID, "SELL slice %d size %d", s, w));
     }
     const size_t total = (size_t)m->sell_slice_ptr[ns];
-    // Column ranges of the kernel's work-groups; a slice that reaches into
-    // several counts for each.
     const int rows = m->matinfo.height, cols = std::max(m->matinfo.width, 1);
     const int* sp = m->sell_slice_ptr;
-    constexpr int R = launch::kEllRows;
-    std::vector<ColRange> range((rows + R - 1) / R);
     ColRange all;
-    all.widen(m->sell_col_id, sp[0]);
-    for (int s = 0; s < ns; ++s) {
-        ColRange one;
-        one.widen(m->sell_col_id + sp[s], sp[s + 1] - sp[s]);
-        all.lo = std::min(all.lo, one.lo), all.hi = std::max(all.hi, one.hi);
-        const long long r0 = (long long)s * h, r1 = std::min<long long>(rows, r0 + h);
-        for (long long g = r0 / R; g * R < r1; ++g) {
-            range[g].lo = std::min(range[g].lo, one.lo);
-            range[g].hi = std::max(range[g].hi, one.hi);
-        }
-    }
+    all.widen(m->sell_col_id, total);
     if (total > 0 && !all.within(cols)) UPLOAD_CHECK(check_cols(m->sell_col_id, total, cols, 1, "sell"));
+    constexpr size_t R = launch::kEllRows;
+    const size_t words = ((size_t)sp[ns] / h + ns + 1) / 2 * h;
+    StageBuild stage;
+    stage.start(m->matinfo.width, (rows + R - 1) / R, m->sell_col_id, total, 2 * words, [=](size_t g, auto&& f) {
+        const size_t r1 = std::min<size_t>(rows, (g + 1) * R);
+        for (size_t r = g * R; r < r1;) {  // the group's part of each slice
+            const size_t sl = r / h, i = r - sl * h, n = std::min(r1, (sl + 1) * h) - r;
+            const size_t word = ((size_t)sp[sl] / h + sl) / 2 * h + i, slots = (size_t)(sp[sl + 1] - sp[sl]) / h;
+            for (size_t k = 0; k < slots; ++k) f(sp[sl] + k * h + i, n, 2 * (word + k / 2 * h) + k % 2, 2);
+            r += n;
+        }
+    });
     d->info.slice_height = h;
     d->info.stored = (long long)total;
     UPLOAD_CHECK(upload_array(d, m->sell_slice_ptr, (size_t)ns + 1, &d->sptr));
     UPLOAD_CHECK(upload_array(d, m->sell_col_id, total, &d->col));
     UPLOAD_CHECK(upload_array(d, m->sell_data, total, &d->val));
-    UPLOAD_CHECK(add_windows(d, range, launch::kEllWinMax, [&](size_t g, int* line) {
-        for (int i = 0; i < 64; ++i) {  // the middle slot of each of 64 rows
-            const int r = (int)g * R + i, s = r / h;
-            if (r >= rows || sp[s + 1] == sp[s]) return false;
-            line[i] = m->sell_col_id[sp[s] + (sp[s + 1] - sp[s]) / h / 2 * h + r % h];
-        }
-        return true;
-    }));
+    UPLOAD_CHECK(stage.finish(d));
     *out = d;
     return CLSPMV_OK;
 }

@@ -21,7 +21,7 @@ struct clspmv_dmat {
     std::vector<std::pair<void*, size_t>> bufs;  // device allocations owned by the matrix
 
     // CSR: rp/col/val (col and val padded by launch::kWaveNnz entries);
-    // row blocks of the verification kernel; blocks, long rows and x windows
+    // row blocks of the verification kernel; blocks and long rows
     // of the wave and multi-vector kernels (launch::CsrWave); lanes per row of
     // the vector kernel.
     int* rp = nullptr;
@@ -34,10 +34,10 @@ struct clspmv_dmat {
     int4* wblk = nullptr;
     int* wlong = nullptr;
     int nwblk = 0, nwlong = 0;
-    // x windows of CSR's wave kernel, ELL and SELL (null: absent), the
-    // columns of the widest one.
-    int2* wwin = nullptr;
-    int wwin_max = 0;
+    // Staged x of CSR's wave kernel, ELL and SELL (launch::XStage; null: absent).
+    int* xlist = nullptr;
+    unsigned short* xidx = nullptr;
+    int xstride = 0;
     // COO: row/col/val, carry slots (2 per chunk).
     int* row = nullptr;
     int* carry_row = nullptr;
@@ -159,8 +159,8 @@ void release_array(clspmv_dmat* m, T** p) {
 }
 
 // Builds and uploads the wave kernel's tables of a CSR matrix from its host
-// row pointers; col (or null: no x windows) its host columns.
-int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, const int* col);
+// row pointers; the blocks also to `blocks`.
+int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks = nullptr);
 
 // x-panel encoding (k_panel.hip) of row-sorted entries, built on the host
 // and uploaded into `d`.  pw: panel width (multiple of 8, at most

@@ -475,6 +475,30 @@ def test_ell_windows(ctx, oracle, name, fmt, x_offset, repeat):
         _run(ctx, oracle, A, owned, 0, x_offset=x_offset)
 
 
+@pytest.mark.parametrize("chunks", [40, 511, 512, 513])
+@pytest.mark.parametrize("x_offset", [0, 1])
+def test_staged_x(ctx, oracle, chunks, x_offset):
+    """CSR, ELL and SELL work-groups of up to 512 rows of 11 entries (the last one
+    partial) that touch `chunks` runs of 16 columns, up to the most that are
+    staged and one past it, the last run cut off by the matrix; odd slot
+    counts, an empty slice, slices that reach into two work-groups; dyadic
+    inputs, exact sums."""
+    rows, cols = 3 * 512 + 37, chunks * 16 - 5
+    r = np.repeat(np.arange(rows), 11)
+    c = np.minimum((np.arange(r.size) * 7 % chunks) * 16 + r % 16, cols - 1)
+    key = np.unique(r.astype(np.int64) * cols + c)
+    r, c = key // cols, key % cols
+    v = (np.random.default_rng(chunks).integers(1, 65, r.size) / 64.0).astype(np.float32)
+    A = cs.Coo(r.astype(np.int32), c.astype(np.int32), v, rows, cols)
+    odd = (r % 16 != 3) & (r // 32 != 2) | (r % 8 == 1) & (r // 32 != 2)  # a slice of none
+    B = cs.Coo(A.row[odd], A.col[odd], A.val[odd], rows, cols)
+    _run(ctx, oracle, A, cs.coo2csr(A.copy()), cs.METHOD_AUTO, panel=0, x_offset=x_offset)
+    for M, owned in ((A, cs.coo2ell(A)), (B, cs.coo2sell(B, 32)), (A, cs.coo2sell(A, 48)), (B, cs.coo2sell(B, 700))):
+        _run(ctx, oracle, M, owned, 0, x_offset=x_offset)
+    info = cs.DeviceMatrix(ctx, cs.coo2ell(A)).info
+    assert (info.device_bytes >= 10 * info.stored) == (chunks <= 512)
+
+
 @pytest.mark.parametrize("width", [1, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 24, 27])
 @pytest.mark.parametrize("rows", [100, (1 << 17) + 3])
 def test_ell_slot_groups(ctx, oracle, width, rows):
