@@ -33,6 +33,7 @@ using namespace dev;
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef s16x8 s16x8_a8 __attribute__((aligned(8)));
 typedef _Float16 h16x4 __attribute__((ext_vector_type(4)));
 
 template <bool BF16>
@@ -307,8 +308,9 @@ constexpr int kWinTile = 8 * 4 * NQ + 16;  // bytes per staged tile: 4 * NQ righ
 constexpr int kWinBlock = kBlock;  // (one-wave work-groups measured no faster)
 
 // MULTI: more than 4 * NQ right-hand sides (the chunk loop runs more than
-// once).
-template <bool BF16, int NQ, bool MULTI, bool COLX>
+// once).  ODD (tiled X): an odd number of right-hand sides, or X not 16-byte
+// aligned.
+template <bool BF16, int NQ, bool MULTI, bool COLX, bool ODD>
 __global__ __launch_bounds__(kWinBlock) __attribute__((amdgpu_waves_per_eu(3))) void bspmm4_win_kernel(
     int brows, int rows, int cols, int kall, const int* __restrict__ rp, const unsigned short* __restrict__ val,
     launch::SpmmWindows win, int win_stride, const unsigned short* __restrict__ Xall, int ldx,
@@ -388,8 +390,17 @@ __global__ __launch_bounds__(kWinBlock) __attribute__((amdgpu_waves_per_eu(3))) 
 #pragma unroll
         for (int u = 0; u < kR; ++u) {
             const unsigned pc = (unsigned)(i0 + u * kWave + lane) % PP;
-            v[u] = *reinterpret_cast<const s16x8*>(x_base + (unsigned)tl[u] * x_tile +
-                                                  (2 * pc < (unsigned)kc ? pc * 16 : 0u));
+            if constexpr (ODD) {  // the tiles are 8-byte aligned
+                // The last right-hand side of an odd kc comes with the one before
+                // it (with kc = 1 of the chunk before): none past the tile is read.
+                const bool end = 2 * pc + 1 == (unsigned)kc;
+                v[u] = *reinterpret_cast<const s16x8_a8*>(x_base - 8 + (unsigned)tl[u] * x_tile +
+                                                         (2 * pc < (unsigned)kc ? pc * 16 + (end ? 0u : 8u) : 8u));
+                if (end) v[u].lo = v[u].hi;
+            } else {
+                v[u] = *reinterpret_cast<const s16x8*>(x_base + (unsigned)tl[u] * x_tile +
+                                                      (2 * pc < (unsigned)kc ? pc * 16 : 0u));
+            }
         }
     };
     auto st_store = [&](int i0, const s16x8* v) {
@@ -547,7 +558,7 @@ void launch_kernel(hipStream_t s, unsigned blocks, bool nt, int brows, int rows,
 // carries, a work-group's windows fit kSpmmWinLds and X's byte offsets fit
 // 32 bits (the kernel's staging loads take 32-bit offsets from X); sets
 // `done` when it launched.  One wave per slice for all k right-hand sides.
-template <bool BF16, int NQ, bool COLX>
+template <bool BF16, int NQ, bool COLX, bool ODD>
 hipError_t launch_win(hipStream_t s, bool long_rows, int brows, int rows, int cols, int k, const int* rp,
                       const unsigned short* val, const unsigned short* X, int ldx, float* Y, int ldy, bool acc_y,
                       const launch::SpmmWindows& win, bool& done) {
@@ -560,10 +571,10 @@ hipError_t launch_win(hipStream_t s, bool long_rows, int brows, int rows, int co
     const unsigned wb = (unsigned)((slices * kWave + kWinBlock - 1) / kWinBlock);
     const size_t shm = (size_t)(kWinBlock / kWave) * win_stride;
     if (k > 4 * NQ)
-        hipLaunchKernelGGL((bspmm4_win_kernel<BF16, NQ, true, COLX>), dim3(wb), dim3(kWinBlock), shm, s, brows, rows,
+        hipLaunchKernelGGL((bspmm4_win_kernel<BF16, NQ, true, COLX, ODD>), dim3(wb), dim3(kWinBlock), shm, s, brows, rows,
                            cols, k, rp, val, win, win_stride, X, ldx, Y, ldy, acc_y);
     else
-        hipLaunchKernelGGL((bspmm4_win_kernel<BF16, NQ, false, COLX>), dim3(wb), dim3(kWinBlock), shm, s, brows,
+        hipLaunchKernelGGL((bspmm4_win_kernel<BF16, NQ, false, COLX, ODD>), dim3(wb), dim3(kWinBlock), shm, s, brows,
                            rows, cols, k, rp, val, win, win_stride, X, ldx, Y, ldy, acc_y);
     done = true;
     return hipGetLastError();
@@ -588,14 +599,18 @@ hipError_t launch_nq(hipStream_t s, bool long_rows, int brows, int rows, int col
     // chunk, normal A loads, non-temporal Y accesses (which cost 3-5 us at
     // k = 8 / 16).
     const bool nt = k <= 4 * NQ;
-    // X windows in LDS when the matrix has them (16-byte tile pieces).
+    // X windows in LDS when the matrix has them (pieces of two right-hand
+    // sides, 8-byte aligned ones too: 131,072 block rows x 12, k = 5 / 9 / 17 /
+    // 31: 20.7 / 31.4 / 40.6 / 47.9 us from the tiles directly, 15.7 / 21.6 /
+    // 33.1 / 41.9 through the windows).
     if constexpr (kX16) {
-        if (x16) {
-            bool done = false;
-            const hipError_t e = launch_win<BF16, NQ, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y,
-                                                             ldy, acc_y, win, done);
-            if (done || e != hipSuccess) return e;
-        }
+        bool done = false;
+        const hipError_t e =
+            x16 ? launch_win<BF16, NQ, false, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
+                                                     win, done)
+                : launch_win<BF16, NQ, false, true>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
+                                                    win, done);
+        if (done || e != hipSuccess) return e;
     }
     const unsigned nb = (unsigned)blocks;
     if (long_rows) {
@@ -630,9 +645,9 @@ hipError_t launch_k(hipStream_t s, bool long_rows, int brows, int rows, int cols
         // 8 or 16 right-hand sides per chunk.
         bool done = false;
         const hipError_t e =
-            k <= 8 ? launch_win<BF16, 2, true>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y, win,
+            k <= 8 ? launch_win<BF16, 2, true, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y, win,
                                                done)
-                   : launch_win<BF16, 4, true>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y, win,
+                   : launch_win<BF16, 4, true, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y, win,
                                                done);
         if (done || e != hipSuccess) return e;
     }

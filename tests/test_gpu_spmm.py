@@ -235,3 +235,28 @@ def test_spmm_tiled_overwrite(ctx, name, k):
     y, z = dY.download().reshape(k, ldy), dZ.download().reshape(k, ldy)
     np.testing.assert_array_equal(y[:, :H].view(np.uint32), z[:, :H].view(np.uint32))
     assert np.all(np.isnan(y[:, H:]))  # past the rows: untouched
+
+
+@pytest.mark.parametrize("name", ["block_small", "rand", "win_rounds"])
+@pytest.mark.parametrize("dtype", [cs.DT_BF16, cs.DT_F16])
+@pytest.mark.parametrize("k, offset", [(5, 0), (7, 0), (9, 0), (13, 0), (15, 0), (17, 0), (19, 0), (31, 0), (33, 0),
+                                       (6, 4), (16, 4), (20, 4), (21, 4)])
+def test_spmm_tiled_odd(ctx, name, dtype, k, offset):
+    """Tiled X with an odd number of right-hand sides (its last one alone, in
+    the second chunk too) or starting `offset` 16-bit values into its buffer (8
+    bytes past a 16-byte boundary): the column-major product's bits."""
+    A = CASES[name]
+    rng = np.random.default_rng(300 + k)
+    H, W = A.height, A.width
+    ldx, ldy = (W + 3) // 4 * 4, (H + 3) // 4 * 4
+    Xb = cs.convert_from_f32(rng.uniform(-1, 1, size=(k, ldx)).astype(np.float32), dtype)
+    Y0 = rng.uniform(-1, 1, size=(k, ldy)).astype(np.float32)
+    M = cs.BlockSpmm(ctx, cs.coo2bcsr(A.copy(), 4, 4), dtype)
+    tiles = _tiles(Xb, W).reshape(-1)
+    dX4 = cs.DeviceBuffer(ctx, np.concatenate([np.full(offset, 0x7FFF, np.uint16), tiles]))
+    at = type(dX4.p)(dX4.p.value + 2 * offset)
+    dX, dY, dY4 = cs.DeviceBuffer(ctx, Xb), cs.DeviceBuffer(ctx, Y0), cs.DeviceBuffer(ctx, Y0)
+    M.spmm(k, dX, ldx, dY, ldy)
+    cs.check(cs.lib.clspmv_spmm_tiled(ctx.h, M.h, k, at, dY4.p, ldy), "spmm_tiled")
+    ctx.sync()
+    np.testing.assert_array_equal(dY4.download(), dY.download())
