@@ -48,12 +48,12 @@ __global__ __launch_bounds__(kBlock) void csr_vector_kernel(
 // waves' sums are added in order.  Acc is double for rows longer
 // than kLongRowF64 of 16-bit values: their products are exact and the row is
 // rounded once, into y.
-template <class V, class Acc>
+template <class V, class Acc, int kWaves>
 __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict__ col,
                                              const typename V::T* __restrict__ val,
                                              const float* __restrict__ x, float* __restrict__ y,
                                              Acc* part) {
-    constexpr int U = 4, kThreads = kWave * launch::kCsrWaves;
+    constexpr int U = 4, kThreads = kWave * kWaves;
     const int t = threadIdx.x;
     Acc acc = 0;
     for (int k = s + t; k < e; k += U * kThreads) {
@@ -77,7 +77,7 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
     if (t == 0) {
         Acc tot = 0;
 #pragma unroll
-        for (int w = 0; w < launch::kCsrWaves; ++w) tot += part[w];
+        for (int w = 0; w < kWaves; ++w) tot += part[w];
         *y = sizeof(Acc) == sizeof(double) ? (float)((double)*y + (double)tot) : *y + (float)tot;
     }
 }
@@ -108,8 +108,13 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
 // rows 5.8 -> 7.9 us; 32 no different; 128: 6.4 us on the 30,000 rows).
 constexpr int kWideRow = 64;
 
-template <class V, bool WIN>
-__global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
+// Waves of a work-group that stages no x: the fewer, the sooner a long row's
+// work-group finds room, the more, the shorter its chain (2 / 4 / 8 waves:
+// power-law rows 96,050 13.9 / 11.6 / 12.4 us, 1 M 105.4 / 106.2 / 107.3).
+constexpr int kPlainWaves = 4;
+
+template <class V, bool WIN, int kWaves>
+__global__ __launch_bounds__(kWave* kWaves) void csr_wave_kernel(
     int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
     const int* __restrict__ list, const unsigned short* __restrict__ idx, int stride, int cols,
     const int* __restrict__ rp, const int* __restrict__ col,
@@ -123,16 +128,16 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
         const int r = longs[blockIdx.x], s = rp[r], e = rp[r + 1];
         double* part = reinterpret_cast<double*>(sm);
         if (sizeof(T) == 2 && e - s > launch::kLongRowF64)
-            csr_long_row<V, double>(s, e, col, val, x, y + r, part);
+            csr_long_row<V, double, kWaves>(s, e, col, val, x, y + r, part);
         else
-            csr_long_row<V, float>(s, e, col, val, x, y + r, reinterpret_cast<float*>(part));
+            csr_long_row<V, float, kWaves>(s, e, col, val, x, y + r, reinterpret_cast<float*>(part));
         return;
     }
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int wg = xcd_tile(blockIdx.x - nlong, gridDim.x - nlong);
-    const int b = __builtin_amdgcn_readfirstlane(wg * launch::kCsrWaves + wave);
+    const int b = __builtin_amdgcn_readfirstlane(wg * kWaves + wave);
     if (!WIN && b >= nblk) return;
-    StageX<kWave * launch::kCsrWaves> stage;
+    StageX<kWave * kWaves> stage;
     if constexpr (WIN) stage.ids(list + (size_t)wg * stride, stride);
     int4 B = blk[min(b, nblk - 1)];  // {first row, rows, first entry, entries}
     if (WIN && b >= nblk) B.y = B.w = 0;
@@ -208,16 +213,17 @@ __global__ __launch_bounds__(kWave* launch::kCsrWaves) void csr_wave_kernel(
 template <class V>
 hipError_t csr_wave_v(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
                       int cols, const float* x, float* y) {
-    const dim3 grid(W.nlong + (W.nblk + launch::kCsrWaves - 1) / launch::kCsrWaves), block(kWave * launch::kCsrWaves);
-    const size_t lds = sizeof(float) * launch::kWaveNnz * launch::kCsrWaves;
     const typename V::T* v = static_cast<const typename V::T*>(val);
+    auto launch = [&](auto kernel, int waves, const launch::XStage& X) {
+        const dim3 grid(W.nlong + (W.nblk + waves - 1) / waves), block(kWave * waves);
+        const size_t lds = sizeof(float) * (launch::kWaveNnz * waves + launch::kXChunk * X.stride);
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, X.list, X.idx, X.stride, cols,
+                           rp, col, v, x, y);
+    };
     if (W.stage.list)
-        hipLaunchKernelGGL((csr_wave_kernel<V, true>), grid, block,
-                           lds + sizeof(float) * launch::kXChunk * W.stage.stride, s, W.nlong, W.longs, W.nblk, W.blk,
-                           W.stage.list, W.stage.idx, W.stage.stride, cols, rp, col, v, x, y);
+        launch(csr_wave_kernel<V, true, launch::kCsrWaves>, launch::kCsrWaves, W.stage);
     else
-        hipLaunchKernelGGL((csr_wave_kernel<V, false>), grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, nullptr,
-                           nullptr, 0, cols, rp, col, v, x, y);
+        launch(csr_wave_kernel<V, false, kPlainWaves>, kPlainWaves, launch::XStage{});
     return hipGetLastError();
 }
 

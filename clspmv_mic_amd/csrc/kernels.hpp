@@ -38,7 +38,7 @@ struct XStage {
 // Wave kernel: blk holds {first row, rows (at most 64), first entry, entries
 // (at most kWaveNnz)} per wave, longs the rows with more entries; col and val
 // (and stage.idx) carry kWaveNnz entries of padding (column 0) after the last
-// one.  A work-group takes kCsrWaves blocks.
+// one.  A work-group that stages x takes kCsrWaves blocks.
 constexpr int kWaveNnz = 512;
 constexpr int kCsrWaves = 8;
 static_assert(4 * (kWaveNnz * kCsrWaves + kXChunk * kXChunksMax) <= 64 * 1024, "within the default LDS limit");

@@ -308,7 +308,7 @@ int auto_method(const clspmv_dmat* A) {
     switch (A->info.format) {
         // The wave kernel: lanes striding over rows are no faster at any row
         // length (27-point stencil 77^3 24 against 52 us, 5-point Laplacian
-        // 256^2 4.7 against 4.6 us, power-law rows 1 M 107 against 225 us).
+        // 256^2 4.7 against 4.6 us, power-law rows 1 M 106 against 225 us).
         case CLSPMV_FMT_CSR: return 1;
         // A row per lane: four rows per lane leave a quarter of the waves and
         // gather x four rows apart (27-point stencil 77^3 30 against 19 us,
