@@ -269,7 +269,8 @@ __device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
 
 // Work-group of the CSR kernel: with 512 threads a row over kWaveNnz entries has
 // 1,024 of them in flight (a 5,000-entry row sets the time of a small
-// power-law matrix: 60,000 rows, k = 4: 19.7 us against 27.3 with 256 threads).
+// power-law matrix: 60,000 rows, k = 4: 19.7 us against 27.3 with 256 threads;
+// 17.6 with the longest rows first).
 constexpr int kMultiThreads = 512;
 
 // One row longer than kWaveNnz by the whole work-group, always with four
@@ -340,8 +341,8 @@ __device__ __forceinline__ T group_lane(T v) {
 // a work-group of 1024 entries waited at two barriers, each finished row was
 // added to Y where it ended (a load and a store of one float per right-hand
 // side, waited for) and k not a multiple of 4 gathered single floats.
-// Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 156 / 184 us; 1 M
-// rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 284 / 273 / 311 us (50 G rows/s);
+// Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 138 / 174 us; 1 M
+// rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 266 / 251 / 302 us (53 G rows/s);
 // 27-point stencil 64^3, k = 8: 74 -> 31 us.
 constexpr int kUnit = 8;
 
