@@ -64,14 +64,25 @@ __global__ __launch_bounds__(kBlock) void bcsr_kernel(
 // slice).  A float4 load of 64 block rows is one contiguous run.
 //
 // What bounds it: HBM on large matrices, the chain of slots (block column, then
-// x) on small ones.  The rows of a block go to different waves (kHWaves of
-// them share the block rows and find the columns and x in L1), which gives
-// four times the waves of a lane per block row, and U slots' columns and
+// x) on small ones.  A lane takes HN rows of a block row and HW waves share
+// its block rows (they find the columns and x in L1); U slots' columns and
 // values load at once, the next U's in flight while the present ones' x is
 // fetched (two register sets taking turns; the last group loads no more than
-// its slots).  12 4x4 blocks per block row, BCSR / BELL / SBELL: 20,000 block
-// rows 14.7 / 14.7 / 15.5 -> 6.5 / 6.2 / 6.7 us, 131,072 21.7 / 21.3 / 22.9 ->
-// 21.1 / 21.0 / 21.0 us (6.76 TB/s would be 16.8).
+// its slots).  By the loads that a slot has for the chip, one float4 plane per
+// block row, row and column quad (figures: block rows of 12 4x4 blocks, BCSR /
+// BELL / SBELL, against a lane per block row, one slot after the other):
+//   kSplit    four waves share block rows, two to four slots at a time: 20,000
+//             block rows 14.7 / 14.7 / 15.5 -> 6.5 / 6.2 / 6.7 us, 60,000 15.5 /
+//             15.6 / 16.3 -> 9.9 / 9.7 / 10.1 us;
+//   kAhead    a lane per block row, the next slot in flight, from kAheadPlanes on:
+//             100,000 18.7 / 18.3 / 19.5 -> 14.8 / 14.8 / 15.7 us (kSplit 16.0 /
+//             15.4 / 15.9), 131,072 20.3 / 20.3 / 22.0 -> 17.1 / 17.1 / 18.5
+//             (kSplit 20.4 / 20.2 / 19.8; 6.76 TB/s would be 16.8);
+//   kInOrder  from kInOrderPlanes on the waves cover the chain and more loads in
+//             flight only slow the stream: 200,000 28.8 us (kAhead 30.4, kSplit
+//             28.6), 300,000 39.3 (40.8, 41.9), 524,288 71.8 (70.9, 75.1); 55,000
+//             rows of 8x8 blocks 31.1 (kSplit 39.6).  Not SBELL, whose slot
+//             counts differ by lane: 524,288 73.5 ahead, 77.2 in order.
 //
 // Padding slots of BCSR (column -1) and slots past a lane's last load what is
 // there for another and are not added, so the sum is the row's blocks' in slot
@@ -80,15 +91,19 @@ __global__ __launch_bounds__(kBlock) void bcsr_kernel(
 // the end.
 enum Layout { kBcsrSlots, kBell, kSbell };
 constexpr int kHWaves = kBlock / kWave;  // waves of a work-group
+enum Walk { kSplit, kAhead, kInOrder };
+constexpr long long kAheadPlanes = 3 << 17, kInOrderPlanes = 3 << 18;
+template <int BH, Walk WALK>
+constexpr int kShare = WALK != kSplit ? 1 : BH < kHWaves ? BH : kHWaves;  // waves sharing block rows
 
-template <int BH, int BW4, Layout LAY, bool F4ACC>
+template <int BH, int BW4, Layout LAY, bool F4ACC, Walk WALK>
 __global__ __launch_bounds__(kBlock) void block_rows_kernel(
     int brows, int rows, int cols, int cs, int f4, int nslots, const int* __restrict__ sptr,
     const int* __restrict__ col4, const float* __restrict__ data, const float* __restrict__ x,
     bool x_aligned, float* __restrict__ y) {
-    constexpr int HW = BH < kHWaves ? BH : kHWaves;  // waves sharing block rows
-    constexpr int HN = BH / HW;                      // rows of a block per wave
-    constexpr int U = BW4 * HN == 1 ? 4 : BW4 * HN == 2 ? 3 : 2;  // slots in flight
+    constexpr int HW = kShare<BH, WALK>;
+    constexpr int HN = BH / HW;  // rows of a block per wave
+    constexpr int U = WALK != kSplit ? 1 : BW4 * HN == 1 ? 4 : BW4 * HN == 2 ? 3 : 2;  // slots at a time
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int h0 = wave % HW * HN;
     const int row = (xcd_tile(blockIdx.x, gridDim.x) * (kHWaves / HW) + wave / HW) * kWave + lane;
@@ -170,20 +185,27 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
                 }
         }
     };
-    if (U <= wm) load(0, 0);
-    else load_part(0, 0);
-    int s = 0;
-    for (; s + 3 * U <= wm; s += 2 * U) {
-        load(s + U, 1);
+    if constexpr (WALK == kInOrder) {
+        for (int s = 0; s < wm; ++s) {
+            load(s, 0);
+            add(s, 0);
+        }
+    } else {
+        if (U <= wm) load(0, 0);
+        else load_part(0, 0);
+        int s = 0;
+        for (; s + 3 * U <= wm; s += 2 * U) {
+            load(s + U, 1);
+            add(s, 0);
+            load(s + 2 * U, 0);
+            add(s + U, 1);
+        }
+        if (s + U < wm) load_part(s + U, 1);
         add(s, 0);
-        load(s + 2 * U, 0);
-        add(s + U, 1);
+        if (s + 2 * U < wm) load_part(s + 2 * U, 0);
+        if (s + U < wm) add(s + U, 1);
+        if (s + 2 * U < wm) add(s + 2 * U, 0);
     }
-    if (s + U < wm) load_part(s + U, 1);
-    add(s, 0);
-    if (s + 2 * U < wm) load_part(s + 2 * U, 0);
-    if (s + U < wm) add(s + U, 1);
-    if (s + 2 * U < wm) add(s + 2 * U, 0);
 #pragma unroll
     for (int h = 0; h < HN; ++h) {
         const int at = r * BH + h0 + h;
@@ -195,9 +217,15 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
 template <int BH, int BW4, Layout LAY, bool F4ACC>
 hipError_t block_rows(hipStream_t s, int brows, int rows, int cols, int cs, int f4, int nslots, const int* sptr,
                       const int* col4, const float* data, const float* x, bool xa, float* y) {
-    constexpr int per = kWave * kHWaves / (BH < kHWaves ? BH : kHWaves);  // block rows per work-group
-    hipLaunchKernelGGL((block_rows_kernel<BH, BW4, LAY, F4ACC>), dim3(((long long)brows + per - 1) / per), dim3(kBlock), 0, s,
-                       brows, rows, cols, cs, f4, nslots, sptr, col4, data, x, xa, y);
+    auto launch = [&](auto kernel, int share) {
+        const int per = kBlock / share;  // block rows per work-group
+        hipLaunchKernelGGL(kernel, dim3(((long long)brows + per - 1) / per), dim3(kBlock), 0, s, brows, rows, cols, cs,
+                           f4, nslots, sptr, col4, data, x, xa, y);
+    };
+    const long long planes = (long long)brows * BH * BW4;
+    if (planes < kAheadPlanes) launch(block_rows_kernel<BH, BW4, LAY, F4ACC, kSplit>, kShare<BH, kSplit>);
+    else if (LAY == kSbell || planes < kInOrderPlanes) launch(block_rows_kernel<BH, BW4, LAY, F4ACC, kAhead>, 1);
+    else launch(block_rows_kernel<BH, BW4, LAY, F4ACC, LAY == kSbell ? kAhead : kInOrder>, 1);
     return hipGetLastError();
 }
 

@@ -514,6 +514,28 @@ def test_ell_slot_groups(ctx, oracle, width, rows):
     _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
     _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
 
+@pytest.mark.parametrize("nbr", [(3 << 15) - 1, 3 << 15, (3 << 16) - 1, (3 << 16) + 77])
+@pytest.mark.parametrize("shape, width", [((4, 1), 5), ((4, 2), 2), ((4, 4), 3), ((8, 2), 1)])
+def test_block_walks(ctx, oracle, nbr, shape, width):
+    """Block rows of width and width - 1 blocks on both sides of the block-row
+    counts where the kernels' walk over the slots changes; dyadic inputs, exact
+    sums."""
+    bw, bh = shape
+    lens = np.where(np.arange(nbr) % 12 == 5, width - 1, width)
+    br = np.repeat(np.arange(nbr), lens)
+    bc = (br + 3 * (np.arange(br.size) - (np.cumsum(lens) - lens)[br])) % nbr
+    bc = bc[np.lexsort((bc, br))]
+    r = (br[:, None, None] * bh + np.arange(bh)[:, None] + np.zeros(bw, int)).reshape(-1)
+    c = (bc[:, None, None] * bw + np.zeros((bh, 1), int) + np.arange(bw)).reshape(-1)
+    o = np.argsort(r, kind="stable")
+    v = (np.random.default_rng(nbr).integers(-64, 65, o.size) / 64.0).astype(np.float32)
+    A = cs.Coo(r[o].astype(np.int32), c[o].astype(np.int32), v, nbr * bh, nbr * bw)
+    _run(ctx, oracle, A, cs.coo2b4csr(A.copy(), bw, bh), 0)
+    for m in (0, 1):
+        _run(ctx, oracle, A, cs.coo2b4ell(A.copy(), bw, bh), m)
+    _run(ctx, oracle, A, cs.coo2sbell(A.copy(), bw, bh), 0)
+
+
 @pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16])
 @pytest.mark.parametrize("others", [0, 1, 2, 15, 31, 32, 62, 63])
 def test_csr_wide_rows(ctx, oracle, others, dtype):
