@@ -56,13 +56,16 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
     constexpr int U = 4, kThreads = kWave * kWaves;
     const int t = threadIdx.x;
     Acc acc = 0;
-    // (Unsigned: k may pass 2^31 past the last entries.)
-    for (unsigned k = s + t, end = e; k < end; k += U * kThreads) {
+    // (Indices from the row's start: the sums stay in range near 2^31 entries.)
+    const int n = e - s;
+    col += s;
+    val += s;
+    for (int k = t; k < n; k += U * kThreads) {
         int c[U];
         float v[U], xv[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {  // past the end: the last entry again, not added
-            const unsigned at = min(k + u * kThreads, end - 1);
+            const int at = min(k + u * kThreads, n - 1);
             c[u] = ld_stream(col + at);
             v[u] = V::ld(val + at);
         }
@@ -70,7 +73,7 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
         for (int u = 0; u < U; ++u) xv[u] = x[c[u]];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (k + u * kThreads < end) acc = fma((Acc)v[u], (Acc)xv[u], acc);
+            if (k + u * kThreads < n) acc = fma((Acc)v[u], (Acc)xv[u], acc);
     }
     for (int m = kWave >> 1; m >= 1; m >>= 1) acc += __shfl_xor(acc, m, kWave);
     if (t % kWave == 0) part[t / kWave] = acc;
@@ -148,12 +151,12 @@ __global__ __launch_bounds__(kWave* kWaves) void csr_wave_kernel(
     typename VecOf<T, 4>::type v[U / 4];
 #pragma unroll
     for (int u = 0; u < U / 4; ++u) {
-        const size_t at = (size_t)s + u * P4 + lane * 4;
+        const unsigned at = u * P4 + lane * 4;
         if constexpr (WIN)
-            ix[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<unsigned short, 4>::type*>(idx + at));
+            ix[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<unsigned short, 4>::type*>((idx + s) + at));
         else
-            c[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<int, 4>::type*>(col + at));
-        v[u] = __builtin_nontemporal_load(reinterpret_cast<const T4U*>(val + at));
+            c[u] = __builtin_nontemporal_load(reinterpret_cast<const UVec<int, 4>::type*>((col + s) + at));
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const T4U*>((val + s) + at));
     }
     // Lane groups for the sums: the largest power of two with nrows groups in
     // the wave (a block holds at most kWave rows).

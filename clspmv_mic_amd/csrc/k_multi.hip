@@ -247,13 +247,16 @@ __device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
                                               const typename V::T* __restrict__ val, int j0, int j1,
                                               int step, const float* __restrict__ X, int k, int qb,
                                               bool vec, Acc* a) {
-    // (Unsigned: j may pass 2^31 past the last entries.)
-    for (unsigned j = j0, end = j1; j < end; j += U * step) {
+    // (Indices from j0: the sums stay in range near 2^31 entries.)
+    const int n = j1 - j0;
+    col += j0;
+    val += j0;
+    for (int j = 0; j < n; j += U * step) {
         int c[U];
         float v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const unsigned at = min(j + u * step, end - 1);
+            const int at = min(j + u * step, n - 1);
             c[u] = ld_stream(col + at);
             v[u] = V::ld(val + at);
         }
@@ -262,7 +265,7 @@ __device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
         for (int u = 0; u < U; ++u) load_xq<Q>(X, c[u], k, qb, vec, xv[u]);
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            if (j + u * step < end)
+            if (j + u * step < n)
 #pragma unroll
                 for (int q = 0; q < Q; ++q) a[q] = fma((Acc)v[u], (Acc)xv[u][q], a[q]);
     }
