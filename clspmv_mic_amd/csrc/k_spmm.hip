@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "device_common.hpp"
+#include "index_math.hpp"
 #include "kernels.hpp"
 
 namespace clspmv {
@@ -366,9 +367,9 @@ __global__ __launch_bounds__(kWinBlock) __attribute__((amdgpu_waves_per_eu(3))) 
     // Staging of a chunk's window from tiled X: 16-byte piece p of tile i
     // (right-hand sides 2p, 2p + 1 of the chunk) to wbuf[i * kWinTile + 16p],
     // kR pieces per lane per round, stored with no branch: pieces past the
-    // window go to the spare slot, pieces past the chunk's k (re-reads of its
-    // first piece) stay in their tile, where they feed only right-hand sides
-    // that are never stored.  The first chunk reads the window's tile list
+    // window go to the spare slot, pieces past the chunk's k (re-reads of one
+    // that its tile holds) stay in their tile, where they feed only right-hand
+    // sides that are never stored.  The first chunk reads the window's tile list
     // from memory and keeps it in LDS (after the zero tile) for the later
     // chunks.
     auto st_load = [&](int cc, int i0, s16x8* v) {
@@ -390,12 +391,10 @@ __global__ __launch_bounds__(kWinBlock) __attribute__((amdgpu_waves_per_eu(3))) 
 #pragma unroll
         for (int u = 0; u < kR; ++u) {
             const unsigned pc = (unsigned)(i0 + u * kWave + lane) % PP;
-            if constexpr (ODD) {  // the tiles are 8-byte aligned
-                // The last right-hand side of an odd kc comes with the one before
-                // it (with kc = 1 of the chunk before): none past the tile is read.
-                const bool end = 2 * pc + 1 == (unsigned)kc;
+            if constexpr (ODD) {  // the tiles are 8-byte aligned; none past a tile is read
+                const bool end = launch::spmm_piece_end(pc, (unsigned)kc);
                 v[u] = *reinterpret_cast<const s16x8_a8*>(x_base - 8 + (unsigned)tl[u] * x_tile +
-                                                         (2 * pc < (unsigned)kc ? pc * 16 + (end ? 0u : 8u) : 8u));
+                                                         launch::spmm_piece_offset(pc, (unsigned)kc));
                 if (end) v[u].lo = v[u].hi;
             } else {
                 v[u] = *reinterpret_cast<const s16x8*>(x_base + (unsigned)tl[u] * x_tile +
