@@ -34,24 +34,24 @@ using namespace dev;
 // in LDS: 27-point stencil 30^3 5.6 / 8.8 -> 4.5 / 6.1 us, 97^3 37.0 / 39.2 ->
 // 29.0 / 30.4, mesh of 20,000 rows 9.7 / 10.5 -> 6.2 / 6.9, 700,000 40.1 / 43.3
 // -> 32.0 / 33.7 us.
-template <bool SELL, bool WIN, int kSlots>
-__global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
+template <bool SELL, bool WIN, int kSlots, int kRows>
+__global__ __launch_bounds__(kRows) void ell_row_kernel(
     int rows, int h, int w0, const int* __restrict__ ptr, const int* __restrict__ list, const unsigned short* __restrict__ idx,
     int stride, int cols, const int* __restrict__ col, const float* __restrict__ val, const float* __restrict__ x,
     float* __restrict__ y) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     const int wg = xcd_tile(blockIdx.x, gridDim.x);
-    const int row = wg * launch::kEllRows + (int)threadIdx.x;
+    const int row = wg * kRows + (int)threadIdx.x;
     const int r = min(row, rows - 1);  // lanes past the end shadow the last row
     int w = w0;
     constexpr int kPer = WIN ? 2 : 1;  // slots per column word
     const int* cp = WIN ? reinterpret_cast<const int*>(idx) : col;
     const float* vp = val;
-    StageX<launch::kEllRows> stage;
+    StageX<kRows> stage;
     if constexpr (WIN) stage.ids(list + (size_t)wg * stride, stride);
     if constexpr (SELL) {
-        const int sl = r / h, p0 = ptr[sl], q0 = p0 / h;
-        w = ptr[sl + 1] / h - q0;
+        const int sl = r / h, p0 = ptr[sl], q0 = WIN ? p0 / h : 0;
+        w = WIN ? ptr[sl + 1] / h - q0 : (ptr[sl + 1] - p0) / h;
         // A lane whose slice is empty reads entry 0 beside its neighbours (the
         // matrix has entries when they have any): at p0 there may be none.
         const int i = r - sl * h;
@@ -64,8 +64,12 @@ __global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
     // The widest row of the wave: its slots are walked, and slots past the
     // lane's own last one re-read that one and are not added.
     int wm = w;
-    if constexpr (SELL)
-        for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    if constexpr (SELL) {
+        if (h % 32 == 0)  // a slice per half of the wave, at most
+            wm = max(__builtin_amdgcn_readlane(w, 0), __builtin_amdgcn_readlane(w, 32));
+        else
+            for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    }
     wm = __builtin_amdgcn_readfirstlane(wm);
     int c[2][kSlots / kPer];
     float v[2][kSlots];
@@ -122,6 +126,28 @@ __global__ __launch_bounds__(launch::kEllRows) void ell_row_kernel(
     if (row < rows) y[r] += (a[0] + a[1]) + (a[2] + a[3]);
 }
 
+// SELL with short rows: a row per lane, two slots at a time, nothing clamped.
+__global__ __launch_bounds__(kBlock) void sell_short_kernel(
+    int rows, int h, const int* __restrict__ ptr, const int* __restrict__ col,
+    const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
+    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    if (r >= rows) return;
+    const int sl = r / h, i = r - sl * h;
+    const int p0 = ptr[sl];
+    const int w = (ptr[sl + 1] - p0) / h;
+    const int* c = col + p0 + i;
+    const float* v = val + p0 + i;
+    float a0 = 0.0f, a1 = 0.0f;
+    int k = 0;
+    for (; k + 1 < w; k += 2) {
+        const int c0 = ld_stream(c + (size_t)k * h), c1 = ld_stream(c + (size_t)(k + 1) * h);
+        a0 = fmaf(ld_stream(v + (size_t)k * h), x[c0], a0);
+        a1 = fmaf(ld_stream(v + (size_t)(k + 1) * h), x[c1], a1);
+    }
+    if (k < w) a0 = fmaf(ld_stream(v + (size_t)k * h), x[ld_stream(c + (size_t)k * h)], a0);
+    y[r] += a0 + a1;
+}
+
 // Four consecutive rows per lane; requires hal % 4 == 0.
 __global__ __launch_bounds__(kBlock) void ell4_kernel(
     int rows, int hal, int ellnum, const int* __restrict__ col,
@@ -145,29 +171,55 @@ __global__ __launch_bounds__(kBlock) void ell4_kernel(
     if (r + 3 < rows) y[r + 3] += a.w;
 }
 
-// Slots in flight: eight while there are fewer than two waves per SIMD (131,072
-// rows), where the chain of slots sets the time (stencil 30^3 6.5 against 8.2
-// us), four above, where more waves cover it and the shorter last group
-// matters (stencil 77^3 19 against 22 us, 5-point Laplacian 701^2 5.9 against
-// 6.6 us).
-template <bool SELL, int kSlots>
-hipError_t ell_rows_k(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
-                      const float* val, int cols, const float* x, float* y) {
-    const dim3 grid((rows + launch::kEllRows - 1) / launch::kEllRows), block(launch::kEllRows);
-    if (W.list)
-        hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots>), grid, block, sizeof(float) * launch::kXChunk * W.stride,
-                           s, rows, h, w, ptr, W.list, W.idx, W.stride, cols, col, val, x, y);
-    else
-        hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots>), grid, block, 0, s, rows, h, w, ptr, nullptr, nullptr,
-                           0, cols, col, val, x, y);
+template <bool SELL, int kSlots, int kRows>
+hipError_t ell_rows_plain(hipStream_t s, int rows, int h, int w, const int* ptr, const int* col, const float* val,
+                          int cols, const float* x, float* y) {
+    hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots, kRows>), dim3((rows + kRows - 1) / kRows), dim3(kRows), 0,
+                       s, rows, h, w, ptr, nullptr, nullptr, 0, cols, col, val, x, y);
     return hipGetLastError();
 }
 
+template <bool SELL, int kSlots>
+hipError_t ell_rows_staged(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
+                           const float* val, int cols, const float* x, float* y) {
+    constexpr int R = launch::kEllRows;
+    hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots, R>), dim3((rows + R - 1) / R), dim3(R),
+                       sizeof(float) * launch::kXChunk * W.stride, s, rows, h, w, ptr, W.list, W.idx, W.stride, cols,
+                       col, val, x, y);
+    return hipGetLastError();
+}
+
+// Staged work-groups of 512 rows leave too many CUs idle below 96 of them: the
+// mesh of 20,000 rows (40 work-groups) with 12 / 25 / 40 neighbours 3.1 / 4.0 /
+// 4.5 us staged, 2.8 / 3.6 / 4.4 gathered (ELL), 40,000 rows (79) of 12 3.6 / 3.3
+// (SELL); 50,000 rows (98) of 25 / 40 4.1 / 4.7 staged, 4.0 / 5.9 gathered.
+constexpr int kStagedGroups = 96;
+
+// Slots in flight, staged: eight while there are fewer than two waves per SIMD
+// (131,072 rows), where the chain of slots sets the time (mesh of 100,000 rows
+// of 25 5.1 against 5.8 us), four above, where more waves cover it and the
+// shorter last group matters (mesh of 400,000 rows of 12 6.4 against 8.0 us).
+//
+// Gathered: work-groups of one wave, which fill the CUs evenly (random columns,
+// 40,000 rows, SELL, work-groups of 512 / 256 / 64 rows: 32 slots 17.6 / 9.3 /
+// 8.4 us, 100 slots 66.9 / 30.4 / 24.2 us), of four waves for rows of less than
+// four slots (1 M rows of one slot: 4.8 against 5.9 us).  Slots by the mean row:
+// 16 from 24 slots on (100,000 rows of 32 / 100, ELL: 16.9 / 56.0 us, by eight
+// 18.7 / 64.5, by four 21.5 / 69.4), eight from ten on (1 M rows of 12 76.6
+// against 79.2 us) and on few rows, else four (1 M rows of 5: 9.4 against
+// 9.9).
 template <bool SELL>
-hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
-                    const float* val, int cols, const float* x, float* y) {
-    return rows < (1 << 17) ? ell_rows_k<SELL, 8>(s, rows, h, w, ptr, W, col, val, cols, x, y)
-                            : ell_rows_k<SELL, 4>(s, rows, h, w, ptr, W, col, val, cols, x, y);
+hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, long long stored, launch::XStage W,
+                    const int* col, const float* val, int cols, const float* x, float* y) {
+    const bool few = rows < (1 << 17);
+    if (W.list && (rows + launch::kEllRows - 1) / launch::kEllRows >= kStagedGroups)
+        return few ? ell_rows_staged<SELL, 8>(s, rows, h, w, ptr, W, col, val, cols, x, y)
+                   : ell_rows_staged<SELL, 4>(s, rows, h, w, ptr, W, col, val, cols, x, y);
+    const long long mean = stored / rows;
+    if (mean < 4) return ell_rows_plain<SELL, 4, 256>(s, rows, h, w, ptr, col, val, cols, x, y);
+    if (mean >= 24) return ell_rows_plain<SELL, 16, 64>(s, rows, h, w, ptr, col, val, cols, x, y);
+    return few || mean >= 10 ? ell_rows_plain<SELL, 8, 64>(s, rows, h, w, ptr, col, val, cols, x, y)
+                             : ell_rows_plain<SELL, 4, 64>(s, rows, h, w, ptr, col, val, cols, x, y);
 }
 
 }  // namespace
@@ -177,7 +229,8 @@ namespace launch {
 hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, XStage W,
                const int* col, const float* val, int cols, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
-    if (rows_per_lane != 4) return ell_rows<false>(s, rows, hal, ellnum, nullptr, W, col, val, cols, x, y);
+    if (rows_per_lane != 4)
+        return ell_rows<false>(s, rows, hal, ellnum, nullptr, (long long)rows * ellnum, W, col, val, cols, x, y);
     if (hal % 4 != 0) return hipErrorInvalidValue;
     const int lanes = (rows + 3) / 4;
     hipLaunchKernelGGL(ell4_kernel, dim3((lanes + kBlock - 1) / kBlock),
@@ -185,11 +238,19 @@ hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, 
     return hipGetLastError();
 }
 
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, XStage W,
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, long long stored, XStage W,
                 const int* col, const float* val, int cols, const float* x, float* y) {
     if (rows <= 0) return hipSuccess;
     if (slice_height <= 0) return hipErrorInvalidValue;
-    return ell_rows<true>(s, rows, slice_height, 0, ptr, W, col, val, cols, x, y);
+    // Up to three slots a row the walk's bookkeeping shows: 1 M rows of 1 / 2 / 3
+    // slots 5.6 / 4.8 / 7.4 us by the short kernel, 5.9 / 5.6 / 7.8 by the other; of
+    // 5 11.1 / 10.0.
+    if (stored * 2 <= rows * 7LL) {
+        hipLaunchKernelGGL(sell_short_kernel, dim3((rows + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rows,
+                           slice_height, ptr, col, val, x, y);
+        return hipGetLastError();
+    }
+    return ell_rows<true>(s, rows, slice_height, 0, ptr, stored, W, col, val, cols, x, y);
 }
 
 }  // namespace launch

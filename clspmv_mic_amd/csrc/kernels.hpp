@@ -121,11 +121,11 @@ hipError_t panel_pass2(hipStream_t s, const float* seg_val, int nblocks, const i
                        const int* longs, float* y);
 
 // ---- ELL / SELL --------------------------------------------------------------
-// A work-group takes kEllRows rows.
+// A work-group that stages x takes kEllRows rows.  stored: slots of all slices.
 constexpr int kEllRows = 512;
 hipError_t ell(hipStream_t s, int rows, int hal, int ellnum, int rows_per_lane, XStage W,
                const int* col, const float* val, int cols, const float* x, float* y);
-hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, XStage W,
+hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, long long stored, XStage W,
                 const int* col, const float* val, int cols, const float* x, float* y);
 
 // ---- DIA / BDIA -------------------------------------------------------------

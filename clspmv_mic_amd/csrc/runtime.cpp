@@ -137,9 +137,12 @@ struct ColRange {
 // entries per chunk CSR 13.6 / 18.7, ELL 10.1 / 14.8, 9 per chunk 11.5 / 14.7
 // and 8.8 / 10.9; rows of 2 and 1 entries, ELL: 6.7 / 6.6 and 6.3 / 5.2).
 // Matrices of few work-groups wait for the list and the chunks: 60,000 rows
-// of 4, 5 entries per chunk, CSR 6.2 / 5.8, ELL 6.0 / 5.4; the 27-point stencil
-// 30^3, 40 per chunk, gains: CSR 4.2 / 4.8, ELL 4.5 / 5.6.
-constexpr int kEntriesPerChunk = 4, kFewGroups = 256, kEntriesPerChunkFew = 8, kEntriesPerGroup = 1536;
+// of 4, 5 entries per chunk, CSR 6.2 / 5.8, ELL 6.0 / 5.4; 5 consecutive
+// columns a row, ELL 100,000 rows 3.1 / 2.5, 200,000 3.3 / 3.1; 3-D stencil of 7
+// points on 47^3 3.0 / 2.6.  Long rows gain from 50,000 rows on (mesh of 40
+// neighbours, ELL 4.7 / 5.9, CSR 4.7 / 5.9).
+constexpr int kEntriesPerChunk = 4, kFewGroups = 256, kEntriesPerChunkFew = 8;
+constexpr int kEntriesPerGroup = 1536, kShortGroups = 384, kEntriesPerGroupShort = 4096;
 
 // A work-group's chunks and its entries' places in them.  runs(g, f) calls
 // f(first entry, count, to, step) for the entries of group g: entry first + i's
@@ -222,7 +225,8 @@ private:
                     ++looked;
                 }
                 const int per_chunk = groups < kFewGroups ? kEntriesPerChunkFew : kEntriesPerChunk;
-                if (entries < per_chunk * chunks || entries < kEntriesPerGroup * looked) return;
+                const int per_group = groups < kShortGroups ? kEntriesPerGroupShort : kEntriesPerGroup;
+                if (entries < per_chunk * chunks || entries < per_group * looked) return;
             }
             // The groups in `parts` runs of about as many, a thread each.
             const size_t parts = std::min<size_t>(total < (1u << 20) ? 1 : 8, groups);
@@ -412,7 +416,7 @@ int dmat_launch_rest(hipStream_t s, const clspmv_dmat* A, int method,
                             A->col, A->val, I.cols, x, y);
             break;
         case CLSPMV_FMT_SELL:
-            e = launch::sell(s, I.rows, I.slice_height, A->sptr, stage_of(A), A->col,
+            e = launch::sell(s, I.rows, I.slice_height, A->sptr, I.stored, stage_of(A), A->col,
                              A->val, I.cols, x, y);
             break;
         case CLSPMV_FMT_DIA: {

@@ -514,6 +514,28 @@ def test_ell_slot_groups(ctx, oracle, width, rows):
     _run(ctx, oracle, A, cs.coo2ell(A), cs.METHOD_AUTO)
     _run(ctx, oracle, A, cs.coo2sell(A, 32), cs.METHOD_AUTO)
 
+
+@pytest.mark.parametrize("rows, width", [(65, w) for w in (1, 2, 3, 4, 7, 9, 10, 15, 17, 23, 24, 31, 32, 33, 48, 49, 64)] +
+                         [((1 << 17) - 1, 9), ((1 << 17) - 1, 12)] +
+                         [((1 << 17) + 3, w) for w in (2, 3, 4, 9, 10, 23, 24, 25, 33)])
+def test_ell_gathered(ctx, oracle, rows, width):
+    """ELL and SELL without staged x (columns anywhere) at the mean row lengths
+    where the work-group and the slots in flight change; slices of 32 rows, of
+    a multiple of it and of neither, of different widths; dyadic inputs, exact
+    sums."""
+    rng = np.random.default_rng(width)
+    lens = np.where(np.arange(rows) % 64 < 32, width, max(1, width - 3))
+    cols = 50_000
+    r = np.repeat(np.arange(rows), lens)
+    first = np.repeat(np.cumsum(lens) - lens, lens)
+    c = (rng.integers(0, cols, rows)[r] + (np.arange(r.size) - first) * 769) % cols  # distinct in a row
+    o = np.lexsort((c, r))
+    A = cs.Coo(r.astype(np.int32), c[o].astype(np.int32), (rng.integers(-64, 65, r.size) / 64.0).astype(np.float32),
+               rows, cols)
+    _run(ctx, oracle, A, cs.coo2ell(A), 0)
+    for h in (32, 96, 40):
+        _run(ctx, oracle, A, cs.coo2sell(A, h), cs.METHOD_AUTO)
+
 @pytest.mark.parametrize("nbr", [(3 << 15) - 1, 3 << 15, (3 << 16) - 1, (3 << 16) + 77])
 @pytest.mark.parametrize("shape, width", [((4, 1), 5), ((4, 2), 2), ((4, 4), 3), ((8, 2), 1)])
 def test_block_walks(ctx, oracle, nbr, shape, width):
