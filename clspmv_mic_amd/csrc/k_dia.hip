@@ -92,13 +92,20 @@ __global__ __launch_bounds__(kBlock) void dia_row_kernel(
 // The sums are dia_row_kernel's, in diagonal order, bit for bit; x reads zero
 // outside the matrix.  len must be a multiple of 4.
 //
-// 16-bit values only, from 3 << 18 rows and 8 M values on: 27-point stencil 93^3 /
-// 101^3 / 128^3 14.0 / 17.1 / 31.4 -> 13.6 / 14.4 / 28.9 us, 5-point Laplacian
-// 1400^2 11.6 -> 10.6; below, the waves are too few (80^3 8.6 -> 9.6 us, 900^2
-// 5.9 -> 6.9).  FP32 values already set dia_row_kernel's pace (128^3 42.3 against
-// 42.7 us, 1400^2 12.4 against 13.1).
-constexpr int kQuadRows = 3 << 18;
+// 16-bit values only, from 15 << 16 rows and 8 M values on: 27-point stencil 101^3 /
+// 128^3 14.5 / 27.3 -> 13.4 / 26.6 us, 5-point Laplacian of 2 M rows 11.0 -> 9.6,
+// nine-point 13.9 -> 12.1; below, the waves are too few (27-point stencil of
+// 800,000 rows 11.8 -> 12.6 us, 400,000 7.4 -> 11.1).  And few segments, or full
+// runs: a wave walks them one after the other (1 M rows, 16 consecutive diagonals
+// 9.5 -> 11.4 us, 19-point stencil 11.3 -> 12.4; by S = 5 lone ones, 2 M rows, 5 / 7 /
+// 31 of them 11.0 / 11.1 / 31.1 -> 9.0 / 12.3 / 37.0).  FP32 values already set
+// dia_row_kernel's pace (128^3 42.3 against 42.7 us, 1400^2 12.4 against 13.1).
+constexpr int kQuadRows = 15 << 16;
 constexpr long long kQuadValues = 8 << 20;
+bool quad_segments(const launch::DiaSegments& S, int ndiag) {
+    if (S.width == 1) return S.count <= 5;
+    return S.count <= 3 || (S.count <= 9 && ndiag == S.width * S.count);
+}
 template <int W, int S, class V>
 __global__ __launch_bounds__(kBlock) void dia_quad_kernel(
     int rows, int cols, int len, int nseg, const int4* __restrict__ seg,
@@ -302,7 +309,7 @@ hipError_t dia_typed(hipStream_t s, int rows, int cols, int len, int ndiag,
             const dim3 g(ceil_div(rows, kBlock)), b(kBlock);
             if constexpr (sizeof(typename V::T) == 2) {
                 if (ndiag <= 32 && S.count > 0 && rows >= kQuadRows && rows * (long long)ndiag >= kQuadValues &&
-                    len % 4 == 0) {
+                    len % 4 == 0 && quad_segments(S, ndiag)) {
                     const dim3 q(ceil_div(rows, 4 * kBlock));
                     if (S.width == 1)
                         hipLaunchKernelGGL((dia_quad_kernel<1, 5, V>), q, b, 0, s, rows, cols, len, S.count, S.seg,

@@ -423,6 +423,28 @@ def test_dia_multi_tiles(ctx, offsets, n, ks):
             ctx.sync()
             np.testing.assert_array_equal(dY.download()[1:].reshape(k, n + 1), ref.astype(np.float32))
 
+def _dia_by_hand(n, off, align=32, seed=5):
+    """A DIA struct with the diagonals `off` full of dyadic values (zero outside
+    the matrix), and the arrays that it refers to."""
+    length = cs.lib.clspmv_aligned_length(n, align)
+    rng = np.random.default_rng(seed)
+    data, o32 = np.zeros((len(off), length), np.float32), np.array(off, np.int32)
+    for j, o in enumerate(off):
+        r0, r1 = max(0, -o), min(n, n - o)
+        data[j, r0:r1] = rng.integers(-64, 65, r1 - r0) / 64.0
+    m = cs.DiaMatrix(cs.MatInfo(n, n, int(np.count_nonzero(data))), len(off), n, length, cs._ip(o32), cs._fp(data))
+    return m, data, o32
+
+
+def _dia_product(data, off, n, X, Y):
+    """Y (k, n) + A X (n, k) in FP64."""
+    out = Y.astype(np.float64)
+    for j, o in enumerate(off):
+        r0, r1 = max(0, -o), min(n, n - o)
+        out[:, r0:r1] += data[j, r0:r1].astype(np.float64) * X[r0 + o:r1 + o].T
+    return out
+
+
 def _csr_wave_case(name):
     """Dyadic matrices at the edges of the CSR wave kernel: rows at its 512
     entries, runs of empty rows, blocks of 64 rows, and scattered columns in
@@ -637,6 +659,25 @@ def test_csr_multi_units(ctx, dtype, x_offset):
     for k in range(1, 17):
         np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
         np.testing.assert_array_equal(run(dR, Xr, k), wide[:k])
+
+@pytest.mark.parametrize("offsets", [[-900, -30, 0, 31, 1000], [-900, -30, -2, 0, 31, 1000],
+                                     [a + b * 40 for b in range(-4, 5) for a in (-1, 0, 1)],
+                                     [a + b * 40 for b in range(-4, 5) for a in (-1, 0, 1)][:-1],
+                                     [a + b * 40 for b in range(-4, 6) for a in (-1, 0, 1)]])
+@pytest.mark.parametrize("n", [(15 << 16) - 1, (15 << 16) + 37, (7 << 18) + 1])
+def test_dia_quad_segments(ctx, offsets, n):
+    """16-bit DIA at the segment counts where a lane takes four rows or one:
+    five and six lone diagonals, nine and ten full runs, nine with one cut short;
+    dyadic inputs, exact sums."""
+    m, data, _ = _dia_by_hand(n, offsets)
+    x, y0 = matrices.dyadic_vector(n, seed=11), matrices.dyadic_vector(n, seed=12)
+    ref = _dia_product(data, offsets, n, x[:, None], y0[None])
+    dA = cs.DeviceMatrix(ctx, m, dtype=cs.DT_BF16)
+    dx, dy = cs.DeviceVector(ctx, n, x), cs.DeviceVector(ctx, n, y0)
+    dA.spmv(dx, dy, 0)
+    ctx.sync()
+    np.testing.assert_array_equal(dy.download(), ref[0].astype(np.float32))
+
 
 @pytest.mark.parametrize("offsets", sorted(DIA_TILE_OFFSETS))
 @pytest.mark.parametrize("n,align", [((3 << 18) - 1, 32), ((3 << 18) + 37, 32), ((3 << 18) + 37, 1),
