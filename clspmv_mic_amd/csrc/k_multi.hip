@@ -237,6 +237,50 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
     }
 }
 
+// DIA where the chain of segments would set the time: a lane takes one row and
+// right-hand sides Q * (t % L) .. + Q - 1 (the last lane of a row ends at k) and
+// reads the X pieces itself, C diagonals' values and pieces in flight.  The sums
+// are dia_multi_kernel's, bit for bit.
+template <int Q, int L, class V>
+__global__ __launch_bounds__(kBlock) void dia_multi_direct_kernel(
+    int rows, int cols, int len, int ndiag, const int* __restrict__ off,
+    const typename V::T* __restrict__ data, int k, const float* __restrict__ X, float* __restrict__ Y,
+    int ldy, bool accumulate) {
+    constexpr int C = Q == 4 ? 8 : 16;
+    typedef VecOf<float, Q> XV;
+    const int t = threadIdx.x;
+    const int r = xcd_tile(blockIdx.x, gridDim.x) * (kBlock / L) + t / L;
+    if (r >= rows) return;
+    const int q0 = t % L * Q, qs = min(q0, k - Q);
+    float acc[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) acc[q] = 0.0f;
+    for (int j0 = 0; j0 < ndiag; j0 += C) {  // wave-uniform
+        float d[C];
+        typename XV::type xv[C];
+        bool in[C];
+#pragma unroll
+        for (int u = 0; u < C; ++u) {
+            const int j = min(j0 + u, ndiag - 1);
+            d[u] = V::ld(data + (size_t)j * len + r);
+            const int c = r + off[j];
+            in[u] = j0 + u < ndiag && (unsigned)c < (unsigned)cols;
+            xv[u] = *reinterpret_cast<const typename UVec<float, Q>::type*>(X + (size_t)(in[u] ? c : 0) * k + qs);
+        }
+#pragma unroll
+        for (int u = 0; u < C; ++u)
+#pragma unroll
+            for (int q = 0; q < Q; ++q) acc[q] = in[u] ? fmaf(d[u], XV::get(xv[u], q), acc[q]) : acc[q];
+    }
+    if (q0 >= k) return;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        if (qs + q < q0) continue;  // the lane before has this column
+        float* yp = Y + (size_t)(qs + q) * ldy + r;
+        *yp = (accumulate ? *yp : 0.0f) + acc[q];
+    }
+}
+
 // Accumulates a[q] += val[j] * X[col[j]][qb + q] over j = j0, j0 + step, ...
 // below j1 in that order, U nonzeros in flight per lane also in the last round
 // (slots past the end re-read the last one and are not added).  Acc is float,
@@ -521,6 +565,34 @@ hipError_t dia_multi_tile(hipStream_t s, int rows, int cols, int len, int nseg, 
     return hipGetLastError();
 }
 
+template <int Q, int L, class V>
+hipError_t dia_multi_direct(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off, const void* data,
+                            int k, const float* X, float* Y, int ldy, bool accumulate) {
+    hipLaunchKernelGGL((dia_multi_direct_kernel<Q, L, V>), dim3(ceil_div(rows, kBlock / L)), dim3(kBlock), 0, s, rows,
+                       cols, len, ndiag, off, static_cast<const typename V::T*>(data), k, X, Y, ldy, accumulate);
+    return hipGetLastError();
+}
+
+// Whether the direct kernel is the better one.  The staging kernel walks the
+// segments one after the other (about 0.25 us each at k = 1, 0.4 us at k = 8),
+// which sets its time on few rows, and on lone diagonals each staged X row is
+// read once.  Staged / direct, us:
+//   runs: 27-point stencil of 60,000 rows, k = 1 / 8 / 16, 5.2 / 7.5 / 10.5 and 4.4 /
+//     6.9 / 9.8; 120,000 rows 5.6 / 8.6 / 12.2 and 5.0 / 10.3 / 17.0;
+//   31 lone diagonals: 60,000 rows 10.1 / 15.1 / 17.8 and 4.6 / 7.2 / 9.9; 1 M rows
+//     29.5 / 67.3 / 109.5 and 21.6 / 64.4 / 123.9;
+//   14: 120,000 rows, k = 2 / 4 / 8 / 16, 6.8 / 7.7 / 9.3 / 11.9 and 4.4 / 5.2 / 7.9 /
+//     12.6; 650,000 rows 14.1 / 17.0 / 26.5 / 42.5 and 12.8 / 17.7 / 32.5 / 58.4;
+//   three: 120,000 rows 3.5 / 4.0 / 4.8 / 6.3 and 3.9 / 3.6 / 5.0 / 7.7.
+bool dia_multi_chain(int rows, int nseg, int w, int k) {
+    if (w > 1) return k == 1 ? rows < 300000 || nseg >= 10 : rows < 100000;
+    if (nseg >= 24) return k <= 8 || rows < 350000;
+    if (k == 1) return nseg >= 7;
+    if (k <= 3) return rows < 40000LL * nseg && rows < 600000;
+    if (k == 4) return nseg >= 7 || rows < 250000;
+    return rows < (k <= 8 && nseg >= 7 ? 200000 : 100000);
+}
+
 // Rows per lane: more of them reuse each staged X row more often but leave
 // fewer waves, each with a longer chain of segments.  On the 27-point stencil
 // the wider tile wins from 80^3 to 96^3 rows on (96^3, k = 4 / 8: 31 / 41 us
@@ -530,8 +602,19 @@ hipError_t dia_multi_tile(hipStream_t s, int rows, int cols, int len, int nseg, 
 // a wave has 64 / 4 lane groups, and four rows each win from 32^3 rows on
 // (32^3: 9.8 us, 22^3: 10.3 against 7.9 us).
 template <class V>
-hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int nseg, int w, const int4* seg,
-                       const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
+hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off, int nseg, int w,
+                       const int4* seg, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
+    if (dia_multi_chain(rows, nseg, w, k)) {
+#define CLSPMV_DIA_DIRECT(Q, L) dia_multi_direct<Q, L, V>(s, rows, cols, len, ndiag, off, data, k, X, Y, ldy, accumulate)
+        switch (k) {
+            case 1: return CLSPMV_DIA_DIRECT(1, 1);
+            case 2: return CLSPMV_DIA_DIRECT(2, 1);
+            case 3: return CLSPMV_DIA_DIRECT(3, 1);
+            case 4: return CLSPMV_DIA_DIRECT(4, 1);
+            default: return k <= 8 ? CLSPMV_DIA_DIRECT(4, 2) : CLSPMV_DIA_DIRECT(4, 4);
+        }
+#undef CLSPMV_DIA_DIRECT
+    }
     const bool large = rows >= (1 << 19);
     const bool deep = large && nseg >= 6;
 #define CLSPMV_DIA_MULTI(Q, L, R) dia_multi_tile<Q, L, R, V>(s, rows, cols, len, nseg, w, seg, data, k, X, Y, ldy, accumulate)
@@ -576,14 +659,14 @@ hipError_t csr_multi_v(hipStream_t s, const launch::CsrWave& W, const int* rp, c
 
 namespace launch {
 
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, DiaSegments S,
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off, DiaSegments S,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate) {
     if (rows <= 0 || cols <= 0 || S.count <= 0 || k <= 0) return hipSuccess;
     if (k > kMultiMax) return hipErrorInvalidValue;
     switch (dtype) {
-        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
-        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
-        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
+        case 0: return dia_multi_v<ValF32>(s, rows, cols, len, ndiag, off, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
+        case 1: return dia_multi_v<ValBF16>(s, rows, cols, len, ndiag, off, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
+        case 2: return dia_multi_v<ValF16>(s, rows, cols, len, ndiag, off, S.count, S.width, S.seg, data, k, X, Y, ldy, accumulate);
         default: return hipErrorInvalidValue;
     }
 }

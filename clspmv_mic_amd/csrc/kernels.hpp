@@ -173,7 +173,7 @@ hipError_t sbell(hipStream_t s, int brows, int rows, int cols, int bh, int bw,
 // Y[:, q] += A X[:, q], or without `accumulate` Y[:, q] = 0 + A X[:, q], Y not
 // read; X row-major (X[c*k + q]), Y column-major (ldy).
 constexpr int kMultiMax = 16;
-hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, DiaSegments S,
+hipError_t dia_multi(hipStream_t s, int rows, int cols, int len, int ndiag, const int* off, DiaSegments S,
                      int dtype, const void* data, int k, const float* X, float* Y, int ldy, bool accumulate);
 // CSR over the wave kernel's blocks and long rows.  A right-hand side's
 // result does not depend on k, nor does DIA's.

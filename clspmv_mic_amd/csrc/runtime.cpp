@@ -486,7 +486,7 @@ int multi_launch(hipStream_t s, const clspmv_dmat* A, int k, const float* X, flo
     const clspmv_dmat_info& I = A->info;
     hipError_t e;
     if (I.format == CLSPMV_FMT_DIA) {
-        e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, segments_of(A), A->dtype,
+        e = launch::dia_multi(s, std::min(I.rows, A->len), I.cols, A->len, A->ndiag, A->offs, segments_of(A), A->dtype,
                               A->dtype ? (const void*)A->lpval : (const void*)A->val, k, X, Y, ldy, accumulate);
     } else if (I.format == CLSPMV_FMT_CSR && A->plain) {
         e = launch::csr_multi(s, csr_wave_of(A), A->rp, A->col, A->dtype,

@@ -445,6 +445,31 @@ def _dia_product(data, off, n, X, Y):
     return out
 
 
+@pytest.mark.parametrize("n", [39_999, 99_999, 100_003, 200_000, 240_001, 300_007, 600_011])
+@pytest.mark.parametrize("name, offsets", [("three", [-9, 0, 11]), ("six", [-300, -9, 0, 11, 30, 4000]),
+                                           ("seven", [-400, -20, -9, 0, 11, 30, 4000]),
+                                           ("runs", [-301, -300, -299, -1, 0, 1, 299, 300, 301]),
+                                           ("thirty", [i * 17 for i in range(-15, 15)])])
+def test_dia_multi_routes(ctx, name, offsets, n):
+    """The multi-vector DIA kernels, staging and direct, at the row and segment
+    counts where the choice between them lies; dyadic inputs, exact sums, X and Y
+    aligned to one float only."""
+    m, data, _ = _dia_by_hand(n, offsets)
+    rng = np.random.default_rng(n)
+    dAs = [cs.DeviceMatrix(ctx, m, dtype=dt) for dt in (cs.DT_F32, cs.DT_F16)]
+    for k in (1, 2, 3, 4, 7, 8, 13):
+        X = (rng.integers(-64, 65, size=(n, k)) / 64.0).astype(np.float32)
+        Y0 = (rng.integers(-64, 65, size=(k, n + 1)) / 64.0).astype(np.float32)
+        ref = Y0.astype(np.float64)
+        ref[:, :n] = _dia_product(data, offsets, n, X, Y0[:, :n])
+        dX = cs.DeviceVector(ctx, X.size + 1, np.concatenate([[0.0], X.reshape(-1)]).astype(np.float32)).view(1)
+        for dA in dAs:
+            dY = cs.DeviceVector(ctx, Y0.size + 1, np.concatenate([[0.0], Y0.reshape(-1)]).astype(np.float32))
+            dA.spmv_multi(k, dX, dY.view(1), n + 1)
+            ctx.sync()
+            np.testing.assert_array_equal(dY.download()[1:].reshape(k, n + 1), ref.astype(np.float32))
+
+
 def _csr_wave_case(name):
     """Dyadic matrices at the edges of the CSR wave kernel: rows at its 512
     entries, runs of empty rows, blocks of 64 rows, and scattered columns in
