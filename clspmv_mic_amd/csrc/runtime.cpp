@@ -310,10 +310,18 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* b
 
 int auto_method(const clspmv_dmat* A) {
     switch (A->info.format) {
-        // The wave kernel: lanes striding over rows are no faster at any row
-        // length (27-point stencil 77^3 24 against 52 us, 5-point Laplacian
-        // 256^2 4.7 against 4.6 us, power-law rows 1 M 106 against 225 us).
-        case CLSPMV_FMT_CSR: return 1;
+        // Lanes striding over rows of about equal lengths where a row is one or
+        // two entries (2 M rows of one 8.5 us, by the wave kernel 12.8; 1 M of two
+        // random columns 17.2 / 19.5; of three 26.1 / 25.6) and on matrices so small
+        // that the wave kernel's longer chain shows (mesh of 5,000 rows of 8 2.8 /
+        // 3.1 us, 50,000 of 8 2.8 / 3.3, 20,000 of 25 3.1 / 3.1; 27-point stencil
+        // 30^3, 0.7 M entries, 3.9 / 3.1).  The wave kernel elsewhere (27-point
+        // stencil 77^3 52 / 15 us, power-law rows 1 M 225 / 106).
+        case CLSPMV_FMT_CSR: {
+            const double avg = A->info.rows ? (double)A->info.nnz / A->info.rows : 0.0;
+            const bool even = A->max_row <= 8.0 * std::max(avg, 4.0);
+            return even && (avg <= 2.0 || (avg <= 64.0 && A->info.nnz < (1 << 19))) ? 0 : 1;
+        }
         // A row per lane: four rows per lane leave a quarter of the waves and
         // gather x four rows apart (27-point stencil 77^3 30 against 19 us,
         // 30^3 21 against 6.5 us; 5-point Laplacian 701^2 7.9 against 5.9 us).

@@ -605,6 +605,27 @@ def test_block_walks(ctx, oracle, nbr, shape, width):
     _run(ctx, oracle, A, cs.coo2sbell(A.copy(), bw, bh), 0)
 
 
+@pytest.mark.parametrize("rows, lens", [(30_000, 2), (30_000, 3), (262_143, 2), (262_144, 2), (20_000, 26), (20_000, 27),
+                                        (8_000, 64), (8_000, 65), (300, 300)])
+@pytest.mark.parametrize("skew", [False, True])
+def test_csr_auto(ctx, oracle, rows, lens, skew):
+    """The automatic CSR method around the sizes where it changes kernels, with
+    rows of equal lengths and with one long one; dyadic inputs, exact sums."""
+    n = np.full(rows, lens)
+    if skew:
+        n[rows // 2] = 9 * max(lens, 4)
+    r = np.repeat(np.arange(rows), n)
+    first = np.repeat(np.cumsum(n) - n, n)
+    width = 9 * 65 + rows
+    c = (r + (np.arange(r.size) - first)) % width
+    o = np.lexsort((c, r))
+    A = cs.Coo(r.astype(np.int32), c[o].astype(np.int32),
+               (np.random.default_rng(lens).integers(-64, 65, r.size) / 64.0).astype(np.float32), rows, width)
+    for dtype in (cs.DT_F32, cs.DT_F16):
+        for method in (cs.METHOD_AUTO, 1):
+            _run(ctx, oracle, A, cs.coo2csr(A.copy()), method, panel=0, dtype=dtype)
+
+
 @pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_BF16])
 @pytest.mark.parametrize("others", [0, 1, 2, 15, 31, 32, 62, 63])
 def test_csr_wide_rows(ctx, oracle, others, dtype):
