@@ -21,33 +21,6 @@ namespace {
 using namespace dev;
 using launch::kDiaRun;
 
-// Loads right-hand sides qb .. qb+Q-1 of row c of X (zero where q >= k).
-template <int Q>
-__device__ __forceinline__ void load_xq(const float* __restrict__ X, int c, int k, int qb, bool vec,
-                                        float* xv) {
-    const float* p = X + (size_t)c * k + qb;
-    if (qb >= k) {  // a lane quad past k (e.g. k = 12 with KB = 16): nothing to load
-#pragma unroll
-        for (int q = 0; q < Q; ++q) xv[q] = 0.0f;
-        return;
-    }
-    if constexpr (Q == 4) {
-        if (vec) {  // k % 4 == 0, X 16-byte aligned
-            const float4 t = *reinterpret_cast<const float4*>(p);
-            xv[0] = t.x; xv[1] = t.y; xv[2] = t.z; xv[3] = t.w;
-            return;
-        }
-    } else if constexpr (Q == 2) {
-        if (vec) {  // k == 2, X 8-byte aligned
-            const float2 t = *reinterpret_cast<const float2*>(p);
-            xv[0] = t.x; xv[1] = t.y;
-            return;
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) xv[q] = qb + q < k ? p[q] : 0.0f;
-}
-
 // DIA.  The diagonals come as segments {first diagonal, its offset, how many
 // (at most W) consecutive offsets, 0} in diagonal order.  A wave owns NR
 // consecutive rows; lane t takes rows R * (t / L) .. + R - 1 and right-hand
@@ -281,70 +254,121 @@ __global__ __launch_bounds__(kBlock) void dia_multi_direct_kernel(
     }
 }
 
-// Accumulates a[q] += val[j] * X[col[j]][qb + q] over j = j0, j0 + step, ...
-// below j1 in that order, U nonzeros in flight per lane also in the last round
-// (slots past the end re-read the last one and are not added).  Acc is float,
-// or double for rows longer than kLongRowF64 (the products are exact in
-// double).
-template <int Q, class V, class Acc, int U>
-__device__ __forceinline__ void csr_multi_run(const int* __restrict__ col,
-                                              const typename V::T* __restrict__ val, int j0, int j1,
-                                              int step, const float* __restrict__ X, int k, int qb,
-                                              bool vec, Acc* a) {
-    // (Indices from j0: the sums stay in range near 2^31 entries.)
-    const int n = j1 - j0;
-    col += j0;
-    val += j0;
-    for (int j = 0; j < n; j += U * step) {
+// The value of lane P of each aligned group of L lanes (L at most 4), by a
+// DPP quad permute.
+template <int L, int P, class T>
+__device__ __forceinline__ T group_lane(T v) {
+    if constexpr (L == 1) return v;
+    constexpr int ctrl = L == 4 ? P * 0x55 : P | P << 2 | (P + 2) << 4 | (P + 2) << 6;
+    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false));
+}
+
+// Work-group of the CSR kernel: a row by 512 threads has up to 4,096 entries in
+// flight (a 5,000-entry row sets the time of a small power-law matrix).  Rows of
+// kWaveNnz + 1 to kWideRowNnz entries go to a wave each where there are enough of
+// them to fill the chip (launch::CsrWave::nwide), else, and longer ones, to a
+// work-group each.  Columns of neighbouring rows overlapping / anywhere, k = 1, 4
+// and 16, us: 15,000 rows of 1,100 by waves 28 / 33 / 68 and 112 / 229 / 310, by
+// work-groups 39 / 80 / 101 and 94 / 231 / 297; 500 rows of 700 5.3 / 6.0 / 9.9
+// against 3.6 / 4.5 / 4.6; 3,000 rows of 5,000 by work-groups 25 / 35 / 74 and 98 /
+// 206 / 278.
+constexpr int kMultiThreads = 512;
+
+// One row longer than kWaveNnz by a team of T threads (a wave or the
+// work-group), t its thread: "slot" t of T sums entries t, t + T, ... in order,
+// and the slots are added by the tree of neighbours, neighbours' neighbours, ...
+// whatever k is: a lane loads its slot's entries, L lanes hand them round and
+// keep the sums of their L slots for Q right-hand sides each.  Rounds past the
+// row's end are skipped by the wave, entries past it re-read the last one and
+// are not added.  Returns the wave's sums in sum.
+template <int Q, int L, int T, class V, class Acc>
+__device__ __forceinline__ void csr_multi_row(unsigned t, int s, unsigned n, const int* __restrict__ col,
+                                              const typename V::T* __restrict__ val,
+                                              const float* __restrict__ Xq, int k, Acc* sum) {
+    constexpr int U = (Q >= 3 && L < 4 ? 6 : 8) / L;  // rounds in flight, by the registers that leave three work-groups a CU
+    typedef VecOf<float, Q> XV;
+    const unsigned p = t % L, w0 = __builtin_amdgcn_readfirstlane(t / kWave * kWave);
+    // (Unsigned indices from the row's start: the sums stay in range near 2^31
+    // entries.)
+    col += s;
+    val += s;
+    Acc a[L][Q];
+#pragma unroll
+    for (int i = 0; i < L; ++i)
+#pragma unroll
+        for (int q = 0; q < Q; ++q) a[i][q] = 0;
+    for (unsigned base = 0; base + w0 < n; base += U * T) {
+        const int rounds = (int)((n - base - w0 + T - 1) / T);  // wave-uniform
         int c[U];
         float v[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int at = min(j + u * step, n - 1);
+            if (u >= rounds) break;
+            const unsigned at = min(base + u * T + t, n - 1);
             c[u] = ld_stream(col + at);
             v[u] = V::ld(val + at);
         }
-        float xv[U][Q];
+        typename XV::type xv[U][L];
+        float vs[U][L];
 #pragma unroll
-        for (int u = 0; u < U; ++u) load_xq<Q>(X, c[u], k, qb, vec, xv[u]);
+        for (int u = 0; u < U; ++u) {
+            if (u >= rounds) break;
+            int cs[L];
+            cs[0] = group_lane<L, 0>(c[u]);
+            vs[u][0] = group_lane<L, 0>(v[u]);
+            if constexpr (L >= 2) {
+                cs[1] = group_lane<L, 1>(c[u]);
+                vs[u][1] = group_lane<L, 1>(v[u]);
+            }
+            if constexpr (L == 4) {
+                cs[2] = group_lane<L, 2>(c[u]);
+                vs[u][2] = group_lane<L, 2>(v[u]);
+                cs[3] = group_lane<L, 3>(c[u]);
+                vs[u][3] = group_lane<L, 3>(v[u]);
+            }
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-            if (j + u * step < n)
+            for (int i = 0; i < L; ++i)
+                xv[u][i] = *reinterpret_cast<const typename UVec<float, Q>::type*>(Xq + (size_t)cs[i] * k);
+        }
 #pragma unroll
-                for (int q = 0; q < Q; ++q) a[q] = fma((Acc)v[u], (Acc)xv[u][q], a[q]);
+        for (int u = 0; u < U; ++u) {
+            if (u >= rounds) break;
+#pragma unroll
+            for (int i = 0; i < L; ++i) {
+                const bool in = base + u * T + t - p + i < n;
+#pragma unroll
+                for (int q = 0; q < Q; ++q) {
+                    const Acc f = fma((Acc)vs[u][i], (Acc)XV::get(xv[u][i], q), a[i][q]);
+                    a[i][q] = in ? f : a[i][q];
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        Acc b = a[0][q];
+        if constexpr (L == 2) b += a[1][q];
+        if constexpr (L == 4) b = (b + a[1][q]) + (a[2][q] + a[3][q]);
+        for (int m = L; m < kWave; m <<= 1) b += __shfl_xor(b, m, kWave);
+        sum[q] = b;
     }
 }
 
-// Work-group of the CSR kernel: with 512 threads a row over kWaveNnz entries has
-// 1,024 of them in flight (a 5,000-entry row sets the time of a small
-// power-law matrix: 60,000 rows, k = 4: 19.7 us against 27.3 with 256 threads;
-// 17.6 with the longest rows first).
-constexpr int kMultiThreads = 512;
-
-// One row longer than kWaveNnz by the whole work-group, always with four
-// lanes per entry, so that a column's sum does not depend on k: each lane
-// group strides the row with 8 entries in flight, the eight waves' sums are
-// combined in a fixed order through LDS, and Y[:, r] is updated once per
-// right-hand side.
-template <class V, class Acc>
+// A row by the work-group: the eight waves' sums are combined in a fixed order
+// through LDS, and Y[:, r] is updated once per right-hand side (rows summed in
+// FP64 rounded once).
+template <int Q, int L, class V, class Acc>
 __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__ val,
-                                               const int* __restrict__ col, int r, int j0, int j1,
-                                               const float* __restrict__ X, int k, bool vec,
-                                               float* __restrict__ Y, int ldy, bool accumulate,
-                                               Acc (*part)[launch::kMultiMax]) {
-    constexpr int Q = 4, L = launch::kMultiMax / Q;
-    const int t = threadIdx.x;
-    const int qb = (t % L) * Q;
-    Acc a[Q];
+                                               const int* __restrict__ col, int r, int s, int n,
+                                               const float* __restrict__ X, int k, float* __restrict__ Y, int ldy,
+                                               bool accumulate, Acc (*part)[launch::kMultiMax]) {
+    const int t = threadIdx.x, q0 = t % L * Q, qs = min(q0, k - Q);
+    Acc sum[Q];
+    csr_multi_row<Q, L, kMultiThreads, V, Acc>(t, s, n, col, val, X + qs, k, sum);
+    if (t % kWave < L && q0 < k) {
 #pragma unroll
-    for (int q = 0; q < Q; ++q) a[q] = 0;
-    csr_multi_run<Q, V, Acc, 8>(col, val, j0 + t / L, j1, kMultiThreads / L, X, k, qb, vec, a);
-#pragma unroll
-    for (int q = 0; q < Q; ++q)
-        for (int m = kWave >> 1; m >= L; m >>= 1) a[q] += __shfl_xor(a[q], m, kWave);
-    if ((t & (kWave - 1)) < L) {
-#pragma unroll
-        for (int q = 0; q < Q; ++q) part[t / kWave][qb + q] = a[q];
+        for (int q = 0; q < Q; ++q)
+            if (qs + q >= q0) part[t / kWave][qs + q] = sum[q];
     }
     __syncthreads();
     if (t < k) {
@@ -354,19 +378,73 @@ __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__
         float* yp = Y + (size_t)t * ldy + r;
         const float y0 = accumulate ? *yp : 0.0f;
         if constexpr (sizeof(Acc) == sizeof(double))
-            *yp = (float)((double)y0 + tot);  // one rounding of the whole row
+            *yp = (float)((double)y0 + tot);
         else
             *yp = y0 + tot;
     }
 }
 
-// The value of lane P of each aligned group of L lanes (L at most 4), by a
-// DPP quad permute.
-template <int L, int P, class T>
-__device__ __forceinline__ T group_lane(T v) {
-    if constexpr (L == 1) return v;
-    constexpr int ctrl = L == 4 ? P * 0x55 : P | P << 2 | (P + 2) << 4 | (P + 2) << 6;
-    return __builtin_bit_cast(T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), ctrl, 0xF, 0xF, false));
+// Entries of a unit (below).
+constexpr int kUnit = 8;
+
+// A block whose rows hold at most four entries each: a lane per row, without
+// the units' pass through LDS (2 M rows of one entry, k = 1 / 2 / 4: 22.2 / 28.9 /
+// 36.8 -> 11.5 / 14.6 / 22.1 us).  The sums are the units', bit for bit: a row's
+// entries up to the next multiple of kUnit from the block's start in one chain,
+// those after it in another.  False: some row is longer, nothing was done.
+template <int Q, class V>
+__device__ __forceinline__ bool csr_multi_short(int lane, int r0, int nrows, int s, int n, const int* __restrict__ rp,
+                                                const int* __restrict__ col, const typename V::T* __restrict__ val,
+                                                int k, const float* __restrict__ X, float* __restrict__ Y, int ldy,
+                                                bool accumulate) {
+    constexpr int M = 4;
+    typedef VecOf<float, Q> XV;
+    if (n > M * kWave) return false;
+    const bool row = lane < nrows;
+    const int b0 = rp[r0 + min(lane, nrows)] - s, b1 = rp[r0 + min(lane + 1, nrows)] - s, len = b1 - b0;
+    if (__ballot(len > M)) return false;
+    float first[Q], a[Q], y[Q];
+    bool two = false;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) first[q] = a[q] = y[q] = 0.0f;
+    const bool write = row && !(len == 0 && accumulate);  // empty rows leave Y as it is
+    if (write && accumulate) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) y[q] = Y[(size_t)q * ldy + r0 + lane];
+    }
+    col += s;
+    val += s;
+    int c[M];
+    float v[M];
+    typename XV::type xv[M];
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+        if (e >= len) continue;
+        c[e] = ld_stream(col + b0 + e);
+        v[e] = V::ld(val + b0 + e);
+    }
+#pragma unroll
+    for (int e = 0; e < M; ++e)
+        if (e < len) xv[e] = *reinterpret_cast<const typename UVec<float, Q>::type*>(X + (size_t)c[e] * k);
+#pragma unroll
+    for (int e = 0; e < M; ++e) {
+        if (e >= len) continue;
+        if (e > 0 && (b0 + e) % kUnit == 0) {
+            two = true;
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                first[q] = a[q];
+                a[q] = 0.0f;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) a[q] = fmaf(v[e], XV::get(xv[e], q), a[q]);
+    }
+    if (write) {
+#pragma unroll
+        for (int q = 0; q < Q; ++q) Y[(size_t)q * ldy + r0 + lane] = y[q] + (two ? first[q] + a[q] : a[q]);
+    }
+    return true;
 }
 
 // CSR: a wave per block of short rows (the wave kernel's blocks), L lanes per
@@ -392,13 +470,11 @@ __device__ __forceinline__ T group_lane(T v) {
 // Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 138 / 174 us; 1 M
 // rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 266 / 251 / 302 us (53 G rows/s);
 // 27-point stencil 64^3, k = 8: 74 -> 31 us.
-constexpr int kUnit = 8;
-
 template <int Q, int L, class V>
-__global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
-    int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
+__global__ __launch_bounds__(kMultiThreads, L == 4 ? 4 : 6) void csr_multi_kernel(
+    int nlong, int nwide, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
     const int* __restrict__ rp, const int* __restrict__ col, const typename V::T* __restrict__ val, int k,
-    const float* __restrict__ X, bool vec, float* __restrict__ Y, int ldy, bool accumulate) {
+    const float* __restrict__ X, float* __restrict__ Y, int ldy, bool accumulate) {
     typedef typename V::T T;
     constexpr int QP = Q == 3 ? 4 : Q;              // LDS floats per piece
     constexpr int KB = QP * L;                      // and per row or unit
@@ -419,24 +495,43 @@ __global__ __launch_bounds__(kMultiThreads) void csr_multi_kernel(
         float part[kWaves][launch::kMultiMax];
         double part64[kWaves][launch::kMultiMax];
     } lds;
-    if ((int)blockIdx.x < nlong) {  // the longest work first
-        const int r = longs[blockIdx.x], j0 = rp[r], j1 = rp[r + 1];
-        if (j1 - j0 > launch::kLongRowF64)
-            csr_multi_long<V, double>(val, col, r, j0, j1, X, k, vec, Y, ldy, accumulate, lds.part64);
+    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int q0 = lane % L * Q, qs = min(q0, k - Q);  // the last piece ends at k
+    const int nlwg = nwide + (nlong - nwide + kWaves - 1) / kWaves;
+    if ((int)blockIdx.x < nwide) {  // the longest work first
+        const int r = longs[blockIdx.x], j0 = rp[r], n = rp[r + 1] - j0;
+        if (n > launch::kLongRowF64)
+            csr_multi_long<Q, L, V, double>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part64);
         else
-            csr_multi_long<V, float>(val, col, r, j0, j1, X, k, vec, Y, ldy, accumulate, lds.part);
+            csr_multi_long<Q, L, V, float>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part);
         return;
     }
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int b = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x - nlong, gridDim.x - nlong) * kWaves + wave);
+    if ((int)blockIdx.x < nlwg) {  // a wave per row
+        const int at = nwide + ((int)blockIdx.x - nwide) * kWaves + wave;
+        if (at >= nlong) return;
+        const int r = longs[at], j0 = rp[r], n = rp[r + 1] - j0;
+        float sum[Q], y[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) y[q] = accumulate ? Y[(size_t)(qs + q) * ldy + r] : 0.0f;
+        csr_multi_row<Q, L, kWave, V, float>(lane, j0, n, col, val, X + qs, k, sum);
+        if (lane < L && q0 < k) {
+#pragma unroll
+            for (int q = 0; q < Q; ++q)
+                if (qs + q >= q0) Y[(size_t)(qs + q) * ldy + r] = y[q] + sum[q];
+        }
+        return;
+    }
+    const int b = __builtin_amdgcn_readfirstlane(xcd_tile(blockIdx.x - nlwg, gridDim.x - nlwg) * kWaves + wave);
     if (b >= nblk) return;  // the whole wave
     const int4 B = blk[b];  // {first row, rows, first entry, entries}
     const int r0 = B.x, nrows = B.y, s = B.z, n = B.w;
     WaveLds& W = lds.w[wave];
     const int gi = lane / L, p = lane % L;
-    const int q0 = p * Q, qs = min(q0, k - Q);  // the last piece ends at k
     const bool act = q0 < k;
     const float* Xq = X + qs;
+    if constexpr (L == 1) {
+        if (csr_multi_short<Q, V>(lane, r0, nrows, s, n, rp, col, val, k, Xq, Y, ldy, accumulate)) return;
+    }
     typedef VecOf<int, NE> CV;
     typedef VecOf<T, NE> TV;
     typename CV::type cn;
@@ -633,11 +728,10 @@ hipError_t dia_multi_v(hipStream_t s, int rows, int cols, int len, int ndiag, co
 template <int Q, int L, class V>
 hipError_t csr_multi_tile(hipStream_t s, const launch::CsrWave& W, const int* rp, const int* col, const void* val,
                           int k, const float* X, float* Y, int ldy, bool accumulate) {
-    const bool vec = k % 4 == 0 && ((uintptr_t)X % 16) == 0;  // long rows: aligned 16-byte pieces
-    hipLaunchKernelGGL((csr_multi_kernel<Q, L, V>), dim3(W.nlong + ceil_div(W.nblk, kMultiThreads / kWave)),
-                       dim3(kMultiThreads), 0, s,
-                       W.nlong, W.longs, W.nblk, W.blk, rp, col, static_cast<const typename V::T*>(val), k, X, vec, Y,
-                       ldy, accumulate);
+    constexpr int kWaves = kMultiThreads / kWave;
+    const int groups = W.nwide + ceil_div(W.nlong - W.nwide, kWaves) + ceil_div(W.nblk, kWaves);
+    hipLaunchKernelGGL((csr_multi_kernel<Q, L, V>), dim3(groups), dim3(kMultiThreads), 0, s, W.nlong, W.nwide, W.longs,
+                       W.nblk, W.blk, rp, col, static_cast<const typename V::T*>(val), k, X, Y, ldy, accumulate);
     return hipGetLastError();
 }
 

@@ -41,12 +41,18 @@ struct XStage {
 // one.  A work-group that stages x takes kCsrWaves blocks.
 constexpr int kWaveNnz = 512;
 constexpr int kCsrWaves = 8;
+constexpr int kWideRowNnz = 2048;
+constexpr int kWaveRows = 4096;  // rows of up to kWideRowNnz entries before waves take them
+static_assert(kWideRowNnz <= kLongRowF64, "rows by one wave are summed in FP32");
 static_assert(4 * (kWaveNnz * kCsrWaves + kXChunk * kXChunksMax) <= 64 * 1024, "within the default LDS limit");
 struct CsrWave {
     const int4* blk = nullptr;
     int nblk = 0;
     const int* longs = nullptr;
     int nlong = 0;
+    // Multi-vector kernel: the first nwide go to a work-group each, the others (of
+    // at most kWideRowNnz entries) to a wave each.
+    int nwide = 0;
     XStage stage;
 };
 hipError_t csr_wave(hipStream_t s, const CsrWave& W, const int* rp, const int* col, int dtype, const void* val,

@@ -302,6 +302,9 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* b
     // (power-law rows, 96,050: 15.3 -> 12.4 us, 1 M: 113.5 -> 107 us).
     std::stable_sort(longs.begin(), longs.end(), [&](int a, int b) { return rp[a + 1] - rp[a] > rp[b + 1] - rp[b]; });
     d->nwlong = (int)longs.size();
+    d->nwwide = (int)std::count_if(longs.begin(), longs.end(),
+                                   [&](int r) { return rp[r + 1] - rp[r] > launch::kWideRowNnz; });
+    if (d->nwlong - d->nwwide < launch::kWaveRows) d->nwwide = d->nwlong;
     int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
     if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
     if (blocks) *blocks = std::move(blk);
@@ -367,7 +370,7 @@ launch::DiaSegments segments_of(const clspmv_dmat* A) { return launch::DiaSegmen
 launch::XStage stage_of(const clspmv_dmat* A) { return launch::XStage{A->xlist, A->xidx, A->xstride}; }
 
 launch::CsrWave csr_wave_of(const clspmv_dmat* A) {
-    return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, stage_of(A)};
+    return launch::CsrWave{A->wblk, A->nwblk, A->wlong, A->nwlong, A->nwwide, stage_of(A)};
 }
 
 int resolve_method(const clspmv_dmat* A, int* method) {

@@ -33,7 +33,7 @@ struct clspmv_dmat {
     int max_row = 0;
     int4* wblk = nullptr;
     int* wlong = nullptr;
-    int nwblk = 0, nwlong = 0;
+    int nwblk = 0, nwlong = 0, nwwide = 0;
     // Staged x of CSR's wave kernel, ELL and SELL (launch::XStage; null: absent).
     int* xlist = nullptr;
     unsigned short* xidx = nullptr;

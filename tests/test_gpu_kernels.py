@@ -706,6 +706,46 @@ def test_csr_multi_units(ctx, dtype, x_offset):
         np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
         np.testing.assert_array_equal(run(dR, Xr, k), wide[:k])
 
+@pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_F16])
+@pytest.mark.parametrize("medium", [4095, 4096, 4100])
+def test_csr_multi_long_rows(ctx, medium, dtype):
+    """Rows longer than a block, by a wave or a work-group each as their number
+    decides, around the kernels' rounds (513, 576, 577, 1024, 2047..2049 and
+    longer), and blocks of rows of 0..4 entries, which have a path of their own up
+    to four right-hand sides: dyadic inputs, so Y equals the FP64 product, and
+    each right-hand side's bits on random inputs do not depend on k."""
+    rng = np.random.default_rng(medium)
+    width = 6000
+    lens = np.concatenate([rng.choice([513, 514, 576, 577, 640, 1024, 2047, 2048], medium), rng.integers(0, 5, 3000),
+                           [2049, 4096, 4097, 5000, 4, 5, 0, 3], rng.integers(0, 3, 700)])
+    rng.shuffle(lens)
+    r = np.repeat(np.arange(lens.size), lens)
+    first = np.repeat(np.cumsum(lens) - lens, lens)
+    c = np.sort((rng.integers(0, width, lens.size)[r] + np.arange(r.size) - first) % width + r * np.int64(width)) % width
+    Ad = cs.Coo(r.astype(np.int32), c.astype(np.int32), (rng.integers(-8, 9, r.size) / 8.0).astype(np.float32),
+                lens.size, width)
+    Ar = cs.Coo(Ad.row, Ad.col, rng.standard_normal(r.size).astype(np.float32), lens.size, width)
+    dA, dR = (cs.DeviceMatrix(ctx, cs.coo2csr(m.copy()), panel=0, dtype=dtype) for m in (Ad, Ar))
+    Xd = (rng.integers(-8, 9, size=(width, 16)) / 8.0).astype(np.float32)
+    Xr = rng.uniform(-1, 1, size=(width, 16)).astype(np.float32)
+    Y0 = (rng.integers(-8, 9, size=(16, lens.size)) / 8.0).astype(np.float32)
+    import scipy.sparse as sp
+    S = sp.csr_matrix((Ad.val.astype(np.float64), (Ad.row, Ad.col)), shape=(lens.size, width))
+    ref = Y0 + (S @ Xd.astype(np.float64)).T
+
+    def run(m, X, k):
+        dX = cs.DeviceVector(ctx, k * width, np.ascontiguousarray(X[:, :k]).reshape(-1))
+        dY = cs.DeviceVector(ctx, k * lens.size, Y0[:k].reshape(-1))
+        m.spmv_multi(k, dX, dY, lens.size)
+        ctx.sync()
+        return dY.download().reshape(k, lens.size)
+
+    wide = run(dR, Xr, 16)
+    for k in (1, 2, 3, 4, 5, 7, 8, 9, 12, 15, 16):
+        np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
+        np.testing.assert_array_equal(run(dR, Xr, k), wide[:k])
+
+
 @pytest.mark.parametrize("offsets", [[-900, -30, 0, 31, 1000], [-900, -30, -2, 0, 31, 1000],
                                      [a + b * 40 for b in range(-4, 5) for a in (-1, 0, 1)],
                                      [a + b * 40 for b in range(-4, 5) for a in (-1, 0, 1)][:-1],
