@@ -602,13 +602,20 @@ hipError_t launch_nq(hipStream_t s, bool long_rows, int brows, int rows, int col
     // sides, 8-byte aligned ones too: 131,072 block rows x 12, k = 5 / 9 / 17 /
     // 31: 20.7 / 31.4 / 40.6 / 47.9 us from the tiles directly, 15.7 / 21.6 /
     // 33.1 / 41.9 through the windows).
+    // Several chunks through the windows are one wave per slice, from the tiles a
+    // wave per slice and chunk: 8-byte pieces (odd k) take the tiles while the
+    // slices are too few to fill the chip by themselves (500 block rows, 32 slices,
+    // k = 17 / 33: 5.5 / 5.7 us from the tiles, 6.6 / 8.4 through the windows; 9,000,
+    // k = 33: 7.6 / 8.9; k = 17: 6.9 / 6.6).
     if constexpr (kX16) {
         bool done = false;
-        const hipError_t e =
-            x16 ? launch_win<BF16, NQ, false, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
-                                                     win, done)
-                : launch_win<BF16, NQ, false, true>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
-                                                    win, done);
+        hipError_t e = hipSuccess;
+        if (x16)
+            e = launch_win<BF16, NQ, false, false>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
+                                                   win, done);
+        else if (chunks == 1 || slices >= 256 * chunks)
+            e = launch_win<BF16, NQ, false, true>(s, long_rows, brows, rows, cols, k, rp, val, X, ldx, Y, ldy, acc_y,
+                                                  win, done);
         if (done || e != hipSuccess) return e;
     }
     const unsigned nb = (unsigned)blocks;
