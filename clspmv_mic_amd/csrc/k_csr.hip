@@ -86,6 +86,42 @@ __device__ __forceinline__ void csr_long_row(int s, int e, const int* __restrict
     }
 }
 
+// A row over kWaveNnz by a wave, where there are enough of them to fill the chip
+// (launch::CsrWave::nwide): 30,000 rows of 513 / 15,000 of 1,100 overlapping
+// columns 27 / 27.5 us, by a work-group each 35 / 31 us.  Not 16-bit values, whose
+// long rows the work-groups already take in 33 / 28 us (by waves 33 / 32.6).
+template <class V>
+__device__ __forceinline__ float csr_wave_row(int lane, int s, int n, const int* __restrict__ col,
+                                              const typename V::T* __restrict__ val, const float* __restrict__ x) {
+    constexpr int U = 8;
+    float acc = 0.0f;
+    col += s;
+    val += s;
+    for (int base = 0; base < n; base += U * kWave) {
+        const int rounds = (n - base + kWave - 1) / kWave;
+        int c[U];
+        float v[U], xv[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {  // past the end: the last entry again, not added
+            if (u >= rounds) break;
+            const int at = min(base + u * kWave + lane, n - 1);
+            c[u] = ld_stream(col + at);
+            v[u] = V::ld(val + at);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u >= rounds) break;
+            xv[u] = x[c[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (u >= rounds) break;
+            acc = base + u * kWave + lane < n ? fmaf(v[u], xv[u], acc) : acc;
+        }
+    }
+    return group_sum<kWave>(acc);
+}
+
 // What bounds it: the gathers of x, and before that the waves' chain of
 // dependent loads (block, columns, x).  A wave loads the up to kWaveNnz entries
 // of its block at once as 16-byte pieces (the arrays carry kWaveNnz entries
@@ -119,7 +155,7 @@ constexpr int kPlainWaves = 4;
 
 template <class V, bool WIN, int kWaves>
 __global__ __launch_bounds__(kWave* kWaves) void csr_wave_kernel(
-    int nlong, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
+    int nlong, int nwide, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,
     const int* __restrict__ list, const unsigned short* __restrict__ idx, int stride, int cols,
     const int* __restrict__ rp, const int* __restrict__ col,
     const typename V::T* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
@@ -128,7 +164,8 @@ __global__ __launch_bounds__(kWave* kWaves) void csr_wave_kernel(
     typedef typename UVec<T, 4>::type T4U;
     typedef VecOf<unsigned short, 4> I4;
     extern __shared__ __attribute__((aligned(16))) float sm[];  // x chunks, then the products of each wave
-    if ((int)blockIdx.x < nlong) {  // the longest work first
+    const int nlwg = nwide + (nlong - nwide + kWaves - 1) / kWaves;
+    if ((int)blockIdx.x < nwide) {  // the longest work first
         const int r = longs[blockIdx.x], s = rp[r], e = rp[r + 1];
         double* part = reinterpret_cast<double*>(sm);
         if (sizeof(T) == 2 && e - s > launch::kLongRowF64)
@@ -138,7 +175,15 @@ __global__ __launch_bounds__(kWave* kWaves) void csr_wave_kernel(
         return;
     }
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int wg = xcd_tile(blockIdx.x - nlong, gridDim.x - nlong);
+    if (sizeof(T) == 4 && (int)blockIdx.x < nlwg) {
+        const int at = nwide + ((int)blockIdx.x - nwide) * kWaves + wave;
+        if (at >= nlong) return;
+        const int r = longs[at], s = rp[r];
+        const float sum = csr_wave_row<V>(lane, s, rp[r + 1] - s, col, val, x);
+        if (lane == 0) y[r] += sum;
+        return;
+    }
+    const int wg = xcd_tile(blockIdx.x - nlwg, gridDim.x - nlwg);
     const int b = __builtin_amdgcn_readfirstlane(wg * kWaves + wave);
     if (!WIN && b >= nblk) return;
     StageX<kWave * kWaves> stage;
@@ -219,10 +264,12 @@ hipError_t csr_wave_v(hipStream_t s, const launch::CsrWave& W, const int* rp, co
                       int cols, const float* x, float* y) {
     const typename V::T* v = static_cast<const typename V::T*>(val);
     auto launch = [&](auto kernel, int waves, const launch::XStage& X) {
-        const dim3 grid(W.nlong + (W.nblk + waves - 1) / waves), block(kWave * waves);
+        const int nwide = sizeof(typename V::T) == 4 ? W.nwide : W.nlong;  // rows by a work-group each
+        const dim3 grid(nwide + (W.nlong - nwide + waves - 1) / waves + (W.nblk + waves - 1) / waves),
+            block(kWave * waves);
         const size_t lds = sizeof(float) * (launch::kWaveNnz * waves + launch::kXChunk * X.stride);
-        hipLaunchKernelGGL(kernel, grid, block, lds, s, W.nlong, W.longs, W.nblk, W.blk, X.list, X.idx, X.stride, cols,
-                           rp, col, v, x, y);
+        hipLaunchKernelGGL(kernel, grid, block, lds, s, W.nlong, nwide, W.longs, W.nblk, W.blk, X.list, X.idx,
+                           X.stride, cols, rp, col, v, x, y);
     };
     if (W.stage.list)
         launch(csr_wave_kernel<V, true, launch::kCsrWaves>, launch::kCsrWaves, W.stage);

@@ -50,8 +50,8 @@ struct CsrWave {
     int nblk = 0;
     const int* longs = nullptr;
     int nlong = 0;
-    // Multi-vector kernel: the first nwide go to a work-group each, the others (of
-    // at most kWideRowNnz entries) to a wave each.
+    // The first nwide go to a work-group each, the others (of at most kWideRowNnz
+    // entries) to a wave each.
     int nwide = 0;
     XStage stage;
 };

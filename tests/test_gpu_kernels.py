@@ -709,8 +709,8 @@ def test_csr_multi_units(ctx, dtype, x_offset):
 @pytest.mark.parametrize("dtype", [cs.DT_F32, cs.DT_F16])
 @pytest.mark.parametrize("medium", [4095, 4096, 4100])
 def test_csr_multi_long_rows(ctx, medium, dtype):
-    """Rows longer than a block, by a wave or a work-group each as their number
-    decides, around the kernels' rounds (513, 576, 577, 1024, 2047..2049 and
+    """Rows longer than a block (single-vector FP32 and multi-vector kernels), by a
+    wave or a work-group each as their number decides, around the kernels' rounds (513, 576, 577, 1024, 2047..2049 and
     longer), and blocks of rows of 0..4 entries, which have a path of their own up
     to four right-hand sides: dyadic inputs, so Y equals the FP64 product, and
     each right-hand side's bits on random inputs do not depend on k."""
@@ -740,6 +740,10 @@ def test_csr_multi_long_rows(ctx, medium, dtype):
         ctx.sync()
         return dY.download().reshape(k, lens.size)
 
+    dx, dy = cs.DeviceVector(ctx, width, Xd[:, 3].copy()), cs.DeviceVector(ctx, lens.size, Y0[3])
+    dA.spmv(dx, dy, 1)
+    ctx.sync()
+    np.testing.assert_array_equal(dy.download(), ref[3].astype(np.float32))
     wide = run(dR, Xr, 16)
     for k in (1, 2, 3, 4, 5, 7, 8, 9, 12, 15, 16):
         np.testing.assert_array_equal(run(dA, Xd, k), ref[:k].astype(np.float32))
