@@ -201,18 +201,7 @@ int make_flat(hipStream_t s, int format, int dim, int width, int slice_h, clspmv
             if (!st) st = fillf(s, m->val, nnz + launch::kWaveNnz, 1.0f);
             std::vector<int> rp(dim + 1);
             for (int r = 0; r <= dim; ++r) rp[r] = r * width;
-            if (!st) st = build_csr_wave(m, rp.data(), dim);
-            // Row blocks for constant row length.
-            std::vector<int> blocks{0};
-            if (width > launch::kAdaptiveNnz) {
-                for (int r = 1; r <= dim; ++r) blocks.push_back(r);
-            } else {
-                const int per = std::max(1, std::min(launch::kAdaptiveRows, launch::kAdaptiveNnz / std::max(width, 1)));
-                for (int r = per; r < dim; r += per) blocks.push_back(r);
-                blocks.push_back(dim);
-            }
-            m->nblocks = (int)blocks.size() - 1;
-            if (!st) st = upload_array(m, blocks.data(), blocks.size(), &m->blocks);
+            if (!st) st = build_csr_tables(m, rp.data(), dim);
             break;
         }
         case CLSPMV_FMT_COO: {

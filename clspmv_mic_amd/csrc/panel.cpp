@@ -365,9 +365,8 @@ void drop_encoding(clspmv_dmat* d, bool panel) {
     release_array(d, &d->lpval);
     release_array(d, &d->carry_row);
     release_array(d, &d->carry_val);
-    release_array(d, &d->blocks);
     release_array(d, &d->wblk);
-    release_array(d, &d->wlong);
+    d->wlong = d->blocks = nullptr;  // behind wblk
     release_array(d, &d->xlist);
     release_array(d, &d->xidx);
     d->plain = false;

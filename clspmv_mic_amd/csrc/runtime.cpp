@@ -148,9 +148,11 @@ constexpr int kEntriesPerGroup = 1536, kShortGroups = 384, kEntriesPerGroupShort
 // f(first entry, count, to, step) for the entries of group g: entry first + i's
 // place goes to idx[to + i * step].
 struct ChunkMap {
-    std::vector<long long> seen;  // per chunk: the last group that touched it, + 1
-    std::vector<int> place;       // and its place in that group's list
-    explicit ChunkMap(int cols) : seen((size_t)cols / launch::kXChunk + 1), place(seen.size()) {}
+    struct Chunk {
+        int seen, place;  // the last group that touched it, + 1; its first column's place in that group's list
+    };
+    std::vector<Chunk> chunks;
+    explicit ChunkMap(int cols) : chunks((size_t)cols / launch::kXChunk + 1) {}
     // idx null: only counts.  Returns the chunks (more than kXChunksMax: idx is
     // not complete), adds the entries.
     template <class Runs>
@@ -161,13 +163,14 @@ struct ChunkMap {
         runs(g, [&](size_t first, size_t count, size_t to, size_t step) {
             total += (long long)count;
             for (size_t e = first; e < first + count && n <= launch::kXChunksMax; ++e, to += step) {
-                const size_t c = (size_t)(col[e] / launch::kXChunk);
-                if (seen[c] != (long long)g + 1) {
-                    seen[c] = (long long)g + 1;
-                    place[c] = n++;
-                    if (list) list->push_back((int)c);
+                const unsigned c = (unsigned)col[e];
+                Chunk& chunk = chunks[c / launch::kXChunk];
+                if (chunk.seen != (int)g + 1) {
+                    chunk.seen = (int)g + 1;
+                    chunk.place = n++ * launch::kXChunk;
+                    if (list) list->push_back((int)(c / launch::kXChunk));
                 }
-                if (idx) idx[to] = (unsigned short)(place[c] * launch::kXChunk + col[e] % launch::kXChunk);
+                if (idx) idx[to] = (unsigned short)(chunk.place + c % launch::kXChunk);
             }
         });
         *entries += total;
@@ -189,7 +192,7 @@ public:
     template <class Runs>
     void start(int cols, size_t groups, const int* col, size_t total, size_t places, Runs runs) {
         if (groups == 0 || total == 0) return;
-        if (total >= (1u << 18)) {
+        if (total >= 2 * kEntriesPerThread) {
             try {
                 main_ = std::thread([=] { build(cols, groups, col, total, places, runs); });
                 return;
@@ -229,7 +232,8 @@ private:
                 if (entries < per_chunk * chunks || entries < per_group * looked) return;
             }
             // The groups in `parts` runs of about as many, a thread each.
-            const size_t parts = std::min<size_t>(total < (1u << 20) ? 1 : 8, groups);
+            const size_t parts = std::min<size_t>(
+                {std::max<size_t>(total / kEntriesPerThread, 1), groups, 8, std::max(std::thread::hardware_concurrency(), 1u)});
             idx_.reset(new unsigned short[places]);  // the threads' pages are theirs to touch first
             const size_t pad = std::min<size_t>(places, launch::kWaveNnz);
             std::fill_n(idx_.get() + places - pad, pad, (unsigned short)0);
@@ -275,6 +279,8 @@ private:
         }
     }
 
+    // A thread's start costs about what it takes to place this many entries.
+    static constexpr size_t kEntriesPerThread = 1 << 16;
     std::thread main_;
     std::vector<int> list_;
     std::unique_ptr<unsigned short[]> idx_;
@@ -284,7 +290,7 @@ private:
 
 }  // namespace
 
-int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks) {
+int build_csr_tables(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks) {
     std::vector<int4> blk;
     std::vector<int> longs;
     for (int r = 0; r < rows;) {
@@ -305,8 +311,18 @@ int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* b
     d->nwwide = (int)std::count_if(longs.begin(), longs.end(),
                                    [&](int r) { return rp[r + 1] - rp[r] > launch::kWideRowNnz; });
     if (d->nwlong - d->nwwide < launch::kWaveRows) d->nwwide = d->nwlong;
-    int st = upload_array(d, blk.data(), blk.size(), &d->wblk);
-    if (!st) st = upload_array(d, longs.data(), longs.size(), &d->wlong);
+    const std::vector<int> rows_of = csr_row_blocks(rp, rows);
+    d->nblocks = (int)rows_of.size() - 1;
+    // One allocation: the blocks, the long rows, the verification kernel's blocks.
+    std::vector<int4> table = blk;
+    table.resize(blk.size() + (longs.size() + rows_of.size() + 3) / 4);
+    int* tail = reinterpret_cast<int*>(table.data() + blk.size());
+    std::copy(rows_of.begin(), rows_of.end(), std::copy(longs.begin(), longs.end(), tail));
+    const int st = upload_array(d, table.data(), table.size(), &d->wblk);
+    if (!st) {
+        d->wlong = reinterpret_cast<int*>(d->wblk + blk.size());
+        d->blocks = d->wlong + longs.size();
+    }
     if (blocks) *blocks = std::move(blk);
     return st;
 }
@@ -727,14 +743,20 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     if (nnz > 0 && !all.within(m->matinfo.width))
         UPLOAD_CHECK(check_cols(m->csr_col_id, nnz, m->matinfo.width, 1, "csr"));
     std::vector<int4> blk;
-    UPLOAD_CHECK(build_csr_wave(d, m->csr_row_ptr, rows, &blk));
+    UPLOAD_CHECK(build_csr_tables(d, m->csr_row_ptr, rows, &blk));
+    // x is staged by the own arrays' kernel only: built here, beside the upload, or
+    // below once a panel encoding that may replace them turned out not to.
     constexpr size_t W = launch::kCsrWaves;
     StageBuild stage;
-    stage.start(m->matinfo.width, (blk.size() + W - 1) / W, m->csr_col_id, nnz, (size_t)nnz + launch::kWaveNnz,
-                [&blk](size_t g, auto&& f) {
-                    for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
-                        f(blk[b].z, blk[b].w, blk[b].z, 1);
-                });
+    auto build_stage = [&] {
+        stage.start(m->matinfo.width, (blk.size() + W - 1) / W, m->csr_col_id, nnz, (size_t)nnz + launch::kWaveNnz,
+                    [&blk](size_t g, auto&& f) {
+                        for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
+                            f(blk[b].z, blk[b].w, blk[b].z, 1);
+                    });
+    };
+    const bool keeps_own = o.panel_width == 0 || o.panel_width == CLSPMV_PANEL_BOTH;
+    if (keeps_own) build_stage();
     UPLOAD_CHECK(upload_array(d, m->csr_row_ptr, (size_t)rows + 1, &d->rp));
     UPLOAD_CHECK(upload_padded(d, m->csr_col_id, nnz, launch::kWaveNnz, &d->col));
     if (o.dtype != CLSPMV_DT_F32) {
@@ -746,10 +768,6 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     } else {
         UPLOAD_CHECK(upload_padded(d, m->csr_data, nnz, launch::kWaveNnz, &d->val));
     }
-    UPLOAD_CHECK(stage.finish(d));
-    std::vector<int> blocks = csr_row_blocks(m->csr_row_ptr, rows);
-    d->nblocks = (int)blocks.size() - 1;
-    UPLOAD_CHECK(upload_array(d, blocks.data(), blocks.size(), &d->blocks));
 
     if (o.panel_width != 0 && nnz > 0) {
         std::vector<int> row_of(nnz);
@@ -757,6 +775,8 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
             std::fill(row_of.begin() + m->csr_row_ptr[r], row_of.begin() + m->csr_row_ptr[r + 1], r);
         UPLOAD_CHECK(add_panel(d, o, row_of.data(), m->csr_col_id, m->csr_data));
     }
+    if (!keeps_own && d->plain) build_stage();
+    UPLOAD_CHECK(stage.finish(d));  // last: what the matrix can do without
     *out = d;
     return CLSPMV_OK;
 }

@@ -27,12 +27,12 @@ struct clspmv_dmat {
     int* rp = nullptr;
     int* col = nullptr;
     float* val = nullptr;
-    int* blocks = nullptr;
+    int* blocks = nullptr;  // in wblk's allocation
     int nblocks = 0;
     int lanes = 1;
     int max_row = 0;
     int4* wblk = nullptr;
-    int* wlong = nullptr;
+    int* wlong = nullptr;  // in wblk's allocation
     int nwblk = 0, nwlong = 0, nwwide = 0;
     // Staged x of CSR's wave kernel, ELL and SELL (launch::XStage; null: absent).
     int* xlist = nullptr;
@@ -135,10 +135,15 @@ int upload_array(clspmv_dmat* m, const T* host, size_t n, T** out) {
 // The same with `pad` zeros after the last element.
 template <class T>
 int upload_padded(clspmv_dmat* m, const T* host, size_t n, size_t pad, T** out) {
+    if (n < (1 << 16)) {  // one copy
+        std::vector<T> all(n + pad, T(0));
+        std::copy_n(host, n, all.begin());
+        return upload_array(m, all.data(), all.size(), out);
+    }
     const int st = upload_array<T>(m, nullptr, n + pad, out);
     if (st) return st;
     const std::vector<T> zero(pad, T(0));
-    hipError_t e = n ? hipMemcpy(*out, host, sizeof(T) * n, hipMemcpyHostToDevice) : hipSuccess;
+    hipError_t e = hipMemcpy(*out, host, sizeof(T) * n, hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemcpy(*out + n, zero.data(), sizeof(T) * pad, hipMemcpyHostToDevice);
     if (e != hipSuccess) return fail(CLSPMV_ERR_HIP, "hipMemcpy failed: %s", hipGetErrorString(e));
     return CLSPMV_OK;
@@ -158,9 +163,10 @@ void release_array(clspmv_dmat* m, T** p) {
     *p = nullptr;
 }
 
-// Builds and uploads the wave kernel's tables of a CSR matrix from its host
-// row pointers; the blocks also to `blocks`.
-int build_csr_wave(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks = nullptr);
+// Builds and uploads the row blocks and long rows of a CSR matrix (wave and
+// verification kernels) from its host row pointers; the wave kernel's blocks
+// also to `blocks`.
+int build_csr_tables(clspmv_dmat* d, const int* rp, int rows, std::vector<int4>* blocks = nullptr);
 
 // x-panel encoding (k_panel.hip) of row-sorted entries, built on the host
 // and uploaded into `d`.  pw: panel width (multiple of 8, at most

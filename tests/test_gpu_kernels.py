@@ -546,6 +546,48 @@ def test_staged_x(ctx, oracle, chunks, x_offset):
     assert (info.device_bytes >= 10 * info.stored) == (chunks <= 512)
 
 
+@pytest.mark.parametrize("chunks", [127, 128, 129, 256, 257, 384, 511, 512, 513])
+@pytest.mark.parametrize("fmt", ["csr", "csr_bf16", "ell", "sell"])
+def test_staged_x_rounds(ctx, oracle, fmt, chunks):
+    """Staged x with exactly `chunks` runs of 16 columns in every work-group, in
+    one to four rounds of its loads, up to the most that are staged (and one past
+    it: none are), the last run cut off by the matrix and a last partial
+    work-group; dyadic inputs, exact sums."""
+    csr = fmt.startswith("csr")
+    per_row = 32 if csr else 8  # 4,096 entries a work-group: 8 blocks of 16 rows, or 512 rows
+    groups, rows = 390, 390 * (4096 // per_row) + 37
+    cols = chunks * 16 - 5
+    r = np.repeat(np.arange(rows), per_row)
+    i = np.arange(r.size)
+    chunk = (i * 11 + i // 4096 * 5) % chunks  # 11 shares no factor with the counts: all of them, distinct in a row
+    c = np.minimum(chunk * 16 + (i * 7) % 16, cols - 1)
+    key = np.unique(r.astype(np.int64) * cols + c)
+    assert key.size == r.size and all(np.unique(chunk[g * 4096:(g + 1) * 4096]).size == chunks for g in (0, 7, groups - 1))
+    v = (np.random.default_rng(chunks).integers(1, 65, r.size) / 64.0).astype(np.float32)
+    A = cs.Coo(r.astype(np.int32), (key % cols).astype(np.int32), v, rows, cols)
+    dtype = cs.DT_BF16 if fmt == "csr_bf16" else cs.DT_F32
+    owned = cs.coo2csr(A.copy()) if csr else cs.coo2ell(A) if fmt == "ell" else cs.coo2sell(A, 48)
+    kw = dict(panel=0, dtype=dtype) if csr else {}
+    for x_offset in (0, 1):
+        _run(ctx, oracle, A, owned, 1 if csr else 0, x_offset=x_offset, **kw)
+    info = cs.DeviceMatrix(ctx, owned, **kw).info
+    own = (6 if fmt == "csr_bf16" else 8) * info.stored
+    assert (info.device_bytes >= own + 2 * info.stored) == (chunks <= 512)
+
+
+def test_staged_x_with_panels(ctx, oracle):
+    """A CSR upload that keeps its own arrays stages x for them (2 bytes an entry
+    beside the 8 of columns and values), with panels beside them too."""
+    A = matrices.banded(60_000, list(range(-13, 14)), seed=3, dyadic=True)
+    csr = cs.coo2csr(A.copy())
+    own, panels, both = (cs.DeviceMatrix(ctx, csr, panel=p).info for p in (0, cs.PANEL_AUTO, cs.PANEL_BOTH))
+    assert own.plain and both.plain and both.panel_active and not panels.plain
+    assert own.device_bytes >= 10 * A.nnz
+    assert both.device_bytes - panels.device_bytes >= 10 * A.nnz
+    for p in (0, cs.PANEL_AUTO, cs.PANEL_BOTH):
+        _run(ctx, oracle, A, csr, 1, panel=p)
+
+
 @pytest.mark.parametrize("width", [1, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 24, 27])
 @pytest.mark.parametrize("rows", [100, (1 << 17) + 3])
 def test_ell_slot_groups(ctx, oracle, width, rows):
