@@ -4,6 +4,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "index_math.hpp"
 #include "kernels.hpp"
 
 namespace clspmv {

@@ -17,5 +17,20 @@ constexpr unsigned spmm_piece_offset(unsigned piece, unsigned kc) {
 }
 constexpr bool spmm_piece_end(unsigned piece, unsigned kc) { return 2 * piece + 1 == kc; }
 
+// The row that thread `row` of a grid works on: threads past the last row
+// shadow it.  (row is unsigned: with rows near 2^31 the last work-group's go past
+// the signed range.)
+constexpr int shadow_row(unsigned row, int rows) { return row < (unsigned)rows ? (int)row : rows - 1; }
+
+// Floats from one (slot, row, column quad) plane of a slot-major block matrix of
+// `aligned` block rows to the next: a float4 per block row.
+constexpr long long block_plane(int aligned) { return 4LL * aligned; }
+
+// f(first), f(first + step), ... below n.
+template <class F>
+constexpr void strided(long long first, long long step, long long n, F f) {
+    for (long long i = first; i < n; i += step) f(i);
+}
+
 }  // namespace launch
 }  // namespace clspmv

@@ -98,7 +98,7 @@ constexpr int kShare = WALK != kSplit ? 1 : BH < kHWaves ? BH : kHWaves;  // wav
 
 template <int BH, int BW4, Layout LAY, bool F4ACC, Walk WALK>
 __global__ __launch_bounds__(kBlock) void block_rows_kernel(
-    int brows, int rows, int cols, int cs, int f4, int nslots, const int* __restrict__ sptr,
+    int brows, int rows, int cols, int cs, long long f4, int nslots, const int* __restrict__ sptr,
     const int* __restrict__ col4, const float* __restrict__ data, const float* __restrict__ x,
     bool x_aligned, float* __restrict__ y) {
     constexpr int HW = kShare<BH, WALK>;
@@ -106,16 +106,16 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
     constexpr int U = WALK != kSplit ? 1 : BW4 * HN == 1 ? 4 : BW4 * HN == 2 ? 3 : 2;  // slots at a time
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
     const int h0 = wave % HW * HN;
-    const int row = (xcd_tile(blockIdx.x, gridDim.x) * (kHWaves / HW) + wave / HW) * kWave + lane;
-    const int r = min(row, brows - 1);  // lanes past the end shadow the last block row
+    const unsigned row = ((unsigned)xcd_tile(blockIdx.x, gridDim.x) * (kHWaves / HW) + wave / HW) * kWave + lane;
+    const int r = launch::shadow_row(row, brows);
     int w = nslots;
     const int* cp = col4 + r;
     const float* dp = data + (size_t)r * 4;
-    int P = f4;  // floats per (slot, w4, h) plane
+    long long P = f4;  // floats per (slot, w4, h) plane
     if constexpr (LAY == kSbell) {  // cs: the slice height
         const int sl = r / cs, p0 = sptr[sl];
         w = (sptr[sl + 1] - p0) / cs;
-        P = cs * 4;
+        P = launch::block_plane(cs);
         // A lane whose slice is empty reads entry 0 beside its neighbours.
         const int at = w > 0 ? p0 + (r - sl * cs) : 0;
         cp = col4 + at;
@@ -208,14 +208,14 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
     }
 #pragma unroll
     for (int h = 0; h < HN; ++h) {
-        const int at = r * BH + h0 + h;
+        const unsigned at = (unsigned)r * BH + h0 + h;
         const float v = F4ACC ? (acc4[h].x + acc4[h].y) + (acc4[h].z + acc4[h].w) : acc[h];
-        if (row < brows && at < rows) y[at] += v;
+        if (row < (unsigned)brows && at < (unsigned)rows) y[at] += v;
     }
 }
 
 template <int BH, int BW4, Layout LAY, bool F4ACC>
-hipError_t block_rows(hipStream_t s, int brows, int rows, int cols, int cs, int f4, int nslots, const int* sptr,
+hipError_t block_rows(hipStream_t s, int brows, int rows, int cols, int cs, long long f4, int nslots, const int* sptr,
                       const int* col4, const float* data, const float* x, bool xa, float* y) {
     auto launch = [&](auto kernel, int share) {
         const int per = kBlock / share;  // block rows per work-group
@@ -280,7 +280,8 @@ hipError_t bcsr_slots(hipStream_t s, int brows, int rows, int cols, int bh, int 
                       const int* col4, const float* data, const float* x, bool x_aligned, float* y) {
     if (brows <= 0 || nslots <= 0) return hipSuccess;
     if (hal < brows || nslots > kBcsrSlotsMax) return hipErrorInvalidValue;
-    SHAPE_DISPATCH(block_rows, LAYOUT(kBcsrSlots, false), s, brows, rows, cols, hal, 4 * hal, nslots, nullptr, col4,
+    SHAPE_DISPATCH(block_rows, LAYOUT(kBcsrSlots, false), s, brows, rows, cols, hal, block_plane(hal), nslots, nullptr,
+                   col4,
                    data, x, x_aligned, y)
 }
 

@@ -112,10 +112,11 @@ __global__ __launch_bounds__(kBlock) void dia_quad_kernel(
     const typename V::T* __restrict__ data, const float* __restrict__ x, float* __restrict__ y) {
     constexpr int R = 4, NX = R + W - 1;
     typedef typename V::T T;
-    const int r0 = (xcd_tile(blockIdx.x, gridDim.x) * kBlock + (int)threadIdx.x) * R;
-    const int w0 = __builtin_amdgcn_readfirstlane(r0);
-    if (w0 >= rows) return;  // the whole wave
-    const int dl = min(r0, len - R) - w0, xl = r0 - w0;
+    const unsigned r0u = ((unsigned)xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x) * R;
+    const unsigned w0u = __builtin_amdgcn_readfirstlane(r0u);
+    if (w0u >= (unsigned)rows) return;  // the whole wave
+    const int w0 = (int)w0u, xl = (int)(r0u - w0u), r0 = w0 + min(xl, rows - w0);
+    const int dl = min(xl, len - R - w0);
     float acc[R] = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int s = 0; s < nseg; s += S) {
         float xv[S][NX];
@@ -157,7 +158,8 @@ __global__ __launch_bounds__(kBlock) void dia_quad_kernel(
                     for (int r = 0; r < R; ++r) acc[r] = fmaf(V::cvt(d[i][n][r]), xv[i][n + r], acc[r]);
         }
     }
-    if (r0 + R <= rows) {
+    const int left = rows - w0 - xl;  // rows from the lane's first on
+    if (left >= R) {
         typedef UVec<float, R>::type YU;
         f32x4 v = *reinterpret_cast<const YU*>(y + r0);
 #pragma unroll
@@ -166,7 +168,7 @@ __global__ __launch_bounds__(kBlock) void dia_quad_kernel(
     } else {
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            if (r0 + r < rows) y[r0 + r] += acc[r];
+            if (r < left) y[r0 + r] += acc[r];
     }
 }
 

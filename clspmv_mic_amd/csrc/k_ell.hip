@@ -41,8 +41,8 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
     float* __restrict__ y) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
     const int wg = xcd_tile(blockIdx.x, gridDim.x);
-    const int row = wg * kRows + (int)threadIdx.x;
-    const int r = min(row, rows - 1);  // lanes past the end shadow the last row
+    const unsigned row = (unsigned)wg * kRows + threadIdx.x;
+    const int r = launch::shadow_row(row, rows);
     int w = w0;
     constexpr int kPer = WIN ? 2 : 1;  // slots per column word
     const int* cp = WIN ? reinterpret_cast<const int*>(idx) : col;
@@ -123,16 +123,16 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
     if (s + 2 * kSlots < wm) load_part(s + 2 * kSlots, c[0], v[0]);
     if (s + kSlots < wm) add(s + kSlots, c[1], v[1]);
     if (s + 2 * kSlots < wm) add(s + 2 * kSlots, c[0], v[0]);
-    if (row < rows) y[r] += (a[0] + a[1]) + (a[2] + a[3]);
+    if (row < (unsigned)rows) y[r] += (a[0] + a[1]) + (a[2] + a[3]);
 }
 
 // SELL with short rows: a row per lane, two slots at a time, nothing clamped.
 __global__ __launch_bounds__(kBlock) void sell_short_kernel(
     int rows, int h, const int* __restrict__ ptr, const int* __restrict__ col,
     const float* __restrict__ val, const float* __restrict__ x, float* __restrict__ y) {
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (r >= rows) return;
-    const int sl = r / h, i = r - sl * h;
+    const unsigned r = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    if (r >= (unsigned)rows) return;
+    const int sl = (int)r / h, i = (int)r - sl * h;
     const int p0 = ptr[sl];
     const int w = (ptr[sl + 1] - p0) / h;
     const int* c = col + p0 + i;
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(kBlock) void ell4_kernel(
 template <bool SELL, int kSlots, int kRows>
 hipError_t ell_rows_plain(hipStream_t s, int rows, int h, int w, const int* ptr, const int* col, const float* val,
                           int cols, const float* x, float* y) {
-    hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots, kRows>), dim3((rows + kRows - 1) / kRows), dim3(kRows), 0,
+    hipLaunchKernelGGL((ell_row_kernel<SELL, false, kSlots, kRows>), dim3(((unsigned)rows + kRows - 1) / kRows), dim3(kRows), 0,
                        s, rows, h, w, ptr, nullptr, nullptr, 0, cols, col, val, x, y);
     return hipGetLastError();
 }
@@ -183,7 +183,7 @@ template <bool SELL, int kSlots>
 hipError_t ell_rows_staged(hipStream_t s, int rows, int h, int w, const int* ptr, launch::XStage W, const int* col,
                            const float* val, int cols, const float* x, float* y) {
     constexpr int R = launch::kEllRows;
-    hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots, R>), dim3((rows + R - 1) / R), dim3(R),
+    hipLaunchKernelGGL((ell_row_kernel<SELL, true, kSlots, R>), dim3(((unsigned)rows + R - 1) / R), dim3(R),
                        sizeof(float) * launch::kXChunk * W.stride, s, rows, h, w, ptr, W.list, W.idx, W.stride, cols,
                        col, val, x, y);
     return hipGetLastError();
@@ -193,7 +193,7 @@ hipError_t ell_rows_staged(hipStream_t s, int rows, int h, int w, const int* ptr
 // mesh of 20,000 rows (40 work-groups) with 12 / 25 / 40 neighbours 3.1 / 4.0 /
 // 4.5 us staged, 2.8 / 3.6 / 4.4 gathered (ELL), 40,000 rows (79) of 12 3.6 / 3.3
 // (SELL); 50,000 rows (98) of 25 / 40 4.1 / 4.7 staged, 4.0 / 5.9 gathered.
-constexpr int kStagedGroups = 96;
+constexpr unsigned kStagedGroups = 96;
 
 // Slots in flight, staged: eight while there are fewer than two waves per SIMD
 // (131,072 rows), where the chain of slots sets the time (mesh of 100,000 rows
@@ -212,7 +212,7 @@ template <bool SELL>
 hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, long long stored, launch::XStage W,
                     const int* col, const float* val, int cols, const float* x, float* y) {
     const bool few = rows < (1 << 17);
-    if (W.list && (rows + launch::kEllRows - 1) / launch::kEllRows >= kStagedGroups)
+    if (W.list && ((unsigned)rows + launch::kEllRows - 1) / launch::kEllRows >= kStagedGroups)
         return few ? ell_rows_staged<SELL, 8>(s, rows, h, w, ptr, W, col, val, cols, x, y)
                    : ell_rows_staged<SELL, 4>(s, rows, h, w, ptr, W, col, val, cols, x, y);
     const long long mean = stored / rows;
@@ -246,7 +246,7 @@ hipError_t sell(hipStream_t s, int rows, int slice_height, const int* ptr, long 
     // slots 5.6 / 4.8 / 7.4 us by the short kernel, 5.9 / 5.6 / 7.8 by the other; of
     // 5 11.1 / 10.0.
     if (stored * 2 <= rows * 7LL) {
-        hipLaunchKernelGGL(sell_short_kernel, dim3((rows + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rows,
+        hipLaunchKernelGGL(sell_short_kernel, dim3(((unsigned)rows + kBlock - 1) / kBlock), dim3(kBlock), 0, s, rows,
                            slice_height, ptr, col, val, x, y);
         return hipGetLastError();
     }

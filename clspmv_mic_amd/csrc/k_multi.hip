@@ -68,8 +68,10 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
     __shared__ __attribute__((aligned(16))) float sx[kWaves][(NX + R - 1) / R * CS];
     __shared__ __attribute__((aligned(16))) float sd[kWaves][W * NR];
     const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-    const int w0 = __builtin_amdgcn_readfirstlane((xcd_tile(blockIdx.x, gridDim.x) * kWaves + wave) * NR);
-    if (w0 >= rows) return;  // the whole wave
+    const unsigned w0u =
+        __builtin_amdgcn_readfirstlane(((unsigned)xcd_tile(blockIdx.x, gridDim.x) * kWaves + wave) * NR);
+    if (w0u >= (unsigned)rows) return;  // the whole wave
+    const int w0 = (int)w0u, left = rows - w0;  // rows from the wave's first on
     float* xl = sx[wave];
     float* dl = sd[wave];
     const int g = lane / L, p = lane % L;
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
     for (int r = 0; r < R; ++r)
 #pragma unroll
         for (int q = 0; q < Q; ++q) acc[r][q] = 0.0f;
-    const bool tail = w0 + NR > len;  // rows past the stored length
+    const bool tail = len - w0 < NR;  // rows past the stored length
     typename XV::type xr[NLD];
     typename DV::type dr[W];
     const unsigned xo = (unsigned)(g * k + qs), xlast = (unsigned)((NX - 1) * k + qs);
@@ -189,13 +191,12 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
         }
         wave_lds_order();
     }
-    const int r0 = w0 + g * R;
     if (q0 >= k) return;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         if (qs + q < q0) continue;  // the lane before has this column
-        float* yp = Y + (size_t)(qs + q) * ldy + r0;
-        if (r0 + R <= rows) {
+        float* yp = Y + (size_t)(qs + q) * ldy + w0 + g * R;
+        if (g * R + R <= left) {
             typedef typename UVec<float, R>::type YU;
             typename RV::type v{};
             if (accumulate) v = *reinterpret_cast<const YU*>(yp);
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(kBlock) void dia_multi_kernel(
         } else {
 #pragma unroll
             for (int r = 0; r < R; ++r)
-                if (r0 + r < rows) yp[r] = (accumulate ? yp[r] : 0.0f) + acc[r][q];
+                if (g * R + r < left) yp[r] = (accumulate ? yp[r] : 0.0f) + acc[r][q];
         }
     }
 }
@@ -222,8 +223,9 @@ __global__ __launch_bounds__(kBlock) void dia_multi_direct_kernel(
     constexpr int C = Q == 4 ? 8 : 16;
     typedef VecOf<float, Q> XV;
     const int t = threadIdx.x;
-    const int r = xcd_tile(blockIdx.x, gridDim.x) * (kBlock / L) + t / L;
-    if (r >= rows) return;
+    const unsigned ru = (unsigned)xcd_tile(blockIdx.x, gridDim.x) * (kBlock / L) + t / L;
+    if (ru >= (unsigned)rows) return;
+    const int r = (int)ru;
     const int q0 = t % L * Q, qs = min(q0, k - Q);
     float acc[Q];
 #pragma unroll
@@ -236,8 +238,8 @@ __global__ __launch_bounds__(kBlock) void dia_multi_direct_kernel(
         for (int u = 0; u < C; ++u) {
             const int j = min(j0 + u, ndiag - 1);
             d[u] = V::ld(data + (size_t)j * len + r);
-            const int c = r + off[j];
-            in[u] = j0 + u < ndiag && (unsigned)c < (unsigned)cols;
+            const unsigned c = ru + (unsigned)off[j];
+            in[u] = j0 + u < ndiag && c < (unsigned)cols;
             xv[u] = *reinterpret_cast<const typename UVec<float, Q>::type*>(X + (size_t)(in[u] ? c : 0) * k + qs);
         }
 #pragma unroll

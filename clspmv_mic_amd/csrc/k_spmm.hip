@@ -24,7 +24,6 @@
 #include <type_traits>
 
 #include "device_common.hpp"
-#include "index_math.hpp"
 #include "kernels.hpp"
 
 namespace clspmv {

@@ -33,6 +33,7 @@
 #include <unordered_set>
 
 #include "clspmv_serve.h"
+#include "index_math.hpp"
 #include "kernels.hpp"
 #include "rng.hpp"
 #include "runtime.hpp"
@@ -125,8 +126,8 @@ __global__ __launch_bounds__(kStageRows) void stage_rows_kernel(unsigned long lo
 
 // Columns of y (leading dimension ldy) to the caller's (rows floats each).
 __global__ void copy_y_kernel(int rows, int ldy, const float* __restrict__ y, float* __restrict__ out) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < rows; i += gridDim.x * blockDim.x)
-        out[(size_t)blockIdx.y * rows + i] = y[(size_t)blockIdx.y * ldy + i];
+    launch::strided((long long)blockIdx.x * blockDim.x + threadIdx.x, (long long)gridDim.x * blockDim.x, rows,
+                    [&](long long i) { out[(size_t)blockIdx.y * rows + i] = y[(size_t)blockIdx.y * ldy + i]; });
 }
 
 __global__ void zero_kernel(long long n, float* y) {
@@ -367,7 +368,7 @@ int stage_x(hipStream_t s, const SMatrix& M, const clspmv_request& r, int K, int
         for (int j = 0; j < r.k;) {  // the request's columns of each chunk
             const int c = (g0 + j) / kMultiCols, off = (g0 + j) % kMultiCols;
             const int n = std::min(r.k - j, kMultiCols - off);
-            hipLaunchKernelGGL(stage_rows_kernel, dim3((M.cols + kStageRows - 1) / kStageRows), dim3(kStageRows), 0, s,
+            hipLaunchKernelGGL(stage_rows_kernel, dim3(((unsigned)M.cols + kStageRows - 1) / kStageRows), dim3(kStageRows), 0, s,
                                r.seed, j, src ? src + (size_t)j * src_ld : nullptr, src_ld, n, M.cols,
                                std::min(kMultiCols, K - c * kMultiCols), off,
                                static_cast<float*>(M.X) + (size_t)c * kMultiCols * M.ldx);
@@ -387,7 +388,7 @@ int copy_y(hipStream_t s, const SMatrix& M, const clspmv_request& r, int g0, flo
     const float* y = M.Y + (size_t)g0 * M.ldy;
     const size_t row_bytes = sizeof(float) * M.rows;
     if (r.device_y && M.rows > 0 && r.k <= 65535) {  // the grid's y limit
-        hipLaunchKernelGGL(copy_y_kernel, dim3(std::min((M.rows + 255) / 256, 2048), r.k), dim3(256), 0, s, M.rows,
+        hipLaunchKernelGGL(copy_y_kernel, dim3(std::min(((unsigned)M.rows + 255) / 256, 2048u), r.k), dim3(256), 0, s, M.rows,
                            M.ldy, y, r.device_y);
         CLSPMV_HIP(hipGetLastError());
     } else if (r.device_y) {
