@@ -122,8 +122,12 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
         dp = data + (w > 0 ? (size_t)p0 * BH * BW4 * 4 + (size_t)(r - sl * cs) * 4 : 0);
     }
     int wm = w;  // the most slots of the wave's block rows
-    if constexpr (LAY == kSbell)
-        for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    if constexpr (LAY == kSbell) {
+        if (cs % 32 == 0)  // a slice per half of the wave, at most
+            wm = max(__builtin_amdgcn_readlane(w, 0), __builtin_amdgcn_readlane(w, 32));
+        else
+            for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+    }
     wm = __builtin_amdgcn_readfirstlane(wm);
     dp += (size_t)h0 * P;
     float acc[HN];
