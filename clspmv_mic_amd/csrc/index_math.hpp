@@ -1,5 +1,6 @@
-// Index and address arithmetic of kernels, as constexpr functions that the
-// kernels and the host's tests share (no HIP headers).
+// Index and address arithmetic of kernels and the rules on a caller's pointers,
+// as constexpr functions that the library and the host's tests share (no HIP
+// headers).
 #pragma once
 
 namespace clspmv {
@@ -30,6 +31,14 @@ constexpr long long block_plane(int aligned) { return 4LL * aligned; }
 template <class F>
 constexpr void strided(long long first, long long step, long long n, F f) {
     for (long long i = first; i < n; i += step) f(i);
+}
+
+// Whether a server's kernels write a request's device_y themselves: device memory
+// of the server's own GPU.  Everything else that the runtime can copy to (another
+// device's memory, with or without peer access, host memory) is left to its copy.
+// known: the runtime knows the pointer.
+constexpr bool kernel_writes_y(bool known, bool device_memory, int memory_device, int server_device) {
+    return known && device_memory && memory_device == server_device;
 }
 
 }  // namespace launch

@@ -218,6 +218,7 @@ struct SRequest {
     int state = 0;  // 0 waiting, 1 running, 2 done, < 0 failed (status)
     int col = 0;    // first column in its batch
     size_t pin = kNone;  // pinned staging of host_y
+    bool y_here = false;  // device_y is written by kernels (kernel_writes_y)
 };
 
 struct SBatch {
@@ -383,13 +384,22 @@ int stage_x(hipStream_t s, const SMatrix& M, const clspmv_request& r, int K, int
     return CLSPMV_OK;
 }
 
+// launch::kernel_writes_y for a request's device_y (null: false).
+bool y_here(const float* device_y, int device) {
+    if (!device_y) return false;
+    hipPointerAttribute_t a{};
+    const bool known = hipPointerGetAttributes(&a, device_y) == hipSuccess;
+    if (!known) (void)hipGetLastError();
+    return launch::kernel_writes_y(known, a.type == hipMemoryTypeDevice, a.device, device);
+}
+
 // y of one request (columns [g0, g0 + k) of Y) to the caller.
-int copy_y(hipStream_t s, const SMatrix& M, const clspmv_request& r, int g0, float* pinned) {
+int copy_y(hipStream_t s, const SMatrix& M, const clspmv_request& r, bool y_here, int g0, float* pinned) {
     const float* y = M.Y + (size_t)g0 * M.ldy;
     const size_t row_bytes = sizeof(float) * M.rows;
-    if (r.device_y && M.rows > 0 && r.k <= 65535) {  // the grid's y limit
-        hipLaunchKernelGGL(copy_y_kernel, dim3(std::min(((unsigned)M.rows + 255) / 256, 2048u), r.k), dim3(256), 0, s, M.rows,
-                           M.ldy, y, r.device_y);
+    if (r.device_y && y_here && M.rows > 0 && r.k <= 65535) {  // the grid's y limit
+        hipLaunchKernelGGL(copy_y_kernel, dim3(std::min(((unsigned)M.rows + 255) / 256, 2048u), r.k), dim3(256), 0, s,
+                           M.rows, M.ldy, y, r.device_y);
         CLSPMV_HIP(hipGetLastError());
     } else if (r.device_y) {
         CLSPMV_HIP(hipMemcpy2DAsync(r.device_y, row_bytes, y, sizeof(float) * M.ldy, row_bytes, r.k,
@@ -436,8 +446,9 @@ int launch_batch(clspmv_server* S, SMatrix& M, SBatch& b) {
     }
     // One request with its y on the device alone: the multi-vector pass writes
     // there, without the copy.
-    const clspmv_request& r0 = S->reqs[b.tickets[0]].r;
-    const bool direct = M.path == kMulti && b.tickets.size() == 1 && r0.device_y && !r0.host_y &&
+    const SRequest& q0 = S->reqs[b.tickets[0]];
+    const clspmv_request& r0 = q0.r;
+    const bool direct = M.path == kMulti && b.tickets.size() == 1 && q0.y_here && !r0.host_y &&
                         pass_launches(M, K) <= kPlainLaunches;
     if (direct) {
         int st = enqueue_pass(s, M, K, r0.device_y, M.rows);
@@ -454,7 +465,7 @@ int launch_batch(clspmv_server* S, SMatrix& M, SBatch& b) {
     for (long long t : b.tickets) {
         if (direct) break;
         SRequest& q = S->reqs[t];
-        int st = copy_y(s, M, q.r, q.col, q.pin != kNone ? S->pinned + q.pin / sizeof(float) : nullptr);
+        int st = copy_y(s, M, q.r, q.y_here, q.col, q.pin != kNone ? S->pinned + q.pin / sizeof(float) : nullptr);
         if (st) return st;
     }
     if (S->free_events.empty()) {
@@ -675,7 +686,7 @@ int run_plain(clspmv_server* S, SMatrix& M, const clspmv_request& r, float* pinn
             st = dmat_launch(s, P.A, P.method, static_cast<const float*>(P.X) + (size_t)j * P.ldx,
                              P.Y + (size_t)j * P.ldy);
     }
-    if (!st) st = copy_y(s, P, r, 0, pinned);
+    if (!st) st = copy_y(s, P, r, y_here(r.device_y, S->cfg.device_ordinal), 0, pinned);
     if (!st) CLSPMV_HIP(hipStreamSynchronize(s));
     if (!st && r.host_y) std::memcpy(r.host_y, pinned, sizeof(float) * (size_t)P.rows * r.k);
     if (st) (void)hipStreamSynchronize(s);
@@ -803,6 +814,7 @@ double clspmv_server_clock(clspmv_server* S) { return S ? S->now() : 0.0; }
 
 int clspmv_server_submit(clspmv_server* S, const clspmv_request* r, long long* ticket) {
     if (!S || !r || !ticket) return fail(CLSPMV_ERR_INVALID, "null argument");
+    const bool here = y_here(r->device_y, S->cfg.device_ordinal);
     std::lock_guard<std::mutex> lk(S->mu);
     if (S->stop) return fail(CLSPMV_ERR_INVALID, "server is shutting down");
     if (r->matrix < 0 || r->matrix >= (int)S->mats.size())
@@ -814,6 +826,7 @@ int clspmv_server_submit(clspmv_server* S, const clspmv_request* r, long long* t
                     r->k, S->pin_arena.size);
     SRequest q;
     q.r = *r;
+    q.y_here = here;
     q.arrival = r->arrival > 0 ? r->arrival : S->now();
     const long long t = S->next_ticket++;
     S->reqs.emplace(t, q);

@@ -58,7 +58,8 @@ typedef struct {
     int    streams;       /* HIP streams passes are spread over (>= 1)        */
     int    max_batch;     /* most requests coalesced into one pass (>= 1)     */
     size_t hbm_budget;    /* device pool for the matrices' working buffers    */
-    int    use_graphs;    /* 1: replay captured graphs; 0: plain launches     */
+    int    use_graphs;    /* 1: replay captured graphs for passes of more
+                             than four kernel launches; 0: plain launches     */
     size_t host_staging;  /* pinned bytes for copies to host_y; 0: 256 MiB    */
 } clspmv_server_config;
 
@@ -93,7 +94,9 @@ typedef struct {
     const float* x;           /* NULL, or cols * k floats, column-major       */
     int    x_on_device;       /* x is a device pointer (server's GPU)         */
     float* host_y;            /* NULL, or rows * k floats (column-major)      */
-    float* device_y;          /* NULL, or rows * k floats on the device       */
+    float* device_y;          /* NULL, or rows * k floats on a device: written
+                                 by the pass or a copy kernel where it is the
+                                 server's GPU, else copied by the runtime     */
     double arrival;           /* server clock; <= 0 means "now"               */
 } clspmv_request;
 

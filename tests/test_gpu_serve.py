@@ -9,6 +9,9 @@ evicts and still serves everything identically; one device matrix
 registered twice (in one server and in two) is never run by two passes at
 once."""
 
+import ctypes
+import types
+
 import numpy as np
 import pytest
 
@@ -221,4 +224,34 @@ def test_device_y_direct_and_batched(ctx, oracle, fmt):
             y64, bound = oracle.spmv_f64(A.row, A.col, A.val, x[j * A.width:(j + 1) * A.width].copy(), A.height)
             err, worst = oracle.scaled_error(host[j * A.height:(j + 1) * A.height].copy(), y64, bound)
             assert err <= TOL, f"k {k} rhs {j}: {err:.3e} at row {worst}"
+    s.close()
+
+
+@pytest.mark.parametrize("fmt", ["dia", "csr", "sell"])
+def test_device_y_in_pinned_host_memory(ctx, fmt):
+    """device_y in pinned host memory, which the runtime's copy reaches (no kernel
+    of the server writes it): the same bits as in device memory, alone and in a
+    batch."""
+    def pinned(n):
+        p = ctypes.c_void_p()
+        assert cs.lib.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(4 * n), ctypes.c_uint(0)) == 0
+        a = np.ctypeslib.as_array(ctypes.cast(p, ctypes.POINTER(ctypes.c_float)), (n,))
+        a[:] = np.nan
+        return a, types.SimpleNamespace(p=p)
+
+    A = matrices.laplacian_2d(150)
+    dm = (cs.DeviceMatrix(ctx, cs.coo2dia(A.copy())) if fmt == "dia" else
+          cs.DeviceMatrix(ctx, cs.coo2csr(A.copy()), panel=0) if fmt == "csr" else cs.DeviceMatrix(ctx, cs.coo2sell(A)))
+    s = cs.Server(streams=2, max_batch=4, hbm_budget=64 << 20)
+    i = s.add(dm, kmax=20)
+    for k in (1, 5, 17):
+        dy = [cs.DeviceVector(ctx, A.height * k, np.full(A.height * k, np.nan, np.float32)) for _ in range(3)]
+        py, ptr = zip(*[pinned(A.height * k) for _ in range(3)])
+        s.wait(s.submit(i, k, 70, device_y=ptr[0]))
+        s.wait(s.submit(i, k, 70, device_y=dy[0]))
+        for t in [s.submit(i, k, 70 + j, device_y=v) for j in (1, 2) for v in (ptr[j], dy[j])]:
+            s.wait(t)
+        for j in range(3):
+            np.testing.assert_array_equal(py[j], dy[j].download())
+            cs.lib.hipHostFree(ptr[j].p)
     s.close()

@@ -16,6 +16,9 @@ extern "C" {
 unsigned piece_offset(unsigned piece, unsigned kc) { return spmm_piece_offset(piece, kc); }
 int piece_end(unsigned piece, unsigned kc) { return spmm_piece_end(piece, kc); }
 int shadow(unsigned row, int rows) { return shadow_row(row, rows); }
+int writes_y(int known, int device_memory, int at, int server) {
+    return kernel_writes_y(known, device_memory, at, server);
+}
 long long plane(int aligned) { return block_plane(aligned); }
 // Visits of strided(); -1: one of them outside [0, n).
 long long visits(long long first, long long step, long long n) {
@@ -86,3 +89,13 @@ def test_strided_ends_at_n(lib, n):
     for first in (0, 1, step - 1):
         if first >= 0 and step:
             assert lib.visits(first, step, n) == max(0, (n - first + step - 1) // step)
+
+
+@pytest.mark.parametrize("known, device_memory, at, server, kernel", [
+    (1, 1, 0, 0, 1), (1, 1, 3, 3, 1),  # the server's GPU
+    (1, 1, 1, 0, 0), (1, 1, 0, 1, 0),  # another device: there may be no peer access
+    (1, 0, 0, 0, 0),                   # host memory
+    (0, 0, 0, 0, 0), (0, 1, 0, 0, 0),  # a pointer that the runtime does not know
+])
+def test_who_writes_device_y(lib, known, device_memory, at, server, kernel):
+    assert lib.writes_y(known, device_memory, at, server) == kernel
