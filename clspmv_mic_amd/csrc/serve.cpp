@@ -393,21 +393,35 @@ bool y_here(const float* device_y, int device) {
     return launch::kernel_writes_y(known, a.type == hipMemoryTypeDevice, a.device, device);
 }
 
+// Up to this many bytes of y go to the pinned staging by the copy kernel: small
+// copies by the DMA engines waited 130 us or 250 us at times, behind plain
+// launches above all (one request with x and y on the host, one right-hand side,
+// power-law 50,000 rows: 136 us by graph and copy, 150 to 250 by launches and
+// copy, 70 by launches and kernel; larger ones overlap other passes).
+constexpr size_t kKernelToHost = 1 << 20;
+
 // y of one request (columns [g0, g0 + k) of Y) to the caller.
 int copy_y(hipStream_t s, const SMatrix& M, const clspmv_request& r, bool y_here, int g0, float* pinned) {
     const float* y = M.Y + (size_t)g0 * M.ldy;
     const size_t row_bytes = sizeof(float) * M.rows;
-    if (r.device_y && y_here && M.rows > 0 && r.k <= 65535) {  // the grid's y limit
+    auto by_kernel = [&](float* out) {
         hipLaunchKernelGGL(copy_y_kernel, dim3(std::min(((unsigned)M.rows + 255) / 256, 2048u), r.k), dim3(256), 0, s,
-                           M.rows, M.ldy, y, r.device_y);
-        CLSPMV_HIP(hipGetLastError());
+                           M.rows, M.ldy, y, out);
+        return hipGetLastError();
+    };
+    const bool kernel = M.rows > 0 && r.k <= 65535;  // the grid's y limit
+    if (r.device_y && y_here && kernel) {
+        CLSPMV_HIP(by_kernel(r.device_y));
     } else if (r.device_y) {
         CLSPMV_HIP(hipMemcpy2DAsync(r.device_y, row_bytes, y, sizeof(float) * M.ldy, row_bytes, r.k,
                                     hipMemcpyDeviceToDevice, s));
     }
-    if (r.host_y && pinned)
+    if (r.host_y && pinned && kernel && row_bytes * r.k <= kKernelToHost) {
+        CLSPMV_HIP(by_kernel(pinned));
+    } else if (r.host_y && pinned) {
         CLSPMV_HIP(hipMemcpy2DAsync(pinned, row_bytes, y, sizeof(float) * M.ldy, row_bytes, r.k,
                                     hipMemcpyDeviceToHost, s));
+    }
     return CLSPMV_OK;
 }
 
