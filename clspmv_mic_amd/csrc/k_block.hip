@@ -70,7 +70,9 @@ __global__ __launch_bounds__(kBlock) void bcsr_kernel(
 // fetched (two register sets taking turns; the last group loads no more than
 // its slots).  By the loads that a slot has for the chip, one float4 plane per
 // block row, row and column quad (figures: block rows of 12 4x4 blocks, BCSR /
-// BELL / SBELL, against a lane per block row, one slot after the other):
+// BELL / SBELL, against a lane per block row, one slot after the other; passes
+// over one matrix in turn, which up to about 250 MB the memory-side cache holds:
+// read from HBM each time, 131,072 block rows take the same by every walk):
 //   kSplit    four waves share block rows, two to four slots at a time: 20,000
 //             block rows 14.7 / 14.7 / 15.5 -> 6.5 / 6.2 / 6.7 us, 60,000 15.5 /
 //             15.6 / 16.3 -> 9.9 / 9.7 / 10.1 us;

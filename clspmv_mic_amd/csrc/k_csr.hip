@@ -129,17 +129,16 @@ __device__ __forceinline__ float csr_wave_row(int lane, int s, int n, const int*
 // at once, and leaves the products in its own part of LDS, where lane groups
 // sized to the row count sum the rows: no barrier, 32 waves per CU.  Against
 // lanes striding over rows (csr_vector) and a work-group per 1024 entries
-// with a barrier: 27-point stencil 77^3 52 / 31 -> 24 us, 5-point Laplacian
-// 701^2 15 / 10.5 -> 8 us.
+// with a barrier: 27-point stencil 77^3 52 / 31 -> 23.5 us, 5-point Laplacian
+// 701^2 15 / 10.5 -> 7 us.
 //
 // WIN: gathers through L1 return in order behind the streams; without them
 // the 27-point stencil 97^3 (24.6 M entries) ran in 31.8 us instead of 47.7.
 // Where the rows of a work-group share x, it stages their chunks of x in LDS
 // (launch::XStage) while the entries are in flight and gathers there, by
-// 16-bit places instead of 32-bit columns (6 bytes an entry): 77^3 23.9 -> 16.5
-// us, 97^3 48.1 -> 33.2, 5-point Laplacian 1300^2 20.9 -> 16.9, mesh of 700,000
-// rows 34.9 -> 28.6 us (with one window of consecutive columns staged and
-// 32-bit columns), the stencil 30^3 4.8 -> 4.2 us.
+// 16-bit places instead of 32-bit columns (6 bytes an entry): 27-point stencil
+// 77^3 23.5 -> 15.1 us (81.6 MB of HBM traffic), 47^3 7.3 -> 5.4, 5-point Laplacian
+// 1000^2 11.4 -> 9.7, mesh of 700,000 rows of 25 48.2 -> 24.6 us.
 //
 // A skewed block (a row of 400 entries among 50 of a few) would leave the long
 // row's sum to the one or two lanes its row count gives each row; rows of more

@@ -22,18 +22,16 @@ using namespace dev;
 // values load at once, and the next kSlots' are in flight while the present
 // ones' x values are gathered (two register sets taking turns, nothing
 // copied; the last, shorter group loads no more than its slots).  Two slots
-// at a time took 9.8 / 10.4 us (ELL / SELL) on the 27-point stencil 30^3 and
-// 14.4 / 15.2 us on a mesh of 40,000 rows; this takes 6.5 / 7.1 and 10.2 /
-// 11.1 us.
+// at a time took 9.8 / 10.4 us (ELL / SELL) on the 27-point stencil 30^3; this
+// takes 3.6 / 4.2 us.
 //
 // WIN: the work-group stages the chunks of x that its rows touch in LDS and
 // gathers there, by 16-bit places instead of 32-bit columns (launch::XStage;
 // two slots to a word, so that a word is loaded as it is used: single 16-bit
 // loads were widened behind a wait for the next slots').  ELL / SELL, against
-// gathering from memory, for meshes against one window of consecutive columns
-// in LDS: 27-point stencil 30^3 5.6 / 8.8 -> 4.5 / 6.1 us, 97^3 37.0 / 39.2 ->
-// 29.0 / 30.4, mesh of 20,000 rows 9.7 / 10.5 -> 6.2 / 6.9, 700,000 40.1 / 43.3
-// -> 32.0 / 33.7 us.
+// gathering from memory: 27-point stencil 60^3 8.6 / 9.2 -> 7.5 / 8.3 us, 77^3 16.1 /
+// 18.7 -> 13.2 / 14.6, mesh of 100,000 rows of 25 5.9 / 6.8 -> 5.1 / 5.8, of 700,000
+// 51.3 / 53.3 -> 20.0 / 21.9 us.
 template <bool SELL, bool WIN, int kSlots, int kRows>
 __global__ __launch_bounds__(kRows) void ell_row_kernel(
     int rows, int h, int w0, const int* __restrict__ ptr, const int* __restrict__ list, const unsigned short* __restrict__ idx,

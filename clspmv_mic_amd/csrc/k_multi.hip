@@ -282,12 +282,11 @@ constexpr int kMultiThreads = 512;
 // whatever k is: a lane loads its slot's entries, L lanes hand them round and
 // keep the sums of their L slots for Q right-hand sides each.  Rounds past the
 // row's end are skipped by the wave, entries past it re-read the last one and
-// are not added.  Returns the wave's sums in sum.
-template <int Q, int L, int T, class V, class Acc>
+// are not added.  U rounds are in flight.  Returns the wave's sums in sum.
+template <int Q, int L, int T, int U, class V, class Acc>
 __device__ __forceinline__ void csr_multi_row(unsigned t, int s, unsigned n, const int* __restrict__ col,
                                               const typename V::T* __restrict__ val,
                                               const float* __restrict__ Xq, int k, Acc* sum) {
-    constexpr int U = (Q >= 3 && L < 4 ? 6 : 8) / L;  // rounds in flight, by the registers that leave three work-groups a CU
     typedef VecOf<float, Q> XV;
     const unsigned p = t % L, w0 = __builtin_amdgcn_readfirstlane(t / kWave * kWave);
     // (Unsigned indices from the row's start: the sums stay in range near 2^31
@@ -356,17 +355,27 @@ __device__ __forceinline__ void csr_multi_row(unsigned t, int s, unsigned n, con
     }
 }
 
-// A row by the work-group: the eight waves' sums are combined in a fixed order
+// Rounds of a long row in flight, by the registers that leave three work-groups a
+// CU.  Up to kBesideNnz entries beside as many blocks of short rows, one: more
+// loads in flight only slow the blocks (power-law rows, FP32, k = 4 / 8 / 16, 600,000:
+// 111 / 149 / 182 -> 104 / 136 / 177 us, 1 M: 225 / 274 / 317 -> 200 / 261 / 309).  By
+// themselves the rows gain from them (3,000 of 5,000 overlapping columns, k = 1 / 8:
+// 38.6 / 54.4 -> 25.6 / 45.9 us; one of 1 M, k = 1: 1172 -> 312).
+constexpr int kBesideNnz = 8192;
+template <int Q, int L>
+constexpr int kRounds = (Q >= 3 && L < 4 ? 6 : 8) / L;
+
+// A row by the work-group (ROUNDS in flight): the eight waves' sums are combined in a fixed order
 // through LDS, and Y[:, r] is updated once per right-hand side (rows summed in
 // FP64 rounded once).
-template <int Q, int L, class V, class Acc>
+template <int Q, int L, int ROUNDS, class V, class Acc>
 __device__ __forceinline__ void csr_multi_long(const typename V::T* __restrict__ val,
                                                const int* __restrict__ col, int r, int s, int n,
                                                const float* __restrict__ X, int k, float* __restrict__ Y, int ldy,
                                                bool accumulate, Acc (*part)[launch::kMultiMax]) {
     const int t = threadIdx.x, q0 = t % L * Q, qs = min(q0, k - Q);
     Acc sum[Q];
-    csr_multi_row<Q, L, kMultiThreads, V, Acc>(t, s, n, col, val, X + qs, k, sum);
+    csr_multi_row<Q, L, kMultiThreads, ROUNDS, V, Acc>(t, s, n, col, val, X + qs, k, sum);
     if (t % kWave < L && q0 < k) {
 #pragma unroll
         for (int q = 0; q < Q; ++q)
@@ -502,10 +511,15 @@ __global__ __launch_bounds__(kMultiThreads, L == 4 ? 4 : 6) void csr_multi_kerne
     const int nlwg = nwide + (nlong - nwide + kWaves - 1) / kWaves;
     if ((int)blockIdx.x < nwide) {  // the longest work first
         const int r = longs[blockIdx.x], j0 = rp[r], n = rp[r + 1] - j0;
-        if (n > launch::kLongRowF64)
-            csr_multi_long<Q, L, V, double>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part64);
-        else
-            csr_multi_long<Q, L, V, float>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part);
+        auto row = [&](auto rounds) {
+            constexpr int R = decltype(rounds)::value;
+            if (n > launch::kLongRowF64)
+                csr_multi_long<Q, L, R, V, double>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part64);
+            else
+                csr_multi_long<Q, L, R, V, float>(val, col, r, j0, n, X, k, Y, ldy, accumulate, lds.part);
+        };
+        if (nblk >= nwide && n <= kBesideNnz) row(std::integral_constant<int, 1>{});
+        else row(std::integral_constant<int, kRounds<Q, L>>{});
         return;
     }
     if ((int)blockIdx.x < nlwg) {  // a wave per row
@@ -515,7 +529,7 @@ __global__ __launch_bounds__(kMultiThreads, L == 4 ? 4 : 6) void csr_multi_kerne
         float sum[Q], y[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) y[q] = accumulate ? Y[(size_t)(qs + q) * ldy + r] : 0.0f;
-        csr_multi_row<Q, L, kWave, V, float>(lane, j0, n, col, val, X + qs, k, sum);
+        csr_multi_row<Q, L, kWave, kRounds<Q, L>, V, float>(lane, j0, n, col, val, X + qs, k, sum);
         if (lane < L && q0 < k) {
 #pragma unroll
             for (int q = 0; q < Q; ++q)

@@ -335,7 +335,7 @@ int auto_method(const clspmv_dmat* A) {
         // that the wave kernel's longer chain shows (mesh of 5,000 rows of 8 2.8 /
         // 3.1 us, 50,000 of 8 2.8 / 3.3, 20,000 of 25 3.1 / 3.1; 27-point stencil
         // 30^3, 0.7 M entries, 3.9 / 3.1).  The wave kernel elsewhere (27-point
-        // stencil 77^3 52 / 15 us, power-law rows 1 M 225 / 106).
+        // stencil 77^3 52 / 15.1 us, power-law rows 1 M 225 / 106).
         case CLSPMV_FMT_CSR: {
             const double avg = A->info.rows ? (double)A->info.nnz / A->info.rows : 0.0;
             const bool even = A->max_row <= 8.0 * std::max(avg, 4.0);
