@@ -145,9 +145,11 @@ def measured_traffic(workload, kernel_prefix):
     return None
 
 
-# Kernel-name prefix of each format's dominant kernel (rocprofv3 names).
-KERNEL_OF = {"dia": "dia", "bdia": "bdia", "coo": "panel_pass", "csr": "panel_pass", "bcsr": "bcsr",
-             "bell": "bell_kernel", "sbell": "sbell_kernel", "ell": "ell", "sell": "sell_kernel"}
+# Each format's dominant kernel as the counter table names it (rocprofv3 names;
+# the layouts that share a kernel in brackets).
+KERNEL_OF = {"dia": "dia", "bdia": "dia", "coo": "panel_pass", "csr": "panel_pass",
+             "bcsr": "block_rows_kernel (BCSR", "bell": "block_rows_kernel (BELL", "sbell": "block_rows_kernel (SBELL",
+             "ell": "ell_row_kernel (ELL", "sell": "ell_row_kernel (SELL"}
 
 
 def measure_cocktail(args, name):

@@ -37,10 +37,10 @@ using launch::kDiaRun;
 // segment's loads are in flight in registers meanwhile; no work-group barrier.
 // LDS rows are padded by KB floats every R rows, which keeps the 16-byte reads
 // of lanes R rows apart on different banks.  96^3 27-point stencil, FP32,
-// k = 2 / 4 / 7 / 8 / 16: 26 / 31 / 38 / 41 / 73 us against 41 / 49 / 135 /
-// 94 / 183 us for lanes loading every diagonal's X row themselves (1.7 to 3.8
-// TB/s of the bytes that cannot be avoided); 5-point Laplacian on 900^2, k = 8 /
-// 16: 19 / 42 against 30 / 59 us.
+// k = 2 / 4 / 7 / 8 / 16: 25 / 30 / 38 / 41 / 52 us (16: 73 over three matrices in
+// turn) against 41 / 49 / 135 / 94 / 183 us for lanes loading every diagonal's X
+// row themselves (1.7 to 3.8 TB/s of the bytes that cannot be avoided); 5-point
+// Laplacian on 900^2, k = 8 / 16: 19 / 31 against 30 / 59 us.
 //
 // Each column is summed alone in diagonal order, one product at a time,
 // skipping columns outside x, whatever the tile: its result does not depend
@@ -478,9 +478,9 @@ __device__ __forceinline__ bool csr_multi_short(int lane, int r0, int nrows, int
 // a work-group of 1024 entries waited at two barriers, each finished row was
 // added to Y where it ended (a load and a store of one float per right-hand
 // side, waited for) and k not a multiple of 4 gathered single floats.
-// Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 138 / 174 us; 1 M
-// rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 266 / 251 / 302 us (53 G rows/s);
-// 27-point stencil 64^3, k = 8: 74 -> 31 us.
+// Power-law rows: 600,011 rows, BF16, k = 8 / 16: 191 / 318 -> 132 / 172 us; 1 M
+// rows, FP32, k = 5 / 8 / 16: 357 / 329 / 528 -> 247 / 260 / 300 us (52 G rows/s);
+// 27-point stencil 64^3, k = 8: 74 -> 28 us.
 template <int Q, int L, class V>
 __global__ __launch_bounds__(kMultiThreads, L == 4 ? 4 : 6) void csr_multi_kernel(
     int nlong, int nwide, const int* __restrict__ longs, int nblk, const int4* __restrict__ blk,

@@ -575,6 +575,28 @@ def test_staged_x_rounds(ctx, oracle, fmt, chunks):
     assert (info.device_bytes >= own + 2 * info.stored) == (chunks <= 512)
 
 
+@pytest.mark.parametrize("chunks", [40, 301])
+@pytest.mark.parametrize("x_offset", [0, 1])
+def test_staged_x_slices(ctx, oracle, chunks, x_offset):
+    """ELL and SELL with staged x where the launch takes it (101 work-groups, the
+    last one partial): odd slot counts, empty slices beside full ones, slices that
+    reach into two work-groups; dyadic inputs, exact sums."""
+    rows, cols = 100 * 512 + 37, chunks * 16 - 5
+    r = np.repeat(np.arange(rows), 11)
+    c = np.minimum((np.arange(r.size) * 13 % chunks) * 16 + r % 16, cols - 1)
+    key = np.unique(r.astype(np.int64) * cols + c)
+    r, c = key // cols, key % cols
+    v = (np.random.default_rng(chunks).integers(1, 65, r.size) / 64.0).astype(np.float32)
+    A = cs.Coo(r.astype(np.int32), c.astype(np.int32), v, rows, cols)
+    keep = (r // 32 % 9 != 2) & ((r % 16 != 3) | (c // 16 % 2 == 0))  # slices of none, rows of fewer
+    B = cs.Coo(A.row[keep], A.col[keep], A.val[keep], rows, cols)
+    for M, owned in ((A, cs.coo2ell(A)), (B, cs.coo2ell(B)), (B, cs.coo2sell(B, 32)), (A, cs.coo2sell(A, 48)),
+                     (B, cs.coo2sell(B, 48)), (B, cs.coo2sell(B, 700))):
+        _run(ctx, oracle, M, owned, 0, x_offset=x_offset)
+        info = cs.DeviceMatrix(ctx, owned).info
+        assert info.device_bytes >= 10 * info.stored
+
+
 def test_staged_x_with_panels(ctx, oracle):
     """A CSR upload that keeps its own arrays stages x for them (2 bytes an entry
     beside the 8 of columns and values), with panels beside them too."""
