@@ -87,7 +87,10 @@ __global__ __launch_bounds__(kBlock) void bcsr_kernel(
 //             counts differ by lane: 524,288 73.5 ahead, 77.2 in order.
 //
 // Padding slots of BCSR (column -1) and slots past a lane's last load what is
-// there for another and are not added, so the sum is the row's blocks' in slot
+// there for another (SBELL: the wave's widest block row's blocks, one address for
+// all such lanes; each its own last block, power-law rows, 300,000 of 4 on average:
+// slices of eight rows of 4x1 / 4x4 / 8x2 blocks 140 / 240 / 300 us, so 83 / 173 /
+// 223) and are not added, so the sum is the row's blocks' in slot
 // order, one float4 dot per w4.  F4ACC = true (BELL method 1, the reference's
 // "_mad" variant, kernels/spmv_bell.cl:24-42): float4 accumulators reduced at
 // the end.
@@ -106,22 +109,24 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
     constexpr int HW = kShare<BH, WALK>;
     constexpr int HN = BH / HW;  // rows of a block per wave
     constexpr int U = WALK != kSplit ? 1 : BW4 * HN == 1 ? 4 : BW4 * HN == 2 ? 3 : 2;  // slots at a time
-    const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int h0 = wave % HW * HN;
     const unsigned row = ((unsigned)xcd_tile(blockIdx.x, gridDim.x) * (kHWaves / HW) + wave / HW) * kWave + lane;
     const int r = launch::shadow_row(row, brows);
     int w = nslots;
-    const int* cp = col4 + r;
-    const float* dp = data + (size_t)r * 4;
+    const int* cp = LAY == kSbell ? col4 : col4 + r;
+    const float* dp = LAY == kSbell ? data : data + (size_t)r * 4;
+    // SBELL: the first column and float of the lane's block row, and of the wave's
+    // widest, whose blocks lanes past their own last one load.
+    unsigned ci = 0, cw = 0;
+    size_t di = 0, dw = 0;
     long long P = f4;  // floats per (slot, w4, h) plane
     if constexpr (LAY == kSbell) {  // cs: the slice height
         const int sl = r / cs, p0 = sptr[sl];
         w = (sptr[sl + 1] - p0) / cs;
         P = launch::block_plane(cs);
-        // A lane whose slice is empty reads entry 0 beside its neighbours.
-        const int at = w > 0 ? p0 + (r - sl * cs) : 0;
-        cp = col4 + at;
-        dp = data + (w > 0 ? (size_t)p0 * BH * BW4 * 4 + (size_t)(r - sl * cs) * 4 : 0);
+        ci = (unsigned)(p0 + (r - sl * cs));
+        di = (size_t)p0 * BH * BW4 * 4 + (size_t)(r - sl * cs) * 4;
     }
     int wm = w;  // the most slots of the wave's block rows
     if constexpr (LAY == kSbell) {
@@ -131,6 +136,12 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
             for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
     }
     wm = __builtin_amdgcn_readfirstlane(wm);
+    if constexpr (LAY == kSbell) {
+        const int widest = __builtin_ctzll(__ballot(w == wm));
+        cw = (unsigned)__builtin_amdgcn_readlane((int)ci, widest);
+        dw = (unsigned)__builtin_amdgcn_readlane((int)di, widest) |
+             (size_t)(unsigned)__builtin_amdgcn_readlane((int)(di >> 32), widest) << 32;
+    }
     dp += (size_t)h0 * P;
     float acc[HN];
     float4 acc4[HN];
@@ -142,13 +153,14 @@ __global__ __launch_bounds__(kBlock) void block_rows_kernel(
     int c[2][U];
     float4 d[2][U][BW4][HN];
     auto load_slot = [&](int s, int& cc, float4 (*dd)[HN]) {
-        const size_t at = LAY == kSbell ? (size_t)max(min(s, w - 1), 0) : (size_t)s;
-        cc = ld_stream(cp + at * cs);
+        const bool own = LAY != kSbell || s < w;
+        cc = ld_stream(cp + (size_t)s * cs + (own ? ci : cw));
+        const float* from = dp + (own ? di : dw);
 #pragma unroll
         for (int w4 = 0; w4 < BW4; ++w4)
 #pragma unroll
             for (int h = 0; h < HN; ++h)
-                dd[w4][h] = ld_stream(reinterpret_cast<const float4*>(dp + ((at * BW4 + w4) * BH + h) * P));
+                dd[w4][h] = ld_stream(reinterpret_cast<const float4*>(from + (((size_t)s * BW4 + w4) * BH + h) * P));
     };
     auto load = [&](int s, int b) {
 #pragma unroll

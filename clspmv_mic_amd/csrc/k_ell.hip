@@ -6,6 +6,8 @@
 // own consecutive rows and every slot load is one contiguous 256-byte wave
 // access.  The 4-rows-per-lane ELL variant issues 128-bit loads.
 
+#include <type_traits>
+
 #include "device_common.hpp"
 #include "kernels.hpp"
 
@@ -47,20 +49,25 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
     const float* vp = val;
     StageX<kRows> stage;
     if constexpr (WIN) stage.ids(list + (size_t)wg * stride, stride);
+    // SELL: the first column word and value of the lane's row, and of the wave's
+    // widest; slot indices fit 31 bits with them (ptr is int).
+    unsigned ci = 0, vi = 0, cw = 0, vw = 0;
     if constexpr (SELL) {
         const int sl = r / h, p0 = ptr[sl], q0 = WIN ? p0 / h : 0;
         w = WIN ? ptr[sl + 1] / h - q0 : (ptr[sl + 1] - p0) / h;
-        // A lane whose slice is empty reads entry 0 beside its neighbours (the
-        // matrix has entries when they have any): at p0 there may be none.
         const int i = r - sl * h;
-        cp += w > 0 ? (WIN ? (size_t)((q0 + sl) >> 1) * h + i : (size_t)p0 + i) : 0;
-        vp += w > 0 ? p0 + i : 0;
+        ci = WIN ? (unsigned)((q0 + sl) >> 1) * h + i : (unsigned)(p0 + i);
+        vi = (unsigned)(p0 + i);
     } else {
         cp += r;
         vp += r;
     }
-    // The widest row of the wave: its slots are walked, and slots past the
-    // lane's own last one re-read that one and are not added.
+    // The widest row of the wave: its slots are walked.  A lane past its own last
+    // one loads the widest row's, one address for all such lanes, and does not add
+    // it: lanes re-reading each its own last slot keep as many cache lines busy as
+    // live ones (power-law rows, 300,000 of 4 on average and at most 60: slices of
+    // 1 / 4 / 8 / 32 rows 112 / 132 / 107 / 87 us, with the widest's 38 / 53 / 54 /
+    // 71; lanes leaving the walk one by one, two slots at a time, 43 / 65 / 70 / 80).
     int wm = w;
     if constexpr (SELL) {
         if (h % 32 == 0)  // a slice per half of the wave, at most
@@ -69,12 +76,22 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
             for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
     }
     wm = __builtin_amdgcn_readfirstlane(wm);
+    if constexpr (SELL) {
+        const int lane = __builtin_ctzll(__ballot(w == wm));
+        cw = (unsigned)__builtin_amdgcn_readlane((int)ci, lane);
+        vw = (unsigned)__builtin_amdgcn_readlane((int)vi, lane);
+    }
     int c[2][kSlots / kPer];
     float v[2][kSlots];
     auto load_slot = [&](int s, int u, int* cc, float* vv) {
-        const int at = SELL ? max(min(s + u, w - 1), 0) : s + u;
-        if (u % kPer == 0) cc[u / kPer] = ld_stream(cp + (size_t)(at / kPer) * h);
-        vv[u] = ld_stream(vp + (size_t)at * h);
+        if constexpr (SELL) {
+            const bool own = s + u < w;
+            if (u % kPer == 0) cc[u / kPer] = ld_stream(cp + ((own ? ci : cw) + (unsigned)((s + u) / kPer) * h));
+            vv[u] = ld_stream(vp + ((own ? vi : vw) + (unsigned)(s + u) * h));
+        } else {
+            if (u % kPer == 0) cc[u / kPer] = ld_stream(cp + (size_t)((s + u) / kPer) * h);
+            vv[u] = ld_stream(vp + (size_t)(s + u) * h);
+        }
     };
     auto load = [&](int s, int* cc, float* vv) {
 #pragma unroll
@@ -92,35 +109,45 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
     if constexpr (WIN) stage.fetch(stride, cols, x, xs);
     const unsigned last = (unsigned)stride * launch::kXChunk - 1u;
     float a[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    auto add = [&](int s, const int* cc, const float* vv) {
+    auto add = [&](auto full, int s, const int* cc, const float* vv) {  // full: all slots below wm
         float xv[kSlots];
         if constexpr (WIN) {  // entry 0 may be another work-group's: clamped, not added
 #pragma unroll
             for (int u = 0; u < kSlots; ++u) {
                 const unsigned i = u % 2 ? (unsigned)cc[u / 2] >> 16 : cc[u / 2] & 0xFFFFu;
-                if (s + u < wm) xv[u] = xs[SELL ? min(i, last) : i];
+                if (full || s + u < wm) xv[u] = xs[SELL ? min(i, last) : i];
             }
         } else {
 #pragma unroll
             for (int u = 0; u < kSlots; ++u)
-                if (s + u < wm) xv[u] = x[cc[u]];
+                if (full || s + u < wm) xv[u] = x[cc[u]];
         }
 #pragma unroll
         for (int u = 0; u < kSlots; ++u)
-            if (s + u < wm) a[u % 4] = s + u < w ? fmaf(vv[u], xv[u], a[u % 4]) : a[u % 4];
+            if (full || s + u < wm) {
+                // Two selects: a single one is made a branch around the gather, with
+                // a wait for the next slots in it.
+                const bool own = !SELL || s + u < w;
+                const float t = fmaf(own ? vv[u] : 0.0f, xv[u], a[u % 4]);
+                a[u % 4] = own ? t : a[u % 4];
+            }
     };
+    constexpr std::true_type whole{};
+    constexpr std::false_type part{};
     int s = 0;
     for (; s + 3 * kSlots <= wm; s += 2 * kSlots) {
         load(s + kSlots, c[1], v[1]);
-        add(s, c[0], v[0]);
+        __builtin_amdgcn_sched_barrier(0);  // the next slots' loads stay ahead of the gathers' waits
+        add(whole, s, c[0], v[0]);
         load(s + 2 * kSlots, c[0], v[0]);
-        add(s + kSlots, c[1], v[1]);
+        __builtin_amdgcn_sched_barrier(0);
+        add(whole, s + kSlots, c[1], v[1]);
     }
     if (s + kSlots < wm) load_part(s + kSlots, c[1], v[1]);
-    add(s, c[0], v[0]);
+    add(part, s, c[0], v[0]);
     if (s + 2 * kSlots < wm) load_part(s + 2 * kSlots, c[0], v[0]);
-    if (s + kSlots < wm) add(s + kSlots, c[1], v[1]);
-    if (s + 2 * kSlots < wm) add(s + 2 * kSlots, c[0], v[0]);
+    if (s + kSlots < wm) add(part, s + kSlots, c[1], v[1]);
+    if (s + 2 * kSlots < wm) add(part, s + 2 * kSlots, c[0], v[0]);
     if (row < (unsigned)rows) y[r] += (a[0] + a[1]) + (a[2] + a[3]);
 }
 

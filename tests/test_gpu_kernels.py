@@ -647,6 +647,40 @@ def test_ell_gathered(ctx, oracle, rows, width):
     for h in (32, 96, 40):
         _run(ctx, oracle, A, cs.coo2sell(A, h), cs.METHOD_AUTO)
 
+
+@pytest.mark.parametrize("height", [1, 8, 20, 32, 100])
+@pytest.mark.parametrize("rows, least", [(5_003, 3), (5_003, 12), (200_003, 3)])
+def test_skewed_slices(ctx, oracle, rows, least, height):
+    """SELL and SBELL slices of few rows whose widths differ a lot within a wave,
+    empty ones and a first wave of none among them: a row adds nothing of the
+    wave's widest, infinite x that only that one has included; dyadic inputs,
+    exact sums."""
+    rng = np.random.default_rng(least)
+    lens = np.minimum((least / rng.random(rows) ** 0.9).astype(int), 150)
+    lens[rng.random(rows) < 0.2] = 0
+    lens[:80] = 0
+    lens[3_000] = 160
+    cols = 50_000
+    r = np.repeat(np.arange(rows), lens)
+    at = np.arange(r.size) - np.repeat(np.cumsum(lens) - lens, lens)
+    c = (rng.integers(0, cols, rows)[r] + at * 769) % cols  # distinct in a row
+    o = np.lexsort((c, r))
+    A = cs.Coo(r.astype(np.int32), c[o].astype(np.int32), (rng.integers(-64, 65, r.size) / 64.0).astype(np.float32),
+               rows, cols + 8)
+    _run(ctx, oracle, A, cs.coo2sell(A, height), 0)
+    for bw, bh in ((4, 1), (4, 4), (8, 2)):
+        _run(ctx, oracle, A, cs.coo2sbell(A.copy(), bw, bh, height, cap=False), 0)
+    last = (A.row == 3_000).nonzero()[0][-1]
+    A.col[last], A.val[last] = cols + 3, 1.0
+    x = matrices.dyadic_vector(cols + 8, seed=11)
+    x[cols + 3] = np.inf
+    dx, dy = cs.DeviceVector(ctx, cols + 8, x), cs.DeviceVector(ctx, rows, np.zeros(rows, np.float32))
+    cs.DeviceMatrix(ctx, cs.coo2sell(A, height)).spmv(dx, dy, 0)
+    ctx.sync()
+    y = dy.download()
+    assert np.isinf(y[3_000]) and np.isfinite(np.delete(y, 3_000)).all()
+
+
 @pytest.mark.parametrize("nbr", [(3 << 15) - 1, 3 << 15, (3 << 16) - 1, (3 << 16) + 77])
 @pytest.mark.parametrize("shape, width", [((4, 1), 5), ((4, 2), 2), ((4, 4), 3), ((8, 2), 1)])
 def test_block_walks(ctx, oracle, nbr, shape, width):
