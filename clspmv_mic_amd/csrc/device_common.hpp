@@ -170,6 +170,21 @@ __device__ __forceinline__ float dpp_row(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
 }
 
+template <int CTRL>
+__device__ __forceinline__ int dpp_row(int v) {
+    return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false);
+}
+
+// The largest v of the wave, all of whose lanes are active.
+__device__ __forceinline__ int wave_max(int v) {
+    v = max(v, dpp_row<0xB1>(v));
+    v = max(v, dpp_row<0x4E>(v));
+    v = max(v, dpp_row<0x141>(v));
+    v = max(v, dpp_row<0x140>(v));
+    return max(max(__builtin_amdgcn_readlane(v, 0), __builtin_amdgcn_readlane(v, 16)),
+               max(__builtin_amdgcn_readlane(v, 32), __builtin_amdgcn_readlane(v, 48)));
+}
+
 // The value of lane ^ M (M a power of two below 64): DPP quad permutes for
 // 1 and 2, a ds_swizzle in bit-mask mode (and-mask 0x1F, xor-mask M: no
 // address computation, unlike ds_bpermute) within each 32 lanes for 4..16,

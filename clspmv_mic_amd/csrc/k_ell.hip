@@ -73,7 +73,7 @@ __global__ __launch_bounds__(kRows) void ell_row_kernel(
         if (h % 32 == 0)  // a slice per half of the wave, at most
             wm = max(__builtin_amdgcn_readlane(w, 0), __builtin_amdgcn_readlane(w, 32));
         else
-            for (int m = kWave >> 1; m >= 1; m >>= 1) wm = max(wm, __shfl_xor(wm, m, kWave));
+            wm = wave_max(w);
     }
     wm = __builtin_amdgcn_readfirstlane(wm);
     if constexpr (SELL) {

@@ -140,9 +140,15 @@ struct ColRange {
 // of 4, 5 entries per chunk, CSR 6.2 / 5.8, ELL 6.0 / 5.4; 5 consecutive
 // columns a row, ELL 100,000 rows 3.1 / 2.5, 200,000 3.3 / 3.1; 3-D stencil of 7
 // points on 47^3 3.0 / 2.6.  Long rows gain from 50,000 rows on (mesh of 40
-// neighbours, ELL 4.7 / 5.9, CSR 4.7 / 5.9).
+// neighbours, ELL 4.7 / 5.9, CSR 4.7 / 5.9).  Slots that a wave gathers from
+// few chunks (kCoalesced and more entries of a chunk follow each other: ELL, and
+// SELL slices of about 20 rows and more) do without for longer: 2-D stencil of 5
+// points on 550^2, ELL 4.6 / 3.7, SELL 5.1 / 4.4, 3-D one of 7 on 65^3 4.6 / 4.0 and
+// 5.2 / 4.7; where the columns are random in a band, SELL, 250,000 rows of 5 4.4 /
+// 5.6, 220,000 of 7 4.8 / 6.3.
 constexpr int kEntriesPerChunk = 4, kFewGroups = 256, kEntriesPerChunkFew = 8;
 constexpr int kEntriesPerGroup = 1536, kShortGroups = 384, kEntriesPerGroupShort = 4096;
+constexpr int kCoalesced = 8, kShortGroupsCoalesced = 640;
 
 // A work-group's chunks and its entries' places in them.  runs(g, f) calls
 // f(first entry, count, to, step) for the entries of group g: entry first + i's
@@ -152,6 +158,7 @@ struct ChunkMap {
         int seen, place;  // the last group that touched it, + 1; its first column's place in that group's list
     };
     std::vector<Chunk> chunks;
+    long long turns = 0;  // counted entries (idx null) of another chunk than the one before
     explicit ChunkMap(int cols) : chunks((size_t)cols / launch::kXChunk + 1) {}
     // idx null: only counts.  Returns the chunks (more than kXChunksMax: idx is
     // not complete), adds the entries.
@@ -160,6 +167,7 @@ struct ChunkMap {
               long long* entries) {
         int n = 0;
         long long total = 0;
+        unsigned before = ~0u;
         runs(g, [&](size_t first, size_t count, size_t to, size_t step) {
             total += (long long)count;
             for (size_t e = first; e < first + count && n <= launch::kXChunksMax; ++e, to += step) {
@@ -170,6 +178,8 @@ struct ChunkMap {
                     chunk.place = n++ * launch::kXChunk;
                     if (list) list->push_back((int)(c / launch::kXChunk));
                 }
+                turns += !idx && c / launch::kXChunk != before;
+                before = c / launch::kXChunk;
                 if (idx) idx[to] = (unsigned short)(chunk.place + c % launch::kXChunk);
             }
         });
@@ -182,24 +192,25 @@ struct ChunkMap {
 // in `groups` work-groups, when every group's chunks fit and the entries per
 // chunk pay for the staging.  start() builds it on threads of its own while
 // the caller uploads the matrix (col and what `runs` refers to must outlive
-// the object); finish() uploads it.  places: 16-bit words of idx.  Without the
-// host or device memory for it the matrix goes without.
+// the object); finish() uploads it.  places: 16-bit words of idx.  by_slot: `runs`
+// goes slot by slot, as a wave gathers.  Without the host or device memory for
+// it the matrix goes without.
 class StageBuild {
 public:
     ~StageBuild() {
         if (main_.joinable()) main_.join();
     }
     template <class Runs>
-    void start(int cols, size_t groups, const int* col, size_t total, size_t places, Runs runs) {
+    void start(int cols, size_t groups, const int* col, size_t total, size_t places, bool by_slot, Runs runs) {
         if (groups == 0 || total == 0) return;
         if (total >= 2 * kEntriesPerThread) {
             try {
-                main_ = std::thread([=] { build(cols, groups, col, total, places, runs); });
+                main_ = std::thread([=] { build(cols, groups, col, total, places, by_slot, runs); });
                 return;
             } catch (const std::exception&) {  // no thread: here
             }
         }
-        build(cols, groups, col, total, places, runs);
+        build(cols, groups, col, total, places, by_slot, runs);
     }
     int finish(clspmv_dmat* d) {
         if (main_.joinable()) main_.join();
@@ -216,7 +227,7 @@ public:
 
 private:
     template <class Runs>
-    void build(int cols, size_t groups, const int* col, size_t total, size_t places, const Runs& runs) {
+    void build(int cols, size_t groups, const int* col, size_t total, size_t places, bool by_slot, const Runs& runs) {
         try {
             {  // a look at up to 64 groups
                 ChunkMap map(cols);
@@ -228,7 +239,9 @@ private:
                     ++looked;
                 }
                 const int per_chunk = groups < kFewGroups ? kEntriesPerChunkFew : kEntriesPerChunk;
-                const int per_group = groups < kShortGroups ? kEntriesPerGroupShort : kEntriesPerGroup;
+                const bool coalesced = by_slot && entries >= kCoalesced * map.turns;
+                const size_t short_groups = coalesced ? kShortGroupsCoalesced : kShortGroups;
+                const int per_group = groups < short_groups ? kEntriesPerGroupShort : kEntriesPerGroup;
                 if (entries < per_chunk * chunks || entries < per_group * looked) return;
             }
             // The groups in `parts` runs of about as many, a thread each.
@@ -749,7 +762,7 @@ int clspmv_upload_csr_ex(clspmv_ctx* ctx, const clspmv_csr_matrix* m,
     constexpr size_t W = launch::kCsrWaves;
     StageBuild stage;
     auto build_stage = [&] {
-        stage.start(m->matinfo.width, (blk.size() + W - 1) / W, m->csr_col_id, nnz, (size_t)nnz + launch::kWaveNnz,
+        stage.start(m->matinfo.width, (blk.size() + W - 1) / W, m->csr_col_id, nnz, (size_t)nnz + launch::kWaveNnz, false,
                     [&blk](size_t g, auto&& f) {
                         for (size_t b = g * W; b < std::min(blk.size(), (g + 1) * W); ++b)
                             f(blk[b].z, blk[b].w, blk[b].z, 1);
@@ -829,7 +842,7 @@ int clspmv_upload_ell(clspmv_ctx* ctx, const clspmv_ell_matrix* m, clspmv_dmat**
     constexpr size_t R = launch::kEllRows;
     const size_t words = (size_t)(m->ell_num + 1) / 2 * hal;
     StageBuild stage;
-    stage.start(m->matinfo.width, (rows + R - 1) / R, m->ell_col_id, total, 2 * words, [=](size_t g, auto&& f) {
+    stage.start(m->matinfo.width, (rows + R - 1) / R, m->ell_col_id, total, 2 * words, true, [=](size_t g, auto&& f) {
         for (size_t s = 0; s < (size_t)m->ell_num; ++s)
             f(s * hal + g * R, std::min(R, rows - g * R), 2 * (s / 2 * hal + g * R) + s % 2, 2);
     });
@@ -861,7 +874,7 @@ int clspmv_upload_sell(clspmv_ctx* ctx, const clspmv_sell_matrix* m, clspmv_dmat
     constexpr size_t R = launch::kEllRows;
     const size_t words = ((size_t)sp[ns] / h + ns + 1) / 2 * h;
     StageBuild stage;
-    stage.start(m->matinfo.width, (rows + R - 1) / R, m->sell_col_id, total, 2 * words, [=](size_t g, auto&& f) {
+    stage.start(m->matinfo.width, (rows + R - 1) / R, m->sell_col_id, total, 2 * words, true, [=](size_t g, auto&& f) {
         const size_t r1 = std::min<size_t>(rows, (g + 1) * R);
         for (size_t r = g * R; r < r1;) {  // the group's part of each slice
             const size_t sl = r / h, i = r - sl * h, n = std::min(r1, (sl + 1) * h) - r;

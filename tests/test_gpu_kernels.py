@@ -597,6 +597,23 @@ def test_staged_x_slices(ctx, oracle, chunks, x_offset):
         assert info.device_bytes >= 10 * info.stored
 
 
+@pytest.mark.parametrize("groups, near, staged", [(639, 1, False), (640, 1, True), (383, 7, False), (384, 7, True)])
+def test_staged_x_short_rows(ctx, oracle, groups, near, staged):
+    """Five slots a row: where consecutive rows' columns follow each other x is
+    staged from more work-groups of 512 rows on; exact sums on both sides."""
+    rows = (groups - 1) * 512 + 200
+    off = np.array([-700, -1, 0, 1, 700])
+    r = np.repeat(np.arange(rows), 5)
+    c = r + np.tile(off, rows) + (np.arange(rows) % near * 40)[r]
+    ok = (c >= 0) & (c < rows)
+    v = (np.random.default_rng(near).integers(1, 65, r.size) / 64.0).astype(np.float32)
+    A = cs.Coo(r[ok].astype(np.int32), c[ok].astype(np.int32), v[ok], rows, rows)
+    for owned in (cs.coo2ell(A), cs.coo2sell(A, 32)):
+        _run(ctx, oracle, A, owned, 0)
+        info = cs.DeviceMatrix(ctx, owned).info
+        assert (info.device_bytes >= 10 * info.stored) == staged
+
+
 def test_staged_x_with_panels(ctx, oracle):
     """A CSR upload that keeps its own arrays stages x for them (2 bytes an entry
     beside the 8 of columns and values), with panels beside them too."""
