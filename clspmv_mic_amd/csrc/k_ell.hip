@@ -25,15 +25,15 @@ using namespace dev;
 // ones' x values are gathered (two register sets taking turns, nothing
 // copied; the last, shorter group loads no more than its slots).  Two slots
 // at a time took 9.8 / 10.4 us (ELL / SELL) on the 27-point stencil 30^3; this
-// takes 3.6 / 4.2 us.
+// takes 3.6 / 4.3 us.
 //
 // WIN: the work-group stages the chunks of x that its rows touch in LDS and
 // gathers there, by 16-bit places instead of 32-bit columns (launch::XStage;
 // two slots to a word, so that a word is loaded as it is used: single 16-bit
 // loads were widened behind a wait for the next slots').  ELL / SELL, against
-// gathering from memory: 27-point stencil 60^3 8.6 / 9.2 -> 7.5 / 8.3 us, 77^3 16.1 /
-// 18.7 -> 13.2 / 14.6, mesh of 100,000 rows of 25 5.9 / 6.8 -> 5.1 / 5.8, of 700,000
-// 51.3 / 53.3 -> 20.0 / 21.9 us.
+// gathering from memory: 27-point stencil 60^3 8.4 / 9.1 -> 7.4 / 8.0 us, 77^3 18.3 /
+// 20.5 -> 13.0 / 14.9, mesh of 100,000 rows of 25 6.0 / 6.6 -> 4.6 / 5.6, of 700,000
+// 51.0 / 53.9 -> 18.8 / 21.6 us.
 template <bool SELL, bool WIN, int kSlots, int kRows>
 __global__ __launch_bounds__(kRows) void ell_row_kernel(
     int rows, int h, int w0, const int* __restrict__ ptr, const int* __restrict__ list, const unsigned short* __restrict__ idx,
@@ -215,24 +215,24 @@ hipError_t ell_rows_staged(hipStream_t s, int rows, int h, int w, const int* ptr
 }
 
 // Staged work-groups of 512 rows leave too many CUs idle below 96 of them: the
-// mesh of 20,000 rows (40 work-groups) with 12 / 25 / 40 neighbours 3.1 / 4.0 /
-// 4.5 us staged, 2.8 / 3.6 / 4.4 gathered (ELL), 40,000 rows (79) of 12 3.6 / 3.3
-// (SELL); 50,000 rows (98) of 25 / 40 4.1 / 4.7 staged, 4.0 / 5.9 gathered.
+// mesh of 20,000 rows (40 work-groups) with 12 neighbours 3.1 / 3.7 us staged, 2.8 /
+// 3.3 gathered (ELL / SELL), 27-point stencil 22^3 (21) 4.0 / 4.6 and 3.4 / 4.1;
+// 50,000 rows (98) of 40 4.4 / 5.4 staged, 5.7 / 6.9 gathered.
 constexpr unsigned kStagedGroups = 96;
 
 // Slots in flight, staged: eight while there are fewer than two waves per SIMD
 // (131,072 rows), where the chain of slots sets the time (mesh of 100,000 rows
-// of 25 5.1 against 5.8 us), four above, where more waves cover it and the
-// shorter last group matters (mesh of 400,000 rows of 12 6.4 against 8.0 us).
+// of 25 4.6 against 5.2 us), four above, where more waves cover it and the
+// shorter last group matters (mesh of 400,000 rows of 12, SELL, 7.4 against 8.1 us).
 //
 // Gathered: work-groups of one wave, which fill the CUs evenly (random columns,
 // 40,000 rows, SELL, work-groups of 512 / 256 / 64 rows: 32 slots 17.6 / 9.3 /
 // 8.4 us, 100 slots 66.9 / 30.4 / 24.2 us), of four waves for rows of less than
 // four slots (1 M rows of one slot: 4.8 against 5.9 us).  Slots by the mean row:
-// 16 from 24 slots on (100,000 rows of 32 / 100, ELL: 16.9 / 56.0 us, by eight
-// 18.7 / 64.5, by four 21.5 / 69.4), eight from ten on (1 M rows of 12 76.6
-// against 79.2 us) and on few rows, else four (1 M rows of 5: 9.4 against
-// 9.9).
+// 16 from 24 slots on (100,000 rows of 32 / 100, ELL: 16.6 / 53.2 us, by eight
+// 17.2 / 55.3, by four 20.6 / 66.5), eight from ten on (200,000 rows of 12 13.6
+// against 14.8 us) and on few rows, else four (400,000 rows of 5: 12.0 against
+// 12.6).
 template <bool SELL>
 hipError_t ell_rows(hipStream_t s, int rows, int h, int w, const int* ptr, long long stored, launch::XStage W,
                     const int* col, const float* val, int cols, const float* x, float* y) {
